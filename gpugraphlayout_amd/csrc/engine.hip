@@ -1250,12 +1250,7 @@ int gfa2_stress_setup(gfa2_handle h, int32_t nsources, int32_t targets_per_sourc
         const int j = i + (int)rng.below((uint64_t)(n - i));
         std::swap(perm[i], perm[j]);
     }
-    std::vector<int> src(perm.begin(), perm.begin() + K), tgt((size_t)K * T);
-    for (int k = 0; k < K; ++k)
-        for (int j = 0; j < T; ++j) {
-            int u = (int)rng.below((uint64_t)(n - 1));
-            tgt[(size_t)k * T + j] = u >= src[k] ? u + 1 : u;
-        }
+    std::vector<int> src(perm.begin(), perm.begin() + K);
     int st = GFA2_OK;
     if (!h->stress_part) {
         if ((st = dalloc(h, &h->stress_part, 3 * kStressBlocks)) != GFA2_OK) return st;
@@ -1269,29 +1264,13 @@ int gfa2_stress_setup(gfa2_handle h, int32_t nsources, int32_t targets_per_sourc
     h->stress_K = K;
     h->stress_T = T;
     GFA2_TRY(hipMemcpyAsync(h->stress_src, src.data(), sizeof(int) * K, hipMemcpyHostToDevice, h->stream));
-    GFA2_TRY(hipMemcpyAsync(h->stress_tgt, tgt.data(), sizeof(int) * tgt.size(), hipMemcpyHostToDevice, h->stream));
-    // BFS scratch, freed right after
-    unsigned long long *seen = nullptr, *front = nullptr, *next = nullptr;
-    int* flag = nullptr;
-    GFA2_TRY(hipMalloc(&seen, sizeof(unsigned long long) * n));
-    GFA2_TRY(hipMalloc(&front, sizeof(unsigned long long) * n));
-    GFA2_TRY(hipMalloc(&next, sizeof(unsigned long long) * n));
-    GFA2_TRY(hipMalloc(&flag, sizeof(int)));
-    int rc = stress_hop_distances(h->b, h->stress_src, K, h->stress_tgt, T, h->stress_dist, seen, front, next, flag,
-                                  h->stream);
-    (void)hipStreamSynchronize(h->stream);
-    (void)hipFree(seen);
-    (void)hipFree(front);
-    (void)hipFree(next);
-    (void)hipFree(flag);
-    if (rc != 0) return GFA2_ERR_HIP;
-    if (npairs) {
-        std::vector<int> d((size_t)K * T);
-        GFA2_TRY(hipMemcpy(d.data(), h->stress_dist, sizeof(int) * d.size(), hipMemcpyDeviceToHost));
-        int64_t c = 0;
-        for (int v : d) c += v > 0;
-        *npairs = c;
-    }
+    // the targets take the generator's draws after the K of the shuffle
+    stress_draw_targets(h->stress_src, T, (long long)K * T, seed, (unsigned long long)K, n, h->stress_tgt, h->stream);
+    long long reached = 0;
+    const int rc = stress_hop_distances(h->b, h->stress_src, K, h->stress_tgt, T, h->stress_dist,
+                                        npairs ? &reached : nullptr, h->stream);
+    if (rc != 0) return rc == -2 ? GFA2_ERR_OOM : GFA2_ERR_HIP;
+    if (npairs) *npairs = reached;
     return GFA2_OK;
 }
 
@@ -1306,7 +1285,10 @@ int gfa2_stress_pairs(gfa2_handle h, int64_t cap, int32_t* a, int32_t* b, int32_
     if (b) GFA2_TRY(hipMemcpy(b, h->stress_tgt, sizeof(int) * c, hipMemcpyDeviceToHost));
     if (d) GFA2_TRY(hipMemcpy(d, h->stress_dist, sizeof(int) * c, hipMemcpyDeviceToHost));
     if (a)
-        for (int64_t p = 0; p < c; ++p) a[p] = src[p / h->stress_T];
+        for (int64_t k = 0, p = 0; p < c; ++k) {
+            const int64_t end = std::min<int64_t>(p + h->stress_T, c);
+            for (; p < end; ++p) a[p] = src[(size_t)k];
+        }
     return GFA2_OK;
 }
 

@@ -273,9 +273,12 @@ void launch_edge_weights(const Bufs& b, float delta, hipStream_t s);
 
 // Layout quality (stress.hip): hop distances of K*T sampled pairs by multi-source BFS,
 // and the normalized-stress sums {sum r, sum r^2, pairs} for positions pos.
+// npairs (may be null): the pairs whose target was reached. -2: no device memory for the search.
 int stress_hop_distances(const Bufs& b, const int* d_src, int K, const int* d_tgt, int T, int* d_dist,
-                         unsigned long long* seen, unsigned long long* front, unsigned long long* next, int* d_flag,
-                         hipStream_t s);
+                         long long* npairs, hipStream_t s);
+// The targets of np = K*T pairs: draws first, first + 1, ... of SplitMix64 seeded by `seed`.
+void stress_draw_targets(const int* d_src, int T, long long np, unsigned long long seed, unsigned long long first, int n,
+                         int* d_tgt, hipStream_t s);
 int stress_reduce(const float2* pos, const int* d_src, const int* d_tgt, const int* d_dist, int T, long long np,
                   double* d_part, int nblocks, double out[3], hipStream_t s);
 
