@@ -108,7 +108,8 @@ __global__ __launch_bounds__(256) void k_keys(const float2* __restrict__ pos, co
                                               float4* __restrict__ seg_root,
                                               unsigned long long* __restrict__ k0, unsigned int* __restrict__ v0,
                                               unsigned long long* __restrict__ k1, unsigned int* __restrict__ v1,
-                                              float4* __restrict__ pm, int first, unsigned int* __restrict__ dhist) {
+                                              float4* __restrict__ pm, int first, unsigned int* __restrict__ dhist,
+                                              const SegState* __restrict__ seg, SegState* __restrict__ seg_cur) {
     __shared__ float root[3];
     __shared__ unsigned int h[8][256];
     if (dhist)
@@ -125,6 +126,7 @@ __global__ __launch_bounds__(256) void k_keys(const float2* __restrict__ pos, co
         st->rooty = rooty;
         st->radius = radius;
         seg_root[0] = make_float4(rootx, rooty, radius, 0.0f);
+        *seg_cur = seg[0];        // for k_advance
     }
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         const float2 p = pos[i];
@@ -882,7 +884,7 @@ void launch_keys(const Bufs& b, int first, hipStream_t s) {
     if (blocks > b.grid_cap) blocks = b.grid_cap;
     k_keys<<<blocks, 256, 0, s>>>(b.pos, b.mass, b.n, b.bbox_part, b.st, b.seg_root, b.sort.keys[0], b.sort.vals[0],
                                   b.sort.keys[1], b.sort.vals[1], b.pm, first,
-                                  b.sort.hist_in_keys ? b.sort.digit_hist : nullptr);
+                                  b.sort.hist_in_keys ? b.sort.digit_hist : nullptr, b.seg_st, b.seg_cur);
 }
 
 void launch_tree(Bufs& b, hipStream_t s) {

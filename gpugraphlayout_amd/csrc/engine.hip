@@ -193,7 +193,7 @@ void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
     mark(3, s);
     if (!h->p.exact) {
         if (b.nseg > 1) {
-            launch_seg_bbox(b, s);
+            if (!advance_seg(b)) launch_seg_bbox(b, s);
             launch_seg_keys(b, s);
         } else {
             launch_keys(b, h->sort_first, s);
@@ -254,6 +254,14 @@ int drain_timing(gfa2_engine* h) {
     return GFA2_OK;
 }
 
+// What the displacement leaves for the next iteration, formed from positions that came from
+// elsewhere: the degree-ranked copy, and the bounding box's partials or the batch's roots.
+void positions_changed(gfa2_engine* h) {
+    launch_rank_pos(h->b, h->stream);
+    if (h->b.nseg > 1) launch_seg_bbox(h->b, h->stream);
+    else launch_bbox_partials(h->b, h->stream);
+}
+
 int reset_state(gfa2_engine* h) {
     DevState st{};
     st.global_speed = h->user.global_speed;
@@ -273,7 +281,7 @@ int reset_state(gfa2_engine* h) {
     GFA2_TRY(hipMemsetAsync(h->b.fprev, 0, sizeof(float2) * h->b.n, h->stream));
     GFA2_TRY(hipMemsetAsync(h->b.f, 0, sizeof(float2) * h->b.n, h->stream));
     GFA2_TRY(hipMemsetAsync(h->b.fga, 0, sizeof(float2) * h->b.n, h->stream));
-    if (h->has_pos) launch_bbox_partials(h->b, h->stream);
+    if (h->has_pos) positions_changed(h);
     GFA2_TRY(hipStreamSynchronize(h->stream));
     return GFA2_OK;
 }
@@ -591,6 +599,7 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
     GFA2_ALLOC(b.groups, groups_cap);
     GFA2_ALLOC(b.grp_first, (size_t)nseg + 1);
     GFA2_ALLOC(b.seg_st, nseg);
+    GFA2_ALLOC(b.seg_cur, 1);
     GFA2_ALLOC(b.grp_part, groups_cap);
     if (nseg > 1) {
         int* so = nullptr;
@@ -741,7 +750,7 @@ int gfa2_set_positions(gfa2_handle h, const float* xy) {
     GFA2_TRY(hipSetDevice(h->device));
     GFA2_TRY(full_sort_next(h));
     GFA2_TRY(hipMemcpyAsync(h->b.pos, xy, sizeof(float2) * h->b.n, hipMemcpyHostToDevice, h->stream));
-    launch_bbox_partials(h->b, h->stream);
+    positions_changed(h);
     GFA2_TRY(hipGetLastError());
     GFA2_TRY(hipStreamSynchronize(h->stream));
     h->has_pos = true;
@@ -1137,6 +1146,8 @@ int gfa2_autotune(gfa2_handle h, int32_t iters, gfa2_launch_config* best) {
             cp(b.st, sst, sizeof(DevState));
             cp(b.seg_st, sseg, sizeof(SegState) * b.nseg);
             cp(b.bbox_part, spart, sizeof(float4) * kPartBlocks);
+            launch_rank_pos(b, h->stream);
+            if (b.nseg > 1) launch_seg_bbox(b, h->stream);
         }
         if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
         return e;
@@ -1339,7 +1350,7 @@ bool engine_view(gfa2_engine* h, EngineView* v) {
 int engine_positions_written(gfa2_engine* h) {
     h->has_pos = true;
     GFA2_TRY(full_sort_next(h));
-    if (h->b.nseg == 1) launch_bbox_partials(h->b, h->stream);
+    positions_changed(h);
     GFA2_TRY(hipGetLastError());
     GFA2_TRY(hipStreamSynchronize(h->stream));
     return GFA2_OK;

@@ -178,6 +178,7 @@ struct Bufs {
     int* seg_order = nullptr;         // graphs by decreasing node count (per-graph sort)
     int max_seg = 0;                  // largest graph's node count
     struct SegState* seg_st = nullptr;
+    struct SegState* seg_cur = nullptr;   // one graph: the state before the iteration, copied by its first kernel
     WalkPart* grp_part = nullptr;     // per group
     // Integer masses (all whole numbers, total < 2^24 * 62): a cell lighter than 2^24 has
     // the same float mass in every summation order, so it is summarised from prefix sums;
@@ -263,6 +264,10 @@ void launch_walk(const Bufs& b, const Params& p, bool split, hipStream_t s);
 void launch_combine(const Bufs& b, const Params& p, hipStream_t s);
 void launch_speed(const Bufs& b, hipStream_t s);
 void launch_displacement(const Bufs& b, hipStream_t s);
+// The degree-ranked copy of the positions, after they were written by anything but the displacement.
+void launch_rank_pos(const Bufs& b, hipStream_t s);
+// A batch whose displacement also sets the roots of the next trees (no launch_seg_bbox per iteration).
+bool advance_seg(const Bufs& b);
 // Exact mode: pack {pos, mass} in node order, then all-pairs repulsion per graph with the
 // walk's epilogue (total force, swing/traction partials per group).
 void launch_exact(const Bufs& b, const Params& p, hipStream_t s);

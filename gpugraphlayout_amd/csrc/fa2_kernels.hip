@@ -86,7 +86,8 @@ __global__ __launch_bounds__(256) void k_gather_rank(const int* __restrict__ col
         col_rank[e] = rank[col[e]];
 }
 
-// pos_rank[rank[v]] = pos[v] (every iteration, before the attraction).
+// pos_rank[rank[v]] = pos[v] (for positions that came from outside; the displacement keeps the copy
+// up to date afterwards).
 __global__ __launch_bounds__(256) void k_rank_pos(const float2* __restrict__ pos, const int* __restrict__ rank, int n,
                                                   float2* __restrict__ pos_rank) {
     const int v = blockIdx.x * 256 + threadIdx.x;
@@ -596,74 +597,85 @@ __global__ __launch_bounds__(256) void k_combine(const float4* __restrict__ sbod
 }
 
 // ---------------------------------------------------------------------------------------
-// Speed update, one block per graph. Reference: SpeedKernel's last block,
-// src/RPFA2Kernels.cu:167-219 (Gephi's adaptive speed). The graph's group partials are
-// summed in double in a fixed order (thread-strided, then an LDS tree), the same for a
-// graph alone or inside a batch; the update itself is the reference's float arithmetic,
+// Speed update and displacement.
+//
+// Speed. Reference: SpeedKernel's last block, src/RPFA2Kernels.cu:167-219 (Gephi's adaptive
+// speed). The graph's group partials are summed in double in a fixed order: 1,024 strided sums,
+// then a halving tree over them, the same for a graph alone or inside a batch and whatever the
+// threads of the block that sums them. The update itself is the reference's float arithmetic,
 // including its double literals. Graph 0 is mirrored into DevState.
+//
+// Displacement. Reference: DisplacementKernel, src/RPFA2Kernels.cu:223-251:
+// factor = gs/(1.0 + sqrtf(gs*swg)) (double, because of the literal), p += F*factor, F' = F.
+// The new position also goes to the degree-ranked copy that the next attraction gathers from,
+// and the new bounding box (or its partials) is left for the next tree.
+//
+// Three forms of the pair, with the same results:
+//   k_advance      one graph of up to kAdvanceGroups walk groups: every block sums the partials
+//                  itself (a few tens of KB from L2) and displaces its nodes, one launch
+//   k_advance_seg  a batch of graphs of up to kSegSortMax nodes: one block per graph
+//   k_speed, k_displace   larger graphs
+// Each launch on a small graph costs 4-5 us however little it does: with the attraction's
+// position copy (k_rank_pos) the three launches were 13.9 us of 107 on 10,000 nodes.
 // ---------------------------------------------------------------------------------------
-constexpr int kSpeedThreads = 1024;
+constexpr int kSpeedSums = 1024;
+constexpr int kAdvanceGroups = 2048;
 
-__global__ __launch_bounds__(kSpeedThreads) void k_speed(const WalkPart* __restrict__ part,
-                                                         const int* __restrict__ grp_first,
-                                                         const int* __restrict__ node_off, SegState* __restrict__ seg,
-                                                         DevState* st, const int* __restrict__ kids_part,
-                                                         int kids_blocks) {
-    __shared__ double rs[kSpeedThreads], rt[kSpeedThreads];
-    __shared__ unsigned long long ri[kSpeedThreads];
-    __shared__ int rm[8];
-    if (st->err != 0) return;
-    const int g = blockIdx.x;
+struct GroupSums {
+    double s, t;
+    unsigned long long it;
+};
+
+// The graph's group partials [g0, g1) summed by a block of NT threads; thread 0 gets the result.
+template <int NT>
+__device__ __forceinline__ GroupSums sum_groups(const WalkPart* __restrict__ part, int g0, int g1) {
+    constexpr int V = kSpeedSums / NT;            // strided sums per thread
+    static_assert(V == 1 || V == 2 || V == 4, "a thread folds its sums with the tree's own offsets");
+    __shared__ double rs[NT], rt[NT];
+    __shared__ unsigned long long ri[NT];
     const int tid = threadIdx.x;
-    if (g == 0) {
-        // the tree's largest cell at level 4, 8, ..., 32, from the child-list kernel's blocks
-        if (tid < 8) rm[tid] = 0;
-        __syncthreads();
-        // thread t reads level slot t & 7 of every 128th block (the stride keeps the slot),
-        // eight loads in flight
-        int m = 0;
-        const int nq = kids_blocks * 8;
-        int q = tid;
-        for (; q + 7 * kSpeedThreads < nq; q += 8 * kSpeedThreads) {
-            int v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = kids_part[q + u * kSpeedThreads];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) m = max(m, v[u]);
-        }
-        for (; q < nq; q += kSpeedThreads) m = max(m, kids_part[q]);
-        if (m > 0) atomicMax(&rm[tid & 7], m);
-        __syncthreads();
-    }
-    const int g0 = grp_first[g], g1 = grp_first[g + 1];
-    double s = 0.0, t = 0.0;
+    double s[V], t[V];
     unsigned long long it = 0;
-    // thread-strided sums in group order; 8 partials are loaded before they are added (same
-    // order, so the same bits), keeping 8 loads in flight per thread
-    constexpr int kAhead = 8;
-    int k = g0 + tid;
-    for (; k + (kAhead - 1) * kSpeedThreads < g1; k += kAhead * kSpeedThreads) {
-        WalkPart p[kAhead];
 #pragma unroll
-        for (int j = 0; j < kAhead; ++j) p[j] = part[k + j * kSpeedThreads];
+    for (int v = 0; v < V; ++v) {
+        s[v] = 0.0;
+        t[v] = 0.0;
+        // 8 partials are loaded before they are added, keeping 8 loads in flight per thread
+        constexpr int kAhead = 8;
+        int k = g0 + tid + v * NT;
+        for (; k + (kAhead - 1) * kSpeedSums < g1; k += kAhead * kSpeedSums) {
+            WalkPart p[kAhead];
 #pragma unroll
-        for (int j = 0; j < kAhead; ++j) {
-            s += (double)p[j].swing;
-            t += (double)p[j].traction;
-            it += p[j].interactions;
+            for (int j = 0; j < kAhead; ++j) p[j] = part[k + j * kSpeedSums];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) {
+                s[v] += (double)p[j].swing;
+                t[v] += (double)p[j].traction;
+                it += p[j].interactions;
+            }
+        }
+        for (; k < g1; k += kSpeedSums) {
+            const WalkPart p = part[k];
+            s[v] += (double)p.swing;
+            t[v] += (double)p.traction;
+            it += p.interactions;
         }
     }
-    for (; k < g1; k += kSpeedThreads) {
-        const WalkPart p = part[k];
-        s += (double)p.swing;
-        t += (double)p.traction;
-        it += p.interactions;
+    // the halving tree over the 1,024 sums: offsets 512 and 256 first, as far as a thread holds
+    // both halves itself, then through LDS, then within the first wave
+    double a = s[0], c = t[0];
+    if constexpr (V == 4) {
+        a = (s[0] + s[2]) + (s[1] + s[3]);
+        c = (t[0] + t[2]) + (t[1] + t[3]);
+    } else if constexpr (V == 2) {
+        a = s[0] + s[1];
+        c = t[0] + t[1];
     }
-    rs[tid] = s;
-    rt[tid] = t;
+    rs[tid] = a;
+    rt[tid] = c;
     ri[tid] = it;
     __syncthreads();
-    for (int o = kSpeedThreads / 2; o > 0; o >>= 1) {
+    for (int o = NT / 2; o >= 64; o >>= 1) {
         if (tid < o) {
             rs[tid] += rs[tid + o];
             rt[tid] += rt[tid + o];
@@ -671,69 +683,150 @@ __global__ __launch_bounds__(kSpeedThreads) void k_speed(const WalkPart* __restr
         }
         __syncthreads();
     }
-    if (tid == 0) {
-        const int n = node_off[g + 1] - node_off[g];
-        SegState& q = seg[g];
-        const double S = rs[0], T = rt[0];
-        q.swing = S;
-        q.traction = T;
-        q.interactions = ri[0];
-        const float swg = (float)S, etra = (float)T;
-        float gs = q.global_speed, se = q.speed_efficiency;
-        const float jitter = q.jitter_tolerance, ksmax = q.k_s_max;
-        const float eojt = (float)(0.05 * sqrtf((float)n));
-        const float minjt = sqrtf(eojt);
-        float jt = jitter * fmaxf(minjt, fminf(ksmax, eojt * etra / powf((float)n, 2.0f)));
-        const float min_se = (float)0.05;
-        if (swg / etra > 2.0) {
-            if (se > min_se) se = (float)(se * 0.5);
-            jt = fmaxf(jt, jitter);
-        }
-        const float target = jt * se * etra / swg;
-        if (swg > jt * etra) {
-            if (se > min_se) se = (float)(se * 0.7);
-        } else if (gs < 1000) {
-            se = (float)(se * 1.3);
-        }
-        gs += fminf(target - gs, (float)0.5 * gs);
-        q.global_speed = gs;
-        q.speed_efficiency = se;
-        q.iteration += 1;
-        if (g == 0) {
-            st->swing = S;
-            st->traction = T;
-            st->interactions = ri[0];
-            st->global_speed = gs;
-            st->speed_efficiency = se;
-            // the next path-key sort: p 8-bit passes order the bodies by their top 4p levels,
-            // and the pairs left tied are the bodies of one 4p-level cell, which the fix-up
-            // orders; take the fewest passes whose cells (in this tree) hold at most
-            // kSortRunMax bodies each
-            int p = 1;
-            while (p < 8 && rm[p - 1] > kSortRunMax) ++p;
-            if (st->full_sorts > 0) {
-                st->full_sorts -= 1;      // still settling after new positions
-                p = 8;
-            }
-            st->sort_skip = 8 - p;
-            for (int q = 0; q < 8; ++q) st->runmax[q] = rm[q];
+    GroupSums r{0.0, 0.0, 0ull};
+    if (tid < 64) {
+        r = GroupSums{rs[tid], rt[tid], ri[tid]};
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            r.s += __shfl_down(r.s, o, 64);
+            r.t += __shfl_down(r.t, o, 64);
+            r.it += __shfl_down(r.it, o, 64);
         }
     }
-    // per graph (one block each): no word shared by the blocks of a batch
-    if (tid == 0) seg[g].interactions_total += ri[0];
+    return r;
 }
 
-// ---------------------------------------------------------------------------------------
-// Displacement. Reference: DisplacementKernel, src/RPFA2Kernels.cu:223-251:
-// factor = gs/(1.0 + sqrtf(gs*swg)) (double, because of the literal), p += F*factor,
-// F' = F. A single graph also emits bounding-box partials of the new positions for the
-// next tree (a batch recomputes its per-graph boxes instead).
-// ---------------------------------------------------------------------------------------
+// The adaptive speed after an iteration with these sums, from the graph's state q of n nodes.
+__device__ __forceinline__ SegState speed_update(SegState q, const GroupSums& r, int n) {
+    q.swing = r.s;
+    q.traction = r.t;
+    q.interactions = r.it;
+    const float swg = (float)r.s, etra = (float)r.t;
+    float gs = q.global_speed, se = q.speed_efficiency;
+    const float jitter = q.jitter_tolerance, ksmax = q.k_s_max;
+    const float eojt = (float)(0.05 * sqrtf((float)n));
+    const float minjt = sqrtf(eojt);
+    float jt = jitter * fmaxf(minjt, fminf(ksmax, eojt * etra / powf((float)n, 2.0f)));
+    const float min_se = (float)0.05;
+    if (swg / etra > 2.0) {
+        if (se > min_se) se = (float)(se * 0.5);
+        jt = fmaxf(jt, jitter);
+    }
+    const float target = jt * se * etra / swg;
+    if (swg > jt * etra) {
+        if (se > min_se) se = (float)(se * 0.7);
+    } else if (gs < 1000) {
+        se = (float)(se * 1.3);
+    }
+    gs += fminf(target - gs, (float)0.5 * gs);
+    q.global_speed = gs;
+    q.speed_efficiency = se;
+    q.iteration += 1;
+    q.interactions_total += r.it;
+    return q;
+}
+
+// The tree's largest cell at level 4, 8, ..., 32, from the child-list kernel's blocks, into rm
+// (8 words of LDS; followed by a barrier).
+template <int NT>
+__device__ __forceinline__ void max_runs(const int* __restrict__ kids_part, int kids_blocks, int* rm) {
+    const int tid = threadIdx.x;
+    if (tid < 8) rm[tid] = 0;
+    __syncthreads();
+    // thread t reads level slot t & 7 (the stride keeps the slot), eight loads in flight
+    int m = 0;
+    const int nq = kids_blocks * 8;
+    int q = tid;
+    for (; q + 7 * NT < nq; q += 8 * NT) {
+        int v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = kids_part[q + u * NT];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) m = max(m, v[u]);
+    }
+    for (; q < nq; q += NT) m = max(m, kids_part[q]);
+    if (m > 0) atomicMax(&rm[tid & 7], m);
+    __syncthreads();
+}
+
+// Graph 0's part of the instance state (one thread).
+__device__ __forceinline__ void mirror_state(DevState* st, const SegState& q, const int* rm) {
+    st->swing = q.swing;
+    st->traction = q.traction;
+    st->interactions = q.interactions;
+    st->global_speed = q.global_speed;
+    st->speed_efficiency = q.speed_efficiency;
+    // the next path-key sort: p 8-bit passes order the bodies by their top 4p levels,
+    // and the pairs left tied are the bodies of one 4p-level cell, which the fix-up
+    // orders; take the fewest passes whose cells (in this tree) hold at most
+    // kSortRunMax bodies each
+    int p = 1;
+    while (p < 8 && rm[p - 1] > kSortRunMax) ++p;
+    if (st->full_sorts > 0) {
+        st->full_sorts -= 1;      // still settling after new positions
+        p = 8;
+    }
+    st->sort_skip = 8 - p;
+    for (int k = 0; k < 8; ++k) st->runmax[k] = rm[k];
+}
+
+// One node's new position.
+__device__ __forceinline__ float2 displaced(float2 p, float2 F, float2 P, float gs) {
+    const float dx = F.x - P.x, dy = F.y - P.y;
+    const float swg = sqrtf(dx * dx + dy * dy);
+    const float factor = (float)((double)gs / (1.0 + (double)sqrtf(gs * swg)));
+    p.x = fmaf(F.x, factor, p.x);
+    p.y = fmaf(F.y, factor, p.y);
+    return p;
+}
+
+__device__ __forceinline__ float4 box_add(float4 acc, float2 p) {
+    return make_float4(fminf(acc.x, p.x), fminf(acc.y, p.y), fmaxf(acc.z, p.x), fmaxf(acc.w, p.y));
+}
+
+// The block's box {min x, min y, max x, max y}; thread 0 gets it.
+template <int NT>
+__device__ __forceinline__ float4 box_reduce(float4 acc) {
+    __shared__ float4 red[NT / 64];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+        acc = make_float4(fminf(acc.x, __shfl_xor(acc.x, o, 64)), fminf(acc.y, __shfl_xor(acc.y, o, 64)),
+                          fmaxf(acc.z, __shfl_xor(acc.z, o, 64)), fmaxf(acc.w, __shfl_xor(acc.w, o, 64)));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < NT / 64; ++w) {
+            const float4 v = red[w];
+            acc = make_float4(fminf(acc.x, v.x), fminf(acc.y, v.y), fmaxf(acc.z, v.z), fmaxf(acc.w, v.w));
+        }
+    return acc;
+}
+
+constexpr int kSpeedThreads = 1024;
+
+__global__ __launch_bounds__(kSpeedThreads) void k_speed(const WalkPart* __restrict__ part,
+                                                         const int* __restrict__ grp_first,
+                                                         const int* __restrict__ node_off, SegState* __restrict__ seg,
+                                                         DevState* st, const int* __restrict__ kids_part,
+                                                         int kids_blocks) {
+    __shared__ int rm[8];
+    if (st->err != 0) return;
+    const int g = blockIdx.x;
+    if (g == 0) max_runs<kSpeedThreads>(kids_part, kids_blocks, rm);
+    const GroupSums r = sum_groups<kSpeedThreads>(part, grp_first[g], grp_first[g + 1]);
+    if (threadIdx.x == 0) {
+        // per graph (one block each): no word shared by the blocks of a batch
+        const SegState q = speed_update(seg[g], r, node_off[g + 1] - node_off[g]);
+        seg[g] = q;
+        if (g == 0) mirror_state(st, q, rm);
+    }
+}
+
 __global__ __launch_bounds__(256) void k_displace(float2* __restrict__ pos, const float2* __restrict__ f,
-                                                  float2* __restrict__ fprev, int n, const int* __restrict__ seg_of,
+                                                  float2* __restrict__ fprev, int n, const int* __restrict__ rank,
+                                                  float2* __restrict__ pos_rank, const int* __restrict__ seg_of,
                                                   const SegState* __restrict__ seg, float4* __restrict__ part,
                                                   DevState* st) {
-    __shared__ float4 red[256];
     const int tid = threadIdx.x;
     const bool live = st->err == 0;
     const float gs0 = seg[0].global_speed;
@@ -743,43 +836,136 @@ __global__ __launch_bounds__(256) void k_displace(float2* __restrict__ pos, cons
         if (live) {
             const float gs = seg_of ? seg[seg_of[i]].global_speed : gs0;
             const float2 F = f[i];
-            const float2 P = fprev[i];
-            const float dx = F.x - P.x, dy = F.y - P.y;
-            const float swg = sqrtf(dx * dx + dy * dy);
-            const float factor = (float)((double)gs / (1.0 + (double)sqrtf(gs * swg)));
-            p.x = fmaf(F.x, factor, p.x);
-            p.y = fmaf(F.y, factor, p.y);
+            p = displaced(p, F, fprev[i], gs);
             pos[i] = p;
+            pos_rank[rank[i]] = p;
             fprev[i] = F;
         }
-        acc.x = fminf(acc.x, p.x);
-        acc.y = fminf(acc.y, p.y);
-        acc.z = fmaxf(acc.z, p.x);
-        acc.w = fmaxf(acc.w, p.y);
+        acc = box_add(acc, p);
     }
     if (part == nullptr) {
         if (blockIdx.x == 0 && tid == 0 && live) st->iteration += 1;
         return;
     }
-    red[tid] = acc;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (tid < o) {
-            float4 v = red[tid + o];
-            acc.x = fminf(acc.x, v.x);
-            acc.y = fminf(acc.y, v.y);
-            acc.z = fmaxf(acc.z, v.z);
-            acc.w = fmaxf(acc.w, v.w);
-            red[tid] = acc;
-        }
-        __syncthreads();
-    }
+    acc = box_reduce<256>(acc);
     if (tid == 0) {
-        part[blockIdx.x] = red[0];
+        part[blockIdx.x] = acc;
         if (blockIdx.x == 0) {
             st->nbbox = gridDim.x;
             if (live) st->iteration += 1;
         }
+    }
+}
+
+// One graph: speed and displacement in one launch. Every block forms the new speed from seg_cur,
+// the state before the iteration (copied from seg by the iteration's first kernel); block 0
+// alone writes the new state, to seg, which no block of this launch reads.
+__global__ __launch_bounds__(256) void k_advance(float2* __restrict__ pos, const float2* __restrict__ f,
+                                                 float2* __restrict__ fprev, int n, const int* __restrict__ rank,
+                                                 float2* __restrict__ pos_rank, const WalkPart* __restrict__ wpart,
+                                                 int ngroups, const SegState* __restrict__ seg_cur,
+                                                 SegState* __restrict__ seg, const int* __restrict__ kids_part,
+                                                 int kids_blocks, float4* __restrict__ part, DevState* st) {
+    __shared__ int rm[8];
+    __shared__ float new_speed;
+    const int tid = threadIdx.x;
+    const bool live = st->err == 0;               // nothing in this launch changes it
+    // the block's first nodes are loaded beside the sums
+    const int i0 = blockIdx.x * 256 + tid;
+    float2 p0 = make_float2(0.0f, 0.0f), F0 = p0, P0 = p0;
+    int r0 = 0;
+    if (i0 < n) {
+        p0 = pos[i0];
+        F0 = f[i0];
+        P0 = fprev[i0];
+        r0 = rank[i0];
+    }
+    if (live) {
+        if (blockIdx.x == 0) max_runs<256>(kids_part, kids_blocks, rm);
+        const GroupSums r = sum_groups<256>(wpart, 0, ngroups);
+        if (tid == 0) {
+            const SegState q = speed_update(*seg_cur, r, n);
+            new_speed = q.global_speed;
+            if (blockIdx.x == 0) {
+                seg[0] = q;
+                mirror_state(st, q, rm);
+            }
+        }
+        __syncthreads();
+    }
+    const float gs = live ? new_speed : 0.0f;
+    float4 acc = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
+    for (int i = i0; i < n; i += gridDim.x * 256) {
+        if (i != i0) {
+            p0 = pos[i];
+            F0 = f[i];
+            P0 = fprev[i];
+            r0 = rank[i];
+        }
+        float2 p = p0;
+        if (live) {
+            p = displaced(p0, F0, P0, gs);
+            pos[i] = p;
+            pos_rank[r0] = p;
+            fprev[i] = F0;
+        }
+        acc = box_add(acc, p);
+    }
+    acc = box_reduce<256>(acc);
+    if (tid == 0) {
+        part[blockIdx.x] = acc;
+        if (blockIdx.x == 0) {
+            st->nbbox = gridDim.x;
+            if (live) st->iteration += 1;
+        }
+    }
+}
+
+// A batch, one block per graph (largest first): the graph's speed, its nodes' displacement and
+// the root of its next tree (as k_seg_bbox sets it).
+constexpr int kAdvanceSegThreads = 512;
+
+__global__ __launch_bounds__(kAdvanceSegThreads) void k_advance_seg(
+    float2* __restrict__ pos, const float2* __restrict__ f, float2* __restrict__ fprev, const int* __restrict__ rank,
+    float2* __restrict__ pos_rank, const WalkPart* __restrict__ wpart, const int* __restrict__ grp_first,
+    const int* __restrict__ node_off, const int* __restrict__ order, SegState* __restrict__ seg,
+    const int* __restrict__ kids_part, int kids_blocks, float4* __restrict__ seg_root, DevState* st) {
+    constexpr int NT = kAdvanceSegThreads;
+    __shared__ int rm[8];
+    __shared__ float new_speed;
+    if (st->err != 0) return;
+    const int g = order[blockIdx.x], tid = threadIdx.x;
+    const int a = node_off[g], e = node_off[g + 1];
+    if (g == 0) max_runs<NT>(kids_part, kids_blocks, rm);
+    const GroupSums r = sum_groups<NT>(wpart, grp_first[g], grp_first[g + 1]);
+    if (tid == 0) {
+        const SegState q = speed_update(seg[g], r, e - a);
+        new_speed = q.global_speed;
+        seg[g] = q;
+        if (g == 0) {
+            mirror_state(st, q, rm);
+            st->iteration += 1;
+        }
+    }
+    __syncthreads();
+    const float gs = new_speed;
+    float4 acc = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
+#pragma unroll 2
+    for (int i = a + tid; i < e; i += NT) {
+        const float2 F = f[i];
+        const float2 p = displaced(pos[i], F, fprev[i], gs);
+        pos[i] = p;
+        pos_rank[rank[i]] = p;
+        fprev[i] = F;
+        acc = box_add(acc, p);
+    }
+    acc = box_reduce<NT>(acc);
+    if (tid == 0) {
+        // no ordered coordinate at all (every one NaN): the box k_seg_bbox would form
+        if (!(acc.x <= acc.z)) acc.x = acc.z = NAN;
+        if (!(acc.y <= acc.w)) acc.y = acc.w = NAN;
+        seg_root[g] = make_float4((acc.x + acc.z) * 0.5f, (acc.y + acc.w) * 0.5f,
+                                  fmaxf(acc.z - acc.x, acc.w - acc.y) * 0.5f, 0.0f);
     }
 }
 
@@ -791,7 +977,9 @@ __global__ __launch_bounds__(256) void k_displace(float2* __restrict__ pos, cons
 // interacts with every body of its graph, so the interaction count is the sum of n_g^2.
 // ---------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_pack(const float2* __restrict__ pos, const float* __restrict__ mass, int n,
-                                              float4* __restrict__ body) {
+                                              float4* __restrict__ body, const SegState* __restrict__ seg,
+                                              SegState* __restrict__ seg_cur) {
+    if (seg_cur && blockIdx.x == 0 && threadIdx.x == 0) *seg_cur = seg[0];   // for k_advance
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const float2 p = pos[i];
         body[i] = make_float4(p.x, p.y, mass[i], 0.0f);
@@ -915,7 +1103,6 @@ void launch_col_rank(const Bufs& b, hipStream_t s) {
 }
 
 void launch_attraction(const Bufs& b, const Params& p, hipStream_t s) {
-    k_rank_pos<<<(b.n + 255) / 256, 256, 0, s>>>(b.pos, b.rank, b.n, b.pos_rank);
     const int lb = (b.nlight + 255) / 256;
     const int mb = (b.nmedium + 3) / 4;
     int total = lb + mb + b.nattr_chunks;
@@ -961,20 +1148,45 @@ void launch_combine(const Bufs& b, const Params& p, hipStream_t s) {
                                                               b.node_off, b.fga, b.fprev, b.f, b.rep, b.grp_part, b.st);
 }
 
+namespace {
+
+// How a graph or batch takes speed and displacement (see above k_speed).
+bool advance_one(const Bufs& b) { return b.nseg == 1 && b.ngroups <= kAdvanceGroups; }
+
+}  // namespace
+
+bool advance_seg(const Bufs& b) { return b.nseg > 1 && b.max_seg <= kSegSortMax; }
+
+void launch_rank_pos(const Bufs& b, hipStream_t s) {
+    k_rank_pos<<<(b.n + 255) / 256, 256, 0, s>>>(b.pos, b.rank, b.n, b.pos_rank);
+}
+
 void launch_speed(const Bufs& b, hipStream_t s) {
+    if (advance_one(b) || advance_seg(b)) return;          // done with the displacement
     k_speed<<<b.nseg, kSpeedThreads, 0, s>>>(b.grp_part, b.grp_first, b.node_off, b.seg_st, b.st, b.kids_part,
                                               b.kids_blocks);
 }
 
 void launch_displacement(const Bufs& b, hipStream_t s) {
-    k_displace<<<displacement_blocks(b), 256, 0, s>>>(b.pos, b.f, b.fprev, b.n, b.nseg > 1 ? b.seg_of : nullptr,
-                                                       b.seg_st, b.nseg > 1 ? nullptr : b.bbox_part, b.st);
+    if (advance_seg(b)) {
+        k_advance_seg<<<b.nseg, kAdvanceSegThreads, 0, s>>>(b.pos, b.f, b.fprev, b.rank, b.pos_rank, b.grp_part,
+                                                            b.grp_first, b.node_off, b.seg_order, b.seg_st,
+                                                            b.kids_part, b.kids_blocks, b.seg_root, b.st);
+    } else if (advance_one(b)) {
+        k_advance<<<displacement_blocks(b), 256, 0, s>>>(b.pos, b.f, b.fprev, b.n, b.rank, b.pos_rank, b.grp_part,
+                                                         b.ngroups, b.seg_cur, b.seg_st, b.kids_part, b.kids_blocks,
+                                                         b.bbox_part, b.st);
+    } else {
+        k_displace<<<displacement_blocks(b), 256, 0, s>>>(b.pos, b.f, b.fprev, b.n, b.rank, b.pos_rank,
+                                                           b.nseg > 1 ? b.seg_of : nullptr, b.seg_st,
+                                                           b.nseg > 1 ? nullptr : b.bbox_part, b.st);
+    }
 }
 
 void launch_exact(const Bufs& b, const Params& p, hipStream_t s) {
     int pb = (b.n + 255) / 256;
     if (pb > 4096) pb = 4096;
-    k_pack<<<pb, 256, 0, s>>>(b.pos, b.mass, b.n, b.sbody);
+    k_pack<<<pb, 256, 0, s>>>(b.pos, b.mass, b.n, b.sbody, b.seg_st, b.seg_cur);
     constexpr int BT = 256;
     if (p.group == 64)
         k_exact<64, BT><<<walk_blocks(b.ngroups, 64, BT), BT, 0, s>>>(b.sbody, b.groups, b.ngroups, b.node_off, b.fga,
@@ -989,7 +1201,7 @@ void launch_exact(const Bufs& b, const Params& p, hipStream_t s) {
 void launch_exact_only(const Bufs& b, const Params& p, bool fp64, double2* out, hipStream_t s) {
     int pb = (b.n + 255) / 256;
     if (pb > 4096) pb = 4096;
-    k_pack<<<pb, 256, 0, s>>>(b.pos, b.mass, b.n, b.sbody);
+    k_pack<<<pb, 256, 0, s>>>(b.pos, b.mass, b.n, b.sbody, nullptr, nullptr);
     const int blocks = (b.n + 255) / 256;
     if (fp64)
         k_exact_only<double><<<blocks, 256, 0, s>>>(b.sbody, b.n, b.nseg, b.node_off, p.k_r, p.epssq, out);
