@@ -304,8 +304,6 @@ bool engine_view(struct ::gfa2_engine* h, EngineView* v);
 bool engine_graph(struct ::gfa2_engine* h, const Bufs** b, int* device, hipStream_t* stream);
 int engine_positions_written(struct ::gfa2_engine* h);
 
-// Walk grid sizes (partials count depends on them).
-int walk_blocks(int ngroups, int group, int bt);
 int displacement_blocks(const Bufs& b);
 
 }  // namespace gfa2

@@ -970,11 +970,10 @@ __global__ __launch_bounds__(kAdvanceSegThreads) void k_advance_seg(
 }
 
 // ---------------------------------------------------------------------------------------
-// Exact repulsion (no counterpart in the reference's GPU path). Each lane is one node; the
-// group's G lanes run over all nodes j of their graph in ascending order, reading the packed
-// {x, y, mass} of node j (one address per group: a broadcast load), with the walk's term
-// k_r m_i m_j (p_i - p_j) / (|p_i - p_j|^2 + eps^2) (node i itself adds 0). Every body
-// interacts with every body of its graph, so the interaction count is the sum of n_g^2.
+// Exact repulsion (no counterpart in the reference's GPU path). Each lane is one node and runs
+// over nodes j of its graph in ascending order, reading the packed {x, y, mass} of node j, with
+// the walk's term k_r m_i m_j (p_i - p_j) / (|p_i - p_j|^2 + eps^2) (node i itself adds 0).
+// Every body interacts with every body of its graph, so the interaction count is the sum of n_g^2.
 // ---------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_pack(const float2* __restrict__ pos, const float* __restrict__ mass, int n,
                                               float4* __restrict__ body, const SegState* __restrict__ seg,
@@ -986,47 +985,77 @@ __global__ __launch_bounds__(256) void k_pack(const float2* __restrict__ pos, co
     }
 }
 
-template <int G, int BT>
-__global__ __launch_bounds__(BT) void k_exact(const float4* __restrict__ body, const int2* __restrict__ groups,
-                                              int ngroups, const int* __restrict__ node_off,
-                                              const float2* __restrict__ fga, const float2* __restrict__ fprev,
-                                              float2* __restrict__ f, float2* __restrict__ rep,
-                                              WalkPart* __restrict__ part, float k_r, float epssq,
-                                              const DevState* __restrict__ st) {
+// A block takes 64 bodies and cuts their graph's nodes into kExactSlices runs, one per wave; the
+// runs' sums are added in run order through LDS. The cut depends on the graph's size alone, so a
+// graph in a batch gets the bits it gets alone. The wave's lanes all read the same node, which
+// goes through the scalar cache.
+//
+// Bound by FP32 VALU issue (7 vector instructions and a quarter-rate reciprocal per term) once
+// there are waves enough: with one lane per body and no cut, 12,345 bodies were 193 waves on
+// 1,024 SIMDs, each waiting for one load per term, 1,238 us; with the cut 70 us (the issue alone:
+// 44 cycles per term and wave, 51 us on the 193 compute units that hold a block).
+constexpr int kExactSlices = 16;
+
+template <int G>
+__global__ __launch_bounds__(64 * kExactSlices) void k_exact(const float4* __restrict__ body,
+                                                             const int2* __restrict__ groups, int ngroups,
+                                                             const int* __restrict__ node_off,
+                                                             const float2* __restrict__ fga,
+                                                             const float2* __restrict__ fprev,
+                                                             float2* __restrict__ f, float2* __restrict__ rep,
+                                                             WalkPart* __restrict__ part, float k_r, float epssq,
+                                                             const DevState* __restrict__ st) {
+    __shared__ float2 red[kExactSlices][64];
     if (st->err != 0) return;
-    const int lb = xcd_block();
-    const int gidx = (lb * BT + (int)threadIdx.x) / G;
-    const int gl = (lb * BT + (int)threadIdx.x) % G;
+    const int lane = threadIdx.x & 63;
+    const int slice = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int first = xcd_block() * (64 / G);       // the block's first group
+    const int gidx = first + lane / G;
     const bool group_ok = gidx < ngroups;
-    int2 grp = make_int2(0, 0);
-    if (group_ok) grp = groups[gidx];
+    const int2 grp = groups[min(gidx, ngroups - 1)];
     const int g = grp.y;
-    const int k = grp.x + gl;
+    const int k = grp.x + lane % G;
     const bool active = group_ok && k < node_off[g + 1];
-    float px = 0.0f, py = 0.0f, mi = 0.0f, kmi = 0.0f;
+    float px = 0.0f, py = 0.0f, mi = 0.0f;
     if (active) {
         const float4 me = body[k];
         px = me.x;
         py = me.y;
         mi = me.z;
-        kmi = k_r * mi;
     }
     float ax = 0.0f, ay = 0.0f;
-    unsigned int inter = 0;
-    if (group_ok) {
-        const int j0 = node_off[g], j1 = node_off[g + 1];
-        for (int j = j0; j < j1; ++j) {
+    // the one or (a block of two groups of 32) two graphs of the block's bodies
+#pragma unroll
+    for (int q = 0; q < 64 / G; ++q) {
+        const int gq = __builtin_amdgcn_readlane(g, q * G);
+        if (q > 0 && gq == __builtin_amdgcn_readlane(g, 0)) break;      // uniform
+        const int j0 = node_off[gq], m = node_off[gq + 1] - j0;
+        const int run = (m + kExactSlices - 1) / kExactSlices;
+        const int ja = __builtin_amdgcn_readfirstlane(j0 + min(m, slice * run));
+        const int jb = __builtin_amdgcn_readfirstlane(j0 + min(m, (slice + 1) * run));
+        if (g != gq) continue;
+#pragma unroll 8
+        for (int j = ja; j < jb; ++j) {
             const float4 c = body[j];
             const float dx = px - c.x;
             const float dy = py - c.y;
-            const float d2 = dx * dx + dy * dy + epssq;
-            const float w = kmi * c.z * __builtin_amdgcn_rcpf(d2);
+            const float w = c.z * __builtin_amdgcn_rcpf(fmaf(dx, dx, fmaf(dy, dy, epssq)));
             ax = fmaf(dx, w, ax);
             ay = fmaf(dy, w, ay);
         }
-        inter = active ? (unsigned int)(j1 - j0) : 0u;
     }
-    group_finish<G>(active, group_ok, gl, gidx, (unsigned int)k, mi, ax, ay, inter, fga, fprev, f, rep, part);
+    red[slice][lane] = make_float2(ax, ay);
+    __syncthreads();
+    if (slice != 0) return;
+#pragma unroll
+    for (int q = 1; q < kExactSlices; ++q) {
+        ax += red[q][lane].x;
+        ay += red[q][lane].y;
+    }
+    const float kmi = k_r * mi;                     // taken out of every term
+    const unsigned int inter = active ? (unsigned int)(node_off[g + 1] - node_off[g]) : 0u;
+    group_finish<G>(active, group_ok, lane % G, gidx, (unsigned int)k, mi, kmi * ax, kmi * ay, inter, fga, fprev, f,
+                    rep, part);
 }
 
 // All-pairs repulsion into out, one thread per node, FP32 or FP64 arithmetic; the graph of
@@ -1067,12 +1096,6 @@ __global__ __launch_bounds__(256) void k_edge_pow(const float* __restrict__ w, l
 }
 
 }  // namespace
-
-int walk_blocks(int ngroups, int group, int bt) {
-    const int per_block = bt / group;
-    int b = (ngroups + per_block - 1) / per_block;
-    return b < 1 ? 1 : b;
-}
 
 namespace {
 
@@ -1187,15 +1210,14 @@ void launch_exact(const Bufs& b, const Params& p, hipStream_t s) {
     int pb = (b.n + 255) / 256;
     if (pb > 4096) pb = 4096;
     k_pack<<<pb, 256, 0, s>>>(b.pos, b.mass, b.n, b.sbody, b.seg_st, b.seg_cur);
-    constexpr int BT = 256;
+    const int per_block = 64 / p.group;
+    const int blocks = (b.ngroups + per_block - 1) / per_block;
     if (p.group == 64)
-        k_exact<64, BT><<<walk_blocks(b.ngroups, 64, BT), BT, 0, s>>>(b.sbody, b.groups, b.ngroups, b.node_off, b.fga,
-                                                                      b.fprev, b.f, b.rep, b.grp_part, p.k_r,
-                                                                      p.epssq, b.st);
+        k_exact<64><<<blocks, 64 * kExactSlices, 0, s>>>(b.sbody, b.groups, b.ngroups, b.node_off, b.fga, b.fprev, b.f,
+                                                         b.rep, b.grp_part, p.k_r, p.epssq, b.st);
     else
-        k_exact<32, BT><<<walk_blocks(b.ngroups, 32, BT), BT, 0, s>>>(b.sbody, b.groups, b.ngroups, b.node_off, b.fga,
-                                                                      b.fprev, b.f, b.rep, b.grp_part, p.k_r,
-                                                                      p.epssq, b.st);
+        k_exact<32><<<blocks, 64 * kExactSlices, 0, s>>>(b.sbody, b.groups, b.ngroups, b.node_off, b.fga, b.fprev, b.f,
+                                                         b.rep, b.grp_part, p.k_r, p.epssq, b.st);
 }
 
 void launch_exact_only(const Bufs& b, const Params& p, bool fp64, double2* out, hipStream_t s) {
