@@ -70,6 +70,10 @@ struct gfa2_engine {
     // the lowest path-key sort pass launched: one below the lowest the device ran when the host
     // last read its state (a full sort after new positions or parameters)
     int sort_first = 0;
+    // workspace of calls that need scratch (EngineScratch)
+    std::mutex scratch_mu;
+    void* scratch = nullptr;
+    size_t scratch_bytes = 0;
     // launch shapes (autotuned per graph-size bucket)
     int cus = 256;
     LaunchConfig tune{256, 8, 0, 0};
@@ -135,6 +139,9 @@ void free_all(gfa2_engine* h) {
     h->graph_valid = false;
     for (void* p : h->allocs) hipFree(p);
     h->allocs.clear();
+    if (h->scratch) hipFree(h->scratch);
+    h->scratch = nullptr;
+    h->scratch_bytes = 0;
     h->b = Bufs{};
     h->rep_buf = nullptr;
     h->ew_buf = nullptr;
@@ -1332,6 +1339,34 @@ bool engine_graph(gfa2_engine* h, const Bufs** b, int* device, hipStream_t* stre
     *device = h->device;
     *stream = h->stream;
     return true;
+}
+
+EngineScratch::EngineScratch(gfa2_engine* engine) : h(engine) { h->scratch_mu.lock(); }
+
+EngineScratch::~EngineScratch() {
+    if (own) (void)hipFree(own);
+    h->scratch_mu.unlock();
+}
+
+void* EngineScratch::get(size_t bytes) {
+    if (bytes <= h->scratch_bytes) return h->scratch;
+    if (bytes > kScratchKeep) {
+        if (hipMalloc(&own, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            own = nullptr;
+        }
+        return own;
+    }
+    if (h->scratch) (void)hipFree(h->scratch);      // waits for the device
+    h->scratch = nullptr;
+    h->scratch_bytes = 0;
+    if (hipMalloc(&h->scratch, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        h->scratch = nullptr;
+        return nullptr;
+    }
+    h->scratch_bytes = bytes;
+    return h->scratch;
 }
 
 bool engine_view(gfa2_engine* h, EngineView* v) {

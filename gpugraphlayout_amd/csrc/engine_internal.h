@@ -304,6 +304,23 @@ bool engine_view(struct ::gfa2_engine* h, EngineView* v);
 bool engine_graph(struct ::gfa2_engine* h, const Bufs** b, int* device, hipStream_t* stream);
 int engine_positions_written(struct ::gfa2_engine* h);
 
+// Device scratch of one call, from the engine's own workspace: it grows to the largest request
+// of up to kScratchKeep bytes and is freed with the engine's graph; a larger request is
+// allocated for the call alone. Held for the caller's lifetime: calls of other threads wait.
+constexpr size_t kScratchKeep = 256u << 20;
+
+class EngineScratch {
+public:
+    explicit EngineScratch(struct ::gfa2_engine* h);
+    ~EngineScratch();
+    EngineScratch(const EngineScratch&) = delete;
+    EngineScratch& operator=(const EngineScratch&) = delete;
+    void* get(size_t bytes);             // null: no device memory
+private:
+    struct ::gfa2_engine* h;
+    void* own = nullptr;
+};
+
 int displacement_blocks(const Bufs& b);
 
 }  // namespace gfa2

@@ -8,9 +8,19 @@
 // arithmetic (powers by repeated squaring, IEEE operations), so both produce the same bytes;
 // this file is compiled with -ffp-contract=off, since the *_rn intrinsics alone do not stop
 // a multiply and an add from being fused.
+//
+// gfa2_render counts in LDS: the edges become a list of lines (k_raster_lines), and a block per
+// (picture tile, slice of the lines) finds the lines that cross its tile, walks their samples
+// there and writes the tile's counts to a copy of the tile of its own (k_raster_tiles), so that
+// no counter is shared; k_shade adds the copies. A tile gets slices in proportion to the samples
+// a part of the lines put there (k_raster_cost, k_raster_plan): in a finished layout one tile of
+// fifty can hold a sixth of them. gfa2_render_noalloc, which has no memory
+// for a list or copies, adds every sample to one counter per pixel with device atomics
+// (k_raster_nodes, k_raster_edges).
 #include "engine_internal.h"
 #include "../../include/gfa2.h"
 
+#include <algorithm>
 #include <mutex>
 
 // Fixed scratch of gfa2_render_noalloc (one copy per device, loaded with the code object and
@@ -68,14 +78,18 @@ __global__ __launch_bounds__(256) void k_minmax(const float2* __restrict__ pos, 
     if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-__global__ void k_minmax_final(const float4* __restrict__ part, int nb, float4* __restrict__ out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__global__ __launch_bounds__(64) void k_minmax_final(const float4* __restrict__ part, int nb,
+                                                     float4* __restrict__ out) {
     float4 m = part[0];
-    for (int b = 1; b < nb; ++b) {
+    for (int b = threadIdx.x; b < nb; b += 64) {
         const float4 a = part[b];
         m = make_float4(fminf(m.x, a.x), fmaxf(m.y, a.y), fminf(m.z, a.z), fmaxf(m.w, a.w));
     }
-    *out = m;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+        m = make_float4(fminf(m.x, __shfl_xor(m.x, o, 64)), fmaxf(m.y, __shfl_xor(m.y, o, 64)),
+                        fminf(m.z, __shfl_xor(m.z, o, 64)), fmaxf(m.w, __shfl_xor(m.w, o, 64)));
+    if (threadIdx.x == 0) *out = m;
 }
 
 // Discs of radius 3 around the rounded node centre.
@@ -126,6 +140,365 @@ __global__ __launch_bounds__(256) void k_raster_edges(const float2* __restrict__
     }
 }
 
+// ---- counting in picture tiles ----------------------------------------------------------------
+
+constexpr int kTileW = 256, kTileH = 128;         // 257-word rows: a vertical line's samples fall in different banks
+constexpr int kTileThreads = 1024;
+constexpr int kTilePixels = kTileW * kTileH;
+constexpr int kQueueGo = 32;                      // a wave walks its tile's lines once it has found this many
+constexpr int kSpareSlices = 1024;                // slices beyond the first of each tile: four per compute unit
+constexpr long long kListEntries = 4ll << 20;     // CSR entries whose lines are listed at a time (64 MB at most)
+constexpr int kLineThreads = 256, kLineItems = 16;
+// Lines with an end this far out (in pixels) are drawn sample by sample (k_raster_lines): below it
+// a sample's float rounding stays under half a pixel, and steps under 2^24 (quotient below).
+constexpr float kFarOut = 4194304.0f;
+
+// k / steps correctly rounded, from the correctly rounded y = 1 / steps. q is within two units of
+// the quotient, so r = k - steps q is exact (steps is an integer below 2^24), and q + r y errs from
+// the quotient by under 2^-100 of it before its own rounding; a quotient of integers below 2^24
+// that is no double lies at least 2^-78 of itself from the midpoint of two doubles.
+__device__ __forceinline__ double quotient(double k, double steps, double y) {
+    const double q = __dmul_rn(k, y);
+    return __fma_rn(__fma_rn(-steps, q, k), y, q);
+}
+
+// The samples [k0, k1] of a line that may fall in the pixels [x0, x1) x [y0, y1): pad is two
+// pixels and what a sample's rounding can add, and the ends are widened by a sample.
+__device__ __forceinline__ bool clip_line(const float4 l, int steps, float x0, float x1, float y0, float y1,
+                                          float pad, int* k0, int* k1) {
+    if (fmaxf(l.x, l.z) < x0 - pad || fminf(l.x, l.z) > x1 + pad || fmaxf(l.y, l.w) < y0 - pad ||
+        fminf(l.y, l.w) > y1 + pad)
+        return false;
+    double t0 = 0.0, t1 = 1.0;
+    const double dx = (double)l.z - l.x, dy = (double)l.w - l.y;
+    if (fabs(dx) > 1e-3) {
+        const double a = ((double)x0 - pad - l.x) / dx, b = ((double)x1 + pad - l.x) / dx;
+        t0 = fmax(t0, fmin(a, b));
+        t1 = fmin(t1, fmax(a, b));
+    }
+    if (fabs(dy) > 1e-3) {
+        const double a = ((double)y0 - pad - l.y) / dy, b = ((double)y1 + pad - l.y) / dy;
+        t0 = fmax(t0, fmin(a, b));
+        t1 = fmin(t1, fmax(a, b));
+    }
+    if (!(t0 <= t1)) return false;
+    *k0 = max(0, (int)floor(t0 * steps) - 1);
+    *k1 = min(steps, (int)ceil(t1 * steps) + 1);
+    return true;
+}
+
+// Orders this wave's LDS writes before its later LDS reads by other lanes.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The lines of CSR entries [e0, e1) with i < j, in no order (counts do not depend on it), as
+// {x0, y0, x1, y1} in pixels; the far-out ones are drawn here, into far.
+__global__ __launch_bounds__(kLineThreads) void k_raster_lines(const float2* __restrict__ pos,
+                                                               const int* __restrict__ rowptr,
+                                                               const int* __restrict__ col, int n, long long e0,
+                                                               long long e1, Frame f, float4* __restrict__ lines,
+                                                               unsigned int* __restrict__ nlines,
+                                                               unsigned int* __restrict__ far) {
+    __shared__ unsigned int wsum[kLineThreads / 64];
+    __shared__ unsigned int base;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const long long first = e0 + ((long long)blockIdx.x * kLineThreads + tid) * kLineItems;
+    const long long last = first + kLineItems < e1 ? first + kLineItems : e1;
+    float4 mine[kLineItems];
+    unsigned int take = 0u;                         // bit q: mine[q] is a line
+    if (first < last) {
+        int lo = 0, hi = n;                         // row: rowptr[lo] <= first < rowptr[lo + 1]
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if ((long long)rowptr[mid] <= first) lo = mid;
+            else hi = mid;
+        }
+        int i = lo;
+        long long end = rowptr[i + 1];
+#pragma unroll
+        for (int q = 0; q < kLineItems; ++q) {
+            const long long e = first + q;
+            if (e < last) {
+                while (end <= e) end = rowptr[++i + 1];
+                const int j = col[e];
+                if (i < j) {
+                    const float2 a = pos[i], b = pos[j];
+                    mine[q] = make_float4(to_px(a.x, f.x0, f.sx), to_px(a.y, f.y0, f.sy), to_px(b.x, f.x0, f.sx),
+                                          to_px(b.y, f.y0, f.sy));
+                    take |= 1u << q;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < kLineItems; ++q) {
+        if (!((take >> q) & 1u)) continue;
+        const float4 l = mine[q];
+        const float out = fmaxf(fmaxf(fabsf(l.x), fabsf(l.y)), fmaxf(fabsf(l.z), fabsf(l.w)));
+        const bool nan = l.x != l.x || l.y != l.y || l.z != l.z || l.w != l.w;
+        if (out < kFarOut && !nan) continue;
+        take &= ~(1u << q);
+        const float ddx = __fsub_rn(l.z, l.x), ddy = __fsub_rn(l.w, l.y);
+        const float len = fmaxf(fabsf(ddx), fabsf(ddy));
+        if (!(len < 2147483648.0f) && len == len) continue;   // more samples than can be counted
+        const int steps = (int)ceilf(len);
+        if (steps == 0) {
+            hit(far, f, (int)lroundf(l.x), (int)lroundf(l.y));
+            continue;
+        }
+        int k0 = 0, k1 = steps;
+        // up to 2^30 a sample's float rounding is under 2^-23 of the farthest end (further out, a
+        // pixel's number may wrap: every sample is looked at)
+        if (out < 1073741824.0f && !nan &&
+            !clip_line(l, steps, 0.0f, (float)f.w, 0.0f, (float)f.h, 2.0f + 2.4e-7f * out, &k0, &k1))
+            continue;
+        for (long long k = k0; k <= k1; ++k) {
+            const double t = __ddiv_rn((double)k, (double)steps);
+            const float sx = (float)__dadd_rn((double)l.x, __dmul_rn(t, (double)ddx));
+            const float sy = (float)__dadd_rn((double)l.y, __dmul_rn(t, (double)ddy));
+            hit(far, f, (int)lroundf(sx), (int)lroundf(sy));
+        }
+    }
+    // the block's lines get one run of the list
+    const unsigned int c = (unsigned int)__popc(take);
+    unsigned int inc = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned int t = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += t;
+    }
+    if (lane == 63) wsum[wave] = inc;
+    __syncthreads();
+    unsigned int before = 0u, total = 0u;
+#pragma unroll
+    for (int w = 0; w < kLineThreads / 64; ++w) {
+        if (w < wave) before += wsum[w];
+        total += wsum[w];
+    }
+    if (tid == 0) base = total ? atomicAdd(nlines, total) : 0u;
+    __syncthreads();
+    unsigned int at = base + before + inc - c;
+#pragma unroll
+    for (int q = 0; q < kLineItems; ++q)
+        if ((take >> q) & 1u) lines[at++] = mine[q];
+}
+
+// lroundf (half away from zero) of a value below 2^22 in magnitude: the float steps are exact.
+__device__ __forceinline__ int round_px(float v) {
+    const float t = truncf(v);
+    return (int)(t + (fabsf(__fsub_rn(v, t)) >= 0.5f ? copysignf(1.0f, v) : 0.0f));
+}
+
+// A tile of the picture: columns [c0, c0 + cw), rows [r0, r0 + rh); y is up, so these rows are
+// y = ylo + rh - 1 down to ylo.
+struct Tile {
+    int c0, r0, cw, rh, ylo;
+};
+
+__device__ __forceinline__ Tile tile_of(int t, int tiles_x, const Frame& f) {
+    Tile a;
+    a.c0 = (t % tiles_x) * kTileW;
+    a.r0 = (t / tiles_x) * kTileH;
+    a.cw = min(kTileW, f.w - a.c0);
+    a.rh = min(kTileH, f.h - a.r0);
+    a.ylo = f.h - a.r0 - a.rh;
+    return a;
+}
+
+__device__ __forceinline__ int line_steps(const float4 l) {
+    return (int)ceilf(fmaxf(fabsf(__fsub_rn(l.z, l.x)), fabsf(__fsub_rn(l.w, l.y))));
+}
+
+__device__ __forceinline__ bool clip_to_tile(const float4 l, const Tile& a, int* k0, int* k1) {
+    return clip_line(l, line_steps(l), (float)a.c0, (float)(a.c0 + a.cw), (float)a.ylo, (float)(a.ylo + a.rh), 2.0f, k0,
+                     k1);
+}
+
+__device__ __forceinline__ bool node_in_tile(float2 p, const Frame& f, const Tile& a, int* cx, int* cy) {
+    *cx = (int)lroundf(to_px(p.x, f.x0, f.sx));
+    *cy = (int)lroundf(to_px(p.y, f.y0, f.sy));
+    return *cx >= a.c0 - 3 && *cx <= a.c0 + a.cw + 2 && *cy >= a.ylo - 3 && *cy <= a.ylo + a.rh + 2;
+}
+
+// Work of tile t (lines, t < tiles; nodes, t - tiles) in samples, from every kCostStride-th line
+// or node: its samples, 8 per line or node that crosses it, and a quarter per one looked at.
+constexpr int kCostStride = 16;
+
+__global__ __launch_bounds__(256) void k_raster_cost(const float4* __restrict__ lines,
+                                                     const unsigned int* __restrict__ nlines,
+                                                     const float2* __restrict__ pos, int n, Frame f, int tiles,
+                                                     int tiles_x, unsigned long long* __restrict__ cost) {
+    __shared__ unsigned long long wsum[4];
+    const int t = blockIdx.x;
+    const bool nodes = t >= tiles;
+    const Tile a = tile_of(nodes ? t - tiles : t, tiles_x, f);
+    const unsigned int total = nodes ? (unsigned int)n : *nlines;
+    unsigned long long c = 0ull;
+    for (unsigned int i = (blockIdx.y * 256u + threadIdx.x) * kCostStride; i < total; i += gridDim.y * 256u * kCostStride) {
+        int k0, k1;
+        if (nodes) c += node_in_tile(pos[i], f, a, &k0, &k1) ? 4u * (29 + 8) : 0u;
+        else if (clip_to_tile(lines[i], a, &k0, &k1)) c += 4u * (unsigned int)(k1 - k0 + 1 + 8);
+        c += 1u;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+    if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(&cost[t], wsum[0] + wsum[1] + wsum[2] + wsum[3]);
+}
+
+// first[t]: the first copy of tile t's slices; every tile gets one slice and a share of the spare
+// ones by its cost. One block.
+__global__ __launch_bounds__(1024) void k_raster_plan(const unsigned long long* __restrict__ cost, int count,
+                                                      int spare, int* __restrict__ first) {
+    __shared__ unsigned long long wcost[16];
+    __shared__ int wsum[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    unsigned long long c = 0ull;
+    for (int t = tid; t < count; t += 1024) c += cost[t];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+    if (lane == 0) wcost[wave] = c;
+    __syncthreads();
+    unsigned long long total = 1ull;
+    for (int w = 0; w < 16; ++w) total += wcost[w];
+    int carry = 0;
+    for (int t0 = 0; t0 < count; t0 += 1024) {
+        const int t = t0 + tid;
+        const int s = t < count ? 1 + (int)((double)cost[t] / (double)total * spare) : 0;
+        int inc = s;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += u;
+        }
+        if (lane == 63) wsum[wave] = inc;
+        __syncthreads();
+        int before = 0, all = 0;
+        for (int w = 0; w < 16; ++w) {
+            if (w < wave) before += wsum[w];
+            all += wsum[w];
+        }
+        if (t < count) first[t] = carry + before + inc - s;
+        carry += all;
+        __syncthreads();
+    }
+    if (tid == 0) first[count] = carry;
+}
+
+// One block per copy: its tile (lines or nodes) and slice, counted in LDS and written to the
+// copy, copies[block][pixel of the tile] (added to for the lines beyond the first list).
+//
+// Bound by vector instructions (issued in 80 % of the time a compute unit has a block): about 45 per
+// sample, 10 of them FP64, with 16 lanes per line, and half as much again to find the lines. With one device atomic per sample the 1M edges of an R-MAT layout (275M samples, 1250 x
+// 1250) took 11.9 ms, 23 samples/ns; with equal slices per tile 1.94 ms, with slices by cost and
+// block-wide batches 1.31 ms, as here 1.02 ms, 270 samples/ns.
+__global__ __launch_bounds__(kTileThreads) void k_raster_tiles(const float4* __restrict__ lines,
+                                                               const unsigned int* __restrict__ nlines,
+                                                               const float2* __restrict__ pos, int n, Frame f,
+                                                               int tiles, int tiles_x, const int* __restrict__ first,
+                                                               unsigned int* __restrict__ copies, int more) {
+    __shared__ unsigned int cnt[kTileH * (kTileW + 1)];
+    __shared__ int3 queues[kTileThreads / 64][kQueueGo + 64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int count_all = 2 * tiles, me = blockIdx.x;
+    if (me >= first[count_all]) return;              // uniform
+    int lo = 0, hi = count_all;                      // first[lo] <= me < first[lo + 1]
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (first[mid] <= me) lo = mid;
+        else hi = mid;
+    }
+    const bool nodes = lo >= tiles;
+    if (nodes && more) return;                       // the nodes went with the first list
+    const int slice = me - first[lo], slices = first[lo + 1] - first[lo];
+    const Tile a = tile_of(nodes ? lo - tiles : lo, tiles_x, f);
+    for (int q = tid; q < kTileH * (kTileW + 1); q += kTileThreads) cnt[q] = 0u;
+    __syncthreads();
+    // a pixel counts if it lies in the tile
+    auto count = [&](int x, int y) {
+        const int cx = x - a.c0, cy = y - a.ylo;
+        if ((unsigned)cx < (unsigned)a.cw && (unsigned)cy < (unsigned)a.rh) {
+            const int row = a.rh - 1 - cy;
+            atomicAdd(&cnt[(row << 8) + row + cx], 1u);
+        }
+    };
+    static_assert(kTileW == 256, "a row of the counters is 257 words");
+    const unsigned int total = nodes ? (unsigned int)n : *nlines;
+    const unsigned int i0 = (unsigned int)((unsigned long long)total * slice / slices);
+    const unsigned int i1 = (unsigned int)((unsigned long long)total * (slice + 1) / slices);
+    // nodes: a wave per disc of radius 3 around the rounded centre
+    const int dx = lane % 7 - 3, dy = lane / 7 - 3;
+    const bool disc = lane < 49 && dx * dx + dy * dy <= 9;
+    // Each wave looks at 64 lines (or nodes) at a time, the next ones loaded meanwhile, and keeps
+    // those that cross the tile in a queue of its own: no barrier until the block is done.
+    int3* queue = queues[wave];
+    int have = 0;                                    // uniform
+    float4 next = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    auto load = [&](unsigned int id) {
+        if (id < i1) {
+            if (nodes) {
+                const float2 p = pos[id];
+                next = make_float4(p.x, p.y, 0.0f, 0.0f);
+            } else {
+                next = lines[id];
+            }
+        }
+    };
+    load(i0 + tid);
+    for (unsigned int at = i0 + 64 * wave; at < i1; at += kTileThreads) {  // uniform per wave
+        const float4 l = next;
+        const unsigned int id = at + lane;
+        load(id + kTileThreads);
+        int k0 = 0, k1 = 0;
+        bool in = false;
+        if (id < i1) in = nodes ? node_in_tile(make_float2(l.x, l.y), f, a, &k0, &k1) : clip_to_tile(l, a, &k0, &k1);
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(in);
+        if (in)
+            queue[have + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] =
+                nodes ? make_int3(k0, k1, 0) : make_int3((int)id, k0, k1);
+        have += __popcll(m);
+        if (have < kQueueGo && at + kTileThreads < i1) continue;
+        wave_lds_sync();
+        if (nodes) {
+            for (int q = 0; q < have; ++q)
+                if (disc) count(queue[q].x + dx, queue[q].y + dy);
+        } else {
+            // 16 lanes per line
+            for (int q = lane >> 4; q < have; q += 4) {
+                const int3 it = queue[q];
+                const float4 g = lines[(unsigned int)it.x];
+                const int steps = line_steps(g);
+                if (steps == 0) {
+                    if ((lane & 15) == 0) count(round_px(g.x), round_px(g.y));
+                    continue;
+                }
+                const double ddx = (double)__fsub_rn(g.z, g.x), ddy = (double)__fsub_rn(g.w, g.y);
+                const double lx = (double)g.x, ly = (double)g.y;
+                const double n_steps = (double)steps, y = __ddiv_rn(1.0, n_steps);
+                for (int k = it.y + (lane & 15); k <= it.z; k += 16) {
+                    const double t = quotient((double)k, n_steps, y);
+                    const float sx = (float)__dadd_rn(lx, __dmul_rn(t, ddx));
+                    const float sy = (float)__dadd_rn(ly, __dmul_rn(t, ddy));
+                    count(round_px(sx), round_px(sy));
+                }
+            }
+        }
+        have = 0;
+        wave_lds_sync();
+    }
+    __syncthreads();
+    unsigned int* out = copies + (size_t)me * kTilePixels;
+    for (int q = tid; q < a.rh * kTileW; q += kTileThreads) {
+        const unsigned int v = cnt[q / kTileW * (kTileW + 1) + q % kTileW];
+        out[q] = more ? out[q] + v : v;
+    }
+}
+
 __device__ __forceinline__ float powi(float b, unsigned int k) {
     float r = 1.0f;
     while (k) {
@@ -136,13 +509,35 @@ __device__ __forceinline__ float powi(float b, unsigned int k) {
     return r;
 }
 
+__device__ __forceinline__ unsigned char brightness(float keep_n, unsigned int nodes, float keep_e,
+                                                    unsigned int edges) {
+    const float keep = __fmul_rn(powi(keep_n, nodes), powi(keep_e, edges));
+    return (unsigned char)lroundf(__fmul_rn(255.0f, keep));
+}
+
 __global__ __launch_bounds__(256) void k_shade(const unsigned int* __restrict__ cn, const unsigned int* __restrict__ ce,
                                                long long npix, float keep_n, float keep_e,
                                                unsigned char* __restrict__ out) {
-    for (long long p = blockIdx.x * 256ll + threadIdx.x; p < npix; p += (long long)gridDim.x * 256) {
-        const float keep = __fmul_rn(powi(keep_n, cn[p]), powi(keep_e, ce[p]));
-        out[p] = (unsigned char)lroundf(__fmul_rn(255.0f, keep));
-    }
+    for (long long p = blockIdx.x * 256ll + threadIdx.x; p < npix; p += (long long)gridDim.x * 256)
+        out[p] = brightness(keep_n, cn[p], keep_e, ce[p]);
+}
+
+// The same from the tiles' copies and the far-out lines' counters; a block per row of a tile.
+__global__ __launch_bounds__(kTileW) void k_shade_tiles(const unsigned int* __restrict__ copies,
+                                                        const int* __restrict__ first, int tiles, int tiles_x,
+                                                        const unsigned int* __restrict__ far, Frame f, float keep_n,
+                                                        float keep_e, unsigned char* __restrict__ out) {
+    const int t = blockIdx.x / kTileH, row = blockIdx.x % kTileH;
+    const Tile a = tile_of(t, tiles_x, f);
+    if (row >= a.rh || (int)threadIdx.x >= a.cw) return;
+    const size_t p = (size_t)(a.r0 + row) * f.w + a.c0 + threadIdx.x;
+    const unsigned int* c = copies + (size_t)row * kTileW + threadIdx.x;
+    unsigned int edges = far[p], nodes = 0u;
+    const int e1 = first[t + 1], n1 = first[tiles + t + 1];
+#pragma unroll 8
+    for (int k = first[t]; k < e1; ++k) edges += c[(size_t)k * kTilePixels];
+    for (int k = first[tiles + t]; k < n1; ++k) nodes += c[(size_t)k * kTilePixels];
+    out[p] = brightness(keep_n, nodes, keep_e, edges);
 }
 
 }  // namespace
@@ -160,15 +555,15 @@ int gfa2_get_bbox(gfa2_handle h, float* out) {
     if (!engine_graph(h, &b, &device, &s)) return GFA2_ERR_NO_GRAPH;
     if (hipSetDevice(device) != hipSuccess) return GFA2_ERR_HIP;
     const int nb = 256;
-    float4* part = nullptr;
-    if (hipMalloc(&part, sizeof(float4) * (nb + 1)) != hipSuccess) return GFA2_ERR_OOM;
+    EngineScratch scratch(h);
+    float4* part = static_cast<float4*>(scratch.get(sizeof(float4) * (nb + 1)));
+    if (!part) return GFA2_ERR_OOM;
     k_minmax<<<nb, 256, 0, s>>>(b->pos, b->n, part);
     k_minmax_final<<<1, 64, 0, s>>>(part, nb, part + nb);
     float4 m;
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(&m, part + nb, sizeof(float4), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(part);
     if (e != hipSuccess) return GFA2_ERR_HIP;
     out[0] = m.x;
     out[1] = m.y;
@@ -186,29 +581,58 @@ int gfa2_render(gfa2_handle h, const gfa2_raster* r, uint8_t* gray) {
     if (b->nseg > 1) return GFA2_ERR_UNSUPPORTED;
     if (hipSetDevice(device) != hipSuccess) return GFA2_ERR_HIP;
     const long long npix = (long long)r->width * r->height;
-    unsigned int* cnt = nullptr;
-    unsigned char* img = nullptr;
-    if (hipMalloc(&cnt, sizeof(unsigned int) * 2 * (size_t)npix) != hipSuccess) return GFA2_ERR_OOM;
-    if (hipMalloc(&img, (size_t)npix) != hipSuccess) {
-        (void)hipFree(cnt);
-        return GFA2_ERR_OOM;
-    }
     const Frame f{r->x0, r->y0, r->sx, r->sy, r->width, r->height};
-    hipError_t e = hipMemsetAsync(cnt, 0, sizeof(unsigned int) * 2 * (size_t)npix, s);
+    const int tiles_x = (f.w + kTileW - 1) / kTileW, tiles_y = (f.h + kTileH - 1) / kTileH;
+    const int tiles = tiles_x * tiles_y;
+    const int copies = 2 * tiles + kSpareSlices;
+    const long long lists = std::max<long long>(1, (b->nnz + kListEntries - 1) / kListEntries);
+    const size_t list = (size_t)std::min<long long>(b->nnz, kListEntries);
+    // the scratch: line list, line count, tile costs, far-out lines' counters, plan, copies, picture
+    size_t size = 0;
+    auto place = [&](size_t bytes) {
+        const size_t at = size;
+        size += (bytes + 255) & ~(size_t)255;
+        return at;
+    };
+    const size_t at_lines = place(sizeof(float4) * list), at_count = place(sizeof(unsigned int));
+    const size_t at_cost = place(sizeof(unsigned long long) * 2 * (size_t)tiles);
+    const size_t at_far = place(sizeof(unsigned int) * (size_t)npix);
+    const size_t at_first = place(sizeof(int) * (2 * (size_t)tiles + 1));
+    const size_t at_copies = place(sizeof(unsigned int) * kTilePixels * (size_t)copies), at_img = place((size_t)npix);
+    EngineScratch scratch(h);
+    char* mem = static_cast<char*>(scratch.get(size));
+    if (!mem) return GFA2_ERR_OOM;
+    float4* lines = reinterpret_cast<float4*>(mem + at_lines);
+    unsigned int* nlines = reinterpret_cast<unsigned int*>(mem + at_count);
+    unsigned long long* cost = reinterpret_cast<unsigned long long*>(mem + at_cost);
+    unsigned int* far = reinterpret_cast<unsigned int*>(mem + at_far);
+    int* first = reinterpret_cast<int*>(mem + at_first);
+    unsigned int* copy = reinterpret_cast<unsigned int*>(mem + at_copies);
+    unsigned char* img = reinterpret_cast<unsigned char*>(mem + at_img);
+    hipError_t e = hipMemsetAsync(nlines, 0, at_first - at_count, s);      // count, costs and counters
+    for (long long q = 0; q < lists && e == hipSuccess; ++q) {
+        const long long e0 = q * kListEntries, e1 = std::min<long long>(b->nnz, e0 + kListEntries);
+        if (q > 0) e = hipMemsetAsync(nlines, 0, sizeof(unsigned int), s);
+        constexpr long long kPer = kLineThreads * kLineItems;
+        if (e1 > e0)
+            k_raster_lines<<<(int)((e1 - e0 + kPer - 1) / kPer), kLineThreads, 0, s>>>(b->pos, b->rowptr, b->col, b->n, e0,
+                                                                                     e1, f, lines, nlines, far);
+        if (q == 0) {
+            // the plan of the first list serves the others
+            const long long most = std::max<long long>(b->n, (long long)list) / (256 * kCostStride) + 1;
+            k_raster_cost<<<dim3(2 * tiles, (int)std::min<long long>(most, 8)), 256, 0, s>>>(lines, nlines, b->pos, b->n,
+                                                                                           f, tiles, tiles_x, cost);
+            k_raster_plan<<<1, 1024, 0, s>>>(cost, 2 * tiles, kSpareSlices, first);
+        }
+        k_raster_tiles<<<copies, kTileThreads, 0, s>>>(lines, nlines, b->pos, b->n, f, tiles, tiles_x, first, copy, q > 0);
+    }
     if (e == hipSuccess) {
-        k_raster_nodes<<<(b->n + 255) / 256, 256, 0, s>>>(b->pos, b->n, f, cnt);
-        long long eb = (b->nnz + 255) / 256;
-        if (eb > 8192) eb = 8192;
-        if (eb > 0) k_raster_edges<<<(int)eb, 256, 0, s>>>(b->pos, b->rowptr, b->col, b->n, b->nnz, f, cnt + npix);
-        long long pb = (npix + 255) / 256;
-        if (pb > 8192) pb = 8192;
-        k_shade<<<(int)pb, 256, 0, s>>>(cnt, cnt + npix, npix, 1.0f - r->node_alpha, 1.0f - r->edge_alpha, img);
+        k_shade_tiles<<<tiles * kTileH, kTileW, 0, s>>>(copy, first, tiles, tiles_x, far, f, 1.0f - r->node_alpha,
+                                                        1.0f - r->edge_alpha, img);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(gray, img, (size_t)npix, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(cnt);
-    (void)hipFree(img);
     return e == hipSuccess ? GFA2_OK : GFA2_ERR_HIP;
 }
 
