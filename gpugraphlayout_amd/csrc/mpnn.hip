@@ -24,6 +24,12 @@
 //
 // Every reduction over nodes (weight gradients, column statistics, loss) writes per-block
 // partials that a second kernel sums in a fixed order.
+//
+// Dense products run on the FP32 matrix instructions (v_mfma_f32_16x16x4_f32: 16 x 16 results, 4
+// inner terms, FP32 throughout), which do twice the FP32 work per cycle of a vector FMA. A lane
+// of the instruction holds A[i = lane % 16][k = lane / 16], B[k = lane / 16][j = lane % 16] and
+// four results C[i = 4 (lane / 16) + r][j = lane % 16]; which inner index a (step, lane / 16)
+// slot stands for is free as long as A and B agree.
 #include "engine_internal.h"
 #include "mpnn_internal.h"
 
@@ -120,37 +126,31 @@ __global__ __launch_bounds__(256) void k_colnorm_apply(float* __restrict__ X, in
 
 // ---- neighbour aggregation -----------------------------------------------------------------
 
-// out[i][:] = epilogue(sum over CSR neighbours j of in[j][:], times 1/deg(j) for the transposed
-// form), F features per node (8, 16 or 64):
+// out[i][:] = epilogue(sum over CSR neighbours j of in[j][:]), F features per node (8, 16 or 64):
 //   kAggMean       out = sum / deg(i) (0 for an isolated node)     forward mean
 //   kAggSmooth     out = (in[i] + sum / deg(i)) / 2                 feature smoothing
-//   kAggTranspose  out = sum of in[j] / deg(j)                      backward of the mean
+//   kAggBack       out = H[i] > 0 ? P[i] + sum : 0                  backward of the mean and relu
+//                  (in[j] already divided by deg(j))
 // Rows of at most kHeavyDeg entries: F lanes per row, entries in CSR order (four loads in
 // flight). Longer rows (the hubs of a skewed graph, which would otherwise leave one wave
 // looping over 10^5 entries) are split into chunks of kChunk entries: one wave per chunk sums
 // its entries in 64/F interleaved slots, combined in slot order, into a partial; then one
 // thread per (row, feature) adds the row's partials in chunk order. Every sum has a fixed
 // order, so results are deterministic.
-enum AggMode { kAggMean = 0, kAggSmooth = 1, kAggTranspose = 2 };
+enum AggMode { kAggMean = 0, kAggSmooth = 1, kAggBack = 2 };
 
 template <int MODE>
-__device__ __forceinline__ float agg_add(float s, const int* __restrict__ rowptr, const float* __restrict__ in,
-                                         int j, int F, int f) {
-    const float v = in[(size_t)j * F + f];
-    if (MODE == kAggTranspose) return fmaf(v, 1.0f / (float)(rowptr[j + 1] - rowptr[j]), s);
-    return s + v;
-}
-
-template <int MODE>
-__device__ __forceinline__ float agg_finish(float s, int deg, float self) {
-    if (MODE == kAggTranspose) return s;
+__device__ __forceinline__ float agg_finish(float s, int deg, size_t at, const float* __restrict__ in,
+                                            const float* __restrict__ P, const float* __restrict__ H) {
+    if (MODE == kAggBack) return H[at] > 0.0f ? P[at] + s : 0.0f;
     const float m = deg > 0 ? s / (float)deg : 0.0f;
-    return MODE == kAggSmooth ? 0.5f * (self + m) : m;
+    return MODE == kAggSmooth ? 0.5f * (in[at] + m) : m;
 }
 
 template <int F, int MODE>
 __global__ __launch_bounds__(256) void k_agg_rows(const int* __restrict__ rowptr, const int* __restrict__ col, int n,
-                                                  const float* __restrict__ in, float* __restrict__ out) {
+                                                  const float* __restrict__ in, const float* __restrict__ P,
+                                                  const float* __restrict__ H, float* __restrict__ out) {
     constexpr int kRows = 256 / F;
     const int f = threadIdx.x % F;
     for (long long r0 = (long long)blockIdx.x * kRows; r0 < n; r0 += (long long)gridDim.x * kRows) {
@@ -163,18 +163,19 @@ __global__ __launch_bounds__(256) void k_agg_rows(const int* __restrict__ rowptr
         int e = e0;
         for (; e + 4 <= e1; e += 4) {
             const int j0 = col[e], j1 = col[e + 1], j2 = col[e + 2], j3 = col[e + 3];
-            s = agg_add<MODE>(s, rowptr, in, j0, F, f);
-            s = agg_add<MODE>(s, rowptr, in, j1, F, f);
-            s = agg_add<MODE>(s, rowptr, in, j2, F, f);
-            s = agg_add<MODE>(s, rowptr, in, j3, F, f);
+            s += in[(size_t)j0 * F + f];
+            s += in[(size_t)j1 * F + f];
+            s += in[(size_t)j2 * F + f];
+            s += in[(size_t)j3 * F + f];
         }
-        for (; e < e1; ++e) s = agg_add<MODE>(s, rowptr, in, col[e], F, f);
-        out[(size_t)i * F + f] = agg_finish<MODE>(s, e1 - e0, MODE == kAggSmooth ? in[(size_t)i * F + f] : 0.0f);
+        for (; e < e1; ++e) s += in[(size_t)col[e] * F + f];
+        const size_t at = (size_t)i * F + f;
+        out[at] = agg_finish<MODE>(s, e1 - e0, at, in, P, H);
     }
 }
 
 // One wave per chunk {row, first entry}; part[c][f] = the chunk's sum.
-template <int F, int MODE>
+template <int F>
 __global__ __launch_bounds__(256) void k_agg_chunks(const int* __restrict__ rowptr, const int* __restrict__ col,
                                                     const int2* __restrict__ chunks, int nchunks,
                                                     const float* __restrict__ in, float* __restrict__ part) {
@@ -187,12 +188,12 @@ __global__ __launch_bounds__(256) void k_agg_chunks(const int* __restrict__ rowp
         int e = ch.y + slot;
         for (; e + 3 * S < end; e += 4 * S) {
             const int j0 = col[e], j1 = col[e + S], j2 = col[e + 2 * S], j3 = col[e + 3 * S];
-            s = agg_add<MODE>(s, rowptr, in, j0, F, f);
-            s = agg_add<MODE>(s, rowptr, in, j1, F, f);
-            s = agg_add<MODE>(s, rowptr, in, j2, F, f);
-            s = agg_add<MODE>(s, rowptr, in, j3, F, f);
+            s += in[(size_t)j0 * F + f];
+            s += in[(size_t)j1 * F + f];
+            s += in[(size_t)j2 * F + f];
+            s += in[(size_t)j3 * F + f];
         }
-        for (; e < end; e += S) s = agg_add<MODE>(s, rowptr, in, col[e], F, f);
+        for (; e < end; e += S) s += in[(size_t)col[e] * F + f];
         float tot = 0.0f;
 #pragma unroll
         for (int q = 0; q < S; ++q) tot += __shfl(s, q * F + f, 64);
@@ -205,6 +206,7 @@ template <int F, int MODE>
 __global__ __launch_bounds__(256) void k_agg_heavy(const int* __restrict__ rowptr, const int* __restrict__ heavy_row,
                                                    const int* __restrict__ heavy_c0, int nheavy,
                                                    const float* __restrict__ in, const float* __restrict__ part,
+                                                   const float* __restrict__ P, const float* __restrict__ H,
                                                    float* __restrict__ out) {
     const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
     if (t >= (long long)nheavy * F) return;
@@ -212,137 +214,167 @@ __global__ __launch_bounds__(256) void k_agg_heavy(const int* __restrict__ rowpt
     const int i = heavy_row[h];
     float s = 0.0f;
     for (int c = heavy_c0[h]; c < heavy_c0[h + 1]; ++c) s += part[(size_t)c * F + f];
-    out[(size_t)i * F + f] = agg_finish<MODE>(s, rowptr[i + 1] - rowptr[i],
-                                              MODE == kAggSmooth ? in[(size_t)i * F + f] : 0.0f);
+    const size_t at = (size_t)i * F + f;
+    out[at] = agg_finish<MODE>(s, rowptr[i + 1] - rowptr[i], at, in, P, H);
 }
 
-// H[i][o] = relu(b[o] + sum_k (A[i][k] Ws[k][o] + B[i][k] Wn[k][o])), accumulated in the
-// order b, A_0 Ws_0, B_0 Wn_0, A_1 Ws_1, ... (FMAs). Register-tiled: a block holds the BF16
-// weights as FP32 in LDS and walks tiles of 64 nodes, staging A and B transposed in LDS; each
-// thread owns 4 nodes x 4 outputs (16 accumulators), so one k step is 4 LDS reads of 16 bytes
-// for 32 FMAs.
-template <int K>
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+
+__device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// The weights are read from LDS for every tile: held in registers across tiles (the compiler's own
+// choice, 242 of them) they leave one wave per SIMD.
+__device__ __forceinline__ void keep_in_lds() { asm volatile("" ::: "memory"); }
+
+__device__ __forceinline__ float at4(const float4& v, int m) { return m == 0 ? v.x : m == 1 ? v.y : m == 2 ? v.z : v.w; }
+
+// H[i][o] = relu(b[o] + sum_k (A[i][k] Ws[k][o] + B[i][k] Wn[k][o])) and, with HEAD, Y = H Wo + bo
+// as well (H is then written only if asked for: inference needs none of it). A wave takes 16 nodes
+// and all 64 outputs: four result tiles with i = output and j = node, so that a lane ends up with 4
+// consecutive outputs of one node and node data goes from memory straight into the instruction's
+// operand (four inner indices per 16-byte load, slot (m, lane / 16) standing for 4 (lane / 16) + m).
+// The weights, FP32 from BF16, lie in LDS in operand order.
+//
+// Bound by memory for K = 16 (580,000 nodes read 74 MB and write 148: 50 us, 4.4 TB/s, as the
+// vector kernel before) and by the matrix instructions for K = 64 (9.5 GFLOP and 302 MB in 106 us;
+// register-tiled vector FMAs took 194 us and a head launch 33 more).
+template <int K, bool HEAD>
 __global__ __launch_bounds__(256) void k_dense(const float* __restrict__ A, const float* __restrict__ B, int n,
                                                const unsigned short* __restrict__ Ws,
                                                const unsigned short* __restrict__ Wn,
-                                               const unsigned short* __restrict__ bias, float* __restrict__ H) {
-    __shared__ float4 ws[K * kHid / 4], wn[K * kHid / 4];     // [k][o/4]
-    __shared__ float4 ta[K * 16], tb[K * 16];                 // [k][node/4], 64 nodes
-    for (int q = threadIdx.x; q < K * kHid; q += 256) {
-        reinterpret_cast<float*>(ws)[q] = bf16_to_f32(Ws[q]);
-        reinterpret_cast<float*>(wn)[q] = bf16_to_f32(Wn[q]);
-    }
-    const int oq = threadIdx.x & 15, rq = threadIdx.x >> 4;   // outputs 4*oq.., nodes 4*rq..
-    const float4 bo = make_float4(bf16_to_f32(bias[4 * oq]), bf16_to_f32(bias[4 * oq + 1]),
-                                  bf16_to_f32(bias[4 * oq + 2]), bf16_to_f32(bias[4 * oq + 3]));
-    const int tiles = (n + 63) / 64;
-    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const long long i0 = (long long)tile * 64;
-        __syncthreads();                                      // weights written / last tile read
-        for (int q = threadIdx.x; q < 64 * (K / 4); q += 256) {
-            const int r = q & 63, k4 = q >> 6;                // node r, features 4*k4..
-            float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
-            if (i0 + r < n) {
-                a = reinterpret_cast<const float4*>(A + (i0 + r) * K)[k4];
-                b = reinterpret_cast<const float4*>(B + (i0 + r) * K)[k4];
-            }
-            float* fa = reinterpret_cast<float*>(ta);
-            float* fb = reinterpret_cast<float*>(tb);
-            fa[(4 * k4 + 0) * 64 + r] = a.x;
-            fa[(4 * k4 + 1) * 64 + r] = a.y;
-            fa[(4 * k4 + 2) * 64 + r] = a.z;
-            fa[(4 * k4 + 3) * 64 + r] = a.w;
-            fb[(4 * k4 + 0) * 64 + r] = b.x;
-            fb[(4 * k4 + 1) * 64 + r] = b.y;
-            fb[(4 * k4 + 2) * 64 + r] = b.z;
-            fb[(4 * k4 + 3) * 64 + r] = b.w;
-        }
-        __syncthreads();
-        float z[4][4];
+                                               const unsigned short* __restrict__ bias, float* __restrict__ H,
+                                               const unsigned short* __restrict__ Wo,
+                                               const unsigned short* __restrict__ bo, float2* __restrict__ Y) {
+    constexpr int S = K / 16;                                 // 16-index steps per input
+    __shared__ float4 w[4][2 * S][64];                        // [output tile][step][lane]
+    __shared__ float2 wo[kHid];
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    const int tiles = (n + 15) / 16, stride = gridDim.x * 4;
+    float4 nx[2 * S];                                         // the next tile's inputs, loaded meanwhile
+    auto load = [&](int tile) {
+        const size_t row = (size_t)min(tile * 16 + j, n - 1) * K;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            z[r][0] = bo.x;
-            z[r][1] = bo.y;
-            z[r][2] = bo.z;
-            z[r][3] = bo.w;
+        for (int q = 0; q < S; ++q) {
+            nx[q] = *reinterpret_cast<const float4*>(A + row + 16 * q + 4 * g);
+            nx[S + q] = *reinterpret_cast<const float4*>(B + row + 16 * q + 4 * g);
         }
-#pragma unroll 4
-        for (int k = 0; k < K; ++k) {
-            const float4 a = ta[k * 16 + rq], b = tb[k * 16 + rq];
-            const float4 u = ws[k * 16 + oq], v = wn[k * 16 + oq];
-            const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+    };
+    const int tile0 = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (tile0 < tiles) load(tile0);
+#pragma unroll
+    for (int q0 = 0; q0 < 2 * K * (kHid / 4); q0 += 256) {
+        const int q = q0 + threadIdx.x;
+        const int k = q >> 4, o = 4 * (q & 15);               // inner index, first of four outputs
+        const ushort4 u = *reinterpret_cast<const ushort4*>((k < K ? Ws + k * kHid : Wn + (k - K) * kHid) + o);
+        float* at = reinterpret_cast<float*>(&w[o >> 4][k >> 4][16 * ((k >> 2) & 3) + (o & 15)]) + (k & 3);
+        at[0] = bf16_to_f32(u.x);
+        at[4] = bf16_to_f32(u.y);
+        at[8] = bf16_to_f32(u.z);
+        at[12] = bf16_to_f32(u.w);
+    }
+    if (HEAD && threadIdx.x < kHid)
+        wo[threadIdx.x] = make_float2(bf16_to_f32(Wo[2 * threadIdx.x]), bf16_to_f32(Wo[2 * threadIdx.x + 1]));
+    __syncthreads();
+    f32x4 b0[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) b0[t][r] = bf16_to_f32(bias[16 * t + 4 * g + r]);
+    const float y0 = HEAD ? bf16_to_f32(bo[0]) : 0.0f, y1 = HEAD ? bf16_to_f32(bo[1]) : 0.0f;
+    for (int tile = tile0; tile < tiles; tile += stride) {
+        const int i = tile * 16 + j;
+        float4 x[2 * S];
+#pragma unroll
+        for (int q = 0; q < 2 * S; ++q) x[q] = nx[q];
+        if (tile + stride < tiles) load(tile + stride);
+        keep_in_lds();
+        f32x4 acc[4] = {b0[0], b0[1], b0[2], b0[3]};
+#pragma unroll
+        for (int q = 0; q < 2 * S; ++q) {
+            float4 u[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) u[t] = w[t][q][lane];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) acc[t] = mfma(at4(u[t], m), at4(x[q], m), acc[t]);
+        }
+        float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                z[r][0] = fmaf(bv[r], v.x, fmaf(av[r], u.x, z[r][0]));
-                z[r][1] = fmaf(bv[r], v.y, fmaf(av[r], u.y, z[r][1]));
-                z[r][2] = fmaf(bv[r], v.z, fmaf(av[r], u.z, z[r][2]));
-                z[r][3] = fmaf(bv[r], v.w, fmaf(av[r], u.w, z[r][3]));
+                acc[t][r] = fmaxf(acc[t][r], 0.0f);
+                if (HEAD) {
+                    const float2 u = wo[16 * t + 4 * g + r];
+                    s0 = fmaf(acc[t][r], u.x, s0);
+                    s1 = fmaf(acc[t][r], u.y, s1);
+                }
             }
+            if (i < n && H)
+                *reinterpret_cast<float4*>(H + (size_t)i * kHid + 16 * t + 4 * g) =
+                    make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
         }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const long long i = i0 + 4 * rq + r;
-            if (i < n)
-                reinterpret_cast<float4*>(H + i * kHid)[oq] =
-                    make_float4(fmaxf(z[r][0], 0.f), fmaxf(z[r][1], 0.f), fmaxf(z[r][2], 0.f), fmaxf(z[r][3], 0.f));
+        if (HEAD) {
+            // the node's four lanes hold a quarter of the outputs each
+            s0 += __shfl_xor(s0, 16, 64);
+            s1 += __shfl_xor(s1, 16, 64);
+            s0 += __shfl_xor(s0, 32, 64);
+            s1 += __shfl_xor(s1, 32, 64);
+            if (g == 0 && i < n) Y[i] = make_float2(s0 + y0, s1 + y1);
         }
     }
-}
-
-// Y[i][c] = sum_k H[i][k] Wo[k][c] + bo[c]; thread per node.
-__global__ __launch_bounds__(256) void k_head(const float* __restrict__ H, int n, const unsigned short* __restrict__ Wo,
-                                              const unsigned short* __restrict__ bo, float* __restrict__ Y) {
-    __shared__ float w[kHid * 2];
-    if (threadIdx.x < kHid * 2) w[threadIdx.x] = bf16_to_f32(Wo[threadIdx.x]);
-    __syncthreads();
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    float y0 = bf16_to_f32(bo[0]), y1 = bf16_to_f32(bo[1]);
-    for (int k = 0; k < kHid; ++k) {
-        const float h = H[i * kHid + k];
-        y0 = fmaf(h, w[2 * k], y0);
-        y1 = fmaf(h, w[2 * k + 1], y1);
-    }
-    Y[2 * i] = y0;
-    Y[2 * i + 1] = y1;
 }
 
 // ---- loss ----------------------------------------------------------------------------------
 
-// Per node: loss terms over P(i) and dY[i]; per-block loss partials.
+// Per node: loss terms over P(i) and dY[i]; per-block loss partials. Eight lanes per node take
+// its pairs in turn and add up in a fixed tree.
 __global__ __launch_bounds__(256) void k_loss(const int* __restrict__ rowptr, const int* __restrict__ col, int n,
-                                              const float* __restrict__ Y, const float* __restrict__ T,
+                                              const float2* __restrict__ Y, const float2* __restrict__ T,
                                               const int* __restrict__ offs, int R, double inv_pairs,
-                                              float* __restrict__ dY, double* __restrict__ part) {
+                                              float2* __restrict__ dY, double* __restrict__ part) {
     __shared__ double red[256];
-    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int lane8 = threadIdx.x & 7;
+    const float c = (float)(4.0 * inv_pairs);
     double l = 0.0;
-    if (i < n) {
-        const float yx = Y[2 * i], yy = Y[2 * i + 1], tx = T[2 * i], ty = T[2 * i + 1];
+    for (long long i0 = blockIdx.x * 32ll; i0 < n; i0 += gridDim.x * 32ll) {
+        const long long ii = i0 + (threadIdx.x >> 3);
         float gx = 0.0f, gy = 0.0f;
-        const int e0 = rowptr[i], e1 = rowptr[i + 1];
-        const int cnt = (e1 - e0) + 2 * R;
-        for (int q = 0; q < cnt; ++q) {
-            int j;
-            if (q < e1 - e0) j = col[e0 + q];
-            else {
-                const int k = q - (e1 - e0);
-                const int o = offs[k >> 1];
-                j = (k & 1) ? (int)(((long long)i + n - o) % n) : (int)(((long long)i + o) % n);
+        if (ii < n) {
+            const int i = (int)ii;
+            const float2 y = Y[i], t = T[i];
+            const int e0 = rowptr[i], deg = rowptr[i + 1] - e0;
+            const int cnt = deg + 2 * R;
+#pragma unroll 2
+            for (int q = lane8; q < cnt; q += 8) {
+                int j;
+                if (q < deg) j = col[e0 + q];
+                else {
+                    // offsets are below n
+                    const int k = q - deg;
+                    const int o = (k & 1) ? n - offs[k >> 1] : offs[k >> 1];
+                    j = i < n - o ? i + o : i - (n - o);
+                }
+                const float2 yj = Y[j], tj = T[j];
+                const float dx = y.x - yj.x, dy = y.y - yj.y;
+                const float ex = t.x - tj.x, ey = t.y - tj.y;
+                const float d = sqrtf(dx * dx + dy * dy) + 1e-12f;
+                const float r = d - sqrtf(ex * ex + ey * ey);
+                l += (double)r * r;
+                const float s = r / d;
+                gx = fmaf(s, dx, gx);
+                gy = fmaf(s, dy, gy);
             }
-            const float dx = yx - Y[2 * j], dy = yy - Y[2 * j + 1];
-            const float ex = tx - T[2 * j], ey = ty - T[2 * j + 1];
-            const float d = sqrtf(dx * dx + dy * dy) + 1e-12f;
-            const float t = sqrtf(ex * ex + ey * ey);
-            const float r = d - t;
-            l += (double)r * r;
-            const float s = r / d;
-            gx = fmaf(s, dx, gx);
-            gy = fmaf(s, dy, gy);
         }
-        const float c = (float)(4.0 * inv_pairs);
-        dY[2 * i] = c * gx;
-        dY[2 * i + 1] = c * gy;
+#pragma unroll
+        for (int o = 4; o > 0; o >>= 1) {
+            gx += __shfl_xor(gx, o, 64);
+            gy += __shfl_xor(gy, o, 64);
+        }
+        if (lane8 == 0 && ii < n) dY[ii] = make_float2(c * gx, c * gy);
     }
     red[threadIdx.x] = l;
     __syncthreads();
@@ -355,90 +387,258 @@ __global__ __launch_bounds__(256) void k_loss(const int* __restrict__ rowptr, co
 
 // ---- backward ------------------------------------------------------------------------------
 
-// dH2[i][k] = sum_c dY[i][c] Wo[k][c], masked by H2 > 0 (relu): thread per (i, k).
-__global__ __launch_bounds__(256) void k_head_back(const float* __restrict__ dY, const float* __restrict__ H2, int n,
-                                                   const unsigned short* __restrict__ Wo, float* __restrict__ dZ2) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= n * kHid) return;
-    const int i = t / kHid, k = t % kHid;
-    const float g = fmaf(dY[2 * i], bf16_to_f32(Wo[2 * k]), dY[2 * i + 1] * bf16_to_f32(Wo[2 * k + 1]));
-    dZ2[t] = H2[t] > 0.0f ? g : 0.0f;
+// dZ2[i][o] = H2[i][o] > 0 ? sum_c dY[i][c] Wo[o][c] : 0, formed wherever it is needed.
+__device__ __forceinline__ float d_z2(float h, float2 dy, float2 wo) {
+    return h > 0.0f ? fmaf(dy.x, wo.x, dy.y * wo.y) : 0.0f;
 }
 
-// D2[i][k] = sum_o D[i][o] W[k][o] (dense input gradient, K = 64), one wave per node.
-__global__ __launch_bounds__(256) void k_dense_back_x(const float* __restrict__ D, int n,
-                                                      const unsigned short* __restrict__ W, float* __restrict__ out) {
-    __shared__ float w[kHid * kHid];
-    for (int k = threadIdx.x; k < kHid * kHid; k += 256) w[k] = bf16_to_f32(W[k]);
+// P[i][k] = sum_o dZ2[i][o] W2s[k][o], Q[i][k] = sum_o dZ2[i][o] W2n[k][o] / deg(i): both input
+// gradients of the second layer in one pass over H2 and dY, laid out as k_dense (four result
+// tiles each, i = input, j = node).
+//
+// Bound by memory (H2 read, P and Q written): one wave per node with shuffled inputs took 124 us
+// for each of the two products on 50,000 nodes, after a launch that wrote dZ2; both take 19 us here.
+__global__ __launch_bounds__(256) void k_back(const float2* __restrict__ dY, const float* __restrict__ H2, int n,
+                                              const int* __restrict__ rowptr, const unsigned short* __restrict__ Wo,
+                                              const unsigned short* __restrict__ W2s,
+                                              const unsigned short* __restrict__ W2n, float* __restrict__ P,
+                                              float* __restrict__ Q) {
+    __shared__ float4 w[8][4][64];                            // [P's tiles, Q's tiles][step][lane]
+    __shared__ float2 wo[kHid];
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    const int tiles = (n + 15) / 16, stride = gridDim.x * 4;
+    float4 nx[4];                                             // the next tile's inputs, loaded meanwhile
+    float2 ndy = make_float2(0.0f, 0.0f);
+    int ndeg = 0;
+    auto load = [&](int tile) {
+        const int ic = min(tile * 16 + j, n - 1);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) nx[q] = *reinterpret_cast<const float4*>(H2 + (size_t)ic * kHid + 16 * q + 4 * g);
+        ndy = dY[ic];
+        ndeg = rowptr[ic + 1] - rowptr[ic];
+    };
+    const int tile0 = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (tile0 < tiles) load(tile0);
+#pragma unroll
+    for (int q0 = 0; q0 < 2 * kHid * (kHid / 4); q0 += 256) {
+        const int q = q0 + threadIdx.x;
+        const int k = (q >> 4) & 63, o = 4 * (q & 15), n2 = q >> 10;      // row, first of four inner indices, matrix
+        const ushort4 u = *reinterpret_cast<const ushort4*>((n2 ? W2n : W2s) + k * kHid + o);
+        w[4 * n2 + (k >> 4)][o >> 4][16 * ((o >> 2) & 3) + (k & 15)] =
+            make_float4(bf16_to_f32(u.x), bf16_to_f32(u.y), bf16_to_f32(u.z), bf16_to_f32(u.w));
+    }
+    if (threadIdx.x < kHid)
+        wo[threadIdx.x] = make_float2(bf16_to_f32(Wo[2 * threadIdx.x]), bf16_to_f32(Wo[2 * threadIdx.x + 1]));
     __syncthreads();
-    const int lane = threadIdx.x & 63;
-    for (int i = blockIdx.x * 4 + (threadIdx.x >> 6); i < n; i += gridDim.x * 4) {
-        const float d = D[i * kHid + lane];
-        float s = 0.0f;
-#pragma unroll 16
-        for (int o = 0; o < kHid; ++o) s = fmaf(__shfl(d, o, 64), w[lane * kHid + o], s);
-        out[i * kHid + lane] = s;
-    }
-}
-
-// dH1 = P + Q masked by H1 > 0.
-__global__ __launch_bounds__(256) void k_add_mask(const float* __restrict__ P, const float* __restrict__ Q,
-                                                  const float* __restrict__ H, int total, float* __restrict__ out) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= total) return;
-    out[t] = H[t] > 0.0f ? P[t] + Q[t] : 0.0f;
-}
-
-// Weight-gradient partials: for a chunk of 64 nodes, G[k][o] = sum_i A[i][k] D[i][o]
-// (A: K columns; column K stands for the bias, A = 1). Thread per (k, o) pairs.
-template <int K>
-__global__ __launch_bounds__(256) void k_wgrad(const float* __restrict__ A, const float* __restrict__ D, int n,
-                                               float* __restrict__ part) {
-    __shared__ float sa[64 * K];
-    __shared__ float sd[64 * kHid];
-    const int i0 = blockIdx.x * 64;
-    for (int t = threadIdx.x; t < 64 * K; t += 256) {
-        const int i = i0 + t / K;
-        sa[t] = i < n ? A[i * K + t % K] : 0.0f;
-    }
-    for (int t = threadIdx.x; t < 64 * kHid; t += 256) {
-        const int i = i0 + t / kHid;
-        sd[t] = i < n ? D[i * kHid + t % kHid] : 0.0f;
-    }
-    __syncthreads();
-    float* out = part + (size_t)blockIdx.x * (K + 1) * kHid;
-    for (int t = threadIdx.x; t < (K + 1) * kHid; t += 256) {
-        const int k = t / kHid, o = t % kHid;
-        float s = 0.0f;
-        for (int r = 0; r < 64; ++r) s = fmaf(k < K ? sa[r * K + k] : 1.0f, sd[r * kHid + o], s);
-        out[t] = s;
-    }
-}
-
-// Head gradient partials: chunk of 64 nodes, G[k][c] = sum_i H2[i][k] dY[i][c], k = 64 -> bias.
-__global__ __launch_bounds__(256) void k_head_wgrad(const float* __restrict__ H, const float* __restrict__ dY, int n,
-                                                    float* __restrict__ part) {
-    const int i0 = blockIdx.x * 64;
-    float* out = part + (size_t)blockIdx.x * (kHid + 1) * 2;
-    for (int t = threadIdx.x; t < (kHid + 1) * 2; t += 256) {
-        const int k = t >> 1, c = t & 1;
-        float s = 0.0f;
-        for (int r = 0; r < 64 && i0 + r < n; ++r) {
-            const int i = i0 + r;
-            s = fmaf(k < kHid ? H[i * kHid + k] : 1.0f, dY[2 * i + c], s);
+    for (int tile = tile0; tile < tiles; tile += stride) {
+        const int i = tile * 16 + j;
+        float4 x[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = nx[q];
+        const float2 dy = ndy;
+        const int deg = ndeg;
+        if (tile + stride < tiles) load(tile + stride);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float2* u = wo + 16 * q + 4 * g;
+            x[q] = make_float4(d_z2(x[q].x, dy, u[0]), d_z2(x[q].y, dy, u[1]), d_z2(x[q].z, dy, u[2]),
+                               d_z2(x[q].w, dy, u[3]));
         }
-        out[t] = s;
+        keep_in_lds();
+        f32x4 acc[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float4 u[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) u[t] = w[t][q][lane];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int t = 0; t < 8; ++t) acc[t] = mfma(at4(u[t], m), at4(x[q], m), acc[t]);
+        }
+        if (i >= n) continue;
+        const float inv = deg > 0 ? 1.0f / (float)deg : 0.0f;     // no neighbour reads Q of an isolated node
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const size_t at = (size_t)i * kHid + 16 * t + 4 * g;
+            *reinterpret_cast<float4*>(P + at) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+            *reinterpret_cast<float4*>(Q + at) =
+                make_float4(acc[4 + t][0] * inv, acc[4 + t][1] * inv, acc[4 + t][2] * inv, acc[4 + t][3] * inv);
+        }
     }
 }
 
-// Fixed-order sum of nb partial blocks of `len` floats into grad (accumulated in double).
-__global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ part, int nb, int len,
-                                                   float* __restrict__ grad) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= len) return;
+// Weight gradients: products over the nodes (the inner index; a lane's slot lane / 16 is the node
+// within a step of four). Blocks take runs of 64 nodes in turn; a run is summed in FP32 and added
+// to FP64 sums kept in registers, which become the block's partial at the end. Partials are laid
+// out as the parameters are, so that k_sum_grad writes the gradient itself.
+//
+// A partial per run of 64 nodes (782 of them at 50,000 nodes, each of 4,160 values) summed by one
+// thread per value took 185 us per matrix, 925 of the gradient's 1,530 us on 50,000 nodes, and the
+// products 130; here both layers' products take 31 us and the sum 7. A run's loads are issued
+// together: left to the compiler they were waited for step by step (35 and 37 us).
+constexpr int kRun = 64;
+
+// Layer 1: W1s (16 rows, from X), W1n (16 rows, from A0), b1. Each wave has 16 of the outputs.
+__global__ __launch_bounds__(256) void k_wgrad1(const float* __restrict__ X, const float* __restrict__ A0,
+                                                const float* __restrict__ dZ1, int n, double* __restrict__ part) {
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4, b = threadIdx.x >> 6;
+    double sum[2][4] = {}, bias = 0.0;
+    for (long long i0 = (long long)blockIdx.x * kRun; i0 < n; i0 += (long long)gridDim.x * kRun) {
+        f32x4 acc[2] = {f32x4{0, 0, 0, 0}, f32x4{0, 0, 0, 0}};
+        float bs = 0.0f;
+        // the run's loads together, then its products
+        float x[kRun / 4], a0[kRun / 4], z[kRun / 4];
+#pragma unroll
+        for (int st = 0; st < kRun / 4; ++st) {
+            const size_t r = (size_t)min(i0 + 4 * st + g, (long long)n - 1);
+            x[st] = X[r * kIn + j];
+            a0[st] = A0[r * kIn + j];
+            z[st] = dZ1[r * kHid + 16 * b + j];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int st = 0; st < kRun / 4; ++st) {
+            const float zi = i0 + 4 * st + g < n ? z[st] : 0.0f;
+            acc[0] = mfma(x[st], zi, acc[0]);
+            acc[1] = mfma(a0[st], zi, acc[1]);
+            bs += zi;
+        }
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum[a][r] += (double)acc[a][r];
+        bias += (double)bs;
+    }
+    double* out = part + (size_t)blockIdx.x * kGrad1;
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[(16 * a + 4 * g + r) * kHid + 16 * b + j] = sum[a][r];
+    bias += __shfl_xor(bias, 16, 64);
+    bias += __shfl_xor(bias, 32, 64);
+    if (g == 0) out[2 * kIn * kHid + 16 * b + j] = bias;
+}
+
+// Layer 2 and head: W2s (64 rows, from H1), W2n (64 rows, from A1), b2, Wo, bo. Each wave has 32
+// of the rows, and one of the small sums.
+__global__ __launch_bounds__(256) void k_wgrad2(const float* __restrict__ H1, const float* __restrict__ A1,
+                                                const float* __restrict__ H2, const float2* __restrict__ dY, int n,
+                                                const unsigned short* __restrict__ Wo, double* __restrict__ part) {
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const float* src = wave < 2 ? H1 : A1;
+    const int c0 = 32 * (wave & 1);
+    float2 wo[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+        wo[b] = make_float2(bf16_to_f32(Wo[2 * (16 * b + j)]), bf16_to_f32(Wo[2 * (16 * b + j) + 1]));
+    double sum[2][4][4] = {}, small[8] = {};
+    for (long long i0 = (long long)blockIdx.x * kRun; i0 < n; i0 += (long long)gridDim.x * kRun) {
+        f32x4 acc[2][4];
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0, 0, 0, 0};
+        float sm[8] = {};
+        constexpr int kPart = 8;                         // steps whose loads go together
+        for (int s0 = 0; s0 < kRun / 4; s0 += kPart) {
+            float2 dy[kPart];
+            float x0[kPart], x1[kPart], h[kPart][4];
+#pragma unroll
+            for (int st = 0; st < kPart; ++st) {
+                const size_t r = (size_t)min(i0 + 4 * (s0 + st) + g, (long long)n - 1);
+                dy[st] = dY[r];
+                x0[st] = src[r * kHid + c0 + j];
+                x1[st] = src[r * kHid + c0 + 16 + j];
+#pragma unroll
+                for (int b = 0; b < 4; ++b) h[st][b] = H2[r * kHid + 16 * b + j];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int st = 0; st < kPart; ++st) {
+                const float2 d = i0 + 4 * (s0 + st) + g < n ? dy[st] : make_float2(0.0f, 0.0f);
+                float z[4];
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    z[b] = d_z2(h[st][b], d, wo[b]);       // 0 past the last node
+                    acc[0][b] = mfma(x0[st], z[b], acc[0][b]);
+                    acc[1][b] = mfma(x1[st], z[b], acc[1][b]);
+                }
+                if (wave == 0) {
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) sm[b] += z[b];
+                } else if (wave == 1) {
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        sm[2 * b] = fmaf(h[st][b], d.x, sm[2 * b]);
+                        sm[2 * b + 1] = fmaf(h[st][b], d.y, sm[2 * b + 1]);
+                    }
+                } else if (wave == 2) {
+                    sm[0] += d.x;
+                    sm[1] += d.y;
+                }
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sum[a][b][r] += (double)acc[a][b][r];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) small[q] += (double)sm[q];
+    }
+    double* out = part + (size_t)blockIdx.x * kGrad2;
+    const int row0 = 32 * wave;
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[(row0 + 16 * a + 4 * g + r) * kHid + 16 * b + j] = sum[a][b][r];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        small[q] += __shfl_xor(small[q], 16, 64);
+        small[q] += __shfl_xor(small[q], 32, 64);
+    }
+    if (g != 0) return;
+    double* b2 = out + 2 * kHid * kHid;
+    if (wave == 0) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) b2[16 * b + j] = small[b];
+    } else if (wave == 1) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            b2[kHid + 2 * (16 * b + j)] = small[2 * b];
+            b2[kHid + 2 * (16 * b + j) + 1] = small[2 * b + 1];
+        }
+    } else if (wave == 2 && j == 0) {
+        b2[kHid + 2 * kHid] = small[0];
+        b2[kHid + 2 * kHid + 1] = small[1];
+    }
+}
+
+// grad[p] = the sum of parameter p's partials, in FP64 and a fixed order: 64 parameters per block,
+// four runs of the partials each.
+__global__ __launch_bounds__(256) void k_sum_grad(const double* __restrict__ part1, const double* __restrict__ part2,
+                                                  int nb, float* __restrict__ grad) {
+    __shared__ double red[4][64];
+    const int p = blockIdx.x * 64 + (threadIdx.x & 63), run = threadIdx.x >> 6;
     double s = 0.0;
-    for (int b = 0; b < nb; ++b) s += part[(size_t)b * len + t];
-    grad[t] = (float)s;
+    if (p < kParams) {
+        const double* src = p < kGrad1 ? part1 + p : part2 + (p - kGrad1);
+        const size_t len = p < kGrad1 ? kGrad1 : kGrad2;
+        const int b1 = nb * (run + 1) / 4;
+#pragma unroll 8
+        for (int b = nb * run / 4; b < b1; ++b) s += src[b * len];
+    }
+    red[run][threadIdx.x & 63] = s;
+    __syncthreads();
+    if (run == 0 && p < kParams)
+        grad[p] = (float)(((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) + red[3][threadIdx.x]);
 }
 
 // Adam on the FP32 masters, then the BF16 copies.
@@ -518,15 +718,23 @@ int blocks_for(long long work) {
     return (int)(b < 1 ? 1 : b);
 }
 
+// Waves of 16 nodes; at most the four blocks per compute unit that the weights' LDS lets run at a
+// time (each stages the weights once).
+int dense_blocks(int n) {
+    const int b = (n + 63) / 64;
+    return b < 1024 ? b : 1024;
+}
+
 template <int F, int MODE>
-void aggregate(const MpnnGraph& g, const float* in, float* out, hipStream_t st) {
+void aggregate(const MpnnGraph& g, const float* in, float* out, hipStream_t st, const float* P = nullptr,
+               const float* H = nullptr) {
     const long long rb = ((long long)g.n * F + 255) / 256;
-    k_agg_rows<F, MODE><<<(int)(rb < 1 ? 1 : (rb > 65536 ? 65536 : rb)), 256, 0, st>>>(g.rowptr, g.col, g.n, in, out);
+    k_agg_rows<F, MODE><<<(int)(rb < 1 ? 1 : (rb > 65536 ? 65536 : rb)), 256, 0, st>>>(g.rowptr, g.col, g.n, in, P, H, out);
     if (g.nchunks > 0) {
         const int cb = (g.nchunks + 3) / 4;
-        k_agg_chunks<F, MODE><<<cb < 8192 ? cb : 8192, 256, 0, st>>>(g.rowptr, g.col, g.chunks, g.nchunks, in, g.part);
+        k_agg_chunks<F><<<cb < 8192 ? cb : 8192, 256, 0, st>>>(g.rowptr, g.col, g.chunks, g.nchunks, in, g.part);
         k_agg_heavy<F, MODE><<<blocks_for((long long)g.nheavy * F), 256, 0, st>>>(g.rowptr, g.heavy_row, g.heavy_c0,
-                                                                                 g.nheavy, in, g.part, out);
+                                                                                 g.nheavy, in, g.part, P, H, out);
     }
 }
 
@@ -565,13 +773,15 @@ void mpnn_features(const MpnnGraph& g, unsigned long long seed, int steps, MpnnS
     aggregate<kIn, kAggMean>(g, g.X, g.A0, st);
 }
 
-void mpnn_forward(const MpnnGraph& g, const MpnnWeights& w, MpnnScratch& s, hipStream_t st) {
+void mpnn_forward(const MpnnGraph& g, const MpnnWeights& w, MpnnScratch& s, bool keep, hipStream_t st) {
     const int n = g.n;
-    const int db = (n + 63) / 64 < 1024 ? (n + 63) / 64 : 1024;
-    k_dense<kIn><<<db, 256, 0, st>>>(g.X, g.A0, n, w.bf + kOffW1s, w.bf + kOffW1n, w.bf + kOffB1, s.H1);
+    const int db = dense_blocks(n);
+    k_dense<kIn, false><<<db, 256, 0, st>>>(g.X, g.A0, n, w.bf + kOffW1s, w.bf + kOffW1n, w.bf + kOffB1, s.H1, nullptr,
+                                            nullptr, nullptr);
     aggregate<kHid, kAggMean>(g, s.H1, s.A1, st);
-    k_dense<kHid><<<db, 256, 0, st>>>(s.H1, s.A1, n, w.bf + kOffW2s, w.bf + kOffW2n, w.bf + kOffB2, s.H2);
-    k_head<<<blocks_for(n), 256, 0, st>>>(s.H2, n, w.bf + kOffWo, w.bf + kOffBo, s.Y);
+    k_dense<kHid, true><<<db, 256, 0, st>>>(s.H1, s.A1, n, w.bf + kOffW2s, w.bf + kOffW2n, w.bf + kOffB2,
+                                            keep ? s.H2 : nullptr, w.bf + kOffWo, w.bf + kOffBo,
+                                            reinterpret_cast<float2*>(s.Y));
 }
 
 int mpnn_loss_backward(const MpnnGraph& g, const MpnnWeights& w, MpnnScratch& s, const int* d_offs, int R,
@@ -579,36 +789,20 @@ int mpnn_loss_backward(const MpnnGraph& g, const MpnnWeights& w, MpnnScratch& s,
     const int n = g.n;
     const long long pairs = (long long)g.nnz + 2ll * R * n;
     const double inv = 1.0 / (double)pairs;
-    const int lb = blocks_for(n);
-    k_loss<<<lb, 256, 0, st>>>(g.rowptr, g.col, n, s.Y, g.T, d_offs, R, inv, s.dY, s.dpart);
-    // head
-    const int chunks = (n + 63) / 64;
-    k_head_wgrad<<<chunks, 256, 0, st>>>(s.H2, s.dY, n, s.wpart);
-    k_sum_parts<<<blocks_for((kHid + 1) * 2), 256, 0, st>>>(s.wpart, chunks, (kHid + 1) * 2, w.grad + kOffWo);
-    k_head_back<<<blocks_for((long long)n * kHid), 256, 0, st>>>(s.dY, s.H2, n, w.bf + kOffWo, s.dZ2);
-    // layer 2: grads of W2s (+b2) from H1, of W2n from A1
-    k_wgrad<kHid><<<chunks, 256, 0, st>>>(s.H1, s.dZ2, n, s.wpart);
-    k_sum_parts<<<blocks_for((kHid + 1) * kHid), 256, 0, st>>>(s.wpart, chunks, (kHid + 1) * kHid, s.gtmp);
-    // gtmp rows 0..63 -> W2s, row 64 -> b2
-    hipMemcpyAsync(w.grad + kOffW2s, s.gtmp, sizeof(float) * kHid * kHid, hipMemcpyDeviceToDevice, st);
-    hipMemcpyAsync(w.grad + kOffB2, s.gtmp + kHid * kHid, sizeof(float) * kHid, hipMemcpyDeviceToDevice, st);
-    k_wgrad<kHid><<<chunks, 256, 0, st>>>(s.A1, s.dZ2, n, s.wpart);
-    k_sum_parts<<<blocks_for(kHid * kHid), 256, 0, st>>>(s.wpart, chunks, (kHid + 1) * kHid, s.gtmp);
-    hipMemcpyAsync(w.grad + kOffW2n, s.gtmp, sizeof(float) * kHid * kHid, hipMemcpyDeviceToDevice, st);
-    // dH1 = dZ2 W2s^T + agg^T(dZ2 W2n^T), masked
-    const int db = (n + 3) / 4 < 2048 ? (n + 3) / 4 : 2048;
-    k_dense_back_x<<<db, 256, 0, st>>>(s.dZ2, n, w.bf + kOffW2s, s.P);
-    k_dense_back_x<<<db, 256, 0, st>>>(s.dZ2, n, w.bf + kOffW2n, s.Q);
-    aggregate<kHid, kAggTranspose>(g, s.Q, s.A1, st);
-    k_add_mask<<<blocks_for((long long)n * kHid), 256, 0, st>>>(s.P, s.A1, s.H1, n * kHid, s.dZ1);
+    const int lb = (n + 31) / 32 < kLossBlocks ? (n + 31) / 32 : kLossBlocks;
+    float2* dY = reinterpret_cast<float2*>(s.dY);
+    k_loss<<<lb, 256, 0, st>>>(g.rowptr, g.col, n, reinterpret_cast<const float2*>(s.Y),
+                               reinterpret_cast<const float2*>(g.T), d_offs, R, inv, dY, s.dpart);
+    // layer 2 and head
+    const int runs = (n + kRun - 1) / kRun, nb = runs < kGradBlocks ? runs : kGradBlocks;
+    k_wgrad2<<<nb, 256, 0, st>>>(s.H1, s.A1, s.H2, dY, n, w.bf + kOffWo, s.part2);
+    // dZ1 = (dZ2 W2s^T + agg^T(dZ2 W2n^T)) masked by H1 > 0
+    k_back<<<dense_blocks(n), 256, 0, st>>>(dY, s.H2, n, g.rowptr, w.bf + kOffWo, w.bf + kOffW2s, w.bf + kOffW2n, s.P,
+                                            s.Q);
+    aggregate<kHid, kAggBack>(g, s.Q, s.dZ1, st, s.P, s.H1);
     // layer 1
-    k_wgrad<kIn><<<chunks, 256, 0, st>>>(g.X, s.dZ1, n, s.wpart);
-    k_sum_parts<<<blocks_for((kIn + 1) * kHid), 256, 0, st>>>(s.wpart, chunks, (kIn + 1) * kHid, s.gtmp);
-    hipMemcpyAsync(w.grad + kOffW1s, s.gtmp, sizeof(float) * kIn * kHid, hipMemcpyDeviceToDevice, st);
-    hipMemcpyAsync(w.grad + kOffB1, s.gtmp + kIn * kHid, sizeof(float) * kHid, hipMemcpyDeviceToDevice, st);
-    k_wgrad<kIn><<<chunks, 256, 0, st>>>(g.A0, s.dZ1, n, s.wpart);
-    k_sum_parts<<<blocks_for(kIn * kHid), 256, 0, st>>>(s.wpart, chunks, (kIn + 1) * kHid, s.gtmp);
-    hipMemcpyAsync(w.grad + kOffW1n, s.gtmp, sizeof(float) * kIn * kHid, hipMemcpyDeviceToDevice, st);
+    k_wgrad1<<<nb, 256, 0, st>>>(g.X, g.A0, s.dZ1, n, s.part1);
+    k_sum_grad<<<(kParams + 63) / 64, 256, 0, st>>>(s.part1, s.part2, nb, w.grad);
     if (loss) {
         std::vector<double> h((size_t)lb);
         if (hipMemcpyAsync(h.data(), s.dpart, sizeof(double) * lb, hipMemcpyDeviceToHost, st) != hipSuccess) return -1;

@@ -58,10 +58,9 @@ int ensure_scratch(gfa2_mpnn* m, int n) {
     MpnnScratch& s = m->s;
     if (n <= s.cap) return GFA2_OK;
     for (void* p : {(void*)s.z0, (void*)s.z1, (void*)s.H1, (void*)s.A1, (void*)s.H2, (void*)s.Y, (void*)s.dY,
-                    (void*)s.dZ2, (void*)s.P, (void*)s.Q, (void*)s.dZ1, (void*)s.wpart})
+                    (void*)s.P, (void*)s.Q, (void*)s.dZ1})
         if (p) (void)hipFree(p);
     const size_t nh = (size_t)n * kHid;
-    const size_t chunks = ((size_t)n + 63) / 64;
     MP_TRY(hipMalloc(&s.z0, sizeof(float) * (size_t)n * 8));
     MP_TRY(hipMalloc(&s.z1, sizeof(float) * (size_t)n * 8));
     MP_TRY(hipMalloc(&s.H1, sizeof(float) * nh));
@@ -69,11 +68,9 @@ int ensure_scratch(gfa2_mpnn* m, int n) {
     MP_TRY(hipMalloc(&s.H2, sizeof(float) * nh));
     MP_TRY(hipMalloc(&s.Y, sizeof(float) * (size_t)n * 2));
     MP_TRY(hipMalloc(&s.dY, sizeof(float) * (size_t)n * 2));
-    MP_TRY(hipMalloc(&s.dZ2, sizeof(float) * nh));
     MP_TRY(hipMalloc(&s.P, sizeof(float) * nh));
     MP_TRY(hipMalloc(&s.Q, sizeof(float) * nh));
     MP_TRY(hipMalloc(&s.dZ1, sizeof(float) * nh));
-    MP_TRY(hipMalloc(&s.wpart, sizeof(float) * chunks * (kHid + 1) * kHid));
     s.cap = n;
     return GFA2_OK;
 }
@@ -129,7 +126,8 @@ int gfa2_mpnn_create(int device, uint64_t seed, gfa2_mpnn_t* out) {
         (st = mp_alloc(m->allocs, &m->w.v, kParams)) != GFA2_OK ||
         (st = mp_alloc(m->allocs, &m->s.dpart, 8192)) != GFA2_OK ||
         (st = mp_alloc(m->allocs, &m->s.musd, 2 * kIn)) != GFA2_OK ||
-        (st = mp_alloc(m->allocs, &m->s.gtmp, (kHid + 1) * kHid)) != GFA2_OK) {
+        (st = mp_alloc(m->allocs, &m->s.part1, (size_t)kGradBlocks * kGrad1)) != GFA2_OK ||
+        (st = mp_alloc(m->allocs, &m->s.part2, (size_t)kGradBlocks * kGrad2)) != GFA2_OK) {
         gfa2_mpnn_destroy(m);
         return st != GFA2_OK ? st : GFA2_ERR_HIP;
     }
@@ -316,7 +314,7 @@ int gfa2_mpnn_loss_grad(gfa2_mpnn_t m, int32_t graph_id, const int32_t* offsets,
         m->offs_cap = R;
     }
     if (R) MP_TRY(hipMemcpyAsync(m->offs, offsets, sizeof(int) * R, hipMemcpyHostToDevice, m->stream));
-    mpnn_forward(g, m->w, m->s, m->stream);
+    mpnn_forward(g, m->w, m->s, true, m->stream);
     if (mpnn_loss_backward(g, m->w, m->s, m->offs, R, loss, m->stream) != 0) return GFA2_ERR_HIP;
     if (grad) {
         MP_TRY(hipMemcpyAsync(grad, m->w.grad, sizeof(float) * kParams, hipMemcpyDeviceToHost, m->stream));
@@ -347,7 +345,7 @@ int gfa2_mpnn_train(gfa2_mpnn_t m, int32_t steps, float lr, int32_t R, uint64_t 
     MP_TRY(hipMemcpyAsync(m->offs, offs.data(), sizeof(int) * offs.size(), hipMemcpyHostToDevice, m->stream));
     for (int s = 0; s < steps; ++s) {
         const MpnnGraph& g = m->graphs[ids[s % ids.size()]];
-        mpnn_forward(g, m->w, m->s, m->stream);
+        mpnn_forward(g, m->w, m->s, true, m->stream);
         double* lp = (s == steps - 1) ? last_loss : nullptr;
         if (mpnn_loss_backward(g, m->w, m->s, m->offs + (size_t)s * R, R, lp, m->stream) != 0) return GFA2_ERR_HIP;
         mpnn_adam(m->w, lr, ++m->adam_step, m->stream);
@@ -374,7 +372,7 @@ int gfa2_mpnn_infer(gfa2_mpnn_t m, int32_t graph_id, float scale, float* xy) {
     if (st != GFA2_OK || !xy) return st != GFA2_OK ? st : GFA2_ERR_INVALID_ARG;
     const MpnnGraph& g = m->graphs[graph_id];
     MP_TRY(hipSetDevice(m->device));
-    mpnn_forward(g, m->w, m->s, m->stream);
+    mpnn_forward(g, m->w, m->s, false, m->stream);
     mpnn_place(g, m->s, scale, reinterpret_cast<float2*>(m->s.dY), m->stream);
     MP_TRY(hipMemcpyAsync(xy, m->s.dY, sizeof(float) * 2 * g.n, hipMemcpyDeviceToHost, m->stream));
     MP_TRY(hipStreamSynchronize(m->stream));
@@ -390,7 +388,7 @@ int gfa2_mpnn_infer_to_engine(gfa2_mpnn_t m, int32_t graph_id, float scale, gfa2
     if (v.n != g.n || v.device != m->device) return GFA2_ERR_INVALID_ARG;
     MP_TRY(hipSetDevice(m->device));
     MP_TRY(hipStreamSynchronize(v.stream));
-    mpnn_forward(g, m->w, m->s, m->stream);
+    mpnn_forward(g, m->w, m->s, false, m->stream);
     mpnn_place(g, m->s, scale, v.pos, m->stream);
     MP_TRY(hipGetLastError());
     MP_TRY(hipStreamSynchronize(m->stream));
@@ -406,7 +404,7 @@ int gfa2_mpnn_destroy(gfa2_mpnn_t m) {
     for (void* p : m->allocs) (void)hipFree(p);
     MpnnScratch& s = m->s;
     for (void* p : {(void*)s.z0, (void*)s.z1, (void*)s.H1, (void*)s.A1, (void*)s.H2, (void*)s.Y, (void*)s.dY,
-                    (void*)s.dZ2, (void*)s.P, (void*)s.Q, (void*)s.dZ1, (void*)s.wpart})
+                    (void*)s.P, (void*)s.Q, (void*)s.dZ1})
         if (p) (void)hipFree(p);
     if (m->offs) (void)hipFree(m->offs);
     if (m->stream) (void)hipStreamDestroy(m->stream);

@@ -19,6 +19,12 @@ constexpr int kOffWo = kOffB2 + kHid;
 constexpr int kOffBo = kOffWo + kHid * 2;
 constexpr int kParams = kOffBo + 2;
 
+// Gradient partials: layer 1 (W1s, W1n, b1) and layer 2 with the head (W2s, W2n, b2, Wo, bo).
+constexpr int kGrad1 = kOffW2s;
+constexpr int kGrad2 = kParams - kOffW2s;
+constexpr int kGradBlocks = 256;
+constexpr int kLossBlocks = 2048;
+
 // Rows longer than kHeavyDeg entries are aggregated in chunks of kChunk entries.
 constexpr int kHeavyDeg = 512;
 constexpr int kChunk = 512;
@@ -51,19 +57,19 @@ struct MpnnWeights {
 struct MpnnScratch {
     int cap = 0;            // nodes the buffers hold
     float *z0 = nullptr, *z1 = nullptr;
-    double* dpart = nullptr;    // >= 4096 doubles
+    double* dpart = nullptr;    // 8192 doubles: column statistics, loss partials
     float* musd = nullptr;      // 2 * kIn
     float *H1 = nullptr, *A1 = nullptr, *H2 = nullptr, *Y = nullptr, *dY = nullptr;
-    float *dZ2 = nullptr, *P = nullptr, *Q = nullptr, *dZ1 = nullptr;
-    float* wpart = nullptr;     // chunks * (kHid+1) * kHid
-    float* gtmp = nullptr;      // (kHid+1) * kHid
+    float *P = nullptr, *Q = nullptr, *dZ1 = nullptr;
+    double *part1 = nullptr, *part2 = nullptr;  // kGradBlocks x kGrad1 and kGrad2: weight-gradient partials
 };
 
 // Host side: the heavy rows and chunk list of a CSR given by its row offsets.
 void mpnn_agg_plan(const int* rowptr, int n, std::vector<int>& heavy_row, std::vector<int>& heavy_c0,
                    std::vector<int2>& chunks);
 void mpnn_features(const MpnnGraph& g, unsigned long long seed, int steps, MpnnScratch& s, hipStream_t st);
-void mpnn_forward(const MpnnGraph& g, const MpnnWeights& w, MpnnScratch& s, hipStream_t st);
+// keep: H2 is written too (the backward pass reads it).
+void mpnn_forward(const MpnnGraph& g, const MpnnWeights& w, MpnnScratch& s, bool keep, hipStream_t st);
 int mpnn_loss_backward(const MpnnGraph& g, const MpnnWeights& w, MpnnScratch& s, const int* d_offs, int R,
                        double* loss, hipStream_t st);
 void mpnn_adam(MpnnWeights& w, float lr, int step, hipStream_t st);

@@ -1,0 +1,46 @@
+"""The network's matrix-instruction kernels at the edges of their tiles (16 nodes per wave, runs of
+64 nodes per gradient partial) and past one round of their grids (16,384, 65,536 and 131,072
+nodes): loss, gradient and placed positions against the FP64 oracle."""
+import numpy as np
+import pytest
+
+from gpugraphlayout_amd import Mpnn
+from oracle import mpnn_oracle as mo
+
+pytestmark = pytest.mark.gpu
+
+
+def sparse_csr(n, seed):
+    """About 1.5 random edges per node, some nodes with none."""
+    rng = np.random.default_rng(seed)
+    a, b = rng.integers(0, n, (2, 3 * n // 2 + 1))
+    key = np.unique(np.concatenate([a[a != b] * n + b[a != b], b[a != b] * n + a[a != b]]))
+    rowptr = np.zeros(n + 1, np.int64)
+    rowptr[1:] = np.cumsum(np.bincount(key // n, minlength=n))
+    return rowptr, (key % n).astype(np.int32)
+
+
+@pytest.mark.parametrize("n", [3, 15, 16, 17, 63, 64, 65, 1000, 16_385, 65_600, 131_090])
+def test_gradient_and_positions(n):
+    print(f"case mpnn sizes n={n}", flush=True)
+    rowptr, col = sparse_csr(n, n)
+    rng = np.random.default_rng(n + 1)
+    T = rng.normal(size=(n, 2)).astype(np.float32)
+    m = Mpnn(seed=3)
+    gid = m.add_graph(n, rowptr, col, target=T, feature_seed=n, steps=1)
+    X = m.features(gid)
+    offsets = sorted({1, n // 2, n - 1} - {0})
+    loss, grad = m.loss_grad(gid, offsets)
+    t = T.astype(np.float64) - T.mean(0, dtype=np.float64)
+    t /= np.sqrt((t ** 2).sum(1).mean())
+    p = m.params().astype(np.float64)
+    L, G = mo.loss_grad(p, rowptr, col, X, t, offsets, round_bf16=True)
+    # the bars of the other gradient tests (float32 products against the FP64 network)
+    assert loss == pytest.approx(L, rel=1e-5)
+    assert np.linalg.norm(grad - G) < 1e-4 * np.linalg.norm(G)
+    Y, _ = mo.forward(p, rowptr, col, X)
+    Y -= Y.mean(0)
+    want = Y * (25.0 / np.sqrt((Y ** 2).sum(1).mean()))
+    got = m.infer(gid, 25.0)
+    assert np.linalg.norm(got - want) < 1e-4 * np.linalg.norm(want)
+    m.close()
