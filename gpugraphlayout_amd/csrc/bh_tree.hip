@@ -724,6 +724,205 @@ __global__ __launch_bounds__(256) void k_kids(const float4* __restrict__ rec, co
     if (threadIdx.x < 8) kids_part[blockIdx.x * 8 + threadIdx.x] = rmax[threadIdx.x];
 }
 
+// k_nodes and k_kids in one launch for graphs of up to kCellsNodes nodes, where the chain of
+// dependent loads of the longest search decides, not their number. A cell gets 16 lanes: they read
+// the 16 keys after the cell's first body at once, which settles cells of up to 16 bodies (most),
+// their extent and where their children start; a larger cell is searched by the whole wave, 16
+// lanes for each of the four bounds (the three changes of the next digit and the end), 16 probes
+// at a time: 7 loads in a row for 10,000 bodies where one thread made 26.
+//
+// A child that starts at sorted position p > i has the record index p + S[p]: p - 1 and p share
+// exactly the cell's L levels, so the first cell opened at p is that child (or, with none opened,
+// p's body is).
+//
+// Measured per iteration: 10,000 nodes k_nodes 11.5 + k_kids 4.1 -> 10.9 us and a launch less; SBM
+// 50,000 nodes 12.3 + 4.9 -> 18.5 us, so larger graphs keep the two (kCellsNodes between them).
+constexpr int kCellsThreads = 1024;
+
+// Positions of [lo, lim) whose keys share their top `top` bits' worth of digits with ki, counted
+// from lo, all of which come first: the first position past them. Every lane of the 16 gets it.
+// `before(key)` says whether a position lies before the bound; it holds up to the bound only.
+template <typename F>
+__device__ __forceinline__ int bound16(const unsigned long long* __restrict__ keys, int lo, int lim, int lane, F before) {
+    // lo: a position before the bound
+    const int q = lane & 15, shift = lane & 48;
+    int step = 1;
+    for (;;) {                       // grows until a probe lies past the bound
+        const int p = lo + (q + 1) * step;
+        const bool in = p < lim && before(keys[p < lim ? p : lo]);
+        const int c = __popc((unsigned)(__builtin_amdgcn_ballot_w64(in) >> shift) & 0xffffu);
+        lo += c * step;
+        if (c < 16) break;
+        step <<= 4;
+    }
+    while (step > 1) {
+        step >>= 4;
+        const int p = lo + (q + 1) * step;
+        const bool in = q < 15 && p < lim && before(keys[p < lim ? p : lo]);
+        lo += step * __popc((unsigned)(__builtin_amdgcn_ballot_w64(in) >> shift) & 0xffffu);
+    }
+    return lo + 1;
+}
+
+__global__ __launch_bounds__(kCellsThreads) void k_cells(const unsigned long long* __restrict__ keys,
+                                                         const signed char* __restrict__ lcp,
+                                                         const int* __restrict__ sg, int n,
+                                                         const int* __restrict__ S, float4* __restrict__ rec,
+                                                         int4* __restrict__ kids, int* __restrict__ rcount,
+                                                         int* __restrict__ cell_rec,
+                                                         unsigned char* __restrict__ cell_lvl,
+                                                         int* __restrict__ rec_begin, DevState* st,
+                                                         const Moment* __restrict__ pmass,
+                                                         const float4* __restrict__ seg_root,
+                                                         int* __restrict__ big_rc, unsigned char* __restrict__ big_lvl,
+                                                         const int* __restrict__ node_off,
+                                                         int* __restrict__ kids_part) {
+    __shared__ int hist[kMaxLevels + 1];
+    __shared__ int rmax[8];
+    __shared__ int lmax;
+    const int tid = threadIdx.x, lane = tid & 63, q = lane & 15;
+    if (tid <= kMaxLevels) hist[tid] = 0;
+    if (tid < 8) rmax[tid] = 0;
+    if (tid == 0) lmax = 0;
+    __syncthreads();
+    const int ncells = st->err == 0 ? S[n] : 0;
+    const int stride = gridDim.x * (kCellsThreads / 16);
+    const int ord0 = (blockIdx.x * kCellsThreads + tid) / 64 * 4;      // the wave's first cell: uniform
+    for (int w0 = ord0; w0 < ncells; w0 += stride) {
+        const int ord = w0 + (lane >> 4);
+        const bool live = ord < ncells;
+        const int i = live ? cell_rec[ord] : 0;
+        const int gi = sg ? sg[i] : 0;
+        const int lim = sg ? node_off[gi + 1] : n;
+        const unsigned long long ki = keys[i];
+        const int wp = i + 1 + q;
+        const unsigned long long kw = keys[wp < lim ? wp : i];
+        const int Si = S[i];
+        const int L = lcp_prev(lcp, sg, i) + 1 + (ord - Si);
+        // digit of the next level (bits 63 - 2L, 62 - 2L); a level-32 cell has none
+        const int dsh = 62 - 2 * min(L, 31);
+        const bool in = live && wp < lim && (L == 0 || lcp_levels(ki, kw) >= L);
+        const unsigned int inm = (unsigned)(__builtin_amdgcn_ballot_w64(in) >> (lane & 48)) & 0xffffu;
+        int end = i + 1 + __popc(inm);           // one past the cell's last body
+        // where its 2nd, 3rd and 4th child start (-1: none)
+        int c1 = -1, c2 = -1, c3 = -1;
+        if (L >= 32) {
+            // children are the bodies themselves
+            if (end > i + 1) c1 = i + 1;
+            if (end > i + 2) c2 = i + 2;
+            if (end > i + 3) c3 = i + 3;
+        } else {
+            const unsigned int dw = (unsigned)(kw >> dsh) & 3u;
+            unsigned int dp = __shfl_up(dw, 1, 16);
+            if (q == 0) dp = (unsigned)(ki >> dsh) & 3u;
+            unsigned int m = (unsigned)(__builtin_amdgcn_ballot_w64(in && dw != dp) >> (lane & 48)) & 0xffffu;
+            if (m) c1 = i + __ffs(m), m &= m - 1;
+            if (m) c2 = i + __ffs(m), m &= m - 1;
+            if (m) c3 = i + __ffs(m);
+        }
+        // cells that fill the window, one after another, by the whole wave
+        unsigned long long large = __builtin_amdgcn_ballot_w64(live && inm == 0xffffu);
+        while (large) {
+            const int src = __builtin_ctzll(large);          // the cell's first lane
+            large &= ~(0xffffull << src);
+            const int bi = __builtin_amdgcn_readlane(i, src), bl = __builtin_amdgcn_readlane(L, src);
+            const int blim = __builtin_amdgcn_readlane(lim, src);
+            const unsigned long long bk =
+                ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(ki >> 32), src) << 32) |
+                (unsigned)__builtin_amdgcn_readlane((int)(unsigned)ki, src);
+            const int bsh = 62 - 2 * min(bl, 31);
+            const unsigned int d0 = (unsigned)(bk >> bsh) & 3u;
+            // 16 lanes look for the first body whose next digit is at least d (4: the cell's end)
+            const unsigned int d = 1 + (lane >> 4);
+            const bool digits = bl < 32;
+            int p = bi;
+            if (d == 4 && bl == 0) p = blim;
+            else if (d == 4 || (digits && d > d0))
+                p = bound16(keys, bi, blim, lane, [&](unsigned long long k) {
+                    return (bl == 0 || lcp_levels(bk, k) >= bl) && (d == 4 || ((unsigned)(k >> bsh) & 3u) < d);
+                });
+            const int p1 = __builtin_amdgcn_readlane(p, 0), p2 = __builtin_amdgcn_readlane(p, 16);
+            const int p3 = __builtin_amdgcn_readlane(p, 32), p4 = __builtin_amdgcn_readlane(p, 48);
+            if ((lane & 48) == src) {
+                end = p4;
+                c1 = c2 = c3 = -1;
+                if (!digits) {
+                    c1 = bi + 1;
+                    c2 = bi + 2;
+                    c3 = bi + 3;
+                } else {
+                    // digit d has bodies where its bound lies before the next digit's
+                    int found = 0;
+                    const int at[4] = {p1, p2, p3, p4};
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+                        if (at[k] > bi && at[k] < at[k + 1]) {
+                            if (found == 0) c1 = at[k];
+                            else if (found == 1) c2 = at[k];
+                            else c3 = at[k];
+                            ++found;
+                        }
+                }
+            }
+        }
+        if (!live) continue;
+        const int rc = i + ord;
+        // lanes 0-3: a child each, and a word of the record each
+        if (q < 4) {
+            const int cp = q == 0 ? i : (q == 1 ? c1 : (q == 2 ? c2 : c3));
+            const int Sc = S[cp >= 0 ? cp : i], Se = S[end];
+            reinterpret_cast<int*>(kids + rc)[q] = q == 0 ? rc + 1 : (cp >= 0 ? cp + Sc : -1);
+            const unsigned int skip = (unsigned int)(end + Se - rc);
+            const unsigned int info = (skip << kInfoLevelBits) | (unsigned int)((L > 0 ? L - 1 : 0) & 31);
+            float out = __uint_as_float(info);               // lane 3
+            bool write = q == 3;
+            if (pmass) {
+                // lane 0: x; lane 1: y; lane 2: mass (see k_nodes)
+                const unsigned long long* a = reinterpret_cast<const unsigned long long*>(pmass + i);
+                const unsigned long long* e = reinterpret_cast<const unsigned long long*>(pmass + end);
+                const int lo = q == 1 ? 2 : 0;
+                const u128 va = ((u128)a[lo + 1] << 64) | a[lo], ve = ((u128)e[lo + 1] << 64) | e[lo];
+                const u128 dv = ve - va;
+                const double M = (double)(e[4] - a[4]);
+                if (M < 16777216.0) {
+                    const float4 c = seg_root[gi];
+                    const double m = i128_to_double((unsigned long long)dv, (unsigned long long)(dv >> 64)) / M;
+                    if (q < 2) out = (float)(ldexp(m, -moment_shift(c.z)) + (q == 0 ? c.x : c.y));
+                    else if (q == 2) out = (float)M;
+                    write = true;
+                } else if (q == 3) {
+                    const int slot = atomicAdd(&st->nbig, 1);
+                    if (slot < kMaxBig) {
+                        big_rc[slot] = rc;
+                        big_lvl[slot] = (unsigned char)L;
+                    } else {
+                        st->err |= kErrTreeOverflow;
+                    }
+                }
+            }
+            if (write) reinterpret_cast<float*>(rec + rc)[q] = out;
+        }
+        if (q == 4) {
+            rcount[rc] = end - i;
+            cell_rec[ord] = rc;       // the cell list of the summary launches
+            if (!pmass) {
+                cell_lvl[ord] = (unsigned char)L;
+                atomicAdd(&hist[L], 1);
+            }
+            if (L == 0 && rec_begin) rec_begin[gi] = rc;
+            atomicMax(&lmax, L);
+            // a cell of level 32 is recorded as level 32 too; level 0 as none of 4, 8, ..., 32
+            if (L > 0 && (L & 3) == 0) atomicMax(&rmax[(L >> 2) - 1], end - i);
+        }
+    }
+    __syncthreads();
+    if (!pmass && tid <= kMaxLevels && hist[tid] != 0) atomicAdd(&st->level_count[tid], hist[tid]);
+    if (tid == 0 && lmax > 0 &&
+        lmax > __hip_atomic_load(&st->max_level, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(&st->max_level, lmax);
+    if (tid < 8) kids_part[blockIdx.x * 8 + tid] = rmax[tid];
+}
+
 // Bucket cells by level (order inside a level is irrelevant).
 __global__ __launch_bounds__(256) void k_levels(const int* __restrict__ cell_rec,
                                                 const unsigned char* __restrict__ cell_lvl,
@@ -910,14 +1109,20 @@ void launch_tree(Bufs& b, hipStream_t s) {
     k_prefix<<<tiles, kTreeThreads, 0, s>>>(b.lcp, sg, n, b.blocksum, b.S, b.sbody, b.rec, b.brec, b.st, b.seg_root,
                                             bm, pm, b.cell_rec, max_cells, fused ? 1 : 0, b.cap_records,
                                             b.rec_begin + b.nseg);
-    // grid-stride over the cells (their number is known on the device only; at most
-    // max_cells, typically below n)
-    const int node_blocks = (n + kTreeThreads - 1) / kTreeThreads;
-    k_nodes<<<node_blocks, kTreeThreads, 0, s>>>(b.sort.keys[0], b.lcp, sg, n, b.S, b.rec, b.rcount, b.cell_rec,
-                                                 b.cell_lvl, b.rec_begin, b.st, pm, b.seg_root, b.big_rc,
-                                                 b.big_lvl, b.node_off);
-    // every record's info word is in place (cells: k_nodes, bodies: k_prefix)
-    k_kids<<<b.kids_blocks, 256, 0, s>>>(b.rec, b.rcount, b.S, n, b.cell_rec, b.kids, b.kids_part, b.st);
+    if (n <= kCellsNodes) {
+        k_cells<<<b.kids_blocks, kCellsThreads, 0, s>>>(b.sort.keys[0], b.lcp, sg, n, b.S, b.rec, b.kids, b.rcount,
+                                                        b.cell_rec, b.cell_lvl, b.rec_begin, b.st, pm, b.seg_root,
+                                                        b.big_rc, b.big_lvl, b.node_off, b.kids_part);
+    } else {
+        // grid-stride over the cells (their number is known on the device only; at most
+        // max_cells, typically below n)
+        const int node_blocks = (n + kTreeThreads - 1) / kTreeThreads;
+        k_nodes<<<node_blocks, kTreeThreads, 0, s>>>(b.sort.keys[0], b.lcp, sg, n, b.S, b.rec, b.rcount, b.cell_rec,
+                                                     b.cell_lvl, b.rec_begin, b.st, pm, b.seg_root, b.big_rc,
+                                                     b.big_lvl, b.node_off);
+        // every record's info word is in place (cells: k_nodes, bodies: k_prefix)
+        k_kids<<<b.kids_blocks, 256, 0, s>>>(b.rec, b.rcount, b.S, n, b.cell_rec, b.kids, b.kids_part, b.st);
+    }
     if (b.int_mass) {
         if (!b.no_big) k_big<<<1, 256, 0, s>>>(b.rec, b.big_rc, b.big_lvl, b.st);
         return;

@@ -586,7 +586,7 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
     GFA2_ALLOC(b.rec, (size_t)cap);
     GFA2_ALLOC(b.kids, (size_t)cap);
     // enough threads for the cells' dependent child hops (about one cell per thread)
-    b.kids_blocks = std::max(1, std::min((n + 255) / 256, 16384));
+    b.kids_blocks = n <= kCellsNodes ? (n + 63) / 64 : std::min((n + 255) / 256, 16384);
     GFA2_ALLOC(b.kids_part, (size_t)b.kids_blocks * 8);
     GFA2_ALLOC(b.brec, n);
     GFA2_ALLOC(b.sbody, n);
