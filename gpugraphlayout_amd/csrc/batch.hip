@@ -10,6 +10,7 @@
 // record range. Walk groups, speed state and displacement are per graph, so a graph laid
 // out in a batch follows exactly the trajectory it follows alone.
 #include "engine_internal.h"
+#include "tree_device.h"
 
 #include <algorithm>
 
@@ -59,20 +60,7 @@ __global__ __launch_bounds__(256) void k_seg_keys(const float2* __restrict__ pos
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         const float4 root = seg_root[seg_of[i]];
         const float2 p = pos[i];
-        float r = root.z * 0.5f;
-        bool bx = root.x < p.x, by = root.y < p.y;
-        float x = root.x + (bx ? r : -r);
-        float y = root.y + (by ? r : -r);
-        unsigned long long key = (unsigned long long)((unsigned)bx | ((unsigned)by << 1)) << 62;
-#pragma unroll
-        for (int l = 1; l < kKeyLevels; ++l) {
-            r *= 0.5f;
-            bx = x < p.x;
-            by = y < p.y;
-            key |= (unsigned long long)((unsigned)bx | ((unsigned)by << 1)) << (62 - 2 * l);
-            x += bx ? r : -r;
-            y += by ? r : -r;
-        }
+        const unsigned long long key = path_key(p, root.x, root.y, root.z);
         keys[i] = key;
         if (pkey) pkey[i] = key;      // kept for the regather after a global graph sort
         vals[i] = (unsigned)i;

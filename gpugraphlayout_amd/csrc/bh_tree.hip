@@ -24,14 +24,10 @@
 //     (src/RPBHKernels.cu:357-506).
 // Nothing waits on another workgroup; every dependency crosses a launch boundary.
 #include "engine_internal.h"
+#include "tree_device.h"
 
 namespace gfa2 {
 namespace {
-
-__device__ __forceinline__ int lcp_levels(unsigned long long a, unsigned long long b) {
-    unsigned long long x = a ^ b;
-    return x == 0ull ? kKeyLevels : (__clzll((long long)x) >> 1);
-}
 
 // Reduce bounding-box partials {minx, miny, maxx, maxy} in LDS (every block does it).
 __device__ void reduce_bbox(const float4* __restrict__ part, int np, float* root /*[3] LDS*/) {
@@ -130,20 +126,7 @@ __global__ __launch_bounds__(256) void k_keys(const float2* __restrict__ pos, co
     }
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         const float2 p = pos[i];
-        float r = radius * 0.5f;
-        bool bx = rootx < p.x, by = rooty < p.y;
-        float x = rootx + (bx ? r : -r);
-        float y = rooty + (by ? r : -r);
-        unsigned long long key = (unsigned long long)((unsigned)bx | ((unsigned)by << 1)) << 62;
-#pragma unroll
-        for (int l = 1; l < kKeyLevels; ++l) {
-            r *= 0.5f;
-            bx = x < p.x;
-            by = y < p.y;
-            key |= (unsigned long long)((unsigned)bx | ((unsigned)by << 1)) << (62 - 2 * l);
-            x += bx ? r : -r;
-            y += by ? r : -r;
-        }
+        const unsigned long long key = path_key(p, rootx, rooty, radius);
         keys[i] = key;
         vals[i] = (unsigned)i;
         pm[i] = make_float4(p.x, p.y, mass[i], 0.0f);   // one gather per body for k_lcp
@@ -205,9 +188,6 @@ __device__ int block_exclusive_scan(int v, int* total) {
     return before + inc - v;
 }
 
-// Exact moments (integer-mass path). Sums are taken modulo 2^128 on two 64-bit limbs.
-using u128 = unsigned __int128;
-
 __device__ __forceinline__ u128 mo_x(const Moment& a) { return ((u128)a.xh << 64) | a.xl; }
 __device__ __forceinline__ u128 mo_y(const Moment& a) { return ((u128)a.yh << 64) | a.yl; }
 
@@ -227,32 +207,6 @@ __device__ __forceinline__ Moment mo_sub(const Moment& a, const Moment& b) {
 __device__ __forceinline__ Moment mo_shfl_up(const Moment& v, int o) {
     return Moment{__shfl_up(v.xl, o, 64), __shfl_up(v.xh, o, 64), __shfl_up(v.yl, o, 64), __shfl_up(v.yh, o, 64),
                   __shfl_up(v.m, o, 64)};
-}
-
-// Fixed-point exponent of a graph whose root radius is R < 2^e: a coordinate relative to the
-// root centre lies within a few R (the centre and radius are rounded floats), so scaled by
-// 2^(58-e) it stays below 2^61 in magnitude. R = 0 (one point) gives coordinates 0.
-__device__ __forceinline__ int moment_shift(float radius) {
-    int e = 0;
-    (void)frexpf(radius, &e);
-    return 58 - e;
-}
-
-__device__ __forceinline__ long long fixed_coord(float p, float c, int s) {
-    double t = ldexp((double)p - (double)c, s);
-    t = fmin(fmax(t, -0x1p62), 0x1p62);
-    return (long long)rint(t);
-}
-
-// The signed 128-bit value hi*2^64 + lo as a double (magnitude converted, so small negative
-// values keep their precision).
-__device__ __forceinline__ double i128_to_double(unsigned long long lo, unsigned long long hi) {
-    u128 v = ((u128)hi << 64) | lo;
-    const bool neg = (long long)hi < 0;
-    if (neg) v = (u128)0 - v;
-    const unsigned long long vh = (unsigned long long)(v >> 64), vl = (unsigned long long)v;
-    const double mag = vh == 0ull ? (double)vl : (double)vh * 0x1p64 + (double)vl;
-    return neg ? -mag : mag;
 }
 
 // Block-wide exclusive scan of one Moment per thread (NT threads); *total gets the sum.

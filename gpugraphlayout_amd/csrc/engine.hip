@@ -180,7 +180,9 @@ void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
     // can run on a second stream: beside the walk (mode 1: the walk is launched split and
     // k_combine forms F afterwards, as the fused epilogue would), or beside keys, sort and tree
     // (mode 2: joined before the walk).
-    const int mode = h->p.exact ? 0 : h->tune.attraction_stream;
+    // A small graph's tree is one launch that carries the attraction along, in every mode.
+    const bool small = !h->p.exact && small_tree(b);
+    const int mode = h->p.exact || small ? 0 : h->tune.attraction_stream;
     auto attraction_on_side = [&]() {
         hipEventRecord(h->fork, s);
         hipStreamWaitEvent(h->side, h->fork, 0);
@@ -192,13 +194,13 @@ void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
     mark(0, s);
     if (mode == 0) {
         mark(1, s);
-        launch_attraction(b, h->p, s);
+        if (!small) launch_attraction(b, h->p, s);
         mark(2, s);
     } else if (mode == 2) {
         attraction_on_side();
     }
     mark(3, s);
-    if (!h->p.exact) {
+    if (!h->p.exact && !small) {
         if (b.nseg > 1) {
             if (!advance_seg(b)) launch_seg_bbox(b, s);
             launch_seg_keys(b, s);
@@ -207,7 +209,7 @@ void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
         }
     }
     mark(4, s);
-    if (!h->p.exact) {
+    if (!h->p.exact && !small) {
         if (b.nseg > 1 && b.max_seg <= kSegSortMax) {
             // every graph fits one block's sort: by (graph, key) in one launch, the low passes
             // skipped as for one graph; the result is in buffer 0 and runs stop at graphs
@@ -224,7 +226,8 @@ void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
         }
     }
     mark(5, s);
-    if (!h->p.exact) launch_tree(b, s);
+    if (small) launch_small_tree(b, h->p, s);
+    else if (!h->p.exact) launch_tree(b, s);
     mark(6, s);
     if (mode == 1) attraction_on_side();
     if (mode == 2) hipStreamWaitEvent(s, h->join, 0);
@@ -337,7 +340,8 @@ int device_error(int err) {
 int read_state(gfa2_engine* h, DevState* st) {
     GFA2_TRY(hipMemcpyAsync(st, h->b.st, sizeof(DevState), hipMemcpyDeviceToHost, h->stream));
     GFA2_TRY(hipStreamSynchronize(h->stream));
-    set_sort_first(h, std::max(0, std::min(st->sort_skip, 7) - 1));
+    // (a small graph's sort is inside its tree's launch)
+    if (!small_tree(h->b)) set_sort_first(h, std::max(0, std::min(st->sort_skip, 7) - 1));
     return GFA2_OK;
 }
 
@@ -644,6 +648,10 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
         b.int_mass = whole && total < 16777216.0 * 62.0;
         // no cell (a part of one graph) can reach 2^24
         b.no_big = total < 16777216.0;
+        if (small_tree(b)) {
+            b.kids_blocks = 1;
+            b.sort.hist_in_keys = false;
+        }
     }
     if (b.int_mass) {
         GFA2_ALLOC(b.pmass, (size_t)n + 1);

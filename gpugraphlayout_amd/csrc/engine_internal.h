@@ -260,6 +260,17 @@ void launch_bbox_partials(const Bufs& b, hipStream_t s);
 // the passes that will run end in buffer 0.
 void launch_keys(const Bufs& b, int first, hipStream_t s);
 void launch_tree(Bufs& b, hipStream_t s);              // after the sort: cells + summaries
+// A graph whose attraction, keys, sort and tree are one launch (two with the keys apart), in
+// place of launch_attraction, launch_keys, the sort and launch_tree. One compute unit does the
+// tree, so its time grows with the bodies while the launches it saves do not. Measured per
+// iteration (Barabasi-Albert, m = 5), launches against one block: 100 nodes 53 / 26 us, 500 72 /
+// 36, 2,048 95 / 56, 4,096 97 / 76; an 8,192-body form took 99 us at 5,000 (launches 99) and 131
+// at 8,000 (103). Up to kSmallOwnKeys the block forms the keys too (a wide launch is quicker
+// beyond) and keeps the prefix moments in LDS.
+constexpr int kSmallTree = 4096;
+constexpr int kSmallOwnKeys = 2048;
+bool small_tree(const Bufs& b);
+void launch_small_tree(const Bufs& b, const Params& p, hipStream_t s);
 // split: the walk writes the repulsion alone (F_ga is not read), and launch_combine, after
 // both the walk and the attraction, forms F and the swing/traction sums.
 void launch_walk(const Bufs& b, const Params& p, bool split, hipStream_t s);

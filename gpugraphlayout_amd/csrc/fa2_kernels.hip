@@ -1,4 +1,5 @@
 // ForceAtlas2 force, speed and displacement kernels for gfx950 (FP32 VALU throughout).
+#include "attract_device.h"
 #include "engine_internal.h"
 
 #include <algorithm>
@@ -17,68 +18,6 @@ namespace {
 //   medium (deg <= 2048): one wave per node, lane-strided sums + butterfly reduction
 //   heavy: one 256-thread block per node, thread-strided sums + LDS tree reduction
 // ---------------------------------------------------------------------------------------
-constexpr int kLightMax = 32;
-
-__device__ __forceinline__ float2 gravity(float2 p, float m, int strong, float k_g) {
-    float fg;
-    if (strong) fg = k_g * m;
-    else if (p.x != 0.0f || p.y != 0.0f) fg = k_g * m * rsqrtf(p.x * p.x + p.y * p.y);
-    else fg = 0.0f;
-    return make_float2(-p.x * fg, -p.y * fg);
-}
-
-// One edge's attraction term on node p from neighbour q. Linear: q - p. With linlog (the
-// reference's CPU rule, src/RPCPUForceAtlas2.cpp:63-67): (q - p) * log(1 + d) / d, and 0 at
-// d = 0 (the reference multiplies the zero vector by FLT_MAX there). With edge weights:
-// times w^delta.
-template <bool GEN>
-__device__ __forceinline__ void attract_term(float2 p, float2 q, int linlog, const float* __restrict__ ew, int e,
-                                             float& ax, float& ay) {
-    const float dx = q.x - p.x;
-    const float dy = q.y - p.y;
-    if constexpr (!GEN) {
-        ax += dx;
-        ay += dy;
-    } else {
-        float fa = 1.0f;
-        if (linlog) {
-            const float d = sqrtf(dx * dx + dy * dy);
-            fa = d == 0.0f ? 0.0f : logf(1.0f + d) / d;
-        }
-        if (ew) fa *= ew[e];
-        ax += dx * fa;
-        ay += dy * fa;
-    }
-}
-
-// The terms of CSR entries e, e + S, e + 2S, ... below e1, added in that order. Four entries at
-// a time: their index and position loads are all issued before the first term is added (the
-// loads past e1 read node 0 and are not added), so a row's tail costs no more round trips to
-// memory than a full group of four.
-// With HUB, the positions of the kHubCache highest-degree nodes come from the block's LDS copy
-// (hub), which spares the L2 the most requested lines.
-constexpr int kHubCache = 2048;
-
-template <bool GEN, int S, bool HUB>
-__device__ __forceinline__ void gather_terms(float2 p, const float2* __restrict__ pos_rank,
-                                             const float2* hub, const int* __restrict__ col, int e, int e1,
-                                             int linlog, const float* __restrict__ ew, float& ax, float& ay) {
-    for (; e < e1; e += 4 * S) {
-        int j[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) j[u] = e + u * S < e1 ? col[e + u * S] : 0;
-        float2 q[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            if (HUB && j[u] < kHubCache) q[u] = hub[j[u]];
-            else q[u] = pos_rank[j[u]];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (e + u * S < e1) attract_term<GEN>(p, q[u], linlog, ew, e + u * S, ax, ay);
-    }
-}
-
 // col_rank[e] = rank[col[e]] (once per graph).
 __global__ __launch_bounds__(256) void k_gather_rank(const int* __restrict__ col, const int* __restrict__ rank,
                                                      long long nnz, int* __restrict__ col_rank) {
@@ -120,42 +59,17 @@ __global__ __launch_bounds__(256) void k_attract(const float2* __restrict__ pos,
         for (int i = tid; i < kHubCache && i < n; i += 256) hub[i] = pos_rank[i];
         __syncthreads();
     }
+    const AttractArgs A{pos, mass, n, pos_rank, rowptr, col, lists, nlight, nmedium, strong, k_g, fga, linlog, ew};
     const int total = light_blocks + medium_blocks + nchunks;
     for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {   // uniform per block
         int blk = vb;
         if (blk < light_blocks) {
-            const int k = blk * 256 + tid;
-            if (k < nlight) {
-                const int v = lists[k];
-                const float2 p = pos[v];
-                float ax = 0.0f, ay = 0.0f;
-                const int e1 = rowptr[v + 1];
-                gather_terms<GEN, 1, HUB>(p, pos_rank, hub, col, rowptr[v], e1, linlog, ew, ax, ay);
-                const float2 g = gravity(p, mass[v], strong, k_g);
-                fga[v] = make_float2(g.x + ax, g.y + ay);
-            }
+            attract_light<GEN, HUB>(blk * 256 + tid, A, hub);
             continue;
         }
         blk -= light_blocks;
         if (blk < medium_blocks) {
-            const int k = blk * 4 + (tid >> 6);
-            if (k < nmedium) {    // uniform per wave
-                const int lane = tid & 63;
-                const int v = lists[nlight + k];
-                const float2 p = pos[v];
-                float ax = 0.0f, ay = 0.0f;
-                const int e1 = rowptr[v + 1];
-                gather_terms<GEN, 64, HUB>(p, pos_rank, hub, col, rowptr[v] + lane, e1, linlog, ew, ax, ay);
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) {
-                    ax += __shfl_xor(ax, o, 64);
-                    ay += __shfl_xor(ay, o, 64);
-                }
-                if (lane == 0) {
-                    const float2 g = gravity(p, mass[v], strong, k_g);
-                    fga[v] = make_float2(g.x + ax, g.y + ay);
-                }
-            }
+            attract_medium<GEN, HUB>(blk * 4 + (tid >> 6), tid & 63, A, hub);
             continue;
         }
         blk -= medium_blocks;
