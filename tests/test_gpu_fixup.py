@@ -33,13 +33,22 @@ def longest_tie(order, key, bits):
     return int(np.diff(edge).max())
 
 
-def test_one_graph():
-    print("case fix-up, one graph", flush=True)
+@pytest.mark.parametrize("weight,least", [(1.0, 2), (1e7, 17), (1e9, 65), (1e14, 500)])
+def test_one_graph(weight, least):
+    """After the full sorts one edge gets the given weight: the bodies it flings away widen the
+    root box, and the others share digits that the previous tree's cells had left to the sort."""
+    print(f"case fix-up, one graph, weight {weight}", flush=True)
     pos, src, dst = clumps(90, 1)
-    eng = Engine(len(pos), src, dst, scale=1e-6, gravity=0.0, strong_gravity=1, cell_factor=40)
+    eng = Engine(len(pos), src, dst, scale=1e-6, gravity=0.0, strong_gravity=1, cell_factor=40,
+                 edge_weight_influence=1.0)
+    eng.set_edge_weights(np.ones(2 * len(src), np.float32))
     eng.set_positions(pos)
     prev, longest = None, 0
-    for it in range(14):
+    for it in range(10):
+        if it == 6:
+            w = np.ones(2 * len(src), np.float32)
+            w[0] = weight             # node 0's first entry
+            eng.set_edge_weights(w)
         p = eng.positions()
         eng.step(1)
         eng.sync()
@@ -49,8 +58,7 @@ def test_one_graph():
         if prev is not None and it > FULL_SORTS_AFTER_NEW:
             longest = max(longest, longest_tie(order, key, 8 * sorted_passes(prev)))
         prev = tree
-    print(f"longest tied run {longest}", flush=True)
-    assert longest >= 2
+    assert longest >= least
     eng.close()
 
 
