@@ -53,62 +53,114 @@ __device__ __forceinline__ void attract_term(float2 p, float2 q, int linlog, con
     }
 }
 
-// The terms of CSR entries e, e + S, e + 2S, ... below e1, added in that order. Four entries at
-// a time: their index and position loads are all issued before the first term is added (the
-// loads past e1 read node 0 and are not added), so a row's tail costs no more round trips to
-// memory than a full group of four.
-// With HUB, the positions of the kHubCache highest-degree nodes come from the block's LDS copy
-// (hub), which spares the L2 the most requested lines.
-constexpr int kHubCache = 2048;
+// One row, or a part of one: len CSR entries from first.
+struct Row {
+    const int* col;
+    const float* ew;
+    int len;
+    __device__ __forceinline__ Row(const AttractArgs& A, int first, int end)
+        : col(A.col + first), ew(A.ew ? A.ew + first : nullptr), len(end - first) {}
+};
 
-template <bool GEN, int S, bool HUB>
-__device__ __forceinline__ void gather_terms(float2 p, const float2* __restrict__ pos_rank,
-                                             const float2* hub, const int* __restrict__ col, int e, int e1,
-                                             int linlog, const float* __restrict__ ew, float& ax, float& ay) {
-    for (; e < e1; e += 4 * S) {
+// Entries i, i + S, i + 2S, i + 3S of the row (0 past its end) ...
+template <int S>
+__device__ __forceinline__ void load_four(const Row& R, int i, int (&j)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) j[u] = i + u * S < R.len ? R.col[i + u * S] : 0;
+}
+
+// ... and their terms, added in that order. The position loads are all issued before the first
+// term is added (those past the end read node 0 and are not added), so a row's tail costs no more
+// round trips to memory than a full group of four.
+// The positions of the HUB highest-degree nodes (HUB > 0) come from the block's LDS copy (hub),
+// which spares the L2 the most requested lines.
+template <int HUB>
+__device__ __forceinline__ void load_positions(const float2* __restrict__ pos_rank, const float2* hub,
+                                               const int (&j)[4], float2 (&q)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        if (j[u] < HUB) q[u] = hub[j[u]];
+        else q[u] = pos_rank[j[u]];
+    }
+}
+
+template <bool GEN, int S>
+__device__ __forceinline__ void add_four(float2 p, const Row& R, int i, const float2 (&q)[4], int linlog, float& ax,
+                                         float& ay) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        if (i + u * S < R.len) attract_term<GEN>(p, q[u], linlog, R.ew, i + u * S, ax, ay);
+}
+
+// The terms of entries i, i + S, i + 2S, ... of the row, four at a time.
+template <bool GEN, int S, int HUB>
+__device__ __forceinline__ void gather_terms(float2 p, const AttractArgs& A, const float2* hub, const Row& R, int i,
+                                             float& ax, float& ay) {
+    for (; i < R.len; i += 4 * S) {
         int j[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) j[u] = e + u * S < e1 ? col[e + u * S] : 0;
+        load_four<S>(R, i, j);
         float2 q[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            if (HUB && j[u] < kHubCache) q[u] = hub[j[u]];
-            else q[u] = pos_rank[j[u]];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (e + u * S < e1) attract_term<GEN>(p, q[u], linlog, ew, e + u * S, ax, ay);
+        load_positions<HUB>(A.pos_rank, hub, j, q);
+        add_four<GEN, S>(p, R, i, q, A.linlog, ax, ay);
     }
 }
 
 // Light row k of the list (one thread): gravity + the row's entries in order.
-template <bool GEN, bool HUB>
+template <bool GEN, int HUB>
 __device__ __forceinline__ void attract_light(int k, const AttractArgs& A, const float2* hub) {
     if (k >= A.nlight) return;
     const int v = A.lists[k];
     const float2 p = A.pos[v];
     float ax = 0.0f, ay = 0.0f;
-    gather_terms<GEN, 1, HUB>(p, A.pos_rank, hub, A.col, A.rowptr[v], A.rowptr[v + 1], A.linlog, A.ew, ax, ay);
+    gather_terms<GEN, 1, HUB>(p, A, hub, Row(A, A.rowptr[v], A.rowptr[v + 1]), 0, ax, ay);
     const float2 g = gravity(p, A.mass[v], A.strong, A.k_g);
     A.fga[v] = make_float2(g.x + ax, g.y + ay);
 }
 
-// Medium row k (one wave): lane-strided sums, then a butterfly.
-template <bool GEN, bool HUB>
-__device__ __forceinline__ void attract_medium(int k, int lane, const AttractArgs& A, const float2* hub) {
-    if (k >= A.nmedium) return;      // uniform per wave
-    const int v = A.lists[A.nlight + k];
-    const float2 p = A.pos[v];
-    float ax = 0.0f, ay = 0.0f;
-    gather_terms<GEN, 64, HUB>(p, A.pos_rank, hub, A.col, A.rowptr[v] + lane, A.rowptr[v + 1], A.linlog, A.ew, ax, ay);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        ax += __shfl_xor(ax, o, 64);
-        ay += __shfl_xor(ay, o, 64);
+// Medium rows k0 to k0 + rows - 1 (one wave, rows <= kMediumBatch): lane-strided sums, then a
+// butterfly. What bounds a row of some hundred entries is its chain of dependent loads (id, bounds,
+// indices, positions). So the rows' ids, bounds and positions are read by a lane each, and the
+// next row's first 256 indices are under way while this row's positions arrive. R-MAT 2^22 (64M
+// entries, 278k such rows): the attraction 462 -> 424 us with the blocks' order in k_attract; batches
+// of 8 are slower where long rows follow one another (BA, 1M bodies: 663 -> 702 us an iteration).
+constexpr int kMediumBatch = 4;
+
+template <bool GEN, int HUB>
+__device__ __forceinline__ void attract_medium(int k0, int rows, int lane, const AttractArgs& A, const float2* hub) {
+    k0 = __builtin_amdgcn_readfirstlane(k0);
+    const int nb = min(rows, A.nmedium - k0);
+    if (nb <= 0) return;             // uniform per wave
+    int v = 0, e0 = 0, e1 = 0;
+    float2 p = make_float2(0.0f, 0.0f), sum = p;
+    if (lane < nb) {
+        v = A.lists[A.nlight + k0 + lane];
+        e0 = A.rowptr[v];
+        e1 = A.rowptr[v + 1];
+        p = A.pos[v];
     }
-    if (lane == 0) {
+    int j[4];
+    load_four<64>(Row(A, __builtin_amdgcn_readlane(e0, 0), __builtin_amdgcn_readlane(e1, 0)), lane, j);
+    for (int r = 0; r < nb; ++r) {
+        const Row R(A, __builtin_amdgcn_readlane(e0, r), __builtin_amdgcn_readlane(e1, r));
+        const float2 pr = make_float2(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(p.x), r)),
+                                      __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p.y), r)));
+        float2 q[4];
+        load_positions<HUB>(A.pos_rank, hub, j, q);
+        if (r + 1 < nb)
+            load_four<64>(Row(A, __builtin_amdgcn_readlane(e0, r + 1), __builtin_amdgcn_readlane(e1, r + 1)), lane, j);
+        float ax = 0.0f, ay = 0.0f;
+        add_four<GEN, 64>(pr, R, lane, q, A.linlog, ax, ay);
+        gather_terms<GEN, 64, HUB>(pr, A, hub, R, lane + 256, ax, ay);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            ax += __shfl_xor(ax, o, 64);
+            ay += __shfl_xor(ay, o, 64);
+        }
+        if (lane == r) sum = make_float2(ax, ay);
+    }
+    if (lane < nb) {
         const float2 g = gravity(p, A.mass[v], A.strong, A.k_g);
-        A.fga[v] = make_float2(g.x + ax, g.y + ay);
+        A.fga[v] = make_float2(g.x + sum.x, g.y + sum.y);
     }
 }
 

@@ -36,49 +36,51 @@ __global__ __launch_bounds__(256) void k_rank_pos(const float2* __restrict__ pos
 // Attraction + gravity, fga[v] = gravity(v) + sum over CSR entries of v (in entry order for the
 // light rows; lane-strided then a shuffle tree for medium rows; see below for heavy rows).
 // Degree classes: light rows (<= 32 entries) one thread each, entries four at a time;
-// medium rows (<= 2,048) one wave each; heavy rows in chunks of kAttrChunk entries, one block
+// medium rows (<= 2,048) one wave each, or up to kMediumBatch to a wave; heavy rows in chunks of kAttrChunk entries, one block
 // per chunk writing its partial (thread-strided, then an LDS tree), added per row in chunk order
 // by k_attract_heavy. Neighbour positions come from the degree-ranked copy. The work is a list
-// of virtual blocks (light, medium, chunks) that the grid strides over: one launch block per
-// virtual block by default, or a smaller grid that leaves room on every compute unit for
-// kernels running beside it on another stream. Every row's sum is the same whatever the grid.
-template <bool GEN, bool HUB>
+// of virtual blocks that the grid strides over: one launch block per virtual block by default, or
+// a smaller grid that leaves room on every compute unit for kernels running beside it on another
+// stream. Every row's sum is the same whatever the grid. The chunks come first, being longest;
+// light and medium blocks then take turns in proportion, since the light rows wait on their
+// serial loads and the medium ones on the L2 (1M bodies, 32M entries, half of them in either: 919 us
+// an iteration with the light blocks first, 934 with them last, 888 in turns).
+constexpr int kHubCache = 2048;      // hubs' positions in LDS: 16 KB, so that 8 blocks fit a CU
+
+template <bool GEN, int HUB>
 __global__ __launch_bounds__(256) void k_attract(const float2* __restrict__ pos, const float* __restrict__ mass,
                                                  int n, const float2* __restrict__ pos_rank,
                                                  const int* __restrict__ rowptr, const int* __restrict__ col,
                                                  const int* __restrict__ lists, int nlight, int nmedium,
                                                  const int2* __restrict__ chunks, int nchunks,
-                                                 int light_blocks, int medium_blocks,
+                                                 int light_blocks, int medium_blocks, int medium_rows,
                                                  int strong, float k_g, float2* __restrict__ fga,
                                                  float2* __restrict__ part, int linlog,
                                                  const float* __restrict__ ew) {
     __shared__ float2 red[256];
-    __shared__ float2 hub[HUB ? kHubCache : 1];
+    __shared__ float2 hub[HUB > 0 ? HUB : 1];
     const int tid = threadIdx.x;
-    if constexpr (HUB) {
-        for (int i = tid; i < kHubCache && i < n; i += 256) hub[i] = pos_rank[i];
+    if constexpr (HUB > 0) {
+        for (int i = tid; i < HUB && i < n; i += 256) hub[i] = pos_rank[i];
         __syncthreads();
     }
     const AttractArgs A{pos, mass, n, pos_rank, rowptr, col, lists, nlight, nmedium, strong, k_g, fga, linlog, ew};
     const int total = light_blocks + medium_blocks + nchunks;
     for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {   // uniform per block
-        int blk = vb;
-        if (blk < light_blocks) {
-            attract_light<GEN, HUB>(blk * 256 + tid, A, hub);
+        if (vb >= nchunks) {
+            const unsigned int i = vb - nchunks, t = light_blocks + medium_blocks;
+            const int m0 = (int)((unsigned long long)i * medium_blocks / t);          // medium blocks before i
+            const int m1 = (int)((i + 1ull) * medium_blocks / t);
+            if (m1 > m0) attract_medium<GEN, HUB>((m0 * 4 + (tid >> 6)) * medium_rows, medium_rows, tid & 63, A, hub);
+            else attract_light<GEN, HUB>(((int)i - m0) * 256 + tid, A, hub);
             continue;
         }
-        blk -= light_blocks;
-        if (blk < medium_blocks) {
-            attract_medium<GEN, HUB>(blk * 4 + (tid >> 6), tid & 63, A, hub);
-            continue;
-        }
-        blk -= medium_blocks;
-        const int2 ch = chunks[blk];
+        const int2 ch = chunks[vb];
         const int v = lists[nlight + nmedium + ch.x];
         const float2 p = pos[v];
         float ax = 0.0f, ay = 0.0f;
-        const int e1 = min(ch.y + kAttrChunk, rowptr[v + 1]);
-        gather_terms<GEN, 256, HUB>(p, pos_rank, hub, col, ch.y + tid, e1, linlog, ew, ax, ay);
+        const int len = min(kAttrChunk, rowptr[v + 1] - ch.y);
+        gather_terms<GEN, 256, HUB>(p, A, hub, Row(A, ch.y, ch.y + len), tid, ax, ay);
         red[tid] = make_float2(ax, ay);
         __syncthreads();
         for (int o = 128; o > 0; o >>= 1) {
@@ -88,7 +90,7 @@ __global__ __launch_bounds__(256) void k_attract(const float2* __restrict__ pos,
             }
             __syncthreads();
         }
-        if (tid == 0) part[blk] = red[0];
+        if (tid == 0) part[vb] = red[0];
         // red[0] is written again only by thread 0, and every other entry only after the
         // barriers above, so the next virtual block may start at once
     }
@@ -1041,7 +1043,10 @@ void launch_col_rank(const Bufs& b, hipStream_t s) {
 
 void launch_attraction(const Bufs& b, const Params& p, hipStream_t s) {
     const int lb = (b.nlight + 255) / 256;
-    const int mb = (b.nmedium + 3) / 4;
+    // several medium rows to a wave once one each would more than fill the card (8 waves on each
+    // of 1,024 SIMDs): with one each, R-MAT 2^18 at 4M entries took 182 us an iteration against 176
+    const int rows = std::max(1, std::min(kMediumBatch, b.nmedium / 8192));
+    const int mb = (b.nmedium + 4 * rows - 1) / (4 * rows);
     int total = lb + mb + b.nattr_chunks;
     if (b.attr_grid > 0 && total > b.attr_grid) total = b.attr_grid;   // the launch grid
     if (total > 0) {
@@ -1051,15 +1056,15 @@ void launch_attraction(const Bufs& b, const Params& p, hipStream_t s) {
         const bool gen = p.linlog || b.ew;
 #define GFA2_ATTRACT(G, H)                                                                                   \
     k_attract<G, H><<<total, 256, 0, s>>>(b.pos, b.mass, b.n, b.pos_rank, b.rowptr, b.col_rank, b.node_lists,   \
-                                          b.nlight, b.nmedium, b.attr_chunks, b.nattr_chunks, lb, mb,         \
+                                          b.nlight, b.nmedium, b.attr_chunks, b.nattr_chunks, lb, mb, rows,     \
                                           p.strong_gravity, p.k_g, b.fga, b.attr_part, G ? p.linlog : 0,      \
                                           G ? b.ew : nullptr)
         if (gen) {
-            if (hub) GFA2_ATTRACT(true, true);
-            else GFA2_ATTRACT(true, false);
+            if (hub) GFA2_ATTRACT(true, kHubCache);
+            else GFA2_ATTRACT(true, 0);
         } else {
-            if (hub) GFA2_ATTRACT(false, true);
-            else GFA2_ATTRACT(false, false);
+            if (hub) GFA2_ATTRACT(false, kHubCache);
+            else GFA2_ATTRACT(false, 0);
         }
 #undef GFA2_ATTRACT
     }

@@ -568,8 +568,8 @@ __global__ __launch_bounds__(kThreads) void k_small_tree(SmallArgs A, AttractArg
     }
     const int sub = threadIdx.x >> 8, tid = threadIdx.x & 255;
     for (int vb = (blockIdx.x - 1) * 4 + sub; vb < virtual_blocks; vb += (gridDim.x - 1) * 4) {
-        if (vb < light_blocks) attract_light<GEN, false>(vb * 256 + tid, at, nullptr);
-        else attract_medium<GEN, false>((vb - light_blocks) * 4 + (tid >> 6), tid & 63, at, nullptr);
+        if (vb < light_blocks) attract_light<GEN, 0>(vb * 256 + tid, at, nullptr);
+        else attract_medium<GEN, 0>((vb - light_blocks) * 4 + (tid >> 6), 1, tid & 63, at, nullptr);
     }
 }
 
