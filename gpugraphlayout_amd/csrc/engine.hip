@@ -187,14 +187,14 @@ void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
         hipEventRecord(h->fork, s);
         hipStreamWaitEvent(h->side, h->fork, 0);
         mark(1, h->side);
-        launch_attraction(b, h->p, h->side);
+        launch_attraction(b, h->p, false, h->side);
         mark(2, h->side);
         hipEventRecord(h->join, h->side);
     };
     mark(0, s);
     if (mode == 0) {
         mark(1, s);
-        if (!small) launch_attraction(b, h->p, s);
+        if (!small) launch_attraction(b, h->p, true, s);
         mark(2, s);
     } else if (mode == 2) {
         attraction_on_side();
@@ -661,6 +661,7 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
         GFA2_ALLOC(b.big_lvl, kMaxBig);
     }
 #undef GFA2_ALLOC
+    b.cus = h->cus;
     b.nlight = nlight;
     b.nmedium = (int)medium.size();
     b.nheavy = (int)heavy.size();
@@ -682,7 +683,12 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
         for (int v = 0; v < n; ++v) ++start[(size_t)(maxdeg - (rp32[v + 1] - rp32[v])) + 1];
         for (int d = 0; d <= maxdeg; ++d) start[(size_t)d + 1] += start[(size_t)d];
         std::vector<int> rank((size_t)n);
-        for (int v = 0; v < n; ++v) rank[v] = start[(size_t)(maxdeg - (rp32[v + 1] - rp32[v]))]++;
+        b.hub_entries = 0;
+        for (int v = 0; v < n; ++v) {
+            const int deg = rp32[v + 1] - rp32[v];
+            rank[v] = start[(size_t)(maxdeg - deg)]++;
+            if (rank[v] < kWideHubs) b.hub_entries += deg;
+        }
         GFA2_TRY(hipMemcpyAsync(b.rank, rank.data(), sizeof(int) * n, hipMemcpyHostToDevice, h->stream));
         launch_col_rank(b, h->stream);
         GFA2_TRY(hipStreamSynchronize(h->stream));   // rank goes out of scope

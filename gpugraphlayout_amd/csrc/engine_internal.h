@@ -109,6 +109,8 @@ struct LaunchConfig {
     int attraction_bpc;     // attraction grid per CU (0: one block per virtual block)
 };
 
+constexpr int kWideHubs = 8192;     // hubs' positions in LDS (k_attract_wide)
+constexpr long long kWideEntries = 1 << 24;     // least entries for it (launch_attraction)
 constexpr int kAttrChunk = 4096;    // entries per block for rows over 2,048 entries
 
 // All device buffers of one instance.
@@ -130,6 +132,8 @@ struct Bufs {
     int2* attr_chunks;      // {heavy index h, first entry}
     int* attr_c0;           // [nheavy + 1] first chunk of each heavy row
     float2* attr_part;      // [nattr_chunks]
+    long long hub_entries;  // entries of the kWideHubs longest rows
+    int cus;
     // Attraction gathers neighbour positions from a copy ordered by decreasing degree: the
     // positions most edges point at share few cache lines. pos_rank[rank[v]] = pos[v] and
     // col_rank[e] = rank[col[e]], so pos_rank[col_rank[e]] is pos[col[e]], bit for bit.
@@ -253,7 +257,8 @@ void segmented_sort_pairs(SortBuffers& buf, const int* node_off, const int* orde
 constexpr int kSegSortMax = 32768;
 
 // Launch groups of one iteration, in order.
-void launch_attraction(const Bufs& b, const Params& p, hipStream_t s);
+// alone: no other kernel is to run beside it
+void launch_attraction(const Bufs& b, const Params& p, bool alone, hipStream_t s);
 void launch_col_rank(const Bufs& b, hipStream_t s);
 void launch_bbox_partials(const Bufs& b, hipStream_t s);
 // first: the lowest path-key sort pass the host launches; the keys go to the buffer from which

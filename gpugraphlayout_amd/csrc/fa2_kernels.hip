@@ -33,6 +33,31 @@ __global__ __launch_bounds__(256) void k_rank_pos(const float2* __restrict__ pos
     if (v < n) pos_rank[rank[v]] = pos[v];
 }
 
+// Block i of the light and medium ones, which take turns in proportion (256 threads).
+template <bool GEN, int HUB>
+__device__ __forceinline__ void attract_rows(int i, int light_blocks, int medium_blocks, int medium_rows, int tid,
+                                             const AttractArgs& A, const float2* hub) {
+    const unsigned int t = light_blocks + medium_blocks;
+    const int m0 = (int)((unsigned long long)i * medium_blocks / t);          // medium blocks before i
+    const int m1 = (int)((i + 1ull) * medium_blocks / t);
+    if (m1 > m0) attract_medium<GEN, HUB>((m0 * 4 + (tid >> 6)) * medium_rows, medium_rows, tid & 63, A, hub);
+    else attract_light<GEN, HUB>((i - m0) * 256 + tid, A, hub);
+}
+
+// red[0] = the sum over 256 threads. red[0] is written again only by thread 0, and every other
+// entry only after the barriers here, so thread 0 may read it after the call.
+__device__ __forceinline__ void sum_chunk(float2* red, int tid, float ax, float ay) {
+    red[tid] = make_float2(ax, ay);
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (tid < o) {
+            const float2 a = red[tid], b = red[tid + o];
+            red[tid] = make_float2(a.x + b.x, a.y + b.y);
+        }
+        __syncthreads();
+    }
+}
+
 // Attraction + gravity, fga[v] = gravity(v) + sum over CSR entries of v (in entry order for the
 // light rows; lane-strided then a shuffle tree for medium rows; see below for heavy rows).
 // Degree classes: light rows (<= 32 entries) one thread each, entries four at a time;
@@ -68,11 +93,7 @@ __global__ __launch_bounds__(256) void k_attract(const float2* __restrict__ pos,
     const int total = light_blocks + medium_blocks + nchunks;
     for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {   // uniform per block
         if (vb >= nchunks) {
-            const unsigned int i = vb - nchunks, t = light_blocks + medium_blocks;
-            const int m0 = (int)((unsigned long long)i * medium_blocks / t);          // medium blocks before i
-            const int m1 = (int)((i + 1ull) * medium_blocks / t);
-            if (m1 > m0) attract_medium<GEN, HUB>((m0 * 4 + (tid >> 6)) * medium_rows, medium_rows, tid & 63, A, hub);
-            else attract_light<GEN, HUB>(((int)i - m0) * 256 + tid, A, hub);
+            attract_rows<GEN, HUB>(vb - nchunks, light_blocks, medium_blocks, medium_rows, tid, A, hub);
             continue;
         }
         const int2 ch = chunks[vb];
@@ -81,19 +102,44 @@ __global__ __launch_bounds__(256) void k_attract(const float2* __restrict__ pos,
         float ax = 0.0f, ay = 0.0f;
         const int len = min(kAttrChunk, rowptr[v + 1] - ch.y);
         gather_terms<GEN, 256, HUB>(p, A, hub, Row(A, ch.y, ch.y + len), tid, ax, ay);
-        red[tid] = make_float2(ax, ay);
-        __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if (tid < o) {
-                float2 a = red[tid], b = red[tid + o];
-                red[tid] = make_float2(a.x + b.x, a.y + b.y);
-            }
-            __syncthreads();
-        }
+        sum_chunk(red, tid, ax, ay);
         if (tid == 0) part[vb] = red[0];
-        // red[0] is written again only by thread 0, and every other entry only after the
-        // barriers above, so the next virtual block may start at once
     }
+}
+
+// The same sums on one stream where many entries are of hubs: blocks of kWideThreads that stay on
+// the chip, two to a compute unit, with the positions of the kWideHubs highest-degree nodes in
+// 64 KB of LDS. The gathers are bound by the L2, which each serves as a request of its own, and by
+// the lines it misses; the copy takes a third of the requests away (R-MAT 2^22: 33% of 64M
+// entries). There 424 -> 368 us.
+constexpr int kWideThreads = 1024, kWideSubs = kWideThreads / 256;
+
+template <bool GEN>
+__global__ __launch_bounds__(kWideThreads) void k_attract_wide(const AttractArgs A, const int2* __restrict__ chunks,
+                                                               int nchunks, int light_blocks, int medium_blocks,
+                                                               int medium_rows, float2* __restrict__ part) {
+    __shared__ float2 hub[kWideHubs];
+    __shared__ float2 red_all[kWideThreads];
+    const int tid = threadIdx.x & 255, sub = threadIdx.x >> 8;
+    float2* red = red_all + sub * 256;
+    for (int i = threadIdx.x; i < kWideHubs && i < A.n; i += kWideThreads) hub[i] = A.pos_rank[i];
+    __syncthreads();
+    // chunks: one to each of the block's quarters at a time (the loop is uniform per block)
+    for (int base = blockIdx.x * kWideSubs; base < nchunks; base += gridDim.x * kWideSubs) {
+        const int c = base + sub;
+        float ax = 0.0f, ay = 0.0f;
+        if (c < nchunks) {
+            const int2 ch = chunks[c];
+            const int v = A.lists[A.nlight + A.nmedium + ch.x];
+            const int len = min(kAttrChunk, A.rowptr[v + 1] - ch.y);
+            gather_terms<GEN, 256, kWideHubs>(A.pos[v], A, hub, Row(A, ch.y, ch.y + len), tid, ax, ay);
+        }
+        sum_chunk(red, tid, ax, ay);
+        if (tid == 0 && c < nchunks) part[c] = red[0];
+    }
+    // rows: no barriers, the quarters go on by themselves
+    for (int i = blockIdx.x * kWideSubs + sub; i < light_blocks + medium_blocks; i += gridDim.x * kWideSubs)
+        attract_rows<GEN, kWideHubs>(i, light_blocks, medium_blocks, medium_rows, tid, A, hub);
 }
 
 // Heavy rows: gravity + the row's chunk partials in chunk order.
@@ -1041,19 +1087,32 @@ void launch_col_rank(const Bufs& b, hipStream_t s) {
     if (b.nnz > 0) k_gather_rank<<<(int)std::min<long long>((b.nnz + 255) / 256, 16384), 256, 0, s>>>(b.col, b.rank, b.nnz, b.col_rank);
 }
 
-void launch_attraction(const Bufs& b, const Params& p, hipStream_t s) {
+void launch_attraction(const Bufs& b, const Params& p, bool alone, hipStream_t s) {
     const int lb = (b.nlight + 255) / 256;
     // several medium rows to a wave once one each would more than fill the card (8 waves on each
     // of 1,024 SIMDs): with one each, R-MAT 2^18 at 4M entries took 182 us an iteration against 176
     const int rows = std::max(1, std::min(kMediumBatch, b.nmedium / 8192));
     const int mb = (b.nmedium + 4 * rows - 1) / (4 * rows);
     int total = lb + mb + b.nattr_chunks;
+    const bool gen = p.linlog || b.ew;
+    // The wide blocks stay until all rows are done, which pays where their staging and their uneven
+    // ends are small beside the work and hubs hold many entries (R-MAT: 8M entries 252 us an
+    // iteration without, 265 with; 20M 402, 397; 64M 1,253, 1,213; BA with 1M bodies, 20M entries,
+    // 9% of them of hubs: 667, 753), and nothing is to run beside them.
+    const bool wide = alone && b.attr_grid == 0 && b.nnz >= kWideEntries && b.hub_entries >= b.nnz / 4;
+    if (wide) {
+        const AttractArgs A{b.pos,    b.mass,    b.n,              b.pos_rank, b.rowptr, b.col_rank, b.node_lists,
+                            b.nlight, b.nmedium, p.strong_gravity, p.k_g,      b.fga,    p.linlog,   b.ew};
+        const int blocks = std::min(2 * b.cus, (total + kWideSubs - 1) / kWideSubs);
+        if (gen) k_attract_wide<true><<<blocks, kWideThreads, 0, s>>>(A, b.attr_chunks, b.nattr_chunks, lb, mb, rows, b.attr_part);
+        else k_attract_wide<false><<<blocks, kWideThreads, 0, s>>>(A, b.attr_chunks, b.nattr_chunks, lb, mb, rows, b.attr_part);
+        total = 0;
+    }
     if (b.attr_grid > 0 && total > b.attr_grid) total = b.attr_grid;   // the launch grid
     if (total > 0) {
         // a grid smaller than the work (beside other kernels): every block stages the hubs'
         // positions once and uses them for several virtual blocks
         const bool hub = b.attr_grid > 0 && lb + mb + b.nattr_chunks > 2 * total;
-        const bool gen = p.linlog || b.ew;
 #define GFA2_ATTRACT(G, H)                                                                                   \
     k_attract<G, H><<<total, 256, 0, s>>>(b.pos, b.mass, b.n, b.pos_rank, b.rowptr, b.col_rank, b.node_lists,   \
                                           b.nlight, b.nmedium, b.attr_chunks, b.nattr_chunks, lb, mb, rows,     \

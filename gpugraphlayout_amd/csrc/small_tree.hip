@@ -612,7 +612,7 @@ void launch_small_tree(const Bufs& b, const Params& p, hipStream_t s) {
                          b.nmedium, p.strong_gravity, p.k_g, b.fga,      p.linlog, b.ew};
     const bool apart = b.nheavy > 0;
     const int lb = apart ? 0 : (b.nlight + 255) / 256, vb = apart ? 0 : lb + (b.nmedium + 3) / 4;
-    if (apart) launch_attraction(b, p, s);
+    if (apart) launch_attraction(b, p, true, s);
     const bool gen = p.linlog || b.ew;
     if (b.n <= kSmallOwnKeys) {
         launch_size<2048, true>(A, at, gen, lb, vb, s);
