@@ -131,91 +131,140 @@ __global__ __launch_bounds__(256) void k_colnorm_apply(float* __restrict__ X, in
 //   kAggSmooth     out = (in[i] + sum / deg(i)) / 2                 feature smoothing
 //   kAggBack       out = H[i] > 0 ? P[i] + sum : 0                  backward of the mean and relu
 //                  (in[j] already divided by deg(j))
-// Rows of at most kHeavyDeg entries: F lanes per row, entries in CSR order (four loads in
-// flight). Longer rows (the hubs of a skewed graph, which would otherwise leave one wave
-// looping over 10^5 entries) are split into chunks of kChunk entries: one wave per chunk sums
-// its entries in 64/F interleaved slots, combined in slot order, into a partial; then one
-// thread per (row, feature) adds the row's partials in chunk order. Every sum has a fixed
-// order, so results are deterministic.
+// Light rows (at most kAggLight entries): kAggSlots slots of F / 4 lanes per row, which read a
+// float4 each of every entry of the slot; medium rows (listed): a wave per row with 256 / F slots;
+// heavy rows (over kAggHeavy entries, the hubs of a skewed graph, which would otherwise leave one
+// wave looping over 10^5 entries): a block per chunk of kAggChunk entries, whose four waves sum a
+// quarter each into a partial, added by k_agg_heavy. A slot has the loads of four or eight entries
+// under way at once, and the slots are added in a fixed tree, so results are deterministic.
+// What bounds it are the lines that the L2s miss, which come at the 4 to 5 TB/s of a plain copy
+// (R-MAT 2^20, 20M entries: F = 64 asks for 40M lines of 128 bytes; halves or quarters of the
+// features to different dies gave nothing, 681 and 862 us). There with 4-byte loads, one row after
+// another per group and 512-entry chunks in a launch of their own: F = 8 325 -> 167 us, F = 16
+// 414 -> 208, F = 64 889 -> 622.
 enum AggMode { kAggMean = 0, kAggSmooth = 1, kAggBack = 2 };
 
-template <int MODE>
-__device__ __forceinline__ float agg_finish(float s, int deg, size_t at, const float* __restrict__ in,
-                                            const float* __restrict__ P, const float* __restrict__ H) {
-    if (MODE == kAggBack) return H[at] > 0.0f ? P[at] + s : 0.0f;
-    const float m = deg > 0 ? s / (float)deg : 0.0f;
-    return MODE == kAggSmooth ? 0.5f * (in[at] + m) : m;
-}
-
-template <int F, int MODE>
-__global__ __launch_bounds__(256) void k_agg_rows(const int* __restrict__ rowptr, const int* __restrict__ col, int n,
-                                                  const float* __restrict__ in, const float* __restrict__ P,
-                                                  const float* __restrict__ H, float* __restrict__ out) {
-    constexpr int kRows = 256 / F;
-    const int f = threadIdx.x % F;
-    for (long long r0 = (long long)blockIdx.x * kRows; r0 < n; r0 += (long long)gridDim.x * kRows) {
-        const long long ii = r0 + threadIdx.x / F;
-        if (ii >= n) continue;
-        const int i = (int)ii;
-        const int e0 = rowptr[i], e1 = rowptr[i + 1];
-        if (e1 - e0 > kHeavyDeg) continue;            // the chunk path writes this row
-        float s = 0.0f;
-        int e = e0;
-        for (; e + 4 <= e1; e += 4) {
-            const int j0 = col[e], j1 = col[e + 1], j2 = col[e + 2], j3 = col[e + 3];
-            s += in[(size_t)j0 * F + f];
-            s += in[(size_t)j1 * F + f];
-            s += in[(size_t)j2 * F + f];
-            s += in[(size_t)j3 * F + f];
-        }
-        for (; e < e1; ++e) s += in[(size_t)col[e] * F + f];
-        const size_t at = (size_t)i * F + f;
-        out[at] = agg_finish<MODE>(s, e1 - e0, at, in, P, H);
-    }
-}
-
-// One wave per chunk {row, first entry}; part[c][f] = the chunk's sum.
+// Slots per light row, and entries under way at once per slot of a medium row (4 in a light one).
 template <int F>
-__global__ __launch_bounds__(256) void k_agg_chunks(const int* __restrict__ rowptr, const int* __restrict__ col,
-                                                    const int2* __restrict__ chunks, int nchunks,
-                                                    const float* __restrict__ in, float* __restrict__ part) {
-    constexpr int S = 64 / F;
-    const int lane = threadIdx.x & 63, slot = lane / F, f = lane % F;
-    for (int c = blockIdx.x * 4 + (threadIdx.x >> 6); c < nchunks; c += gridDim.x * 4) {
-        const int2 ch = chunks[c];
-        const int end = min(ch.y + kChunk, rowptr[ch.x + 1]);
-        float s = 0.0f;
-        int e = ch.y + slot;
-        for (; e + 3 * S < end; e += 4 * S) {
-            const int j0 = col[e], j1 = col[e + S], j2 = col[e + 2 * S], j3 = col[e + 3 * S];
-            s += in[(size_t)j0 * F + f];
-            s += in[(size_t)j1 * F + f];
-            s += in[(size_t)j2 * F + f];
-            s += in[(size_t)j3 * F + f];
-        }
-        for (; e < end; e += S) s += in[(size_t)col[e] * F + f];
-        float tot = 0.0f;
+constexpr int kAggSlots = F == 64 ? 1 : 4;
+template <int F>
+constexpr int kAggAhead = F == 64 ? 8 : 4;
+
+struct AggArgs {
+    const int* rowptr;
+    const int* col;
+    int n;
+    const int* medium;          // rows of more than kAggLight entries up to kAggHeavy
+    int nmedium;
+    const int* heavy;
+    const int2* chunks;         // {index into heavy, first entry}
+    int nchunks;
+    const float* in;
+    const float* P;
+    const float* H;
+    float* out;
+    float* part;                // [4 nchunks][F]
+};
+
+__device__ __forceinline__ float4 add4(float4 a, float4 b) {
+    return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+
+template <int MODE>
+__device__ __forceinline__ float agg_finish(float s, int deg, float in, float P, float H) {
+    if (MODE == kAggBack) return H > 0.0f ? P + s : 0.0f;
+    const float m = deg > 0 ? s / (float)deg : 0.0f;
+    return MODE == kAggSmooth ? 0.5f * (in + m) : m;
+}
+
+// Row i's result from its sum, features at4 to at4 + 3 of the float array.
+template <int MODE>
+__device__ __forceinline__ void agg_store(const AggArgs& A, float4 s, int deg, size_t at) {
+    const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 v = z, P = z, H = z;
+    if (MODE == kAggSmooth) v = *reinterpret_cast<const float4*>(A.in + at);
+    if (MODE == kAggBack) {
+        P = *reinterpret_cast<const float4*>(A.P + at);
+        H = *reinterpret_cast<const float4*>(A.H + at);
+    }
+    *reinterpret_cast<float4*>(A.out + at) =
+        make_float4(agg_finish<MODE>(s.x, deg, v.x, P.x, H.x), agg_finish<MODE>(s.y, deg, v.y, P.y, H.y),
+                    agg_finish<MODE>(s.z, deg, v.z, P.z, H.z), agg_finish<MODE>(s.w, deg, v.w, P.w, H.w));
+}
+
+// The sum of entries slot, slot + S, slot + 2 S, ... of len, for this lane's four features.
+template <int F, int S, int U>
+__device__ __forceinline__ float4 agg_slot(const int* __restrict__ col, int len, int slot, const float* __restrict__ in) {
+    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int e = slot; e < len; e += U * S) {
+        int j[U];
 #pragma unroll
-        for (int q = 0; q < S; ++q) tot += __shfl(s, q * F + f, 64);
-        if (slot == 0) part[(size_t)c * F + f] = tot;
+        for (int u = 0; u < U; ++u) j[u] = e + u * S < len ? col[e + u * S] : 0;
+        float4 v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = *reinterpret_cast<const float4*>(in + (size_t)j[u] * F);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (e + u * S < len) s = add4(s, v[u]);
+    }
+    return s;
+}
+
+// The sum over the slots of a group: lanes that differ by low, 2 low, ... up to high / 2.
+__device__ __forceinline__ float4 agg_fold(float4 s, int low, int high) {
+    for (int o = low; o < high; o <<= 1)
+        s = add4(s, make_float4(__shfl_xor(s.x, o, 64), __shfl_xor(s.y, o, 64), __shfl_xor(s.z, o, 64),
+                                __shfl_xor(s.w, o, 64)));
+    return s;
+}
+
+// Virtual blocks: the chunks, then light and medium blocks in turns.
+template <int F, int MODE>
+__global__ __launch_bounds__(256) void k_agg(const AggArgs A, int light_blocks, int medium_blocks) {
+    constexpr int L = F / 4, G = L * kAggSlots<F>;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int f = 4 * (lane % L);                // this lane's first feature
+    const float* in = A.in + f;
+    const unsigned int vb = blockIdx.x;
+    if (vb < (unsigned int)A.nchunks) {
+        const int2 ch = A.chunks[vb];
+        const int len = min(kAggChunk, A.rowptr[A.heavy[ch.x] + 1] - ch.y);
+        const int first = wave * (kAggChunk / 4);
+        float4 s = agg_slot<F, 64 / L, kAggAhead<F>>(A.col + ch.y + first, min(kAggChunk / 4, len - first), lane / L, in);
+        s = agg_fold(s, L, 64);
+        if (lane < L) *reinterpret_cast<float4*>(A.part + ((size_t)vb * 4 + wave) * F + f) = s;
+        return;
+    }
+    const unsigned int i = vb - A.nchunks, t = light_blocks + medium_blocks;
+    const int m0 = (int)((unsigned long long)i * medium_blocks / t);       // medium blocks before i
+    if ((int)((i + 1ull) * medium_blocks / t) > m0) {
+        const int k = m0 * 4 + wave;
+        if (k >= A.nmedium) return;
+        const int v = A.medium[k], e0 = A.rowptr[v], len = A.rowptr[v + 1] - e0;
+        const float4 s = agg_fold(agg_slot<F, 64 / L, kAggAhead<F>>(A.col + e0, len, lane / L, in), L, 64);
+        if (lane < L) agg_store<MODE>(A, s, len, (size_t)v * F + f);
+    } else {
+        const long long v = (long long)(i - m0) * (256 / G) + threadIdx.x / G;
+        if (v >= A.n) return;
+        const int e0 = A.rowptr[v], len = A.rowptr[v + 1] - e0;
+        if (len > kAggLight) return;
+        const float4 s = agg_fold(agg_slot<F, kAggSlots<F>, 4>(A.col + e0, len, lane % G / L, in), L, G);
+        if (lane % G < L) agg_store<MODE>(A, s, len, (size_t)v * F + f);
     }
 }
 
-// One thread per (heavy row, feature): the row's chunk partials in chunk order.
+// A wave per heavy row: its partials, 256 / F at a time.
 template <int F, int MODE>
-__global__ __launch_bounds__(256) void k_agg_heavy(const int* __restrict__ rowptr, const int* __restrict__ heavy_row,
-                                                   const int* __restrict__ heavy_c0, int nheavy,
-                                                   const float* __restrict__ in, const float* __restrict__ part,
-                                                   const float* __restrict__ P, const float* __restrict__ H,
-                                                   float* __restrict__ out) {
-    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (t >= (long long)nheavy * F) return;
-    const int h = (int)(t / F), f = (int)(t % F);
-    const int i = heavy_row[h];
-    float s = 0.0f;
-    for (int c = heavy_c0[h]; c < heavy_c0[h + 1]; ++c) s += part[(size_t)c * F + f];
-    const size_t at = (size_t)i * F + f;
-    out[at] = agg_finish<MODE>(s, rowptr[i + 1] - rowptr[i], at, in, P, H);
+__global__ __launch_bounds__(256) void k_agg_heavy(const AggArgs A, const int* __restrict__ heavy_c0, int nheavy) {
+    constexpr int L = F / 4, S = 64 / L;
+    const int lane = threadIdx.x & 63, h = blockIdx.x * 4 + (threadIdx.x >> 6), f = 4 * (lane % L);
+    if (h >= nheavy) return;
+    const int v = A.heavy[h], c0 = 4 * heavy_c0[h], c1 = 4 * heavy_c0[h + 1];
+    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 4
+    for (int c = c0 + lane / L; c < c1; c += S) s = add4(s, *reinterpret_cast<const float4*>(A.part + (size_t)c * F + f));
+    s = agg_fold(s, L, 64);
+    if (lane < L) agg_store<MODE>(A, s, A.rowptr[v + 1] - A.rowptr[v], (size_t)v * F + f);
 }
 
 using f32x4 = __attribute__((ext_vector_type(4))) float;
@@ -728,28 +777,29 @@ int dense_blocks(int n) {
 template <int F, int MODE>
 void aggregate(const MpnnGraph& g, const float* in, float* out, hipStream_t st, const float* P = nullptr,
                const float* H = nullptr) {
-    const long long rb = ((long long)g.n * F + 255) / 256;
-    k_agg_rows<F, MODE><<<(int)(rb < 1 ? 1 : (rb > 65536 ? 65536 : rb)), 256, 0, st>>>(g.rowptr, g.col, g.n, in, P, H, out);
-    if (g.nchunks > 0) {
-        const int cb = (g.nchunks + 3) / 4;
-        k_agg_chunks<F><<<cb < 8192 ? cb : 8192, 256, 0, st>>>(g.rowptr, g.col, g.chunks, g.nchunks, in, g.part);
-        k_agg_heavy<F, MODE><<<blocks_for((long long)g.nheavy * F), 256, 0, st>>>(g.rowptr, g.heavy_row, g.heavy_c0,
-                                                                                 g.nheavy, in, g.part, P, H, out);
-    }
+    const AggArgs A{g.rowptr, g.col, g.n, g.medium, g.nmedium, g.heavy_row, g.chunks, g.nchunks, in, P, H, out, g.part};
+    const int light = (int)(((long long)g.n * (F / 4 * kAggSlots<F>) + 255) / 256), medium = (g.nmedium + 3) / 4;
+    k_agg<F, MODE><<<light + medium + g.nchunks, 256, 0, st>>>(A, light, medium);
+    if (g.nheavy > 0) k_agg_heavy<F, MODE><<<(g.nheavy + 3) / 4, 256, 0, st>>>(A, g.heavy_c0, g.nheavy);
 }
 
 }  // namespace
 
-void mpnn_agg_plan(const int* rowptr, int n, std::vector<int>& heavy_row, std::vector<int>& heavy_c0,
-                   std::vector<int2>& chunks) {
+void mpnn_agg_plan(const int* rowptr, int n, std::vector<int>& medium, std::vector<int>& heavy_row,
+                   std::vector<int>& heavy_c0, std::vector<int2>& chunks) {
+    medium.clear();
     heavy_row.clear();
     heavy_c0.assign(1, 0);
     chunks.clear();
     for (int i = 0; i < n; ++i) {
-        const int e0 = rowptr[i], e1 = rowptr[i + 1];
-        if (e1 - e0 <= kHeavyDeg) continue;
+        const int e0 = rowptr[i], len = rowptr[i + 1] - e0;
+        if (len <= kAggLight) continue;
+        if (len <= kAggHeavy) {
+            medium.push_back(i);
+            continue;
+        }
+        for (int e = 0; e < len; e += kAggChunk) chunks.push_back(make_int2((int)heavy_row.size(), e0 + e));
         heavy_row.push_back(i);
-        for (int e = e0; e < e1; e += kChunk) chunks.push_back(make_int2(i, e));
         heavy_c0.push_back((int)chunks.size());
     }
 }

@@ -75,23 +75,29 @@ int ensure_scratch(gfa2_mpnn* m, int n) {
     return GFA2_OK;
 }
 
-// Heavy rows and chunks of a graph's aggregation, from its row offsets on the host.
+// Medium and heavy rows and chunks of a graph's aggregation, from its row offsets on the host.
 int upload_agg_plan(gfa2_mpnn* m, const int* rp, MpnnGraph& g, std::vector<void*>& mine) {
-    std::vector<int> heavy_row, heavy_c0;
+    std::vector<int> medium, heavy_row, heavy_c0;
     std::vector<int2> chunks;
-    mpnn_agg_plan(rp, g.n, heavy_row, heavy_c0, chunks);
+    mpnn_agg_plan(rp, g.n, medium, heavy_row, heavy_c0, chunks);
+    g.nmedium = (int)medium.size();
     g.nheavy = (int)heavy_row.size();
     g.nchunks = (int)chunks.size();
-    if (g.nchunks == 0) return GFA2_OK;
+    if (g.nmedium + g.nchunks == 0) return GFA2_OK;
     int st;
-    if ((st = mp_alloc(mine, &g.heavy_row, heavy_row.size())) != GFA2_OK ||
+    if ((st = mp_alloc(mine, &g.medium, medium.size())) != GFA2_OK ||
+        (st = mp_alloc(mine, &g.heavy_row, heavy_row.size())) != GFA2_OK ||
         (st = mp_alloc(mine, &g.heavy_c0, heavy_c0.size())) != GFA2_OK ||
         (st = mp_alloc(mine, &g.chunks, chunks.size())) != GFA2_OK ||
-        (st = mp_alloc(mine, &g.part, chunks.size() * (size_t)kHid)) != GFA2_OK)
+        (st = mp_alloc(mine, &g.part, chunks.size() * (size_t)(4 * kHid))) != GFA2_OK)
         return st;
-    MP_TRY(hipMemcpyAsync(g.heavy_row, heavy_row.data(), sizeof(int) * heavy_row.size(), hipMemcpyHostToDevice, m->stream));
-    MP_TRY(hipMemcpyAsync(g.heavy_c0, heavy_c0.data(), sizeof(int) * heavy_c0.size(), hipMemcpyHostToDevice, m->stream));
-    MP_TRY(hipMemcpyAsync(g.chunks, chunks.data(), sizeof(int2) * chunks.size(), hipMemcpyHostToDevice, m->stream));
+    if (g.nmedium > 0)
+        MP_TRY(hipMemcpyAsync(g.medium, medium.data(), sizeof(int) * medium.size(), hipMemcpyHostToDevice, m->stream));
+    if (g.nchunks > 0) {
+        MP_TRY(hipMemcpyAsync(g.heavy_row, heavy_row.data(), sizeof(int) * heavy_row.size(), hipMemcpyHostToDevice, m->stream));
+        MP_TRY(hipMemcpyAsync(g.heavy_c0, heavy_c0.data(), sizeof(int) * heavy_c0.size(), hipMemcpyHostToDevice, m->stream));
+        MP_TRY(hipMemcpyAsync(g.chunks, chunks.data(), sizeof(int2) * chunks.size(), hipMemcpyHostToDevice, m->stream));
+    }
     MP_TRY(hipStreamSynchronize(m->stream));   // the host vectors go out of scope
     return GFA2_OK;
 }

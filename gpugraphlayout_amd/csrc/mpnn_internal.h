@@ -25,21 +25,25 @@ constexpr int kGrad2 = kParams - kOffW2s;
 constexpr int kGradBlocks = 256;
 constexpr int kLossBlocks = 2048;
 
-// Rows longer than kHeavyDeg entries are aggregated in chunks of kChunk entries.
-constexpr int kHeavyDeg = 512;
-constexpr int kChunk = 512;
+// Rows of up to kAggLight entries are aggregated by a few lanes each, up to kAggHeavy by a wave
+// each, longer ones in chunks of kAggChunk entries, a block each.
+constexpr int kAggLight = 32;
+constexpr int kAggHeavy = 2048;
+constexpr int kAggChunk = 4096;
 
 struct MpnnGraph {
     int n = 0;
     long long nnz = 0;
     int* rowptr = nullptr;
     int* col = nullptr;
-    int nheavy = 0;             // rows with more than kHeavyDeg entries
+    int nmedium = 0;            // rows of more than kAggLight entries up to kAggHeavy
+    int nheavy = 0;             // longer ones
     int nchunks = 0;
+    int* medium = nullptr;      // [nmedium]
     int* heavy_row = nullptr;   // [nheavy]
     int* heavy_c0 = nullptr;    // [nheavy + 1] first chunk of each heavy row
-    int2* chunks = nullptr;     // [nchunks] {row, first entry}
-    float* part = nullptr;      // [nchunks x kHid] chunk partial sums
+    int2* chunks = nullptr;     // [nchunks] {index into heavy_row, first entry}
+    float* part = nullptr;      // [4 nchunks x kHid] partial sums, one per quarter of a chunk
     float* X = nullptr;     // [n x kIn] features
     float* A0 = nullptr;    // [n x kIn] mean_agg(X)
     float* T = nullptr;     // [n x 2] normalised target, or null
@@ -64,9 +68,9 @@ struct MpnnScratch {
     double *part1 = nullptr, *part2 = nullptr;  // kGradBlocks x kGrad1 and kGrad2: weight-gradient partials
 };
 
-// Host side: the heavy rows and chunk list of a CSR given by its row offsets.
-void mpnn_agg_plan(const int* rowptr, int n, std::vector<int>& heavy_row, std::vector<int>& heavy_c0,
-                   std::vector<int2>& chunks);
+// Host side: the medium and heavy rows and the chunk list of a CSR given by its row offsets.
+void mpnn_agg_plan(const int* rowptr, int n, std::vector<int>& medium, std::vector<int>& heavy_row,
+                   std::vector<int>& heavy_c0, std::vector<int2>& chunks);
 void mpnn_features(const MpnnGraph& g, unsigned long long seed, int steps, MpnnScratch& s, hipStream_t st);
 // keep: H2 is written too (the backward pass reads it).
 void mpnn_forward(const MpnnGraph& g, const MpnnWeights& w, MpnnScratch& s, bool keep, hipStream_t st);

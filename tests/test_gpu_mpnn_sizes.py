@@ -1,6 +1,7 @@
 """The network's matrix-instruction kernels at the edges of their tiles (16 nodes per wave, runs of
 64 nodes per gradient partial) and past one round of their grids (16,384, 65,536 and 131,072
-nodes): loss, gradient and placed positions against the FP64 oracle."""
+nodes), and the aggregation at the borders of its row classes: features, loss, gradient and placed
+positions against the FP64 oracle."""
 import numpy as np
 import pytest
 
@@ -43,4 +44,40 @@ def test_gradient_and_positions(n):
     want = Y * (25.0 / np.sqrt((Y ** 2).sum(1).mean()))
     got = m.infer(gid, 25.0)
     assert np.linalg.norm(got - want) < 1e-4 * np.linalg.norm(want)
+    m.close()
+
+
+def rows_csr(degrees):
+    """Rows of the given lengths over leaves of at most a few entries, numbered in random order."""
+    leaves = max(degrees) + 3
+    n = len(degrees) + leaves
+    new = np.random.default_rng(n).permutation(n)
+    a = np.repeat(np.arange(len(degrees)), degrees)
+    b = len(degrees) + np.concatenate([(np.arange(d) * 7 + 11 * k) % leaves for k, d in enumerate(degrees)])
+    a, b = new[a], new[b]
+    key = np.unique(np.concatenate([a * n + b, b * n + a]))
+    rowptr = np.zeros(n + 1, np.int64)
+    rowptr[1:] = np.cumsum(np.bincount(key // n, minlength=n))
+    return rowptr, (key % n).astype(np.int32)
+
+
+@pytest.mark.parametrize("degrees", [(1, 3, 4, 5, 31, 32, 33, 64, 65, 127, 128, 129), (512, 513, 1023, 1024, 2047, 2048),
+                                     (2049, 3072, 3073, 4096, 4097, 5121, 9000), (8191, 8192, 8193, 70_000)])
+def test_row_lengths(degrees):
+    """Rows at the borders of the aggregation's classes (32, 2,048), of its batches and of its
+    chunks and their quarters (4,096, 1,024)."""
+    print(f"case mpnn rows {degrees}", flush=True)
+    rowptr, col = rows_csr(degrees)
+    n = len(rowptr) - 1
+    T = np.random.default_rng(n).normal(size=(n, 2)).astype(np.float32)
+    m = Mpnn(seed=3)
+    gid = m.add_graph(n, rowptr, col, target=T, feature_seed=n, steps=2)
+    X = m.features(gid)
+    assert np.max(np.abs(X - mo.features(rowptr, col, n, 2))) < 1e-4      # the bar of the other feature tests
+    loss, grad = m.loss_grad(gid, [1, 7])
+    t = T.astype(np.float64) - T.mean(0, dtype=np.float64)
+    t /= np.sqrt((t ** 2).sum(1).mean())
+    L, G = mo.loss_grad(m.params().astype(np.float64), rowptr, col, X, t, [1, 7], round_bf16=True)
+    assert loss == pytest.approx(L, rel=1e-5)
+    assert np.linalg.norm(grad - G) < 1e-4 * np.linalg.norm(G)
     m.close()
