@@ -515,8 +515,8 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
             if (col[e] < node_off[g] || col[e] >= node_off[g + 1] || col[e] == v) return GFA2_ERR_INVALID_GRAPH;
         rp32[v] = (int)a;
         const int64_t deg = e1 - a;
-        if (deg <= 32) lists.push_back(v);
-        else if (deg <= 2048) medium.push_back(v);
+        if (deg <= kAttrLight) lists.push_back(v);
+        else if (deg <= kAttrHeavy) medium.push_back(v);
         else heavy.push_back(v);
         m[v] = mass ? mass[v] : (float)(deg + 1.0);
     }
@@ -1393,6 +1393,12 @@ bool engine_view(gfa2_engine* h, EngineView* v) {
     v->col = h->b.col;
     v->nnz = h->b.nnz;
     v->nseg = h->b.nseg;
+    v->medium = h->b.node_lists + h->b.nlight;
+    v->nmedium = h->b.nmedium;
+    v->nheavy = h->b.nheavy;
+    v->chunk0 = h->b.attr_c0;
+    v->chunks = h->b.attr_chunks;
+    v->nchunks = h->b.nattr_chunks;
     return true;
 }
 

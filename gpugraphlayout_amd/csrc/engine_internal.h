@@ -111,7 +111,9 @@ struct LaunchConfig {
 
 constexpr int kWideHubs = 8192;     // hubs' positions in LDS (k_attract_wide)
 constexpr long long kWideEntries = 1 << 24;     // least entries for it (launch_attraction)
-constexpr int kAttrChunk = 4096;    // entries per block for rows over 2,048 entries
+constexpr int kAttrLight = 32;      // most entries of a light row
+constexpr int kAttrHeavy = 2048;    // and of a medium one
+constexpr int kAttrChunk = 4096;    // entries per block of a heavy row
 
 // All device buffers of one instance.
 struct Bufs {
@@ -316,6 +318,11 @@ struct EngineView {
     const int* col;
     long long nnz;
     int nseg;
+    const int* medium;      // medium rows, then heavy ones
+    int nmedium, nheavy;
+    const int* chunk0;      // [nheavy + 1] first chunk of each heavy row
+    const int2* chunks;     // {heavy row's index, first entry}
+    int nchunks;
 };
 bool engine_view(struct ::gfa2_engine* h, EngineView* v);
 // The buffers, device and stream of an engine holding a graph and positions (rasteriser).

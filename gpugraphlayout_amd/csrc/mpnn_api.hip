@@ -5,9 +5,25 @@
 
 #include <cmath>
 #include <new>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 using namespace gfa2;
+
+static_assert(kAggLight == kAttrLight && kAggHeavy == kAttrHeavy && kAggChunk == kAttrChunk,
+              "the engine's lists of rows are used as they are");
+
+namespace {
+struct GraphBlock {
+    char* p = nullptr;
+    size_t bytes = 0;
+};
+// A released graph's memory is kept for the next graph of the handle up to this size. Allocating and
+// freeing the 160 MB of an R-MAT 2^20 graph (20M entries) in nine pieces, with its row lists built
+// here from offsets read back, took 1.8 of the 3.5 ms of its learned start.
+constexpr size_t kSpareKeep = 256u << 20;
+}  // namespace
 
 struct gfa2_mpnn {
     int device = 0;
@@ -16,7 +32,8 @@ struct gfa2_mpnn {
     MpnnScratch s;
     std::vector<MpnnGraph> graphs;
     std::vector<void*> allocs;          // weights and scratch
-    std::vector<std::vector<void*>> graph_allocs;
+    std::vector<GraphBlock> blocks;     // each graph's device memory
+    GraphBlock spare;                   // a released graph's, for the next one
     int adam_step = 0;
     int* offs = nullptr;                // training offsets, steps x R
     long long offs_cap = 0;
@@ -53,10 +70,16 @@ struct SplitMix {
     double uniform() { return (double)(next() >> 11) * (1.0 / 9007199254740992.0); }
 };
 
+void drop_spare(gfa2_mpnn* m) {
+    if (m->spare.p) (void)hipFree(m->spare.p);
+    m->spare = GraphBlock{};
+}
+
 // Scratch sized for n nodes (grows, never shrinks).
 int ensure_scratch(gfa2_mpnn* m, int n) {
     MpnnScratch& s = m->s;
     if (n <= s.cap) return GFA2_OK;
+    drop_spare(m);
     for (void* p : {(void*)s.z0, (void*)s.z1, (void*)s.H1, (void*)s.A1, (void*)s.H2, (void*)s.Y, (void*)s.dY,
                     (void*)s.P, (void*)s.Q, (void*)s.dZ1})
         if (p) (void)hipFree(p);
@@ -75,32 +98,72 @@ int ensure_scratch(gfa2_mpnn* m, int n) {
     return GFA2_OK;
 }
 
-// Medium and heavy rows and chunks of a graph's aggregation, from its row offsets on the host.
-int upload_agg_plan(gfa2_mpnn* m, const int* rp, MpnnGraph& g, std::vector<void*>& mine) {
-    std::vector<int> medium, heavy_row, heavy_c0;
-    std::vector<int2> chunks;
-    mpnn_agg_plan(rp, g.n, medium, heavy_row, heavy_c0, chunks);
-    g.nmedium = (int)medium.size();
-    g.nheavy = (int)heavy_row.size();
-    g.nchunks = (int)chunks.size();
-    if (g.nmedium + g.nchunks == 0) return GFA2_OK;
-    int st;
-    if ((st = mp_alloc(mine, &g.medium, medium.size())) != GFA2_OK ||
-        (st = mp_alloc(mine, &g.heavy_row, heavy_row.size())) != GFA2_OK ||
-        (st = mp_alloc(mine, &g.heavy_c0, heavy_c0.size())) != GFA2_OK ||
-        (st = mp_alloc(mine, &g.chunks, chunks.size())) != GFA2_OK ||
-        (st = mp_alloc(mine, &g.part, chunks.size() * (size_t)(4 * kHid))) != GFA2_OK)
-        return st;
-    if (g.nmedium > 0)
-        MP_TRY(hipMemcpyAsync(g.medium, medium.data(), sizeof(int) * medium.size(), hipMemcpyHostToDevice, m->stream));
-    if (g.nchunks > 0) {
-        MP_TRY(hipMemcpyAsync(g.heavy_row, heavy_row.data(), sizeof(int) * heavy_row.size(), hipMemcpyHostToDevice, m->stream));
-        MP_TRY(hipMemcpyAsync(g.heavy_c0, heavy_c0.data(), sizeof(int) * heavy_c0.size(), hipMemcpyHostToDevice, m->stream));
-        MP_TRY(hipMemcpyAsync(g.chunks, chunks.data(), sizeof(int2) * chunks.size(), hipMemcpyHostToDevice, m->stream));
+// The block's work is done. The larger of it and the spare one is kept.
+void give_back(gfa2_mpnn* m, GraphBlock& b) {
+    if (b.bytes <= kSpareKeep && b.bytes > m->spare.bytes) std::swap(b, m->spare);
+    if (b.p) (void)hipFree(b.p);
+    b = GraphBlock{};
+}
+
+// The spare block if it is large enough and at least half of it is used.
+int take_block(gfa2_mpnn* m, size_t bytes, GraphBlock& b) {
+    if (m->spare.bytes >= bytes && m->spare.bytes / 2 <= bytes) {
+        std::swap(b, m->spare);
+        return GFA2_OK;
     }
-    MP_TRY(hipStreamSynchronize(m->stream));   // the host vectors go out of scope
+    drop_spare(m);
+    void* p = nullptr;
+    const hipError_t e = hipMalloc(&p, bytes);
+    if (e != hipSuccess) return st_of(e);
+    b.p = static_cast<char*>(p);
+    b.bytes = bytes;
     return GFA2_OK;
 }
+
+// One block for all of a graph's arrays (n, nnz, nmedium, nheavy and nchunks are set).
+int lay_out(gfa2_mpnn* m, MpnnGraph& g, bool target, GraphBlock& b) {
+    size_t at = 0;
+    auto place = [&](auto*& p, size_t count) {
+        p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(b.p ? b.p + at : nullptr);
+        at += (sizeof(*p) * count + 255) / 256 * 256;
+    };
+    auto all = [&]() {
+        const size_t n = (size_t)g.n;
+        at = 0;
+        place(g.rowptr, n + 1);
+        place(g.col, (size_t)g.nnz);
+        place(g.medium, (size_t)g.nmedium + g.nheavy);
+        g.heavy_row = g.medium ? g.medium + g.nmedium : nullptr;
+        place(g.heavy_c0, (size_t)g.nheavy + 1);
+        place(g.chunks, (size_t)g.nchunks);
+        place(g.part, (size_t)g.nchunks * 4 * kHid);
+        place(g.X, n * kIn);
+        place(g.A0, n * kIn);
+        if (target) place(g.T, n * 2);
+    };
+    all();
+    const int st = take_block(m, at, b);
+    if (st == GFA2_OK) all();
+    return st;
+}
+
+// A new graph's block: given back unless the graph is kept.
+struct NewBlock {
+    gfa2_mpnn* m;
+    GraphBlock b;
+    explicit NewBlock(gfa2_mpnn* m_) : m(m_) {}
+    ~NewBlock() {
+        if (!b.p) return;
+        (void)hipStreamSynchronize(m->stream);
+        give_back(m, b);
+    }
+    int keep(const MpnnGraph& g) {
+        m->graphs.push_back(g);
+        m->blocks.push_back(b);
+        b = GraphBlock{};
+        return (int)m->graphs.size() - 1;
+    }
+};
 
 int check_graph(const gfa2_mpnn* m, int id) {
     if (!m || id < 0 || id >= (int)m->graphs.size() || m->graphs[id].n == 0) return GFA2_ERR_INVALID_ARG;
@@ -197,18 +260,24 @@ int gfa2_mpnn_add_graph(gfa2_mpnn_t m, int32_t n, const int64_t* rowptr, const i
     MpnnGraph g;
     g.n = n;
     g.nnz = nnz;
-    std::vector<void*> mine;
-    if ((st = mp_alloc(mine, &g.rowptr, (size_t)n + 1)) != GFA2_OK || (st = mp_alloc(mine, &g.col, (size_t)nnz)) != GFA2_OK ||
-        (st = mp_alloc(mine, &g.X, (size_t)n * kIn)) != GFA2_OK || (st = mp_alloc(mine, &g.A0, (size_t)n * kIn)) != GFA2_OK) {
-        for (void* p : mine) (void)hipFree(p);
-        return st;
-    }
-    MP_TRY(hipMemcpyAsync(g.rowptr, rp.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice, m->stream));
-    if (nnz) MP_TRY(hipMemcpyAsync(g.col, col, sizeof(int) * nnz, hipMemcpyHostToDevice, m->stream));
-    if ((st = upload_agg_plan(m, rp.data(), g, mine)) != GFA2_OK) {
-        for (void* p : mine) (void)hipFree(p);
-        return st;
-    }
+    std::vector<int> medium, heavy_row, heavy_c0;
+    std::vector<int2> chunks;
+    mpnn_agg_plan(rp.data(), n, medium, heavy_row, heavy_c0, chunks);
+    g.nmedium = (int)medium.size();
+    g.nheavy = (int)heavy_row.size();
+    g.nchunks = (int)chunks.size();
+    medium.insert(medium.end(), heavy_row.begin(), heavy_row.end());
+    std::vector<float> t;               // the target, copied by the stream
+    NewBlock mine(m);                   // drains the stream before the vectors go
+    if ((st = lay_out(m, g, target_xy != nullptr, mine.b)) != GFA2_OK) return st;
+    auto upload = [&](void* to, const void* from, size_t bytes) {
+        return bytes ? hipMemcpyAsync(to, from, bytes, hipMemcpyHostToDevice, m->stream) : hipSuccess;
+    };
+    MP_TRY(upload(g.rowptr, rp.data(), sizeof(int) * ((size_t)n + 1)));
+    MP_TRY(upload(g.col, col, sizeof(int) * (size_t)nnz));
+    MP_TRY(upload(g.medium, medium.data(), sizeof(int) * medium.size()));
+    MP_TRY(upload(g.heavy_c0, heavy_c0.data(), sizeof(int) * heavy_c0.size()));
+    MP_TRY(upload(g.chunks, chunks.data(), sizeof(int2) * chunks.size()));
     if (target_xy) {
         // centre and scale to unit RMS radius
         double cx = 0.0, cy = 0.0;
@@ -224,14 +293,10 @@ int gfa2_mpnn_add_graph(gfa2_mpnn_t m, int32_t n, const int64_t* rowptr, const i
             r2 += dx * dx + dy * dy;
         }
         const double rms = std::sqrt(r2 / n);
-        std::vector<float> t((size_t)2 * n);
+        t.resize((size_t)2 * n);
         for (int i = 0; i < n; ++i) {
             t[2 * i] = (float)((target_xy[2 * i] - cx) / (rms > 0 ? rms : 1.0));
             t[2 * i + 1] = (float)((target_xy[2 * i + 1] - cy) / (rms > 0 ? rms : 1.0));
-        }
-        if ((st = mp_alloc(mine, &g.T, (size_t)2 * n)) != GFA2_OK) {
-            for (void* p : mine) (void)hipFree(p);
-            return st;
         }
         g.target_scale = (float)rms;
         MP_TRY(hipMemcpyAsync(g.T, t.data(), sizeof(float) * 2 * n, hipMemcpyHostToDevice, m->stream));
@@ -239,9 +304,8 @@ int gfa2_mpnn_add_graph(gfa2_mpnn_t m, int32_t n, const int64_t* rowptr, const i
     mpnn_features(g, feature_seed, smoothing_steps, m->s, m->stream);
     MP_TRY(hipGetLastError());
     MP_TRY(hipStreamSynchronize(m->stream));
-    m->graphs.push_back(g);
-    m->graph_allocs.push_back(mine);
-    if (graph_id) *graph_id = (int32_t)m->graphs.size() - 1;
+    const int id = mine.keep(g);
+    if (graph_id) *graph_id = id;
     return GFA2_OK;
 }
 
@@ -259,30 +323,29 @@ int gfa2_mpnn_add_engine_graph(gfa2_mpnn_t m, gfa2_handle h, uint64_t feature_se
     MpnnGraph g;
     g.n = n;
     g.nnz = v.nnz;
-    std::vector<void*> mine;
-    if ((st = mp_alloc(mine, &g.rowptr, (size_t)n + 1)) != GFA2_OK || (st = mp_alloc(mine, &g.col, (size_t)g.nnz)) != GFA2_OK ||
-        (st = mp_alloc(mine, &g.X, (size_t)n * kIn)) != GFA2_OK || (st = mp_alloc(mine, &g.A0, (size_t)n * kIn)) != GFA2_OK) {
-        for (void* p : mine) (void)hipFree(p);
-        return st;
-    }
-    // the engine's CSR was validated when it was set; copy it device to device after the
-    // engine's queued work
+    g.nmedium = v.nmedium;
+    g.nheavy = v.nheavy;
+    g.nchunks = v.nchunks;
+    NewBlock mine(m);
+    if ((st = lay_out(m, g, false, mine.b)) != GFA2_OK) return st;
+    // the engine's CSR was validated when it was set; it and the engine's lists of rows, which are
+    // those of the aggregation, are copied device to device after the engine's queued work
     MP_TRY(hipStreamSynchronize(v.stream));
-    MP_TRY(hipMemcpyAsync(g.rowptr, v.rowptr, sizeof(int) * ((size_t)n + 1), hipMemcpyDeviceToDevice, m->stream));
-    if (g.nnz) MP_TRY(hipMemcpyAsync(g.col, v.col, sizeof(int) * (size_t)g.nnz, hipMemcpyDeviceToDevice, m->stream));
-    std::vector<int> rp((size_t)n + 1);
-    MP_TRY(hipMemcpyAsync(rp.data(), v.rowptr, sizeof(int) * ((size_t)n + 1), hipMemcpyDeviceToHost, m->stream));
-    MP_TRY(hipStreamSynchronize(m->stream));
-    if ((st = upload_agg_plan(m, rp.data(), g, mine)) != GFA2_OK) {
-        for (void* p : mine) (void)hipFree(p);
-        return st;
+    auto copy = [&](void* to, const void* from, size_t bytes) {
+        return bytes ? hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToDevice, m->stream) : hipSuccess;
+    };
+    MP_TRY(copy(g.rowptr, v.rowptr, sizeof(int) * ((size_t)n + 1)));
+    MP_TRY(copy(g.col, v.col, sizeof(int) * (size_t)g.nnz));
+    MP_TRY(copy(g.medium, v.medium, sizeof(int) * ((size_t)g.nmedium + g.nheavy)));
+    if (g.nheavy > 0) {
+        MP_TRY(copy(g.heavy_c0, v.chunk0, sizeof(int) * ((size_t)g.nheavy + 1)));
+        MP_TRY(copy(g.chunks, v.chunks, sizeof(int2) * (size_t)g.nchunks));
     }
     mpnn_features(g, feature_seed, smoothing_steps, m->s, m->stream);
     MP_TRY(hipGetLastError());
     MP_TRY(hipStreamSynchronize(m->stream));
-    m->graphs.push_back(g);
-    m->graph_allocs.push_back(mine);
-    if (graph_id) *graph_id = (int32_t)m->graphs.size() - 1;
+    const int id = mine.keep(g);
+    if (graph_id) *graph_id = id;
     return GFA2_OK;
 }
 
@@ -291,8 +354,7 @@ int gfa2_mpnn_release_graph(gfa2_mpnn_t m, int32_t graph_id) {
     if (st != GFA2_OK) return st;
     MP_TRY(hipSetDevice(m->device));
     MP_TRY(hipStreamSynchronize(m->stream));
-    for (void* p : m->graph_allocs[graph_id]) (void)hipFree(p);
-    m->graph_allocs[graph_id].clear();
+    give_back(m, m->blocks[graph_id]);
     m->graphs[graph_id] = MpnnGraph{};     // n = 0, no target: skipped by training, rejected by id
     return GFA2_OK;
 }
@@ -405,8 +467,9 @@ int gfa2_mpnn_destroy(gfa2_mpnn_t m) {
     if (!m) return GFA2_ERR_INVALID_ARG;
     (void)hipSetDevice(m->device);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
-    for (auto& list : m->graph_allocs)
-        for (void* p : list) (void)hipFree(p);
+    for (const GraphBlock& b : m->blocks)
+        if (b.p) (void)hipFree(b.p);
+    drop_spare(m);
     for (void* p : m->allocs) (void)hipFree(p);
     MpnnScratch& s = m->s;
     for (void* p : {(void*)s.z0, (void*)s.z1, (void*)s.H1, (void*)s.A1, (void*)s.H2, (void*)s.Y, (void*)s.dY,
