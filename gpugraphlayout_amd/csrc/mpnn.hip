@@ -66,62 +66,92 @@ __global__ __launch_bounds__(256) void k_normal_fields(int n, unsigned long long
     Z[t] = sqrtf(-2.0f * logf(u1)) * cosf(6.2831853071795864f * u2);
 }
 
-// out[i][f] = (in[i][f] + mean_j in[j][f]) / 2 for 8 columns.
-// X (unnormalised) columns 0..8, zero padding 9..15.
-__global__ __launch_bounds__(256) void k_assemble(const int* __restrict__ rowptr, int n, const float* __restrict__ Z,
-                                                  float* __restrict__ X) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= n * kIn) return;
-    const int i = t / kIn, f = t % kIn;
-    float v = 0.0f;
-    if (f == 0) v = logf((float)(rowptr[i + 1] - rowptr[i]) + 1.0f);
-    else if (f <= 8) v = Z[i * 8 + f - 1];
-    X[t] = v;
+// The features are column 0 log(deg + 1) and columns 1 to 8 Z, each with its mean taken away and
+// divided by its deviation, and zeros. They are written once, normalised: a pass over Z for the
+// columns' sums (each row's entries and offsets are all that it reads), a block that adds the
+// passes' partials, a pass that writes X. All three are bound by memory (R-MAT 2^20, 580k nodes:
+// with the raw features written, read and rewritten and the partials added by one thread per
+// column 144 us, now 28).
+constexpr int kStat = 9;             // columns that are not padding
+constexpr int kStatBlocks = 448;     // partials of 2 kStat doubles each
+static_assert(kStatBlocks * 2 * kStat <= kPartDoubles);
+
+__device__ __forceinline__ float degree_feature(const int* __restrict__ rowptr, int i) {
+    return logf((float)(rowptr[i + 1] - rowptr[i]) + 1.0f);
 }
 
-// Per-block column sums and sums of squares of X (kIn columns).
-__global__ __launch_bounds__(256) void k_colstats(const float* __restrict__ X, int n, double* __restrict__ part) {
-    __shared__ double s1[256], s2[256];
-    const int f = threadIdx.x & (kIn - 1), lane_row = threadIdx.x / kIn;   // 16 rows x 16 columns
-    double a = 0.0, b = 0.0;
-    for (int i = blockIdx.x * 16 + lane_row; i < n; i += gridDim.x * 16) {
-        const double v = X[i * kIn + f];
-        a += v;
-        b += v * v;
-    }
-    s1[threadIdx.x] = a;
-    s2[threadIdx.x] = b;
-    __syncthreads();
-    if (threadIdx.x < kIn) {
-        double A = 0.0, B = 0.0;
-        for (int r = 0; r < 16; ++r) {
-            A += s1[r * kIn + threadIdx.x];
-            B += s2[r * kIn + threadIdx.x];
+__device__ __forceinline__ double wave_sum(double v, int low) {
+    for (int o = low; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+// Per-block sums and sums of squares of the columns. Two lanes per row, a half of Z each; the even
+// one takes the degree too.
+__global__ __launch_bounds__(256) void k_colstats(const int* __restrict__ rowptr, const float* __restrict__ Z, int n,
+                                                  double* __restrict__ part) {
+    __shared__ double sums[4][2 * kStat];
+    const int half = threadIdx.x & 1;
+    double a[5] = {}, b[5] = {};        // the degree, four columns of Z
+    for (long long i = (long long)blockIdx.x * 128 + threadIdx.x / 2; i < n; i += (long long)gridDim.x * 128) {
+        const float4 z = *reinterpret_cast<const float4*>(Z + i * 8 + 4 * half);
+        const float x[5] = {half ? 0.0f : degree_feature(rowptr, (int)i), z.x, z.y, z.z, z.w};
+#pragma unroll
+        for (int c = 0; c < 5; ++c) {
+            const double v = x[c];
+            a[c] += v;
+            b[c] += v * v;
         }
-        part[(blockIdx.x * kIn + threadIdx.x) * 2] = A;
-        part[(blockIdx.x * kIn + threadIdx.x) * 2 + 1] = B;
     }
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+        const double A = wave_sum(a[c], 2), B = wave_sum(b[c], 2);
+        const int f = c == 0 ? 0 : 4 * half + c;
+        if (lane < 2 && (c > 0 || half == 0)) {
+            sums[wave][2 * f] = A;
+            sums[wave][2 * f + 1] = B;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 * kStat)
+        part[blockIdx.x * 2 * kStat + threadIdx.x] = sums[0][threadIdx.x] + sums[1][threadIdx.x] +
+                                                     sums[2][threadIdx.x] + sums[3][threadIdx.x];
 }
 
-__global__ void k_colnorm_finish(const double* __restrict__ part, int nb, int n, float* __restrict__ mu_sd) {
-    const int f = threadIdx.x;
-    if (f >= kIn) return;
+// A wave per column.
+__global__ __launch_bounds__(64 * kStat) void k_colnorm_finish(const double* __restrict__ part, int nb, int n,
+                                                               float* __restrict__ mu_sd) {
+    const int f = threadIdx.x >> 6, lane = threadIdx.x & 63;
     double A = 0.0, B = 0.0;
-    for (int b = 0; b < nb; ++b) {
-        A += part[(b * kIn + f) * 2];
-        B += part[(b * kIn + f) * 2 + 1];
+#pragma unroll 4
+    for (int b = lane; b < nb; b += 64) {
+        A += part[b * 2 * kStat + 2 * f];
+        B += part[b * 2 * kStat + 2 * f + 1];
     }
+    A = wave_sum(A, 1);
+    B = wave_sum(B, 1);
+    if (lane > 0) return;
     const double mu = A / n;
     const double var = B / n - mu * mu;
     mu_sd[2 * f] = (float)mu;
-    mu_sd[2 * f + 1] = (f <= 8 && var > 1e-12) ? (float)(1.0 / sqrt(var)) : 0.0f;
+    mu_sd[2 * f + 1] = var > 1e-12 ? (float)(1.0 / sqrt(var)) : 0.0f;
 }
 
-__global__ __launch_bounds__(256) void k_colnorm_apply(float* __restrict__ X, int n, const float* __restrict__ mu_sd) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= n * kIn) return;
-    const int f = t % kIn;
-    X[t] = (X[t] - mu_sd[2 * f]) * mu_sd[2 * f + 1];
+// Four lanes per row, four columns of X each.
+__global__ __launch_bounds__(256) void k_features(const int* __restrict__ rowptr, const float* __restrict__ Z, int n,
+                                                  const float* __restrict__ mu_sd, float* __restrict__ X) {
+    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+    const long long i = t / 4;
+    if (i >= n) return;
+    const int q = (int)(t % 4);
+    float x[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int f = 4 * q + c;
+        x[c] = 0.0f;
+        if (f < kStat) x[c] = ((f == 0 ? degree_feature(rowptr, (int)i) : Z[i * 8 + f - 1]) - mu_sd[2 * f]) * mu_sd[2 * f + 1];
+    }
+    *reinterpret_cast<float4*>(X + i * kIn + 4 * q) = make_float4(x[0], x[1], x[2], x[3]);
 }
 
 // ---- neighbour aggregation -----------------------------------------------------------------
@@ -744,18 +774,23 @@ __global__ __launch_bounds__(256) void k_ystats(const float* __restrict__ Y, int
 __global__ __launch_bounds__(256) void k_place(const float* __restrict__ Y, int n, const double* __restrict__ part,
                                                int nb, float scale, float2* __restrict__ xy) {
     __shared__ float coef[3];
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {
         double sx = 0.0, sy = 0.0, sq = 0.0;
-        for (int b = 0; b < nb; ++b) {
+        for (int b = threadIdx.x; b < nb; b += 64) {
             sx += part[3 * b];
             sy += part[3 * b + 1];
             sq += part[3 * b + 2];
         }
+        sx = wave_sum(sx, 1);
+        sy = wave_sum(sy, 1);
+        sq = wave_sum(sq, 1);
         const double mx = sx / n, my = sy / n;
         const double var = sq / n - mx * mx - my * my;
-        coef[0] = (float)mx;
-        coef[1] = (float)my;
-        coef[2] = var > 0 ? (float)(scale / sqrt(var)) : scale;
+        if (threadIdx.x == 0) {
+            coef[0] = (float)mx;
+            coef[1] = (float)my;
+            coef[2] = var > 0 ? (float)(scale / sqrt(var)) : scale;
+        }
     }
     __syncthreads();
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
@@ -815,11 +850,10 @@ void mpnn_features(const MpnnGraph& g, unsigned long long seed, int steps, MpnnS
         a = b;
         b = t;
     }
-    k_assemble<<<blocks_for((long long)n * kIn), 256, 0, st>>>(g.rowptr, n, a, g.X);
-    const int nb = 256;
-    k_colstats<<<nb, 256, 0, st>>>(g.X, n, s.dpart);
-    k_colnorm_finish<<<1, 64, 0, st>>>(s.dpart, nb, n, s.musd);
-    k_colnorm_apply<<<blocks_for((long long)n * kIn), 256, 0, st>>>(g.X, n, s.musd);
+    const int nb = (n + 127) / 128 < kStatBlocks ? (n + 127) / 128 : kStatBlocks;
+    k_colstats<<<nb, 256, 0, st>>>(g.rowptr, a, n, s.dpart);
+    k_colnorm_finish<<<1, 64 * kStat, 0, st>>>(s.dpart, nb, n, s.musd);
+    k_features<<<blocks_for((long long)n * 4), 256, 0, st>>>(g.rowptr, a, n, s.musd, g.X);
     aggregate<kIn, kAggMean>(g, g.X, g.A0, st);
 }
 

@@ -193,7 +193,7 @@ int gfa2_mpnn_create(int device, uint64_t seed, gfa2_mpnn_t* out) {
         (st = mp_alloc(m->allocs, &m->w.grad, kParams)) != GFA2_OK ||
         (st = mp_alloc(m->allocs, &m->w.m, kParams)) != GFA2_OK ||
         (st = mp_alloc(m->allocs, &m->w.v, kParams)) != GFA2_OK ||
-        (st = mp_alloc(m->allocs, &m->s.dpart, 8192)) != GFA2_OK ||
+        (st = mp_alloc(m->allocs, &m->s.dpart, kPartDoubles)) != GFA2_OK ||
         (st = mp_alloc(m->allocs, &m->s.musd, 2 * kIn)) != GFA2_OK ||
         (st = mp_alloc(m->allocs, &m->s.part1, (size_t)kGradBlocks * kGrad1)) != GFA2_OK ||
         (st = mp_alloc(m->allocs, &m->s.part2, (size_t)kGradBlocks * kGrad2)) != GFA2_OK) {

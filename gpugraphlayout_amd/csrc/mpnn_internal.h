@@ -24,6 +24,7 @@ constexpr int kGrad1 = kOffW2s;
 constexpr int kGrad2 = kParams - kOffW2s;
 constexpr int kGradBlocks = 256;
 constexpr int kLossBlocks = 2048;
+constexpr int kPartDoubles = 8192;
 
 // Rows of up to kAggLight entries are aggregated by a few lanes each, up to kAggHeavy by a wave
 // each, longer ones in chunks of kAggChunk entries, a block each.
@@ -61,7 +62,7 @@ struct MpnnWeights {
 struct MpnnScratch {
     int cap = 0;            // nodes the buffers hold
     float *z0 = nullptr, *z1 = nullptr;
-    double* dpart = nullptr;    // 8192 doubles: column statistics, loss partials
+    double* dpart = nullptr;    // kPartDoubles: column statistics, loss partials
     float* musd = nullptr;      // 2 * kIn
     float *H1 = nullptr, *A1 = nullptr, *H2 = nullptr, *Y = nullptr, *dY = nullptr;
     float *P = nullptr, *Q = nullptr, *dZ1 = nullptr;

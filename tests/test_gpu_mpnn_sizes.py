@@ -81,3 +81,14 @@ def test_row_lengths(degrees):
     assert loss == pytest.approx(L, rel=1e-5)
     assert np.linalg.norm(grad - G) < 1e-4 * np.linalg.norm(G)
     m.close()
+
+
+@pytest.mark.parametrize("n", [2, 3, 127, 128, 129, 57_344, 57_345, 115_000])
+def test_feature_columns(n):
+    """One to all blocks of the columns' sums (128 rows each, 448 blocks), and past one round."""
+    print(f"case mpnn feature columns n={n}", flush=True)
+    rowptr, col = sparse_csr(n, n)
+    m = Mpnn(seed=3)
+    X = m.features(m.add_graph(n, rowptr, col, feature_seed=n, steps=1))
+    assert np.max(np.abs(X - mo.features(rowptr, col, n, 1))) < 1e-4      # the bar of the other feature tests
+    m.close()
