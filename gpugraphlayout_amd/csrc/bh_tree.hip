@@ -877,7 +877,179 @@ __global__ __launch_bounds__(kCellsThreads) void k_cells(const unsigned long lon
     if (tid < 8) kids_part[blockIdx.x * 8 + tid] = rmax[tid];
 }
 
-// Bucket cells by level (order inside a level is irrelevant).
+// Summaries of all cells in two launches, for trees of up to kSumMaxBlocks * kSumBlock records. A
+// block takes kSumBlock records, which lie in preorder, and sums the cells that end inside it in
+// LDS, deepest level first. The few that reach past its end contain its last record, so they are
+// nested and of different levels: each has a slot of its own (block, level), and one block
+// then sums them all, deepest level first, with their other children read beforehand. What bounds
+// both are the levels' dependent steps, which here cost a barrier each and no launch: 20k bodies
+// with fractional masses 31 us, where a launch per level took 82.
+constexpr int kSumBlock = 4096, kSumThreads = 1024, kSumMaxBlocks = 62;
+constexpr int kSumLevels = 33;       // slots per block: the root, then a cell's info level + 1
+constexpr int kSumOwn = kSumBlock / kSumThreads;
+static_assert(kSumMaxBlocks * kSumLevels <= 2 * kSumThreads, "two slots per thread of k_sum_spill");
+
+constexpr unsigned int kBodyInfo = 0xffffffffu;
+
+__device__ __forceinline__ int info_level(unsigned int info) { return (int)(info & ((1u << kInfoLevelBits) - 1)); }
+
+// Records to the next one beside this one.
+__device__ __forceinline__ int record_hop(unsigned int info) {
+    return info == kBodyInfo ? 1 : max((int)(info >> kInfoLevelBits), 1);
+}
+
+struct CellSum {
+    float m = 0.0f, x = 0.0f, y = 0.0f;
+    __device__ __forceinline__ void add(const float4& c) {
+        x = fmaf(c.x, c.z, x);
+        y = fmaf(c.y, c.z, y);
+        m += c.z;
+    }
+    __device__ __forceinline__ float4 record(float w) const {
+        const float inv = 1.0f / m;
+        return make_float4(x * inv, y * inv, m, w);
+    }
+};
+
+// A cell of info level 0 is the root if a child has that level too (the root's own is 0, as its
+// children's): first is its first child, end past its last, in R.
+__device__ __forceinline__ bool is_root(const float4* R, int first, int end) {
+    for (int r = first; r < end;) {
+        const unsigned int ci = __float_as_uint(R[r].w);
+        if (ci != kBodyInfo && info_level(ci) == 0) return true;
+        r += record_hop(ci);
+    }
+    return false;
+}
+
+__global__ __launch_bounds__(kSumThreads) void k_sum_blocks(float4* __restrict__ rec, int* __restrict__ spill,
+                                                            const DevState* __restrict__ st) {
+    __shared__ float4 R[kSumBlock];
+    __shared__ int slot[kSumLevels];
+    __shared__ int deepest;
+    if (st->err != 0) return;
+    const int tid = threadIdx.x, base = blockIdx.x * kSumBlock, total = st->nrecords;
+    const int len = min(kSumBlock, total - base);
+    if (len <= 0) return;
+    if (tid < kSumLevels) slot[tid] = -1;
+    if (tid == 0) deepest = -1;
+    int level[kSumOwn], end[kSumOwn];            // level -1: no cell, or one that ends in a later block
+#pragma unroll
+    for (int k = 0; k < kSumOwn; ++k) {
+        const int i = tid + k * kSumThreads;
+        level[k] = -1;
+        end[k] = 0;
+        if (i < len) R[i] = rec[base + i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kSumOwn; ++k) {
+        const int i = tid + k * kSumThreads;
+        if (i >= len) continue;
+        const unsigned int info = __float_as_uint(R[i].w);
+        if (info == kBodyInfo) continue;
+        end[k] = min(base + i + (int)(info >> kInfoLevelBits), total) - base;
+        if (end[k] <= len) {
+            level[k] = info_level(info);
+            continue;
+        }
+        const bool root = info_level(info) == 0 && is_root(rec, base + i + 1, base + end[k]);
+        slot[root ? 0 : info_level(info) + 1] = base + i;
+    }
+    int most = level[0];
+#pragma unroll
+    for (int k = 1; k < kSumOwn; ++k) most = max(most, level[k]);
+    for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, 64));
+    if ((tid & 63) == 0 && most >= 0) atomicMax(&deepest, most);
+    __syncthreads();
+    if (tid < kSumLevels) spill[blockIdx.x * kSumLevels + tid] = slot[tid];
+    const int from = deepest;
+    // round -1 is the root's
+    for (int L = from; L >= -1; --L) {
+#pragma unroll
+        for (int k = 0; k < kSumOwn; ++k) {
+            if (level[k] != L || (L == -1 && end[k] >= 0)) continue;
+            const int i = tid + k * kSumThreads;
+            const int stop = L == -1 ? ~end[k] : end[k];
+            if (L == 0 && is_root(R, i + 1, stop)) {
+                level[k] = -1;
+                end[k] = ~stop;
+                continue;
+            }
+            CellSum s;
+            for (int r = i + 1; r < stop;) {
+                const float4 c = R[r];
+                s.add(c);
+                r += record_hop(__float_as_uint(c.w));
+            }
+            R[i] = s.record(R[i].w);
+            rec[base + i] = R[i];
+        }
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(kSumThreads) void k_sum_spill(float4* __restrict__ rec, const int* __restrict__ spill,
+                                                           const DevState* __restrict__ st) {
+    __shared__ float4 sum[2 * kSumThreads];
+    if (st->err != 0) return;
+    const int tid = threadIdx.x, total = st->nrecords;
+    const int slots = (total + kSumBlock - 1) / kSumBlock * kSumLevels;
+    float4 child[2][4], own[2];
+    int ref[2][4];               // a child's slot; -1: it is in child; -2: none
+    int cell[2];
+    bool waits[2] = {false, false};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int q = tid + k * kSumThreads;
+        cell[k] = q < slots ? spill[q] : -1;
+        if (cell[k] < 0) continue;
+        own[k] = rec[cell[k]];
+        const int end = min(cell[k] + (int)(__float_as_uint(own[k].w) >> kInfoLevelBits), total);
+        int r = cell[k] + 1;
+        CellSum s;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            ref[k][u] = -2;
+            if (r >= end) continue;
+            child[k][u] = rec[r];
+            const unsigned int ci = __float_as_uint(child[k][u].w);
+            const int next = r + record_hop(ci);
+            ref[k][u] = -1;
+            if (ci != kBodyInfo && r / kSumBlock != (next - 1) / kSumBlock) {
+                ref[k][u] = r / kSumBlock * kSumLevels + info_level(ci) + 1;
+                waits[k] = true;
+            }
+            s.add(child[k][u]);
+            r = next;
+        }
+        if (waits[k]) continue;          // (such a cell has at most four children)
+        while (r < end) {                // bodies at one point
+            const float4 c = rec[r];
+            s.add(c);
+            r += record_hop(__float_as_uint(c.w));
+        }
+        sum[q] = s.record(own[k].w);
+        rec[cell[k]] = sum[q];
+    }
+    __syncthreads();
+    for (int L = kSumLevels - 1; L >= 0; --L) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int q = tid + k * kSumThreads;
+            if (!waits[k] || q % kSumLevels != L) continue;
+            CellSum s;
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (ref[k][u] != -2) s.add(ref[k][u] >= 0 ? sum[ref[k][u]] : child[k][u]);
+            sum[q] = s.record(own[k].w);
+            rec[cell[k]] = sum[q];
+        }
+        __syncthreads();
+    }
+}
+
+// Larger trees, a launch per level. Bucket cells by level (order inside a level is irrelevant).
 __global__ __launch_bounds__(256) void k_levels(const int* __restrict__ cell_rec,
                                                 const unsigned char* __restrict__ cell_lvl,
                                                 int* __restrict__ level_list, DevState* st) {
@@ -1079,6 +1251,13 @@ void launch_tree(Bufs& b, hipStream_t s) {
     }
     if (b.int_mass) {
         if (!b.no_big) k_big<<<1, 256, 0, s>>>(b.rec, b.big_rc, b.big_lvl, b.st);
+        return;
+    }
+    // the spilled cells fit one block; larger trees fill the chip with a level each
+    const int sum_grid = (b.cap_records + kSumBlock - 1) / kSumBlock;
+    if (sum_grid <= kSumMaxBlocks) {
+        k_sum_blocks<<<sum_grid, kSumThreads, 0, s>>>(b.rec, b.level_list, b.st);
+        k_sum_spill<<<1, kSumThreads, 0, s>>>(b.rec, b.level_list, b.st);
         return;
     }
     k_levels<<<(max_cells + 255) / 256, 256, 0, s>>>(b.cell_rec, b.cell_lvl, b.level_list, b.st);
