@@ -63,18 +63,53 @@ __device__ void reduce_bbox(const float4* __restrict__ part, int np, float* root
     __syncthreads();
 }
 
-__global__ __launch_bounds__(256) void k_bbox_partials(const float2* __restrict__ pos, int n,
-                                                       float4* __restrict__ part, DevState* st) {
+// What the displacement leaves for the next iteration, from positions that came from elsewhere: the
+// degree-ranked copy, the bounding box's partials (one graph) and, with RESET, also cleared forces
+// and the first iteration's state. One launch: at some ten thousand bodies each is little but a
+// launch (20k bodies, positions set, then a reset, before one force evaluation: 366 us in all with
+// the four launches, six fills and two copies that this takes the place of, 343 with it).
+struct NewState {
+    float global_speed, speed_efficiency, jitter_tolerance, k_s_max;
+    int full_sorts;          // without RESET: the next sorts that are full ones (-1: as they were)
+};
+
+template <bool RESET>
+__global__ __launch_bounds__(256) void k_new_positions(const float2* __restrict__ pos, const int* __restrict__ rank,
+                                                       int n, float2* __restrict__ pos_rank,
+                                                       float4* __restrict__ part, DevState* st, NewState init,
+                                                       SegState* __restrict__ seg_st, int nseg,
+                                                       float2* __restrict__ f, float2* __restrict__ fprev,
+                                                       float2* __restrict__ fga) {
     __shared__ float4 red[256];
     const int tid = threadIdx.x;
     float2 p0 = pos[0];
     float4 acc = make_float4(p0.x, p0.y, p0.x, p0.y);
     for (int i = blockIdx.x * 256 + tid; i < n; i += gridDim.x * 256) {
         float2 p = pos[i];
+        pos_rank[rank[i]] = p;
         acc.x = fminf(acc.x, p.x);
         acc.y = fminf(acc.y, p.y);
         acc.z = fmaxf(acc.z, p.x);
         acc.w = fmaxf(acc.w, p.y);
+        if constexpr (RESET) {
+            const float2 z = make_float2(0.0f, 0.0f);
+            f[i] = z;
+            fprev[i] = z;
+            fga[i] = z;
+        }
+    }
+    if constexpr (RESET) {
+        for (int q = blockIdx.x * 256 + tid; q < nseg; q += gridDim.x * 256) {
+            SegState s{};
+            s.global_speed = init.global_speed;
+            s.speed_efficiency = init.speed_efficiency;
+            s.jitter_tolerance = init.jitter_tolerance;
+            s.k_s_max = init.k_s_max;
+            seg_st[q] = s;
+        }
+        static_assert(sizeof(DevState) % 4 == 0, "cleared word by word");
+        if (blockIdx.x == 0)
+            for (int w = tid; w < (int)(sizeof(DevState) / 4); w += 256) reinterpret_cast<int*>(st)[w] = 0;
     }
     red[tid] = acc;
     __syncthreads();
@@ -89,9 +124,18 @@ __global__ __launch_bounds__(256) void k_bbox_partials(const float2* __restrict_
         }
         __syncthreads();
     }
-    if (tid == 0) {
-        part[blockIdx.x] = red[0];
-        if (blockIdx.x == 0) st->nbbox = gridDim.x;
+    if (tid != 0) return;
+    if (nseg == 1) part[blockIdx.x] = red[0];
+    if (blockIdx.x > 0) return;
+    if (nseg == 1) st->nbbox = gridDim.x;
+    if constexpr (RESET) {
+        st->global_speed = init.global_speed;
+        st->speed_efficiency = init.speed_efficiency;
+        st->jitter_tolerance = init.jitter_tolerance;
+        st->k_s_max = init.k_s_max;
+    } else if (init.full_sorts >= 0) {
+        st->sort_skip = 0;
+        st->full_sorts = init.full_sorts;
     }
 }
 
@@ -1200,8 +1244,24 @@ int displacement_blocks(const Bufs& b) {
     return g < 1 ? 1 : (g > cap ? cap : g);
 }
 
-void launch_bbox_partials(const Bufs& b, hipStream_t s) {
-    k_bbox_partials<<<displacement_blocks(b), 256, 0, s>>>(b.pos, b.n, b.bbox_part, b.st);
+namespace {
+
+template <bool RESET>
+void new_positions(const Bufs& b, const NewState& init, hipStream_t s) {
+    k_new_positions<RESET><<<displacement_blocks(b), 256, 0, s>>>(b.pos, b.rank, b.n, b.pos_rank, b.bbox_part, b.st,
+                                                                 init, b.seg_st, b.nseg, b.f, b.fprev, b.fga);
+    if (b.nseg > 1) launch_seg_bbox(b, s);
+}
+
+}  // namespace
+
+void launch_new_positions(const Bufs& b, int full_sorts, hipStream_t s) {
+    new_positions<false>(b, NewState{0.0f, 0.0f, 0.0f, 0.0f, full_sorts}, s);
+}
+
+void launch_reset(const Bufs& b, float global_speed, float speed_efficiency, float jitter_tolerance, float k_s_max,
+                  hipStream_t s) {
+    new_positions<true>(b, NewState{global_speed, speed_efficiency, jitter_tolerance, k_s_max, -1}, s);
 }
 
 void launch_keys(const Bufs& b, int first, hipStream_t s) {

@@ -264,34 +264,10 @@ int drain_timing(gfa2_engine* h) {
     return GFA2_OK;
 }
 
-// What the displacement leaves for the next iteration, formed from positions that came from
-// elsewhere: the degree-ranked copy, and the bounding box's partials or the batch's roots.
-void positions_changed(gfa2_engine* h) {
-    launch_rank_pos(h->b, h->stream);
-    if (h->b.nseg > 1) launch_seg_bbox(h->b, h->stream);
-    else launch_bbox_partials(h->b, h->stream);
-}
-
 int reset_state(gfa2_engine* h) {
-    DevState st{};
-    st.global_speed = h->user.global_speed;
-    st.speed_efficiency = h->user.speed_efficiency;
-    st.jitter_tolerance = h->user.jitter_tolerance;
-    st.k_s_max = h->user.k_s_max;
-    GFA2_TRY(hipMemcpyAsync(h->b.st, &st, sizeof(DevState), hipMemcpyHostToDevice, h->stream));
-    std::vector<SegState> seg((size_t)h->b.nseg);
-    for (SegState& q : seg) {
-        q = SegState{};
-        q.global_speed = h->user.global_speed;
-        q.speed_efficiency = h->user.speed_efficiency;
-        q.jitter_tolerance = h->user.jitter_tolerance;
-        q.k_s_max = h->user.k_s_max;
-    }
-    GFA2_TRY(hipMemcpyAsync(h->b.seg_st, seg.data(), sizeof(SegState) * seg.size(), hipMemcpyHostToDevice, h->stream));
-    GFA2_TRY(hipMemsetAsync(h->b.fprev, 0, sizeof(float2) * h->b.n, h->stream));
-    GFA2_TRY(hipMemsetAsync(h->b.f, 0, sizeof(float2) * h->b.n, h->stream));
-    GFA2_TRY(hipMemsetAsync(h->b.fga, 0, sizeof(float2) * h->b.n, h->stream));
-    if (h->has_pos) positions_changed(h);
+    launch_reset(h->b, h->user.global_speed, h->user.speed_efficiency, h->user.jitter_tolerance, h->user.k_s_max,
+                 h->stream);
+    GFA2_TRY(hipGetLastError());
     GFA2_TRY(hipStreamSynchronize(h->stream));
     return GFA2_OK;
 }
@@ -320,6 +296,12 @@ void set_sort_first(gfa2_engine* h, int first) {
 // tree would underestimate the next one's tied runs (at R-MAT 2^24 from a random start, the
 // second iteration's runs took the fix-up 31 ms).
 constexpr int kFullSortsAfterNew = 3;
+
+// The positions on the device are new ones.
+void positions_changed(gfa2_engine* h) {
+    set_sort_first(h, 0);
+    launch_new_positions(h->b, kFullSortsAfterNew, h->stream);
+}
 
 hipError_t full_sort_next(gfa2_engine* h) {
     set_sort_first(h, 0);
@@ -769,7 +751,6 @@ int gfa2_set_positions(gfa2_handle h, const float* xy) {
     if (!h || !xy) return GFA2_ERR_INVALID_ARG;
     if (!h->has_graph) return GFA2_ERR_NO_GRAPH;
     GFA2_TRY(hipSetDevice(h->device));
-    GFA2_TRY(full_sort_next(h));
     GFA2_TRY(hipMemcpyAsync(h->b.pos, xy, sizeof(float2) * h->b.n, hipMemcpyHostToDevice, h->stream));
     positions_changed(h);
     GFA2_TRY(hipGetLastError());
@@ -1128,9 +1109,8 @@ int gfa2_autotune(gfa2_handle h, int32_t iters, gfa2_launch_config* best) {
     float2 *spos = nullptr, *sfp = nullptr, *sf = nullptr, *sfga = nullptr;
     DevState* sst = nullptr;
     SegState* sseg = nullptr;
-    float4* spart = nullptr;
     auto free_snapshot = [&]() {
-        for (void* p : {(void*)spos, (void*)sfp, (void*)sf, (void*)sfga, (void*)sst, (void*)sseg, (void*)spart})
+        for (void* p : {(void*)spos, (void*)sfp, (void*)sf, (void*)sfga, (void*)sst, (void*)sseg})
             if (p) (void)hipFree(p);
     };
     {
@@ -1140,7 +1120,6 @@ int gfa2_autotune(gfa2_handle h, int32_t iters, gfa2_launch_config* best) {
         if (ea == hipSuccess) ea = hipMalloc(&sfga, sizeof(float2) * n);
         if (ea == hipSuccess) ea = hipMalloc(&sst, sizeof(DevState));
         if (ea == hipSuccess) ea = hipMalloc(&sseg, sizeof(SegState) * b.nseg);
-        if (ea == hipSuccess) ea = hipMalloc(&spart, sizeof(float4) * kPartBlocks);
         if (ea != hipSuccess) {
             free_snapshot();
             return hip_status(ea);
@@ -1158,7 +1137,6 @@ int gfa2_autotune(gfa2_handle h, int32_t iters, gfa2_launch_config* best) {
             cp(sfga, b.fga, sizeof(float2) * n);
             cp(sst, b.st, sizeof(DevState));
             cp(sseg, b.seg_st, sizeof(SegState) * b.nseg);
-            cp(spart, b.bbox_part, sizeof(float4) * kPartBlocks);
         } else {
             cp(b.pos, spos, sizeof(float2) * n);
             cp(b.fprev, sfp, sizeof(float2) * n);
@@ -1166,9 +1144,7 @@ int gfa2_autotune(gfa2_handle h, int32_t iters, gfa2_launch_config* best) {
             cp(b.fga, sfga, sizeof(float2) * n);
             cp(b.st, sst, sizeof(DevState));
             cp(b.seg_st, sseg, sizeof(SegState) * b.nseg);
-            cp(b.bbox_part, spart, sizeof(float4) * kPartBlocks);
-            launch_rank_pos(b, h->stream);
-            if (b.nseg > 1) launch_seg_bbox(b, h->stream);
+            launch_new_positions(b, -1, h->stream);
         }
         if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
         return e;
@@ -1404,7 +1380,6 @@ bool engine_view(gfa2_engine* h, EngineView* v) {
 
 int engine_positions_written(gfa2_engine* h) {
     h->has_pos = true;
-    GFA2_TRY(full_sort_next(h));
     positions_changed(h);
     GFA2_TRY(hipGetLastError());
     GFA2_TRY(hipStreamSynchronize(h->stream));

@@ -262,7 +262,12 @@ constexpr int kSegSortMax = 32768;
 // alone: no other kernel is to run beside it
 void launch_attraction(const Bufs& b, const Params& p, bool alone, hipStream_t s);
 void launch_col_rank(const Bufs& b, hipStream_t s);
-void launch_bbox_partials(const Bufs& b, hipStream_t s);
+// Positions that came from elsewhere: what the displacement leaves for the next iteration, and the
+// number of full sorts that follow (-1: as it was).
+void launch_new_positions(const Bufs& b, int full_sorts, hipStream_t s);
+// The same with cleared forces and the state of a first iteration.
+void launch_reset(const Bufs& b, float global_speed, float speed_efficiency, float jitter_tolerance, float k_s_max,
+                  hipStream_t s);
 // first: the lowest path-key sort pass the host launches; the keys go to the buffer from which
 // the passes that will run end in buffer 0.
 void launch_keys(const Bufs& b, int first, hipStream_t s);
@@ -284,8 +289,6 @@ void launch_walk(const Bufs& b, const Params& p, bool split, hipStream_t s);
 void launch_combine(const Bufs& b, const Params& p, hipStream_t s);
 void launch_speed(const Bufs& b, hipStream_t s);
 void launch_displacement(const Bufs& b, hipStream_t s);
-// The degree-ranked copy of the positions, after they were written by anything but the displacement.
-void launch_rank_pos(const Bufs& b, hipStream_t s);
 // A batch whose displacement also sets the roots of the next trees (no launch_seg_bbox per iteration).
 bool advance_seg(const Bufs& b);
 // Exact mode: pack {pos, mass} in node order, then all-pairs repulsion per graph with the

@@ -25,14 +25,6 @@ __global__ __launch_bounds__(256) void k_gather_rank(const int* __restrict__ col
         col_rank[e] = rank[col[e]];
 }
 
-// pos_rank[rank[v]] = pos[v] (for positions that came from outside; the displacement keeps the copy
-// up to date afterwards).
-__global__ __launch_bounds__(256) void k_rank_pos(const float2* __restrict__ pos, const int* __restrict__ rank, int n,
-                                                  float2* __restrict__ pos_rank) {
-    const int v = blockIdx.x * 256 + threadIdx.x;
-    if (v < n) pos_rank[rank[v]] = pos[v];
-}
-
 // Block i of the light and medium ones, which take turns in proportion (256 threads).
 template <bool GEN, int HUB>
 __device__ __forceinline__ void attract_rows(int i, int light_blocks, int medium_blocks, int medium_rows, int tid,
@@ -578,7 +570,7 @@ __global__ __launch_bounds__(256) void k_combine(const float4* __restrict__ sbod
 //   k_advance_seg  a batch of graphs of up to kSegSortMax nodes: one block per graph
 //   k_speed, k_displace   larger graphs
 // Each launch on a small graph costs 4-5 us however little it does: with the attraction's
-// position copy (k_rank_pos) the three launches were 13.9 us of 107 on 10,000 nodes.
+// position copy the three launches were 13.9 us of 107 on 10,000 nodes.
 // ---------------------------------------------------------------------------------------
 constexpr int kSpeedSums = 1024;
 constexpr int kAdvanceGroups = 2048;
@@ -1157,10 +1149,6 @@ bool advance_one(const Bufs& b) { return b.nseg == 1 && b.ngroups <= kAdvanceGro
 }  // namespace
 
 bool advance_seg(const Bufs& b) { return b.nseg > 1 && b.max_seg <= kSegSortMax; }
-
-void launch_rank_pos(const Bufs& b, hipStream_t s) {
-    k_rank_pos<<<(b.n + 255) / 256, 256, 0, s>>>(b.pos, b.rank, b.n, b.pos_rank);
-}
 
 void launch_speed(const Bufs& b, hipStream_t s) {
     if (advance_one(b) || advance_seg(b)) return;          // done with the displacement
