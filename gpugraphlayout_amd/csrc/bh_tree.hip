@@ -156,7 +156,8 @@ __global__ __launch_bounds__(256) void k_keys(const float2* __restrict__ pos, co
         for (int p = 0; p < 8; ++p) h[p][threadIdx.x] = 0u;
     // the buffer from which the sort passes that will run (8 less the skipped or unlaunched low
     // ones) end in buffer 0
-    const bool odd = ((8 - max(st->sort_skip, first)) & 1) != 0;
+    const int low = max(st->sort_skip, first);
+    const bool odd = ((8 - low) & 1) != 0;
     unsigned long long* __restrict__ keys = odd ? k1 : k0;
     unsigned int* __restrict__ vals = odd ? v1 : v0;
     reduce_bbox(part, st->nbbox, root);
@@ -176,11 +177,12 @@ __global__ __launch_bounds__(256) void k_keys(const float2* __restrict__ pos, co
         pm[i] = make_float4(p.x, p.y, mass[i], 0.0f);   // one gather per body for k_lcp
         if (dhist)
 #pragma unroll
-            for (int d = 0; d < 8; ++d) atomicAdd(&h[d][(unsigned)(key >> (8 * d)) & 255u], 1u);
+            for (int d = 0; d < 8; ++d)
+                if (d >= low) atomicAdd(&h[d][(unsigned)(key >> (8 * d)) & 255u], 1u);
     }
     if (dhist) {
         __syncthreads();
-        for (int d = 0; d < 8; ++d) {
+        for (int d = low; d < 8; ++d) {
             const unsigned int c = h[d][threadIdx.x];
             if (c) atomicAdd(&dhist[d * 256 + threadIdx.x], c);
         }
@@ -1267,6 +1269,10 @@ void launch_reset(const Bufs& b, float global_speed, float speed_efficiency, flo
 void launch_keys(const Bufs& b, int first, hipStream_t s) {
     int blocks = (b.n + 255) / 256;
     if (blocks > b.grid_cap) blocks = b.grid_cap;
+    // Each block that counts digits adds up to 256 counts per pass to the table: at 131,000 bodies
+    // 145.6 us an iteration with 128 blocks, 146.5 with 256, 150.5 with one per 256 bodies; at
+    // 262,000 198.2, 196.5, 207.6
+    if (b.sort.hist_in_keys) blocks = std::min(blocks, std::max(128, (b.n + 1023) / 1024));
     k_keys<<<blocks, 256, 0, s>>>(b.pos, b.mass, b.n, b.bbox_part, b.st, b.seg_root, b.sort.keys[0], b.sort.vals[0],
                                   b.sort.keys[1], b.sort.vals[1], b.pm, first,
                                   b.sort.hist_in_keys ? b.sort.digit_hist : nullptr, b.seg_st, b.seg_cur);

@@ -562,7 +562,7 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
     GFA2_TRY(hipMemsetAsync(b.sort.digit_hist, 0, sizeof(unsigned int) * 8 * 256, h->stream));
     GFA2_ALLOC(b.sort.status, (size_t)256 * sort_tiles);
     GFA2_ALLOC(b.sort.ticket, 1);
-    // look-back state starts empty: no published tile, ticket 0
+    // no tile has published counts, ticket 0
     GFA2_TRY(hipMemsetAsync(b.sort.status, 0, sizeof(unsigned int) * 256 * (size_t)sort_tiles, h->stream));
     GFA2_TRY(hipMemsetAsync(b.sort.ticket, 0, sizeof(unsigned long long), h->stream));
     GFA2_ALLOC(b.lcp, n);

@@ -34,7 +34,7 @@ constexpr int kPartBlocks = 1024;       // bounding-box partials (displacement g
 
 // Error flags raised on the device, read back at synchronisation points.
 constexpr int kErrTreeOverflow = 1;
-constexpr int kErrSortWait = 2;         // a sort look-back wait ran out (results invalid)
+constexpr int kErrSortWait = 2;         // a wait for another tile of a sort pass ran out (results invalid)
 
 // Per-instance scalar state, resident in device memory.
 struct DevState {
@@ -80,13 +80,13 @@ struct SortBuffers {
     unsigned int* vals[2];
     unsigned int* hist;      // 256 x tiles (three-launch passes)
     unsigned int* rowtot;    // 256
-    bool onesweep = true;    // one launch per pass with decoupled look-back
+    bool onesweep = true;    // one launch per pass where that is faster (radix_sort.hip)
     unsigned int* digit_hist = nullptr;   // 8 x 256: digit totals of every pass
     bool hist_in_keys = false;            // k_keys counts the digits; the fix-up clears the table
-    unsigned int* status = nullptr;       // tiles x 256: published tile counts / prefixes
+    unsigned int* status = nullptr;       // tiles x 256: published tile counts
     unsigned long long* ticket = nullptr; // tile tickets, never reset while the tile count holds
     int* err = nullptr;                   // the instance's error word: kErrSortWait is raised there if a
-                                          // look-back wait runs out (never expected)
+                                          // wait for another tile runs out (never expected)
 };
 
 // FA2 scalar parameters (src/RPForceAtlas2.cpp:28-55 defaults).

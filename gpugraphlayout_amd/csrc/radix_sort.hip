@@ -1,16 +1,16 @@
 // LSD radix sort of (u64 key, u32 value) pairs for gfx950.
 //
-// Up to 64 tiles (131,072 pairs): one launch per 8-bit pass ("onesweep"), after one histogram
-// launch for all passes.
+// Up to 262,144 pairs: one launch per 8-bit pass ("onesweep"), after one histogram launch for all
+// passes.
 //   k_sort_hist  digit histograms of every pass at once (order-independent), LDS then global
 //                atomics; the table is cleared by k_sort_zero first
-//   k_onesweep   per tile (2048 pairs): tiles are taken in the order of a global ticket, the
-//                tile's digit counts are published, the exclusive prefix of each digit over the
-//                earlier tiles is found by looking back over their published counts (decoupled
-//                look-back), then the stable rank within the tile (wave64 ballot matching) gives
-//                each pair's destination. A tile only ever waits for tiles with smaller tickets,
-//                which started before it and publish their counts before they wait themselves,
-//                so the waits end; every wait is also bounded and raises an error flag.
+//   k_onesweep   per tile (8 pairs per thread): tiles are taken in the order of a global ticket,
+//                the tile's digit counts are published, and while they travel the tile ranks its
+//                pairs stably (wave64 ballot matching). Then every earlier tile's counts are read,
+//                eight at a time, and added: each digit's exclusive prefix, without a chain from
+//                tile to tile. A tile only ever waits for tiles with smaller tickets, which started
+//                before it and publish their counts before they wait themselves, so the waits end;
+//                every wait is also bounded and raises an error flag.
 // Larger inputs (or SortBuffers::onesweep = false): three launches per pass (per-tile histograms,
 // a scan over tiles per digit, scatter), with every cross-tile dependency through a launch
 // boundary.
@@ -346,11 +346,20 @@ __global__ __launch_bounds__(kSortThreads) void k_seg_sort(unsigned long long* _
 }
 
 // ---- onesweep -------------------------------------------------------------------------------
-constexpr unsigned int kStatAgg = 1u << 30;      // the tile's own digit count is published
-constexpr unsigned int kStatPre = 2u << 30;      // the inclusive prefix over tiles is published
+constexpr unsigned int kStatAgg = 1u << 30;      // the tile's digit count is published, with its pass's epoch
 constexpr unsigned int kStatCount = (1u << 27) - 1;
-constexpr int kOnesweepMaxTiles = 64;
-constexpr int kMaxSpins = 1 << 20;   // per thread and look-back: ~1 s at worst, then an error
+
+// A pass of one launch costs its chain of steps across the chip (ticket, pairs, published counts,
+// the other tiles' counts, destinations), not its bytes. Tiles of 256 threads up to 32,768 pairs, where
+// they spread over more compute units (20,000 bodies: 99.7 us an iteration, 101.0 with 512
+// threads); of 512 up to 262,144, where fewer tiles have to be read (131,000: 145.6, with 256 threads
+// 151.1). Beyond, three launches per pass are as fast (262,000: 198.5 us an iteration against 196.5;
+// 300,000: 225.7 against 224.8; 2M: 1,118 against 1,159). 1,024 threads were slower
+// throughout. With a look-back from tile to tile the iterations took 104.1 us at 20,000, 121.8 (now
+// 115.0) at 50,000 and 158.2 at 131,000.
+constexpr int kSweepSmall = 32768;
+constexpr int kSweepMost = 262144;
+constexpr int kMaxSpins = 1 << 20;   // per thread and pass: ~1 s at worst, then an error
 
 __global__ void k_sort_zero(unsigned int* __restrict__ digit_hist, int npasses) {
     for (int i = threadIdx.x; i < npasses * 256; i += blockDim.x) digit_hist[i] = 0u;
@@ -375,42 +384,70 @@ __global__ __launch_bounds__(256) void k_sort_hist(const unsigned long long* __r
     }
 }
 
-__global__ __launch_bounds__(kSortThreads) void k_onesweep(unsigned long long* __restrict__ k0,
-                                                           unsigned int* __restrict__ v0,
-                                                           unsigned long long* __restrict__ k1,
-                                                           unsigned int* __restrict__ v1, int n, int shift,
-                                                           const unsigned int* __restrict__ digit_hist,
-                                                           unsigned int* __restrict__ status,
-                                                           unsigned long long* __restrict__ ticket, int tiles,
-                                                           int* __restrict__ err, const DevState* __restrict__ st,
-                                                           int first, int lead, int pass) {
+// LDS of a pass of one launch. The tile's keys are staged first, then its values.
+template <int T>
+struct SweepLds {
+    unsigned int wcnt[T / 64][256];              // per-wave digit counts, then the waves' starts
+    unsigned int tcount[256];
+    unsigned int before[T / 256][256];           // counts of the earlier tiles
+    int delta[256];                              // global destination minus tile position, per digit
+    unsigned long long stage[T * kSortItems];
+    unsigned int sh[2][4];
+    int tile;
+    unsigned int epoch;
+};
+
+// Exclusive scan of one value per thread over the block's first 256 threads (one barrier).
+__device__ __forceinline__ unsigned int digit_exscan(unsigned int v, unsigned int* __restrict__ sh) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned int inc = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned int t = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += t;
+    }
+    if (lane == 63 && wave < 4) sh[wave] = inc;
+    __syncthreads();
+    unsigned int off = 0u;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+        if (w < wave) off += sh[w];
+    return off + inc - v;
+}
+
+template <int T>
+__global__ __launch_bounds__(T) void k_onesweep(unsigned long long* __restrict__ k0, unsigned int* __restrict__ v0,
+                                                unsigned long long* __restrict__ k1, unsigned int* __restrict__ v1,
+                                                int n, int shift, const unsigned int* __restrict__ digit_hist,
+                                                unsigned int* __restrict__ status,
+                                                unsigned long long* __restrict__ ticket, int tiles,
+                                                int* __restrict__ err, const DevState* __restrict__ st, int first,
+                                                int lead, int pass) {
+    constexpr int kTile = T * kSortItems, kParts = T / 256, kAhead = 8;
     if (pass_skipped(st, pass)) return;   // takes no ticket: the epochs of later passes stay distinct
     const int src = pass_src(st, first, lead, pass);
     const unsigned long long* __restrict__ kin = src ? k1 : k0;
     const unsigned int* __restrict__ vin = src ? v1 : v0;
     unsigned long long* __restrict__ kout = src ? k0 : k1;
     unsigned int* __restrict__ vout = src ? v0 : v1;
-    __shared__ TileLds L;
-    __shared__ unsigned int tcount[256];
-    __shared__ int s_tile;
-    __shared__ unsigned int s_epoch;
+    __shared__ SweepLds<T> L;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
+    const int digit = tid & 255, part = tid >> 8;
     if (tid == 0) {
         const unsigned long long t = atomicAdd(ticket, 1ull);
-        s_tile = (int)(t % (unsigned long long)tiles);
-        s_epoch = (unsigned int)((t / (unsigned long long)tiles) & 7ull);
+        L.tile = (int)(t % (unsigned long long)tiles);
+        L.epoch = (unsigned int)((t / (unsigned long long)tiles) & 7ull) << 27;
     }
-    tcount[tid] = 0u;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) L.wcnt[w][tid] = 0;
-    // exclusive scan of this pass's digit totals (its barrier also publishes s_tile and the zeros)
-    const unsigned int gstart = block_exscan256(digit_hist[tid], L.sh[0]);
-    const int tile = s_tile;
-    const unsigned int epoch = s_epoch << 27;
-    // the tile's pairs, held in registers (each wave a contiguous quarter), and its digit counts
-    const int wbase = tile * kSortTile + wave * (kSortItems * 64);
+    for (int i = tid; i < T / 64 * 256; i += T) L.wcnt[0][i] = 0u;
+    if (tid < 256) L.tcount[tid] = 0u;
+    const unsigned int total = tid < 256 ? digit_hist[tid] : 0u;
+    __syncthreads();
+    const int tile = L.tile;
+    const unsigned int epoch = L.epoch;
+    // the tile's pairs, held in registers (each wave a contiguous run), and its digit counts
+    const int wbase = tile * kTile + wave * (kSortItems * 64);
     unsigned long long key[kSortItems];
     unsigned int val[kSortItems];
 #pragma unroll
@@ -418,38 +455,87 @@ __global__ __launch_bounds__(kSortThreads) void k_onesweep(unsigned long long* _
         const int e = wbase + r * 64 + lane;
         key[r] = e < n ? kin[e] : 0ull;
         val[r] = e < n ? vin[e] : 0u;
-        if (e < n) atomicAdd(&tcount[(unsigned)(key[r] >> shift) & 255u], 1u);
+    }
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r)
+        if (wbase + r * 64 + lane < n) atomicAdd(&L.tcount[(unsigned)(key[r] >> shift) & 255u], 1u);
+    __syncthreads();
+    const unsigned int count = L.tcount[digit];
+    if (part == 0)
+        __hip_atomic_store(status + (size_t)tile * 256 + digit, kStatAgg | epoch | count, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    // the counts are on their way to the other tiles while this tile ranks its pairs
+    unsigned int rank[kSortItems];
+    rank_rows(key, wbase, n, shift, L.wcnt[wave], rank);
+    unsigned int sum = 0u;
+    int spins = 0;                       // bounded over all of a thread's waits
+    for (int t0 = part; t0 < tile; t0 += kParts * kAhead) {
+        unsigned int v[kAhead];
+        bool ready;
+        do {
+            ready = true;
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int t = t0 + u * kParts;
+                v[u] = t < tile ? __hip_atomic_load(status + (size_t)t * 256 + digit, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT)
+                                : (kStatAgg | epoch);
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) ready = ready && (v[u] & ~kStatCount) == (kStatAgg | epoch);
+        } while (!ready && ++spins < kMaxSpins);
+        if (!ready) {                    // (too small a sum keeps every destination in range)
+            atomicOr(err, kErrSortWait);
+            break;
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) sum += v[u] & kStatCount;
+    }
+    L.before[part][digit] = sum;
+    const unsigned int gstart = digit_exscan(total, L.sh[0]);                       // (barrier)
+    const unsigned int tstart = digit_exscan(tid < 256 ? count : 0u, L.sh[1]);      // (barrier)
+    if (tid < 256) {
+        unsigned int excl = 0u;
+#pragma unroll
+        for (int q = 0; q < kParts; ++q) excl += L.before[q][tid];
+        L.delta[tid] = (int)(gstart + excl) - (int)tstart;
+        unsigned int run = tstart;
+#pragma unroll
+        for (int w = 0; w < T / 64; ++w) {
+            const unsigned int c = L.wcnt[w][tid];
+            L.wcnt[w][tid] = run;
+            run += c;
+        }
     }
     __syncthreads();
-    // publish, look back, publish the inclusive prefix (one digit per thread)
-    unsigned int* my = status + (size_t)tile * 256 + tid;
-    const unsigned int cnt = tcount[tid];
-    unsigned int excl = 0u;
-    if (tile == 0) {
-        __hip_atomic_store(my, kStatPre | epoch | cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-        __hip_atomic_store(my, kStatAgg | epoch | cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        int spins = 0;                       // bounded over the whole look-back
-        for (int t = tile - 1; t >= 0; --t) {
-            const unsigned int* src = status + (size_t)t * 256 + tid;
-            unsigned int v = 0u;
-            for (;;) {
-                v = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if ((v >> 30) != 0u && (v & (7u << 27)) == epoch) break;
-                if (++spins >= kMaxSpins) break;
-                __builtin_amdgcn_s_sleep(1);
-            }
-            if (spins >= kMaxSpins) {
-                atomicOr(err, kErrSortWait);
-                break;
-            }
-            excl += v & kStatCount;
-            if ((v >> 30) == 2u) break;
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r)
+        if (wbase + r * 64 + lane < n) {
+            rank[r] += L.wcnt[wave][(unsigned)(key[r] >> shift) & 255u];
+            L.stage[rank[r]] = key[r];
         }
-        __hip_atomic_store(my, kStatPre | epoch | ((excl + cnt) & kStatCount), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int here = min(kTile, n - tile * kTile);
+    unsigned int dst[kSortItems];
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r) {
+        const int j = tid + r * T;
+        if (j >= here) continue;
+        const unsigned long long k = L.stage[j];
+        dst[r] = (unsigned int)(L.delta[(unsigned)(k >> shift) & 255u] + j);
+        kout[dst[r]] = k;
     }
-    scatter_tile(key, val, tile, n, shift, gstart + excl, L, kout, vout);
+    __syncthreads();
+    unsigned int* sval = reinterpret_cast<unsigned int*>(L.stage);
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r)
+        if (wbase + r * 64 + lane < n) sval[rank[r]] = val[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r) {
+        const int j = tid + r * T;
+        if (j < here) vout[dst[r]] = sval[j];
+    }
 }
 
 // (key, value) pairs in lexicographic order (values are distinct body ids: a total order).
@@ -596,7 +682,7 @@ void launch_sort_fixup(SortBuffers& buf, int n, const DevState* st, hipStream_t 
 }
 
 bool sort_onesweep(const SortBuffers& buf, int n) {
-    return buf.onesweep && (n + kSortTile - 1) / kSortTile <= kOnesweepMaxTiles;
+    return buf.onesweep && n <= kSweepMost;
 }
 
 void segmented_sort_pairs(SortBuffers& buf, const int* node_off, const int* order, int nseg, hipStream_t s,
@@ -616,18 +702,19 @@ void radix_sort_pairs(SortBuffers& buf, int n, int begin_bit, int end_bit, hipSt
     // run may end in buffer 1, and launch_sort_fixup moves the result to buffer 0.
     unsigned long long *k0 = buf.keys[0], *k1 = buf.keys[1];
     unsigned int *v0 = buf.vals[0], *v1 = buf.vals[1];
-    // One launch per pass pays off while the look-back chains stay short; with hundreds of
-    // tiles resident at once the chains grow with the tile count and three launches per pass win.
-    if (buf.onesweep && tiles <= kOnesweepMaxTiles) {
+    if (sort_onesweep(buf, n)) {
         if (!hist_ready) {
             k_sort_zero<<<1, 256, 0, s>>>(buf.digit_hist, npasses);
             int hb = (n + 255) / 256;
             if (hb > 256) hb = 256;
             k_sort_hist<<<hb, 256, 0, s>>>(k0, k1, n, begin_bit, npasses, buf.digit_hist, skip, first, lead);
         }
+        const int threads = n <= kSweepSmall ? 256 : 512;
+        const int sweeps = (n + threads * kSortItems - 1) / (threads * kSortItems);
+        const auto sweep = threads == 256 ? k_onesweep<256> : k_onesweep<512>;
         for (int p = first; p < npasses; ++p)
-            k_onesweep<<<tiles, kSortThreads, 0, s>>>(k0, v0, k1, v1, n, begin_bit + 8 * p, buf.digit_hist + 256 * p,
-                                                      buf.status, buf.ticket, tiles, buf.err, skip, first, lead, p);
+            sweep<<<sweeps, threads, 0, s>>>(k0, v0, k1, v1, n, begin_bit + 8 * p, buf.digit_hist + 256 * p,
+                                             buf.status, buf.ticket, sweeps, buf.err, skip, first, lead, p);
     } else {
         for (int p = first; p < npasses; ++p) {
             const int shift = begin_bit + 8 * p;
