@@ -213,7 +213,7 @@ void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
         if (b.nseg > 1 && b.max_seg <= kSegSortMax) {
             // every graph fits one block's sort: by (graph, key) in one launch, the low passes
             // skipped as for one graph; the result is in buffer 0 and runs stop at graphs
-            segmented_sort_pairs(b.sort, b.node_off, b.seg_order, b.nseg, s, b.st);
+            segmented_sort_pairs(b.sort, b.node_off, b.seg_order, b.nseg, b.max_seg, b.large_segs, s, b.st);
             launch_sort_fixup(b.sort, b.n, b.st, s, 0, true, b.seg_of);
         } else {
             // the previous tree's depth bounds the key bits the order needs (skipped low passes
@@ -611,6 +611,8 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
             return node_off[x + 1] - node_off[x] > node_off[y + 1] - node_off[y];
         });
         b.max_seg = node_off[order[0] + 1] - node_off[order[0]];
+        b.large_segs = 0;
+        for (int q : order) b.large_segs += node_off[q + 1] - node_off[q] > kSegSmall;
         GFA2_ALLOC(b.seg_order, nseg);
         GFA2_TRY(hipMemcpyAsync(b.seg_order, order.data(), sizeof(int) * nseg, hipMemcpyHostToDevice, h->stream));
         GFA2_TRY(hipStreamSynchronize(h->stream));   // order goes out of scope

@@ -183,6 +183,7 @@ struct Bufs {
     int* grp_first = nullptr;         // graph -> first group, nseg + 1
     int* seg_order = nullptr;         // graphs by decreasing node count (per-graph sort)
     int max_seg = 0;                  // largest graph's node count
+    int large_segs = 0;               // graphs of more than kSegSmall nodes
     struct SegState* seg_st = nullptr;
     struct SegState* seg_cur = nullptr;   // one graph: the state before the iteration, copied by its first kernel
     WalkPart* grp_part = nullptr;     // per group
@@ -250,13 +251,16 @@ void launch_sort_fixup(SortBuffers& buf, int n, const DevState* st, hipStream_t 
 // 4p-level cells of the previous tree hold at most this many bodies.
 constexpr int kSortRunMax = 16;
 // Sorts each segment [node_off[g], node_off[g+1]) of buf.keys[0]/vals[0] in place by the full
-// 64-bit key, stable, one block per segment (taken in `order`); for batches whose graphs all
+// 64-bit key, stable, one block per one or four segments (taken in `order`); for batches whose graphs all
 // have at most kSegSortMax nodes.
 // skip: the state whose sort_skip low passes are skipped (then launch_sort_fixup with the
 // graph of each position, and lead, finishes the order); null: all 8 passes.
-void segmented_sort_pairs(SortBuffers& buf, const int* node_off, const int* order, int nseg, hipStream_t s,
-                          const DevState* skip = nullptr);
+// max_seg: pairs of the longest segment; large: how many have more than kSegSmall (the first ones
+// of order).
+void segmented_sort_pairs(SortBuffers& buf, const int* node_off, const int* order, int nseg, int max_seg, int large,
+                          hipStream_t s, const DevState* skip = nullptr);
 constexpr int kSegSortMax = 32768;
+constexpr int kSegSmall = 2048;
 
 // Launch groups of one iteration, in order.
 // alone: no other kernel is to run beside it

@@ -260,89 +260,242 @@ __global__ __launch_bounds__(kSortThreads) void k_scatter(unsigned long long* __
     scatter_tile(key, val, blockIdx.x, n, shift, dglobal, L, kout, vout);
 }
 
-// ---- one block per segment ----------------------------------------------------------------
-// Segment g is [node_off[g], node_off[g+1]) of both buffers; its pairs are sorted in place by
-// the full key, stable, by one block: the digit histograms of all passes first, then per pass
-// the segment's tiles in order, each ranked stably and written to its sorted place in the
-// other buffer (the running digit starts carry from tile to tile). Eight passes end in buffer
-// 0. Blocks take segments in `order` (largest first), so the longest ones start first.
-__global__ __launch_bounds__(kSortThreads) void k_seg_sort(unsigned long long* __restrict__ k0,
-                                                           unsigned int* __restrict__ v0,
-                                                           unsigned long long* __restrict__ k1,
-                                                           unsigned int* __restrict__ v1,
-                                                           const int* __restrict__ node_off,
-                                                           const int* __restrict__ order,
-                                                           const DevState* __restrict__ st) {
-    __shared__ TileLds L;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int g = order[blockIdx.x];
-    // the low passes the previous trees' cells let the sort skip (k_sort_fixup, told the graph
-    // of each position, orders what they would have ordered)
-    const int p0 = st ? st->sort_skip : 0;
-    const int a = node_off[g];
-    const int m = node_off[g + 1] - a;
-    // the 8 digit histograms (8 x 256 words), counted in the not yet used tile staging area when
-    // it holds them, then kept per thread for its own digit: hc[0] is the current pass's count,
-    // shifted down after each pass
-    constexpr bool kAlias = kSortTile >= 8 * 256;
-    __shared__ unsigned int hist_own[kAlias ? 1 : 8 * 256];
-    unsigned int* hist = kAlias ? L.sval : hist_own;
+// ---- one block per segment, or four segments per block ---------------------------------------
+// Segment g is [node_off[g], node_off[g+1]) of both buffers; its pairs are sorted by the full key,
+// stable, into buffer 0. A block of 1,024 threads takes one segment of more than kSegSmall
+// pairs, or four smaller ones, a quarter of its threads each (every quarter runs the same passes
+// and meets the same barriers). A segment of up to 8 pairs per thread stays in registers and LDS
+// from its first pass to its last; a longer one takes its tiles in order in every pass, from one
+// buffer to the other, with the running digit starts of all passes counted beforehand. Blocks take
+// segments in `order` (largest first), so the longest ones start first. What bounds it is the
+// largest segment's chain of tile steps: 192 graphs of 100 to 20,000 bodies 62 us, where blocks of 256
+// threads that went through memory in every pass took 104.
+constexpr int kSegThreads = 1024;
+static_assert(kSegSmall == 256 * kSortItems);
+
+// LDS of a group of T threads.
+template <int T>
+struct SegLds {
+    unsigned int wcnt[T / 64][256];              // per-wave digit counts, then the waves' starts
+    int delta[256];                              // destination minus tile position, per digit
+    unsigned int sh[4];
+    unsigned long long stage[T * kSortItems];
+};
+
+// Exclusive scan of one value per thread over the group's first 256 threads (one barrier).
+__device__ __forceinline__ unsigned int digit_exscan(unsigned int v, unsigned int* __restrict__ sh, int wave) {
+    const int lane = threadIdx.x & 63;
+    unsigned int inc = v;
 #pragma unroll
-    for (int p = 0; p < 8; ++p) hist[p * 256 + tid] = 0u;
-    __syncthreads();
-    for (int e = tid; e < m; e += kSortThreads) {
-        const unsigned long long k = k0[a + e];
-#pragma unroll
-        for (int p = 0; p < 8; ++p) atomicAdd(&hist[p * 256 + ((unsigned)(k >> (8 * p)) & 255u)], 1u);
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned int t = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += t;
     }
+    if (lane == 63 && wave < 4) sh[wave] = inc;
     __syncthreads();
-    unsigned int hc[8];
+    unsigned int off = 0u;
 #pragma unroll
-    for (int p = 0; p < 8; ++p) hc[p] = hist[p * 256 + tid];
-    __syncthreads();                             // the staging area is the tiles' again
-    for (int p = 0; p < p0; ++p) {
+    for (int w = 0; w < 4; ++w)
+        if (w < wave) off += sh[w];
+    return off + inc - v;
+}
+
+// Ranks a tile of m pairs (each wave a contiguous run): rank[r] becomes the pair's place in the
+// tile. Returns the digit's count and start in the tile (the group's first 256 threads). Ends in
+// front of a barrier that the caller has to pass before it reads starts another thread may move.
+template <int T>
+__device__ __forceinline__ unsigned int rank_tile(const unsigned long long (&key)[kSortItems], int m, int shift, int tid,
+                                                  SegLds<T>& L, unsigned int (&rank)[kSortItems],
+                                                  unsigned int& tstart) {
+    const int lane = tid & 63, wave = tid >> 6;
+    const int wbase = wave * (kSortItems * 64);
 #pragma unroll
-        for (int q = 0; q < 7; ++q) hc[q] = hc[q + 1];
+    for (int q = 0; q < 4; ++q) L.wcnt[wave][q * 64 + lane] = 0u;      // this wave's own
+    __builtin_amdgcn_wave_barrier();
+    rank_rows(key, wbase, m, shift, L.wcnt[wave], rank);
+    __syncthreads();
+    unsigned int count = 0u;
+    if (tid < 256)
+#pragma unroll
+        for (int w = 0; w < T / 64; ++w) count += L.wcnt[w][tid];
+    tstart = digit_exscan(count, L.sh, wave);
+    if (tid < 256) {
+        unsigned int run = tstart;
+#pragma unroll
+        for (int w = 0; w < T / 64; ++w) {
+            const unsigned int c = L.wcnt[w][tid];
+            L.wcnt[w][tid] = run;
+            run += c;
+        }
     }
-    const int tiles = (m + kSortTile - 1) / kSortTile;
+    return count;
+}
+
+// The places themselves, after the barrier.
+template <int T>
+__device__ __forceinline__ void add_starts(const unsigned long long (&key)[kSortItems], int m, int shift, int tid,
+                                           const SegLds<T>& L, unsigned int (&rank)[kSortItems]) {
+    const int lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r)
+        if (wave * (kSortItems * 64) + r * 64 + lane < m) rank[r] += L.wcnt[wave][(unsigned)(key[r] >> shift) & 255u];
+}
+
+// A segment of m <= T * kSortItems pairs.
+template <int T>
+__device__ __forceinline__ void sort_in_lds(unsigned long long* __restrict__ k, unsigned int* __restrict__ v, int m,
+                                            int p0, int tid, SegLds<T>& L) {
+    const int base = (tid >> 6) * (kSortItems * 64) + (tid & 63);
+    unsigned int* sval = reinterpret_cast<unsigned int*>(L.stage);
+    unsigned long long key[kSortItems];
+    unsigned int val[kSortItems];
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r) {
+        const int e = base + r * 64;
+        key[r] = e < m ? k[e] : 0ull;
+        val[r] = e < m ? v[e] : 0u;
+    }
     for (int p = p0; p < 8; ++p) {
-        const bool from1 = ((p - p0) & 1) != 0;
-        const unsigned long long* kin = (from1 ? k1 : k0) + a;
-        const unsigned int* vin = (from1 ? v1 : v0) + a;
-        unsigned long long* kout = (from1 ? k0 : k1) + a;
-        unsigned int* vout = (from1 ? v0 : v1) + a;
-        // this thread's digit: its first destination in the segment, advanced tile by tile
-        unsigned int dstart = block_exscan256(hc[0], L.sh[0]);
+        unsigned int rank[kSortItems], tstart;
+        rank_tile<T>(key, m, 8 * p, tid, L, rank, tstart);
+        __syncthreads();
+        add_starts<T>(key, m, 8 * p, tid, L, rank);
 #pragma unroll
-        for (int q = 0; q < 7; ++q) hc[q] = hc[q + 1];
+        for (int r = 0; r < kSortItems; ++r)
+            if (base + r * 64 < m) L.stage[rank[r]] = key[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kSortItems; ++r)
+            if (base + r * 64 < m) key[r] = L.stage[base + r * 64];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kSortItems; ++r)
+            if (base + r * 64 < m) sval[rank[r]] = val[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kSortItems; ++r)
+            if (base + r * 64 < m) val[r] = sval[base + r * 64];
+    }
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r) {
+        const int e = base + r * 64;
+        if (e >= m) continue;
+        k[e] = key[r];
+        v[e] = val[r];
+    }
+}
+
+// A longer segment, by all of the block's threads.
+__device__ __forceinline__ void sort_tiles(unsigned long long* __restrict__ k0, unsigned int* __restrict__ v0,
+                                           unsigned long long* __restrict__ k1, unsigned int* __restrict__ v1, int m,
+                                           int p0, SegLds<kSegThreads>& L, unsigned int* __restrict__ hist) {
+    constexpr int kTile = kSegThreads * kSortItems;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    unsigned int* sval = reinterpret_cast<unsigned int*>(L.stage);
+    // the digit counts of all passes
+    for (int i = tid; i < 8 * 256; i += kSegThreads) hist[i] = 0u;
+    __syncthreads();
+    for (int e = tid; e < m; e += kSegThreads) {
+        const unsigned long long k = k0[e];
+        for (int p = p0; p < 8; ++p) atomicAdd(&hist[p * 256 + ((unsigned)(k >> (8 * p)) & 255u)], 1u);
+    }
+    __syncthreads();
+    const int tiles = (m + kTile - 1) / kTile;
+    for (int p = p0; p < 8; ++p) {
+        const int shift = 8 * p;
+        const bool from1 = ((p - p0) & 1) != 0;
+        const unsigned long long* kin = from1 ? k1 : k0;
+        const unsigned int* vin = from1 ? v1 : v0;
+        unsigned long long* kout = from1 ? k0 : k1;
+        unsigned int* vout = from1 ? v0 : v1;
+        // this thread's digit: its first destination in the segment, advanced tile by tile
+        unsigned int dstart = digit_exscan(tid < 256 ? hist[p * 256 + tid] : 0u, L.sh, wave);
         for (int t = 0; t < tiles; ++t) {
-            const int wbase = t * kSortTile + wave * (kSortItems * 64);
+            const int here = min(kTile, m - t * kTile);
+            const int base = wave * (kSortItems * 64) + lane;
             unsigned long long key[kSortItems];
-            unsigned int val[kSortItems];
+            unsigned int val[kSortItems], rank[kSortItems], dst[kSortItems], tstart;
 #pragma unroll
             for (int r = 0; r < kSortItems; ++r) {
-                const int e = wbase + r * 64 + lane;
-                key[r] = e < m ? kin[e] : 0ull;
-                val[r] = e < m ? vin[e] : 0u;
+                const int e = base + r * 64;
+                key[r] = e < here ? kin[t * kTile + e] : 0ull;
+                val[r] = e < here ? vin[t * kTile + e] : 0u;
             }
-#pragma unroll
-            for (int w = 0; w < kWaves; ++w) L.wcnt[w][tid] = 0;
-            // the counts are cleared (and the previous tile's LDS reads done) before ranking
+            // (the barrier inside also ends the previous tile's and the scan's reads)
+            const unsigned int count = rank_tile<kSegThreads>(key, here, shift, tid, L, rank, tstart);
+            if (tid < 256) L.delta[tid] = (int)dstart - (int)tstart;
+            dstart += count;
             __syncthreads();
-            dstart += scatter_tile(key, val, t, m, 8 * p, dstart, L, kout, vout);
+            add_starts<kSegThreads>(key, here, shift, tid, L, rank);
+#pragma unroll
+            for (int r = 0; r < kSortItems; ++r)
+                if (base + r * 64 < here) L.stage[rank[r]] = key[r];
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kSortItems; ++r) {
+                const int j = tid + r * kSegThreads;
+                if (j >= here) continue;
+                const unsigned long long k = L.stage[j];
+                dst[r] = (unsigned int)(L.delta[(unsigned)(k >> shift) & 255u] + j);
+                kout[dst[r]] = k;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kSortItems; ++r)
+                if (base + r * 64 < here) sval[rank[r]] = val[r];
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kSortItems; ++r) {
+                const int j = tid + r * kSegThreads;
+                if (j < here) vout[dst[r]] = sval[j];
+            }
         }
         // this pass's writes are read by the next one (one block: workgroup-scope visibility)
         __syncthreads();
     }
-    if (((8 - p0) & 1) != 0) {
-        // an odd number of passes ran: the range is sorted in the second buffer
-        for (int e = tid; e < m; e += kSortThreads) {
-            k0[a + e] = k1[a + e];
-            v0[a + e] = v1[a + e];
+    if (((8 - p0) & 1) != 0)
+        for (int e = tid; e < m; e += kSegThreads) {
+            k0[e] = k1[e];
+            v0[e] = v1[e];
         }
+}
+
+// A batch of segments of at most T * kSortItems pairs: a block each.
+template <int T>
+__global__ __launch_bounds__(T) void k_seg_lds(unsigned long long* __restrict__ k0, unsigned int* __restrict__ v0,
+                                               const int* __restrict__ node_off, const int* __restrict__ order,
+                                               const DevState* __restrict__ st) {
+    __shared__ SegLds<T> L;
+    const int g = order[blockIdx.x], a = node_off[g];
+    sort_in_lds<T>(k0 + a, v0 + a, node_off[g + 1] - a, st ? st->sort_skip : 0, threadIdx.x, L);
+}
+
+__global__ __launch_bounds__(kSegThreads) void k_seg_sort(unsigned long long* __restrict__ k0,
+                                                          unsigned int* __restrict__ v0,
+                                                          unsigned long long* __restrict__ k1,
+                                                          unsigned int* __restrict__ v1,
+                                                          const int* __restrict__ node_off,
+                                                          const int* __restrict__ order, int nseg, int large,
+                                                          const DevState* __restrict__ st) {
+    union Lds {
+        SegLds<kSegThreads> one;
+        SegLds<256> four[4];
+    };
+    __shared__ Lds L;
+    __shared__ unsigned int hist[8 * 256];
+    // the low passes the previous trees' cells let the sort skip (k_sort_fixup, told the graph
+    // of each position, orders what they would have ordered)
+    const int p0 = st ? st->sort_skip : 0;
+    if ((int)blockIdx.x >= large) {
+        const int quarter = threadIdx.x >> 8, q = large + ((int)blockIdx.x - large) * 4 + quarter;
+        const int g = q < nseg ? order[q] : 0;
+        const int a = node_off[g], m = q < nseg ? node_off[g + 1] - a : 0;
+        sort_in_lds<256>(k0 + a, v0 + a, m, p0, threadIdx.x & 255, L.four[quarter]);
+        return;
     }
+    const int g = order[blockIdx.x], a = node_off[g], m = node_off[g + 1] - a;
+    if (m <= kSegThreads * kSortItems) sort_in_lds<kSegThreads>(k0 + a, v0 + a, m, p0, threadIdx.x, L.one);
+    else sort_tiles(k0 + a, v0 + a, k1 + a, v1 + a, m, p0, L.one, hist);
 }
 
 // ---- onesweep -------------------------------------------------------------------------------
@@ -396,24 +549,6 @@ struct SweepLds {
     int tile;
     unsigned int epoch;
 };
-
-// Exclusive scan of one value per thread over the block's first 256 threads (one barrier).
-__device__ __forceinline__ unsigned int digit_exscan(unsigned int v, unsigned int* __restrict__ sh) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    unsigned int inc = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const unsigned int t = __shfl_up(inc, o, 64);
-        if (lane >= o) inc += t;
-    }
-    if (lane == 63 && wave < 4) sh[wave] = inc;
-    __syncthreads();
-    unsigned int off = 0u;
-#pragma unroll
-    for (int w = 0; w < 4; ++w)
-        if (w < wave) off += sh[w];
-    return off + inc - v;
-}
 
 template <int T>
 __global__ __launch_bounds__(T) void k_onesweep(unsigned long long* __restrict__ k0, unsigned int* __restrict__ v0,
@@ -492,8 +627,8 @@ __global__ __launch_bounds__(T) void k_onesweep(unsigned long long* __restrict__
         for (int u = 0; u < kAhead; ++u) sum += v[u] & kStatCount;
     }
     L.before[part][digit] = sum;
-    const unsigned int gstart = digit_exscan(total, L.sh[0]);                       // (barrier)
-    const unsigned int tstart = digit_exscan(tid < 256 ? count : 0u, L.sh[1]);      // (barrier)
+    const unsigned int gstart = digit_exscan(total, L.sh[0], wave);                       // (barrier)
+    const unsigned int tstart = digit_exscan(tid < 256 ? count : 0u, L.sh[1], wave);      // (barrier)
     if (tid < 256) {
         unsigned int excl = 0u;
 #pragma unroll
@@ -685,11 +820,19 @@ bool sort_onesweep(const SortBuffers& buf, int n) {
     return buf.onesweep && n <= kSweepMost;
 }
 
-void segmented_sort_pairs(SortBuffers& buf, const int* node_off, const int* order, int nseg, hipStream_t s,
-                          const DevState* skip) {
-    if (nseg > 0)
-        k_seg_sort<<<nseg, kSortThreads, 0, s>>>(buf.keys[0], buf.vals[0], buf.keys[1], buf.vals[1], node_off, order,
-                                                 skip);
+void segmented_sort_pairs(SortBuffers& buf, const int* node_off, const int* order, int nseg, int max_seg, int large,
+                          hipStream_t s, const DevState* skip) {
+    if (nseg <= 0) return;
+    // without a long segment, blocks of just the threads it takes, several to a compute unit (4,000
+    // graphs of 200 bodies: 242 us an iteration, 253 by quarters; 300 of 2,049: 237, 251)
+    if (max_seg <= 256 * kSortItems)
+        k_seg_lds<256><<<nseg, 256, 0, s>>>(buf.keys[0], buf.vals[0], node_off, order, skip);
+    else if (max_seg <= 512 * kSortItems)
+        k_seg_lds<512><<<nseg, 512, 0, s>>>(buf.keys[0], buf.vals[0], node_off, order, skip);
+    else
+        k_seg_sort<<<large + (nseg - large + 3) / 4, kSegThreads, 0, s>>>(buf.keys[0], buf.vals[0], buf.keys[1],
+                                                                         buf.vals[1], node_off, order, nseg, large,
+                                                                         skip);
 }
 
 void radix_sort_pairs(SortBuffers& buf, int n, int begin_bit, int end_bit, hipStream_t s, const DevState* skip,

@@ -1,8 +1,8 @@
 """The sort's pass of one launch at the edges of its tiles (2,048 and 4,096 pairs), of its rounds
 over earlier tiles (8 and 16 of them), of its two tile sizes (32,768 pairs) and of its range
 (262,144), on full sorts and on ones that skip low passes, one key digit shared by almost all
-bodies among them: body orders equal a numpy sort of the restated keys; and in a batch with a graph
-over the per-graph sort's limit."""
+bodies among them: body orders equal a numpy sort of the restated keys. The same of batches, at the
+edges of the per-graph sort's forms (2,048, 4,096, 8,192 and 32,768 bodies) and past them."""
 import numpy as np
 import pytest
 
@@ -36,14 +36,20 @@ def test_orders(n, clumped):
     eng.close()
 
 
-def test_batch_over_the_per_graph_limit():
-    print("case sort pass batch", flush=True)
-    sizes = [40_000, 1, 300, 7000]
+@pytest.mark.parametrize("sizes", [
+    [40_000, 1, 300, 7000],                                               # over the per-graph sort's limit
+    [1, 2, 2047, 2048, 500, 64, 65],                                      # a block of 256 threads each
+    [4096, 2049, 1, 4095, 100],                                           # of 512
+    [8192, 4097, 2048, 2049, 1, 700, 511, 64, 300],                       # of 1,024, or a quarter of one
+    [32_768, 8193, 16_384, 16_385, 2048, 2, 100, 30],                     # and tile by tile
+])
+def test_batches(sizes):
+    print(f"case sort pass batch {sizes}", flush=True)
     chain = [(n, np.arange(n - 1, dtype=np.int32), np.arange(1, n, dtype=np.int32)) for n in sizes]
     eng = BatchEngine(chain, scale=1.0, gravity=1.0)
     eng.set_positions(np.concatenate([positions(n, 0) for n in sizes]))
     off = np.concatenate([[0], np.cumsum(sizes)])
-    for it in range(3):
+    for it in range(5):
         p = eng.positions()
         eng.step(1)
         eng.sync()
