@@ -209,10 +209,11 @@ __device__ __forceinline__ int lcp_prev(const signed char* __restrict__ lcp, con
     return seg_start(sg, i) ? -1 : (int)lcp[i - 1];
 }
 
-// Block-wide exclusive scan of one int per thread (256 threads). Returns the exclusive
+// Block-wide exclusive scan of one int per thread (NT threads). Returns the exclusive
 // prefix; *total gets the block sum.
+template <int NT>
 __device__ int block_exclusive_scan(int v, int* total) {
-    __shared__ int wsum[kTreeThreads / 64];
+    __shared__ int wsum[NT / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int inc = v;
 #pragma unroll
@@ -224,7 +225,7 @@ __device__ int block_exclusive_scan(int v, int* total) {
     __syncthreads();
     int before = 0, all = 0;
 #pragma unroll
-    for (int w = 0; w < kTreeThreads / 64; ++w) {
+    for (int w = 0; w < NT / 64; ++w) {
         int s = wsum[w];
         if (w < wave) before += s;
         all += s;
@@ -279,16 +280,10 @@ __device__ Moment block_exclusive_scan_mo(const Moment& v, Moment* total) {
     return mo_sub(mo_add(before, inc), v);
 }
 
-// Mass and mass-weighted fixed-point position (relative to the graph's root centre) of a
-// sorted body {x, y, mass} of graph g; the mass is a whole number below 2^24.
-__device__ __forceinline__ Moment body_moment(const float4 bd, int g, const float4* __restrict__ seg_root) {
-    const float4 c = seg_root[g];
-    const int s = moment_shift(c.z);
-    const unsigned long long m = (unsigned long long)bd.z;
-    const u128 x = (u128)(__int128)fixed_coord(bd.x, c.x, s) * (u128)m;
-    const u128 y = (u128)(__int128)fixed_coord(bd.y, c.y, s) * (u128)m;
-    return mo_make(x, y, m);
-}
+// Sums over a tile's bodies. They are right for every cell lighter than 2^24, the only ones that
+// take them, and for the tiles inside such a cell; a sum over heavier bodies may wrap.
+using TileSplit = SplitOf<unsigned long long>;
+static_assert(sizeof(TileSplit) == sizeof(Moment));
 
 // lcp per sorted position and the number of cells opened there; block sums (of the
 // cell counts and, on the integer-mass path, of body mass sums). Each sorted body's
@@ -301,12 +296,25 @@ __global__ __launch_bounds__(kTreeThreads) void k_lcp(const unsigned long long* 
                                                       const unsigned int* __restrict__ vals,
                                                       const float4* __restrict__ pm,
                                                       const float4* __restrict__ seg_root,
-                                                      Moment* __restrict__ bmass, float4* __restrict__ sbody) {
+                                                      Moment* __restrict__ bmass, float4* __restrict__ sbody,
+                                                      DevState* __restrict__ st) {
+    if (blockIdx.x == 0) {           // for the launches that follow
+        if (threadIdx.x == 0) {
+            st->max_level = 0;
+            st->nbig = 0;
+        }
+        if (threadIdx.x <= kMaxLevels) {
+            st->level_count[threadIdx.x] = 0;
+            st->level_cursor[threadIdx.x] = 0;
+        }
+    }
     // the tile's keys (with one on each side), graph ids and body ids, read coalesced into
     // LDS; each thread then takes its kTreeItems consecutive positions from there
     __shared__ unsigned long long skey[kTreeTile + 2];
     __shared__ int ssg[kTreeTile + 2];
     __shared__ unsigned int sval[kTreeTile];
+    __shared__ int wsum[kTreeThreads / 64];
+    __shared__ TileSplit wmass[kTreeThreads / 64];
     const int base = blockIdx.x * kTreeTile;
     for (int t = threadIdx.x; t < kTreeTile + 2; t += kTreeThreads) {
         const int gi = base - 1 + t;
@@ -332,7 +340,7 @@ __global__ __launch_bounds__(kTreeThreads) void k_lcp(const unsigned long long* 
 #pragma unroll
     for (int k = 0; k < kTreeItems; ++k) pp[k] = pm[sval[i0 + k - base]];
     int sum = 0;
-    Moment ms{0ull, 0ull, 0ull, 0ull, 0ull};
+    TileSplit ms{};
 #pragma unroll
     for (int k = 0; k < kTreeItems; ++k) {
         int i = i0 + k;
@@ -343,16 +351,25 @@ __global__ __launch_bounds__(kTreeThreads) void k_lcp(const unsigned long long* 
             sum += max(0, l - prev);
             const float4 bd = make_float4(pp[k].x, pp[k].y, pp[k].z, 0.0f);
             sbody[i] = bd;
-            if (bmass) ms = mo_add(ms, body_moment(bd, sg ? ssg[i - base + 1] : 0, seg_root));
+            if (bmass) ms = ms + split_of<unsigned long long>(bd, seg_root[sg ? ssg[i - base + 1] : 0]);
         }
     }
-    int total;
-    block_exclusive_scan(sum, &total);
-    if (threadIdx.x == 0) blocksum[blockIdx.x] = total;
-    if (bmass) {
-        Moment mt;
-        block_exclusive_scan_mo<kTreeThreads>(ms, &mt);
-        if (threadIdx.x == 0) bmass[blockIdx.x] = mt;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    sum = (int)wave_scan((unsigned int)sum);
+    if (bmass) ms = wave_scan(ms);
+    if (lane == 63) {
+        wsum[wave] = sum;
+        if (bmass) wmass[wave] = ms;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kTreeThreads / 64; ++w) wsum[0] += wsum[w];
+        blocksum[blockIdx.x] = wsum[0];
+        if (bmass) {
+            TileSplit all = wmass[0];
+            for (int w = 1; w < kTreeThreads / 64; ++w) all = all + wmass[w];
+            bmass[blockIdx.x] = mo_make(moment_x(all), moment_y(all), all.m);
+        }
     }
 }
 
@@ -366,7 +383,7 @@ __global__ __launch_bounds__(kTileChunk) void k_scan_up(const int* __restrict__ 
                                                         Moment* __restrict__ chunk_mass) {
     const int t = blockIdx.x * kTileChunk + threadIdx.x;
     int total;
-    (void)block_exclusive_scan(t < nb ? blocksum[t] : 0, &total);
+    (void)block_exclusive_scan<kTileChunk>(t < nb ? blocksum[t] : 0, &total);
     if (threadIdx.x == 0) chunk_sum[blockIdx.x] = total;
     if (bmass) {
         Moment mt;
@@ -380,7 +397,7 @@ __global__ __launch_bounds__(kTileChunk) void k_scan_down(int* __restrict__ bloc
                                                           const Moment* __restrict__ chunk_mass) {
     const int t = blockIdx.x * kTileChunk + threadIdx.x;
     int total;
-    const int off = block_exclusive_scan(t < nb ? blocksum[t] : 0, &total) + chunk_sum[blockIdx.x];
+    const int off = block_exclusive_scan<kTileChunk>(t < nb ? blocksum[t] : 0, &total) + chunk_sum[blockIdx.x];
     Moment moff{0ull, 0ull, 0ull, 0ull, 0ull};
     if (bmass) {
         Moment mt;
@@ -393,8 +410,7 @@ __global__ __launch_bounds__(kTileChunk) void k_scan_down(int* __restrict__ bloc
     }
 }
 
-// Single block: exclusive scan of block sums (in place), cell total, capacity check,
-// per-iteration counters reset.
+// Single block: exclusive scan of block sums (in place), cell total, capacity check.
 __global__ __launch_bounds__(1024) void k_scan_blocks(int* __restrict__ blocksum, int nb, int n,
                                                       int cap_records, int* __restrict__ rec_end, DevState* st,
                                                       Moment* __restrict__ bmass) {
@@ -468,459 +484,408 @@ __global__ __launch_bounds__(1024) void k_scan_blocks(int* __restrict__ blocksum
         st->nrecords = n + all;
         *rec_end = n + all;
         if (n + all > cap_records) st->err |= kErrTreeOverflow;
-        st->max_level = 0;
-        st->nbig = 0;
-    }
-    if (tid <= kMaxLevels) {
-        st->level_count[tid] = 0;
-        st->level_cursor[tid] = 0;
     }
 }
 
-// S (exclusive prefix of opened cells), body records and brec. With `fused` (few tiles), the
-// tile offsets are not scanned by a launch of their own: every block sums the totals of the
-// tiles before it (k_lcp's, at most kFuseTiles of them, read from L2), its writes are bounded
-// by its own extent, and the blocks at the ends take over the scan launch's state updates.
-__global__ __launch_bounds__(kTreeThreads) void k_prefix(const signed char* __restrict__ lcp,
-                                                         const int* __restrict__ sg, int n,
-                                                         const int* __restrict__ blockoff,
-                                                         int* __restrict__ S,
-                                                         const float4* __restrict__ sbody,
-                                                         float4* __restrict__ rec, int* __restrict__ brec,
-                                                         DevState* __restrict__ st,
-                                                         const float4* __restrict__ seg_root,
-                                                         const Moment* __restrict__ bmass, Moment* __restrict__ pmass,
-                                                         int* __restrict__ cell_pos, int max_cells, int fused,
-                                                         int cap_records, int* __restrict__ rec_end) {
-    // the tile's sorted bodies and graph ids (one before the tile), read coalesced into LDS
-    __shared__ float4 sbd[kTreeTile];
-    __shared__ int ssg[kTreeTile + 1];
-    const int base = blockIdx.x * kTreeTile;
-    for (int t = threadIdx.x; t < kTreeTile + 1; t += kTreeThreads) {
-        const int gi = base - 1 + t;
-        if (sg) ssg[t] = gi >= 0 && gi < n ? sg[gi] : -1;
-        if (t < kTreeTile) sbd[t] = base + t < n ? sbody[base + t] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+// The tree's cells in two launches. Positions i and j of a graph lie in one cell of level L if every
+// lcp between them is L or more, so a cell that starts at i ends at the first position from i on
+// whose lcp is below L, and its 2nd, 3rd and 4th child start behind the first ones of lcp L.
+//
+// k_tile takes kTreeTile sorted positions: it finds where each cell of the tile ends and where its
+// children start from rows of bits in LDS (row L, bit j: lcp(j) < L), and its summary from prefix
+// sums in LDS, so a cell inside the tile costs no load from memory. A cell that reaches past
+// the tile's end is left to k_cross; such cells contain the tile's last position, so they are nested,
+// at most one per level.
+// What bounds it: the bytes (a body's record and offset, a cell's record, children and count) at
+// 2M bodies, its chain of LDS steps at 50,000. In the place of a pass for the prefix sums over
+// bodies (40 bytes written for each, two read per cell), a pass for the cells by searches over
+// the keys and one for the child lists: 146 -> 109 us at 2M bodies, 27 -> 21 at 50,000.
+constexpr int kTileWords = kTreeTile / 64;
+constexpr int kRows = kKeyLevels + 2;
+constexpr int kTileCells = 2 * kTreeTile;      // cells per round
+
+struct TileArgs {
+    const signed char* lcp;
+    const int* sg;
+    int n;
+    const int* blockoff;        // the tile's first cell, or with fused every tile's cells
+    const Moment* bmass;        // the same of the bodies' sums
+    int fused;
+    int* S;
+    const float4* sbody;
+    float4* rec;
+    int4* kids;
+    int* rcount;
+    int* cell_rec;              // with cell_lvl, for the launches per level: records and levels
+    unsigned char* cell_lvl;
+    DevState* st;
+    const float4* seg_root;
+    TileSplit* pm16;            // the sum over the tile's bodies before every 16th position
+    int cap_records;
+    int* rec_begin;             // each graph's root, then the records' end
+    int nseg;
+    const int* node_off;
+    int* big_rc;
+    unsigned char* big_lvl;
+    int* kids_part;
+    int4* cross;                // per tile up to kCrossMax cells {first position, level, ordinal, graph}
+    TileSplit* cross_sum;       // their sums over the bodies of their own tile
+    int* ncross;
+    signed char* tmin;          // per tile the least lcp
+};
+
+// Row L's first bit at position `from` of the tile or later; kTreeTile: none.
+__device__ __forceinline__ int next_bit(const unsigned long long (*rows)[kTileWords], int L, int from) {
+    if (from >= kTreeTile) return kTreeTile;
+    int w = from >> 6;
+    unsigned long long v = rows[L][w] & (~0ull << (from & 63));
+    while (v == 0ull && ++w < kTileWords) v = rows[L][w];
+    return v ? w * 64 + __builtin_ctzll(v) : kTreeTile;
+}
+
+// A cell's record: its info word, and on the whole-mass path its summary from its moment d. A cell
+// lighter than 2^24 has this exact float mass in any summation order; heavier cells are listed
+// and summed in quadrant order later.
+__device__ __forceinline__ void write_cell(const TileArgs& A, int rc, int L, unsigned int info, const Moment& d, float4 c) {
+    const double M = (double)d.m;
+    if (M < 16777216.0) {
+        const int sh = moment_shift(c.z);
+        A.rec[rc] = make_float4((float)(ldexp(i128_to_double(d.xl, d.xh) / M, -sh) + c.x),
+                                (float)(ldexp(i128_to_double(d.yl, d.yh) / M, -sh) + c.y), (float)M,
+                                __uint_as_float(info));
+        return;
     }
-    __syncthreads();
-    const int i0 = base + threadIdx.x * kTreeItems;
-    int s[kTreeItems];
-    float4 bd[kTreeItems];
-    int sum = 0;
-#pragma unroll
-    for (int k = 0; k < kTreeItems; ++k) {
-        int i = i0 + k;
-        // lcp_prev over the staged graph ids: no graph starts at i
-        const bool start = i == 0 || (sg != nullptr && ssg[i - base] != ssg[i - base + 1]);
-        s[k] = i < n ? max(0, (int)lcp[i] - (start ? -1 : (int)lcp[i - 1])) : 0;
-        bd[k] = sbd[i - base];
-        sum += s[k];
-    }
-    int total;
-    int run = block_exclusive_scan(sum, &total);
-    int off;
-    Moment moff{0ull, 0ull, 0ull, 0ull, 0ull};
-    if (fused) {
-        int acc = 0;
-        Moment macc{0ull, 0ull, 0ull, 0ull, 0ull};
-        for (int t = threadIdx.x; t < (int)blockIdx.x; t += kTreeThreads) {
-            acc += blockoff[t];
-            if (bmass) macc = mo_add(macc, bmass[t]);
-        }
-        (void)block_exclusive_scan(acc, &off);
-        if (bmass) (void)block_exclusive_scan_mo<kTreeThreads>(macc, &moff);
+    A.rec[rc].w = __uint_as_float(info);
+    const int slot = atomicAdd(&A.st->nbig, 1);
+    if (slot < kMaxBig) {
+        A.big_rc[slot] = rc;
+        A.big_lvl[slot] = (unsigned char)L;
     } else {
-        off = blockoff[blockIdx.x];
-        if (bmass) moff = bmass[blockIdx.x];
+        A.st->err |= kErrTreeOverflow;
     }
-    run += off;
-    // records written here: below min(base + tile, n) + off + total (the cells before and in
-    // this tile), within capacity whenever the whole tree is
-    const bool ok = st->err == 0 && (!fused || min(base + kTreeTile, n) + off + total <= cap_records);
-    if (fused && threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) {
-        const int all = off + total;
-        st->ncells = all;
-        st->nrecords = n + all;
-        *rec_end = n + all;
-        if (n + all > cap_records) st->err |= kErrTreeOverflow;
-    }
-    if (fused && blockIdx.x == 0) {
-        if (threadIdx.x == 0) {
-            st->max_level = 0;
-            st->nbig = 0;
-        }
-        if (threadIdx.x <= kMaxLevels) {
-            st->level_count[threadIdx.x] = 0;
-            st->level_cursor[threadIdx.x] = 0;
-        }
-    }
-    if (pmass) {
-        // exclusive prefix of body mass sums over sorted positions
-        Moment mine{0ull, 0ull, 0ull, 0ull, 0ull};
-#pragma unroll
-        for (int k = 0; k < kTreeItems; ++k)
-            if (i0 + k < n) mine = mo_add(mine, body_moment(bd[k], sg ? ssg[i0 + k - base + 1] : 0, seg_root));
-        Moment tot;
-        Moment pre = mo_add(block_exclusive_scan_mo<kTreeThreads>(mine, &tot), moff);
-#pragma unroll
-        for (int k = 0; k < kTreeItems; ++k) {
-            const int i = i0 + k;
-            if (i < n) {
-                pmass[i] = pre;
-                pre = mo_add(pre, body_moment(bd[k], sg ? ssg[i - base + 1] : 0, seg_root));
-                if (i == n - 1) pmass[n] = pre;
-            }
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < kTreeItems; ++k) {
-        int i = i0 + k;
-        if (i < n) {
-            S[i] = run;
-            if (ok)
-                for (int j = 0; j < s[k] && run + j < max_cells; ++j) cell_pos[run + j] = i;
-            run += s[k];
-            int rb = i + run;          // after this position's own cells
-            brec[i] = rb;
-            if (ok) rec[rb] = make_float4(bd[k].x, bd[k].y, bd[k].z, __int_as_float(-1));
-        }
-    }
-    if (i0 + kTreeItems >= n && i0 < n) S[n] = run;   // total cells
 }
 
-// Cell records (skip, level, count) and the cell list, one thread per cell (grid-stride over
-// the S[n] cells). cell_rec[ord] holds the cell's first sorted position on entry (written by
-// k_prefix) and the cell's record index on exit (the list k_kids walks; on the fractional-mass
-// path, with cell_lvl, also the per-level summaries' list). The cells opened at
-// position i have levels lprev+1 .. lcp_i in ord order; each finds its extent end by a
-// galloping search over the keys (sorted within a graph, so a cell's bodies are contiguous),
-// bounded by the graph's end (a graph's root needs no search: it ends where the graph does).
-// One thread per cell keeps the long searches of the top levels in parallel.
-__global__ __launch_bounds__(kTreeThreads) void k_nodes(const unsigned long long* __restrict__ keys,
-                                                        const signed char* __restrict__ lcp,
-                                                        const int* __restrict__ sg, int n,
-                                                        const int* __restrict__ S, float4* __restrict__ rec,
-                                                        int* __restrict__ rcount, int* __restrict__ cell_rec,
-                                                        unsigned char* __restrict__ cell_lvl, int* __restrict__ rec_begin,
-                                                        DevState* st, const Moment* __restrict__ pmass,
-                                                        const float4* __restrict__ seg_root, int* __restrict__ big_rc,
-                                                        unsigned char* __restrict__ big_lvl,
-                                                        const int* __restrict__ node_off) {
-    __shared__ int hist[kMaxLevels + 1];
-    __shared__ int lmax;
-    if (threadIdx.x <= kMaxLevels) hist[threadIdx.x] = 0;
-    if (threadIdx.x == 0) lmax = 0;
-    __syncthreads();
-    const bool ok = st->err == 0;
-    const int ncells = ok ? S[n] : 0;
-    for (int ord = blockIdx.x * blockDim.x + threadIdx.x; ord < ncells; ord += gridDim.x * blockDim.x) {
-        const int i = cell_rec[ord];
-        const int Si = S[i];
-        const int L = lcp_prev(lcp, sg, i) + 1 + (ord - Si);
-        const unsigned long long ki = keys[i];
-        const int gi = sg ? sg[i] : 0;
-        // extent end: largest j < lim (the graph's end) with lcp(k_i, k_j) >= L; the test is
-        // true up to the end and false after it
-        const int lim = sg ? node_off[gi + 1] : n;
-        int lo = i;                   // inside
-        if (L == 0) {
-            lo = lim - 1;             // a graph's root holds the whole graph
-        } else {
-            int step = 1;
-            int hi = lo + 1;
-            while (hi < lim && lcp_levels(ki, keys[hi]) >= L) {
-                lo = hi;
-                step <<= 1;
-                hi = lo + step;
-            }
-            if (hi > lim) hi = lim;
-            while (hi - lo > 1) {
-                const int mid = lo + ((hi - lo) >> 1);
-                if (lcp_levels(ki, keys[mid]) >= L) lo = mid;
-                else hi = mid;
-            }
-        }
-        const int b = lo;
-        const int rc = i + ord;
-        const unsigned int skip = (unsigned int)(b + S[b + 1] + 1 - rc);
-        const unsigned int info = (skip << kInfoLevelBits) | (unsigned int)((L > 0 ? L - 1 : 0) & 31);
-        if (pmass) {
-            // whole-number masses: a cell lighter than 2^24 has this exact float mass in any
-            // summation order; heavier cells are summed in quadrant order later
-            const Moment d = mo_sub(pmass[b + 1], pmass[i]);
-            const double M = (double)d.m;
-            if (M < 16777216.0) {
-                const float4 c = seg_root[gi];
-                const int sh = moment_shift(c.z);
-                rec[rc] = make_float4((float)(ldexp(i128_to_double(d.xl, d.xh) / M, -sh) + c.x),
-                                      (float)(ldexp(i128_to_double(d.yl, d.yh) / M, -sh) + c.y), (float)M,
-                                      __uint_as_float(info));
-            } else {
-                rec[rc].w = __uint_as_float(info);
-                const int slot = atomicAdd(&st->nbig, 1);
-                if (slot < kMaxBig) {
-                    big_rc[slot] = rc;
-                    big_lvl[slot] = (unsigned char)L;
-                } else {
-                    st->err |= kErrTreeOverflow;
-                }
-            }
-        } else {
-            rec[rc].w = __uint_as_float(info);
-        }
-        rcount[rc] = b - i + 1;
-        cell_rec[ord] = rc;       // the cell list of k_kids (and of the summary launches)
-        if (!pmass) {
-            // the per-level cell lists of the summary launches (not needed for integer masses)
-            cell_lvl[ord] = (unsigned char)L;
-            atomicAdd(&hist[L], 1);
-        }
-        if (L == 0 && rec_begin) rec_begin[gi] = rc;
-        atomicMax(&lmax, L);
-    }
-    __syncthreads();
-    if (!pmass && threadIdx.x <= kMaxLevels && hist[threadIdx.x] != 0)
-        atomicAdd(&st->level_count[threadIdx.x], hist[threadIdx.x]);
-    // every block would hit this one word: only blocks above the value seen so far update it
-    // (the maximum only grows, so skipping on a stale value is still correct)
-    if (threadIdx.x == 0 && lmax > 0 &&
-        lmax > __hip_atomic_load(&st->max_level, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(&st->max_level, lmax);
+__device__ __forceinline__ unsigned int cell_info(int skip, int L) {
+    return ((unsigned int)skip << kInfoLevelBits) | (unsigned int)((L > 0 ? L - 1 : 0) & 31);
 }
 
-// Children of every cell record, for the walk: a cell's subtree is the record run
-// [r, r + skip); its children are r + 1 and then each next record past the previous child's
-// subtree (a body spans one record), at most four. Unused slots hold -1.
-__global__ __launch_bounds__(256) void k_kids(const float4* __restrict__ rec, const int* __restrict__ rcount,
-                                              const int* __restrict__ S, int n,
-                                              const int* __restrict__ cell_rec, int4* __restrict__ kids,
-                                              int* __restrict__ kids_part, const DevState* __restrict__ st) {
-    __shared__ int rmax[8];          // largest cell at level 4, 8, ..., 32 seen by the block
-    if (st->err != 0) return;        // uniform
-    if (threadIdx.x < 8) rmax[threadIdx.x] = 0;
-    __syncthreads();
-    const int ncells = S[n];
-    for (int ord = blockIdx.x * 256 + threadIdx.x; ord < ncells; ord += gridDim.x * 256) {
-        const int r = cell_rec[ord];
-        const unsigned int info = __float_as_uint(rec[r].w);
-        // the level bits hold L - 1 (L >= 1): levels 4, 8, ..., 32 are 3, 7, ..., 31
-        const unsigned int lm1 = info & 31u;
-        if ((lm1 & 3u) == 3u) atomicMax(&rmax[lm1 >> 2], rcount[r]);
-        const int end = r + (int)(info >> kInfoLevelBits);
-        int k[4] = {-1, -1, -1, -1};
-        int c = r + 1;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            if (c < end) {
-                k[q] = c;
-                const unsigned int ci = __float_as_uint(rec[c].w);
-                c += ci == 0xffffffffu ? 1 : max((int)(ci >> kInfoLevelBits), 1);
-            }
-        }
-        kids[r] = make_int4(k[0], k[1], k[2], k[3]);
-    }
-    __syncthreads();
-    // per-block maxima, reduced by the speed step (no word shared by the blocks: thousands of
-    // device-scope reads or atomics on one line cost more than the kernel itself)
-    if (threadIdx.x < 8) kids_part[blockIdx.x * 8 + threadIdx.x] = rmax[threadIdx.x];
-}
-
-// k_nodes and k_kids in one launch for graphs of up to kCellsNodes nodes, where the chain of
-// dependent loads of the longest search decides, not their number. A cell gets 16 lanes: they read
-// the 16 keys after the cell's first body at once, which settles cells of up to 16 bodies (most),
-// their extent and where their children start; a larger cell is searched by the whole wave, 16
-// lanes for each of the four bounds (the three changes of the next digit and the end), 16 probes
-// at a time: 7 loads in a row for 10,000 bodies where one thread made 26.
-//
-// A child that starts at sorted position p > i has the record index p + S[p]: p - 1 and p share
-// exactly the cell's L levels, so the first cell opened at p is that child (or, with none opened,
-// p's body is).
-//
-// Measured per iteration: 10,000 nodes k_nodes 11.5 + k_kids 4.1 -> 10.9 us and a launch less; SBM
-// 50,000 nodes 12.3 + 4.9 -> 18.5 us, so larger graphs keep the two (kCellsNodes between them).
-constexpr int kCellsThreads = 1024;
-
-// Positions of [lo, lim) whose keys share their top `top` bits' worth of digits with ki, counted
-// from lo, all of which come first: the first position past them. Every lane of the 16 gets it.
-// `before(key)` says whether a position lies before the bound; it holds up to the bound only.
-template <typename F>
-__device__ __forceinline__ int bound16(const unsigned long long* __restrict__ keys, int lo, int lim, int lane, F before) {
-    // lo: a position before the bound
-    const int q = lane & 15, shift = lane & 48;
-    int step = 1;
-    for (;;) {                       // grows until a probe lies past the bound
-        const int p = lo + (q + 1) * step;
-        const bool in = p < lim && before(keys[p < lim ? p : lo]);
-        const int c = __popc((unsigned)(__builtin_amdgcn_ballot_w64(in) >> shift) & 0xffffu);
-        lo += c * step;
-        if (c < 16) break;
-        step <<= 4;
-    }
-    while (step > 1) {
-        step >>= 4;
-        const int p = lo + (q + 1) * step;
-        const bool in = q < 15 && p < lim && before(keys[p < lim ? p : lo]);
-        lo += step * __popc((unsigned)(__builtin_amdgcn_ballot_w64(in) >> shift) & 0xffffu);
-    }
-    return lo + 1;
-}
-
-__global__ __launch_bounds__(kCellsThreads) void k_cells(const unsigned long long* __restrict__ keys,
-                                                         const signed char* __restrict__ lcp,
-                                                         const int* __restrict__ sg, int n,
-                                                         const int* __restrict__ S, float4* __restrict__ rec,
-                                                         int4* __restrict__ kids, int* __restrict__ rcount,
-                                                         int* __restrict__ cell_rec,
-                                                         unsigned char* __restrict__ cell_lvl,
-                                                         int* __restrict__ rec_begin, DevState* st,
-                                                         const Moment* __restrict__ pmass,
-                                                         const float4* __restrict__ seg_root,
-                                                         int* __restrict__ big_rc, unsigned char* __restrict__ big_lvl,
-                                                         const int* __restrict__ node_off,
-                                                         int* __restrict__ kids_part) {
+template <bool MOMENTS>
+__global__ __launch_bounds__(kTreeTile) void k_tile(const TileArgs A) {
+    __shared__ unsigned long long rows[kRows][kTileWords];
+    __shared__ TileSplit pre[MOMENTS ? kTreeTile + 1 : 1];     // relative to the tile's start
+    __shared__ TileSplit wsum[kTileWords];
+    __shared__ int wopened[kTileWords], wacc[kTileWords];
+    __shared__ int first[kTreeTile + 1];                       // cells opened before each position
+    __shared__ unsigned char level[kTreeTile];                 // the first opened cell's
+    __shared__ unsigned short owner[kTileCells];               // a round's cells' positions
     __shared__ int hist[kMaxLevels + 1];
     __shared__ int rmax[8];
-    __shared__ int lmax;
-    const int tid = threadIdx.x, lane = tid & 63, q = lane & 15;
+    __shared__ int lmax, lmin, ncross, go;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int base = blockIdx.x * kTreeTile, n = A.n, i = base + tid;
+    const bool in = i < n;
+    const int l = in ? (int)A.lcp[i] : -1;
+    int before = in && i > 0 ? (int)A.lcp[i - 1] : -1;
+    const float4 bd = in ? A.sbody[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    int graph = 0;
+    bool ends = !in || i == n - 1;
+    if (A.sg) {
+        graph = in ? A.sg[i] : 0;
+        if (in && i > 0 && A.sg[i - 1] != graph) before = -1;
+        if (!ends && A.sg[i + 1] != graph) ends = true;
+    }
+    const float4 root = A.seg_root[graph];
+    int acc = 0;
+    if (A.fused)
+        for (int t = tid; t < (int)blockIdx.x; t += kTreeTile) acc += A.blockoff[t];
+    else if (tid == 0) acc = A.blockoff[blockIdx.x];
     if (tid <= kMaxLevels) hist[tid] = 0;
     if (tid < 8) rmax[tid] = 0;
-    if (tid == 0) lmax = 0;
+    if (tid == 0) {
+        lmax = ncross = 0;
+        lmin = kMaxLevels;
+        go = A.st->err == 0;
+    }
+    const int opened = in ? max(0, l - before) : 0;
+    const int share = ends ? -1 : l;                           // (a graph of one body has lcp 0)
+    unsigned long long row = 0ull;
+    for (int L = 0; L < kRows; ++L) {
+        const unsigned long long word = __builtin_amdgcn_ballot_w64(share < L);
+        if (lane == L) row = word;
+    }
+    if (lane < kRows) rows[lane][wave] = row;
+    int run = (int)wave_scan((unsigned int)opened);
+    acc = (int)wave_scan((unsigned int)acc);
+    TileSplit own{}, p{};
+    if (MOMENTS) {
+        if (in) own = split_of<unsigned long long>(bd, root);
+        p = wave_scan(own);
+    }
+    if (lane == 63) {
+        wopened[wave] = run;
+        wacc[wave] = acc;
+        if (MOMENTS) wsum[wave] = p;
+    }
     __syncthreads();
-    const int ncells = st->err == 0 ? S[n] : 0;
-    const int stride = gridDim.x * (kCellsThreads / 16);
-    const int ord0 = (blockIdx.x * kCellsThreads + tid) / 64 * 4;      // the wave's first cell: uniform
-    for (int w0 = ord0; w0 < ncells; w0 += stride) {
-        const int ord = w0 + (lane >> 4);
-        const bool live = ord < ncells;
-        const int i = live ? cell_rec[ord] : 0;
-        const int gi = sg ? sg[i] : 0;
-        const int lim = sg ? node_off[gi + 1] : n;
-        const unsigned long long ki = keys[i];
-        const int wp = i + 1 + q;
-        const unsigned long long kw = keys[wp < lim ? wp : i];
-        const int Si = S[i];
-        const int L = lcp_prev(lcp, sg, i) + 1 + (ord - Si);
-        // digit of the next level (bits 63 - 2L, 62 - 2L); a level-32 cell has none
-        const int dsh = 62 - 2 * min(L, 31);
-        const bool in = live && wp < lim && (L == 0 || lcp_levels(ki, kw) >= L);
-        const unsigned int inm = (unsigned)(__builtin_amdgcn_ballot_w64(in) >> (lane & 48)) & 0xffffu;
-        int end = i + 1 + __popc(inm);           // one past the cell's last body
-        // where its 2nd, 3rd and 4th child start (-1: none)
-        int c1 = -1, c2 = -1, c3 = -1;
-        if (L >= 32) {
-            // children are the bodies themselves
-            if (end > i + 1) c1 = i + 1;
-            if (end > i + 2) c2 = i + 2;
-            if (end > i + 3) c3 = i + 3;
-        } else {
-            const unsigned int dw = (unsigned)(kw >> dsh) & 3u;
-            unsigned int dp = __shfl_up(dw, 1, 16);
-            if (q == 0) dp = (unsigned)(ki >> dsh) & 3u;
-            unsigned int m = (unsigned)(__builtin_amdgcn_ballot_w64(in && dw != dp) >> (lane & 48)) & 0xffffu;
-            if (m) c1 = i + __ffs(m), m &= m - 1;
-            if (m) c2 = i + __ffs(m), m &= m - 1;
-            if (m) c3 = i + __ffs(m);
+    // the waves before this one, and all
+    const int wl = lane < kTileWords ? lane : 0;
+    const unsigned int wo = lane < kTileWords ? (unsigned int)wopened[wl] : 0u;
+    const unsigned int wscan = wave_scan(wo);
+    const int total = (int)from_lane(wscan, kTileWords - 1);
+    const int off = (int)from_lane(wave_scan(lane < kTileWords ? (unsigned int)wacc[wl] : 0u), kTileWords - 1);
+    run += (int)from_lane(wscan - wo, wave) - opened;
+    if (MOMENTS) {
+        const TileSplit w = lane < kTileWords ? wsum[wl] : TileSplit{};
+        const TileSplit upto = wave_scan(w);
+        p = p - own + from_lane(upto - w, wave);
+        pre[tid] = p;
+        if (tid == 0) pre[kTreeTile] = from_lane(upto, kTileWords - 1);
+        if (tid % 16 == 0 && in) A.pm16[i / 16] = p;
+    }
+    // records written here: below min(base + tile, n) + off + total (the cells before and in
+    // this tile), within capacity whenever the whole tree is
+    const bool ok = go != 0 && (!A.fused || min(base + kTreeTile, n) + off + total <= A.cap_records);
+    first[tid] = run;
+    level[tid] = (unsigned char)(before + 1);
+    if (tid == 0) {
+        first[kTreeTile] = total;
+        if (base + kTreeTile >= n) A.S[n] = off + total;
+        if (A.fused && blockIdx.x == gridDim.x - 1) {
+            const int all = off + total;
+            A.st->ncells = all;
+            A.st->nrecords = n + all;
+            A.rec_begin[A.nseg] = n + all;
+            if (n + all > A.cap_records) A.st->err |= kErrTreeOverflow;
         }
-        // cells that fill the window, one after another, by the whole wave
-        unsigned long long large = __builtin_amdgcn_ballot_w64(live && inm == 0xffffu);
-        while (large) {
-            const int src = __builtin_ctzll(large);          // the cell's first lane
-            large &= ~(0xffffull << src);
-            const int bi = __builtin_amdgcn_readlane(i, src), bl = __builtin_amdgcn_readlane(L, src);
-            const int blim = __builtin_amdgcn_readlane(lim, src);
-            const unsigned long long bk =
-                ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(ki >> 32), src) << 32) |
-                (unsigned)__builtin_amdgcn_readlane((int)(unsigned)ki, src);
-            const int bsh = 62 - 2 * min(bl, 31);
-            const unsigned int d0 = (unsigned)(bk >> bsh) & 3u;
-            // 16 lanes look for the first body whose next digit is at least d (4: the cell's end)
-            const unsigned int d = 1 + (lane >> 4);
-            const bool digits = bl < 32;
-            int p = bi;
-            if (d == 4 && bl == 0) p = blim;
-            else if (d == 4 || (digits && d > d0))
-                p = bound16(keys, bi, blim, lane, [&](unsigned long long k) {
-                    return (bl == 0 || lcp_levels(bk, k) >= bl) && (d == 4 || ((unsigned)(k >> bsh) & 3u) < d);
-                });
-            const int p1 = __builtin_amdgcn_readlane(p, 0), p2 = __builtin_amdgcn_readlane(p, 16);
-            const int p3 = __builtin_amdgcn_readlane(p, 32), p4 = __builtin_amdgcn_readlane(p, 48);
-            if ((lane & 48) == src) {
-                end = p4;
-                c1 = c2 = c3 = -1;
-                if (!digits) {
-                    c1 = bi + 1;
-                    c2 = bi + 2;
-                    c3 = bi + 3;
-                } else {
-                    // digit d has bodies where its bound lies before the next digit's
-                    int found = 0;
-                    const int at[4] = {p1, p2, p3, p4};
-#pragma unroll
-                    for (int k = 0; k < 3; ++k)
-                        if (at[k] > bi && at[k] < at[k + 1]) {
-                            if (found == 0) c1 = at[k];
-                            else if (found == 1) c2 = at[k];
-                            else c3 = at[k];
-                            ++found;
-                        }
-                }
-            }
-        }
-        if (!live) continue;
-        const int rc = i + ord;
-        // lanes 0-3: a child each, and a word of the record each
-        if (q < 4) {
-            const int cp = q == 0 ? i : (q == 1 ? c1 : (q == 2 ? c2 : c3));
-            const int Sc = S[cp >= 0 ? cp : i], Se = S[end];
-            reinterpret_cast<int*>(kids + rc)[q] = q == 0 ? rc + 1 : (cp >= 0 ? cp + Sc : -1);
-            const unsigned int skip = (unsigned int)(end + Se - rc);
-            const unsigned int info = (skip << kInfoLevelBits) | (unsigned int)((L > 0 ? L - 1 : 0) & 31);
-            float out = __uint_as_float(info);               // lane 3
-            bool write = q == 3;
-            if (pmass) {
-                // lane 0: x; lane 1: y; lane 2: mass (see k_nodes)
-                const unsigned long long* a = reinterpret_cast<const unsigned long long*>(pmass + i);
-                const unsigned long long* e = reinterpret_cast<const unsigned long long*>(pmass + end);
-                const int lo = q == 1 ? 2 : 0;
-                const u128 va = ((u128)a[lo + 1] << 64) | a[lo], ve = ((u128)e[lo + 1] << 64) | e[lo];
-                const u128 dv = ve - va;
-                const double M = (double)(e[4] - a[4]);
-                if (M < 16777216.0) {
-                    const float4 c = seg_root[gi];
-                    const double m = i128_to_double((unsigned long long)dv, (unsigned long long)(dv >> 64)) / M;
-                    if (q < 2) out = (float)(ldexp(m, -moment_shift(c.z)) + (q == 0 ? c.x : c.y));
-                    else if (q == 2) out = (float)M;
-                    write = true;
-                } else if (q == 3) {
-                    const int slot = atomicAdd(&st->nbig, 1);
-                    if (slot < kMaxBig) {
-                        big_rc[slot] = rc;
-                        big_lvl[slot] = (unsigned char)L;
-                    } else {
-                        st->err |= kErrTreeOverflow;
-                    }
-                }
-            }
-            if (write) reinterpret_cast<float*>(rec + rc)[q] = out;
-        }
-        if (q == 4) {
-            rcount[rc] = end - i;
-            cell_rec[ord] = rc;       // the cell list of the summary launches
-            if (!pmass) {
-                cell_lvl[ord] = (unsigned char)L;
+    }
+    if (in) {
+        A.S[i] = off + run;
+        // after its own cells
+        if (ok) A.rec[i + off + run + opened] = make_float4(bd.x, bd.y, bd.z, __int_as_float(-1));
+    }
+    for (int c0 = 0; c0 < total && ok; c0 += kTileCells) {     // uniform
+        if (c0 > 0) __syncthreads();                           // the last round's owners
+        for (int j = max(0, c0 - run); j < opened && run + j < c0 + kTileCells; ++j)
+            owner[run + j - c0] = (unsigned short)tid;
+        __syncthreads();
+        const int here = min(kTileCells, total - c0);
+        for (int c = tid; c < here; c += kTreeTile) {
+            const int p = owner[c], L = level[p] + c0 + c - first[p];
+            const int ord = off + c0 + c, rc = base + p + ord;
+            const int b = next_bit(rows, L, p);                // the cell's last body
+            const int g = A.sg ? A.sg[base + p] : 0;
+            if (L == 0) A.rec_begin[g] = rc;
+            if (A.cell_lvl) {
+                A.cell_rec[ord] = rc;
+                A.cell_lvl[ord] = (unsigned char)L;
                 atomicAdd(&hist[L], 1);
             }
-            if (L == 0 && rec_begin) rec_begin[gi] = rc;
             atomicMax(&lmax, L);
-            // a cell of level 32 is recorded as level 32 too; level 0 as none of 4, 8, ..., 32
+            if (b == kTreeTile) {
+                const int slot = blockIdx.x * kCrossMax + atomicAdd(&ncross, 1);
+                A.cross[slot] = make_int4(base + p, L, ord, g);
+                if (MOMENTS) A.cross_sum[slot] = pre[kTreeTile] - pre[p];
+                continue;
+            }
+            int at[3];
+            int from = p;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                from = from <= b ? next_bit(rows, L + 1, from) + 1 : kTreeTile + 1;
+                at[q] = from <= b ? base + from + off + first[from] : -1;
+            }
+            A.kids[rc] = make_int4(rc + 1, at[0], at[1], at[2]);
+            const unsigned int info = cell_info(base + b + off + first[b + 1] + 1 - rc, L);
+            if (MOMENTS) {
+                const TileSplit d = pre[b + 1] - pre[p];
+                write_cell(A, rc, L, info, mo_make(moment_x(d), moment_y(d), d.m), A.sg ? A.seg_root[g] : root);
+            }
+            if (!MOMENTS) A.rec[rc].w = __uint_as_float(info);
+            A.rcount[rc] = b + 1 - p;
+            if (L > 0 && (L & 3) == 0) atomicMax(&rmax[(L >> 2) - 1], b + 1 - p);
+        }
+    }
+    // the tile's least lcp, for k_cross: the first row with a bit
+    if (tid < kRows) {
+        unsigned long long any = 0ull;
+        for (int w = 0; w < kTileWords; ++w) any |= rows[tid][w];
+        if (any) atomicMin(&lmin, tid - 1);
+    }
+    __syncthreads();
+    if (A.cell_lvl && tid <= kMaxLevels && hist[tid] != 0) atomicAdd(&A.st->level_count[tid], hist[tid]);
+    // every block would hit this one word: only blocks above the value seen so far update it
+    // (the maximum only grows, so skipping on a stale value is still correct)
+    if (tid == 0 && lmax > 0 && lmax > __hip_atomic_load(&A.st->max_level, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(&A.st->max_level, lmax);
+    if (tid == 0) {
+        A.ncross[blockIdx.x] = ncross;
+        A.tmin[blockIdx.x] = (signed char)lmin;
+    }
+    // per-block maxima, reduced by the speed step (no word shared by the blocks: thousands of
+    // device-scope reads or atomics on one line cost more than the kernel itself)
+    if (tid < 8) A.kids_part[blockIdx.x * 8 + tid] = rmax[tid];
+}
+
+// The cells that reach past their tile, a wave each. Where such a cell ends and its children start is
+// found from the tiles' least lcps (1,024 of them per load) and then the 512 lcps of the tiles that
+// hold a bound, at most four besides its own: two or three loads in a row for most.
+constexpr int kCrossThreads = 1024;   // at most
+static_assert(kTreeTile == 64 * 8, "8 lcps per lane");
+
+// Bit b: byte b of v, as a signed number, is below x.
+__device__ __forceinline__ unsigned int bytes_below(const unsigned int (&v)[2], int x) {
+    unsigned int m = 0u;
+#pragma unroll
+    for (int b = 0; b < 8; ++b) m |= (unsigned int)((int)(signed char)(v[b >> 2] >> (8 * (b & 3))) < x) << b;
+    return m;
+}
+
+// Takes the first position out of the lanes' masks of 8 positions each (uniform; -1: none).
+__device__ __forceinline__ int take_first(unsigned int& mask, int lane) {
+    const unsigned long long some = __builtin_amdgcn_ballot_w64(mask != 0u);
+    if (some == 0ull) return -1;
+    const int at = __builtin_ctzll(some);
+    const int bit = __builtin_ctz((unsigned)__builtin_amdgcn_readlane((int)mask, at));
+    if (lane == at) mask &= mask - 1u;
+    return at * 8 + bit;
+}
+
+template <bool MOMENTS>
+__global__ __launch_bounds__(kCrossThreads) void k_cross(const TileArgs A) {
+    __shared__ int rmax[8];
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (tid < 8) rmax[tid] = 0;
+    __syncthreads();
+    const int tile = blockIdx.x, tiles = gridDim.x;
+    const int w1 = (tile + 1) & ~15;                           // the first 1,024 tiles looked at
+    auto lcps = [&](int t) { return reinterpret_cast<const uint2*>(A.lcp + (size_t)t * kTreeTile)[lane]; };
+    auto mins = [&](int w0) {
+        const int t0 = w0 + lane * 16;
+        return t0 < tiles ? reinterpret_cast<const uint4*>(A.tmin)[t0 / 16] : make_uint4(0u, 0u, 0u, 0u);
+    };
+    auto below = [](uint2 w, int x) {
+        const unsigned int v[2] = {w.x, w.y};
+        return bytes_below(v, x);
+    };
+    const uint2 here = lcps(tile);
+    const uint4 next = mins(w1);
+    // (a wave's first cell is read along with their number)
+    const int c0 = tid >> 6;
+    int4 x = A.cross[tile * kCrossMax + c0];
+    TileSplit mine{};
+    if (MOMENTS) mine = A.cross_sum[tile * kCrossMax + c0];
+    const int cells = A.st->err == 0 ? A.ncross[tile] : 0;
+    for (int c = c0; c < cells; c += (int)blockDim.x / 64) {
+        if (c > c0) {
+            x = A.cross[tile * kCrossMax + c];
+            if (MOMENTS) mine = A.cross_sum[tile * kCrossMax + c];
+        }
+        const int i = __builtin_amdgcn_readfirstlane(x.x), L = __builtin_amdgcn_readfirstlane(x.y);
+        const int ord = __builtin_amdgcn_readfirstlane(x.z), g = __builtin_amdgcn_readfirstlane(x.w);
+        const int rc = i + ord;
+        const float4 root = A.seg_root[g];
+        int child[3] = {-1, -1, -1}, found = 0;
+        auto add_child = [&](int p) {
+            if (found == 0) child[0] = p;
+            else if (found == 1) child[1] = p;
+            else child[2] = p;
+            ++found;
+        };
+        // a root ends where its graph does
+        int end = L == 0 ? (A.sg ? A.node_off[g + 1] : A.n) : -1;
+        const int last = L == 0 ? (end - 1) / kTreeTile : tiles - 1;
+        // its own tile: children only
+        {
+            unsigned int m = below(here, L + 1);
+            const int skip = i - tile * kTreeTile - lane * 8;  // positions of this lane before i
+            if (skip > 0) m &= skip >= 8 ? 0u : 0xffu << skip;
+            for (int p; found < 3 && (p = take_first(m, lane)) >= 0;) add_child(tile * kTreeTile + p + 1);
+        }
+        for (int w0 = w1; w0 <= last && (found < 3 || L > 0); w0 += 1024) {
+            // the lane's 16 tiles: least lcp below L + 1, below L
+            unsigned int mc = 0u, me = 0u;
+            const int t0 = w0 + lane * 16;
+            if (t0 <= last) {
+                const uint4 w = w0 == w1 ? next : mins(w0);
+                const unsigned int lo[2] = {w.x, w.y}, hi[2] = {w.z, w.w};
+                mc = bytes_below(lo, L + 1) | bytes_below(hi, L + 1) << 8;
+                me = bytes_below(lo, L) | bytes_below(hi, L) << 8;
+                unsigned int use = 0xffffu;
+                if (t0 <= tile) use &= 0xffffu << (tile + 1 - t0);
+                if (t0 + 15 > last) use &= 0xffffu >> (t0 + 15 - last);
+                mc &= use;
+                me &= use;
+            }
+            bool done = false;
+            for (;;) {
+                // with all children found only the end is missing
+                const unsigned int m = found < 3 ? mc : me;
+                const unsigned long long some = __builtin_amdgcn_ballot_w64(m != 0u);
+                if (some == 0ull) break;
+                const int at = __builtin_ctzll(some);
+                const int bit = __builtin_ctz((unsigned)__builtin_amdgcn_readlane((int)m, at));
+                if (lane < at) mc = me = 0u;                   // tiles before it hold no bound that is wanted
+                else if (lane == at) {
+                    mc &= ~1u << bit;
+                    me &= ~1u << bit;
+                }
+                const int t = w0 + at * 16 + bit;
+                const uint2 there = lcps(t);
+                unsigned int starts = below(there, L + 1);
+                int stop = L == 0 ? end - 1 - t * kTreeTile : -1;          // the cell's last body, if here
+                if (L > 0) {
+                    unsigned int e = below(there, L);
+                    stop = take_first(e, lane);
+                    if (stop < 0) stop = kTreeTile;
+                }
+                for (int p; found < 3 && (p = take_first(starts, lane)) >= 0 && p < stop;) add_child(t * kTreeTile + p + 1);
+                if (L > 0 && stop < kTreeTile) {
+                    end = t * kTreeTile + stop + 1;
+                    done = true;
+                    break;
+                }
+                if (L == 0 && found == 3) break;
+            }
+            if (done) break;
+        }
+        // lanes 0-2: a child each; lane 3: the end
+        const int at = lane == 0 ? child[0] : lane == 1 ? child[1] : lane == 2 ? child[2] : end;
+        const int sat = lane < 4 && at >= 0 ? A.S[at] : 0;
+        Moment m{0ull, 0ull, 0ull, 0ull, 0ull};
+        if (MOMENTS) {
+            // lanes 0-15: the bodies of the last tile from the 16th position before the end; lane 16: those before
+            // them; lane 17: its own tile's; then the tiles between
+            const int from16 = (end - 1) & ~15, t2 = (end - 1) / kTreeTile, j = from16 + lane;
+            TileSplit d{};
+            if (lane < 16 && j < end) d = split_of<unsigned long long>(A.sbody[j], root);
+            if (lane == 16) d = A.pm16[from16 >> 4];
+            if (lane == 17) d = mine;
+            d = from_lane(wave_scan(d), 63);
+            if (!A.fused) {
+                m = mo_sub(A.bmass[t2], A.bmass[tile + 1]);
+            } else if (t2 > tile + 1) {
+                for (int t = tile + 1 + lane; t < t2; t += 64) m = mo_add(m, A.bmass[t]);
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1)
+                    m = mo_add(m, Moment{__shfl_xor(m.xl, o, 64), __shfl_xor(m.xh, o, 64), __shfl_xor(m.yl, o, 64),
+                                         __shfl_xor(m.yh, o, 64), __shfl_xor(m.m, o, 64)});
+            }
+            m = mo_add(m, mo_make(moment_x(d), moment_y(d), d.m));
+        }
+        const int rec = lane < 4 && at >= 0 ? at + sat : -1;
+        const int4 kids = make_int4(rc + 1, __builtin_amdgcn_readlane(rec, 0), __builtin_amdgcn_readlane(rec, 1),
+                                    __builtin_amdgcn_readlane(rec, 2));
+        const unsigned int info = cell_info(__builtin_amdgcn_readlane(rec, 3) - rc, L);
+        if (lane == 0) {
+            A.kids[rc] = kids;
+            A.rcount[rc] = end - i;
+            if (MOMENTS) write_cell(A, rc, L, info, m, root);
+            else A.rec[rc].w = __uint_as_float(info);
             if (L > 0 && (L & 3) == 0) atomicMax(&rmax[(L >> 2) - 1], end - i);
         }
     }
     __syncthreads();
-    if (!pmass && tid <= kMaxLevels && hist[tid] != 0) atomicAdd(&st->level_count[tid], hist[tid]);
-    if (tid == 0 && lmax > 0 &&
-        lmax > __hip_atomic_load(&st->max_level, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(&st->max_level, lmax);
-    if (tid < 8) kids_part[blockIdx.x * 8 + tid] = rmax[tid];
+    if (tid < 8) A.kids_part[(gridDim.x + blockIdx.x) * 8 + tid] = rmax[tid];
 }
 
 // Summaries of all cells in two launches, for trees of up to kSumMaxBlocks * kSumBlock records. A
@@ -1157,7 +1122,7 @@ __global__ __launch_bounds__(256) void k_summarize(int L, const int* __restrict_
     }
 }
 
-// Heavy cells (mass >= 2^24, listed by k_nodes) of the integer-mass path, in one
+// Heavy cells (mass >= 2^24, listed with the cells) of the integer-mass path, in one
 // workgroup: sorted by record index in LDS, then summarised deepest level first, children
 // in quadrant order (mass from 0.0f, centroid (sum m*p)*(1/mass), as
 // src/RPBHKernels.cu:468-494). A heavy child's summary is read from LDS; light children
@@ -1283,10 +1248,9 @@ void launch_tree(Bufs& b, hipStream_t s) {
     const int tiles = (n + kTreeTile - 1) / kTreeTile;
     const int* sg = b.nseg > 1 ? b.sg : nullptr;
     Moment* bm = b.int_mass ? b.bmass : nullptr;
-    Moment* pm = b.int_mass ? b.pmass : nullptr;
     k_lcp<<<tiles, kTreeThreads, 0, s>>>(b.sort.keys[0], sg, n, b.lcp, b.blocksum, b.sort.vals[0], b.pm,
-                                         b.seg_root, bm, b.sbody);
-    // up to kFuseTiles tiles, k_prefix sums the tile totals itself
+                                         b.seg_root, bm, b.sbody, b.st);
+    // up to kFuseTiles tiles, k_tile sums the tile totals itself
     const bool fused = tiles <= kFuseTiles;
     if (tiles > 8 * kTileChunk) {
         const int chunks = (tiles + kTileChunk - 1) / kTileChunk;
@@ -1298,30 +1262,29 @@ void launch_tree(Bufs& b, hipStream_t s) {
         k_scan_blocks<<<1, 1024, 0, s>>>(b.blocksum, tiles, n, b.cap_records, b.rec_begin + b.nseg, b.st, bm);
     }
     const int max_cells = b.cap_records - n;
-    k_prefix<<<tiles, kTreeThreads, 0, s>>>(b.lcp, sg, n, b.blocksum, b.S, b.sbody, b.rec, b.brec, b.st, b.seg_root,
-                                            bm, pm, b.cell_rec, max_cells, fused ? 1 : 0, b.cap_records,
-                                            b.rec_begin + b.nseg);
-    if (n <= kCellsNodes) {
-        k_cells<<<b.kids_blocks, kCellsThreads, 0, s>>>(b.sort.keys[0], b.lcp, sg, n, b.S, b.rec, b.kids, b.rcount,
-                                                        b.cell_rec, b.cell_lvl, b.rec_begin, b.st, pm, b.seg_root,
-                                                        b.big_rc, b.big_lvl, b.node_off, b.kids_part);
+    const int sum_grid = (b.cap_records + kSumBlock - 1) / kSumBlock;
+    const bool by_level = !b.int_mass && sum_grid > kSumMaxBlocks;
+    const TileArgs T{b.lcp,       sg,      n,       b.blocksum,  bm,        fused ? 1 : 0, b.S,     b.sbody,
+                     b.rec,       b.kids,         b.rcount, b.cell_rec, by_level ? b.cell_lvl : nullptr, b.st,
+                     b.seg_root,  reinterpret_cast<TileSplit*>(b.pmass),        b.cap_records, b.rec_begin, b.nseg, b.node_off, b.big_rc, b.big_lvl,
+                     b.kids_part, b.cross,        reinterpret_cast<TileSplit*>(b.cross_sum), b.ncross, b.tmin};
+    // a wave for each of a tile's cells while the tiles fit the chip once (50,000 bodies: 8.4 us with
+    // 1,024 threads, 9.5 with 512), fewer where blocks follow one another (2M bodies: 34 us with
+    // 256 threads, 39 with 512, 84 with 1,024)
+    const int ct = tiles <= 256 ? kCrossThreads : tiles <= 1024 ? 512 : 256;
+    if (b.int_mass) {
+        k_tile<true><<<tiles, kTreeTile, 0, s>>>(T);
+        k_cross<true><<<tiles, ct, 0, s>>>(T);
     } else {
-        // grid-stride over the cells (their number is known on the device only; at most
-        // max_cells, typically below n)
-        const int node_blocks = (n + kTreeThreads - 1) / kTreeThreads;
-        k_nodes<<<node_blocks, kTreeThreads, 0, s>>>(b.sort.keys[0], b.lcp, sg, n, b.S, b.rec, b.rcount, b.cell_rec,
-                                                     b.cell_lvl, b.rec_begin, b.st, pm, b.seg_root, b.big_rc,
-                                                     b.big_lvl, b.node_off);
-        // every record's info word is in place (cells: k_nodes, bodies: k_prefix)
-        k_kids<<<b.kids_blocks, 256, 0, s>>>(b.rec, b.rcount, b.S, n, b.cell_rec, b.kids, b.kids_part, b.st);
+        k_tile<false><<<tiles, kTreeTile, 0, s>>>(T);
+        k_cross<false><<<tiles, ct, 0, s>>>(T);
     }
     if (b.int_mass) {
         if (!b.no_big) k_big<<<1, 256, 0, s>>>(b.rec, b.big_rc, b.big_lvl, b.st);
         return;
     }
     // the spilled cells fit one block; larger trees fill the chip with a level each
-    const int sum_grid = (b.cap_records + kSumBlock - 1) / kSumBlock;
-    if (sum_grid <= kSumMaxBlocks) {
+    if (!by_level) {
         k_sum_blocks<<<sum_grid, kSumThreads, 0, s>>>(b.rec, b.level_list, b.st);
         k_sum_spill<<<1, kSumThreads, 0, s>>>(b.rec, b.level_list, b.st);
         return;

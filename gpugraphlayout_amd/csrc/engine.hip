@@ -565,16 +565,17 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
     // no tile has published counts, ticket 0
     GFA2_TRY(hipMemsetAsync(b.sort.status, 0, sizeof(unsigned int) * 256 * (size_t)sort_tiles, h->stream));
     GFA2_TRY(hipMemsetAsync(b.sort.ticket, 0, sizeof(unsigned long long), h->stream));
-    GFA2_ALLOC(b.lcp, n);
+    GFA2_ALLOC(b.lcp, (size_t)tree_tiles * kTreeTile);      // read by whole tiles
     GFA2_ALLOC(b.blocksum, tree_tiles);
     GFA2_ALLOC(b.chunk_sum, (tree_tiles + kTileChunk - 1) / kTileChunk);
     GFA2_ALLOC(b.S, (size_t)n + 1);
     GFA2_ALLOC(b.rec, (size_t)cap);
     GFA2_ALLOC(b.kids, (size_t)cap);
-    // enough threads for the cells' dependent child hops (about one cell per thread)
-    b.kids_blocks = n <= kCellsNodes ? (n + 63) / 64 : std::min((n + 255) / 256, 16384);
+    b.kids_blocks = 2 * tree_tiles;
     GFA2_ALLOC(b.kids_part, (size_t)b.kids_blocks * 8);
-    GFA2_ALLOC(b.brec, n);
+    GFA2_ALLOC(b.cross, (size_t)tree_tiles * kCrossMax);
+    GFA2_ALLOC(b.ncross, tree_tiles);
+    GFA2_ALLOC(b.tmin, (tree_tiles + 15) / 16 * 16);
     GFA2_ALLOC(b.sbody, n);
     GFA2_ALLOC(b.pm, n);
     GFA2_ALLOC(b.rcount, (size_t)cap);
@@ -638,7 +639,8 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
         }
     }
     if (b.int_mass) {
-        GFA2_ALLOC(b.pmass, (size_t)n + 1);
+        GFA2_ALLOC(b.cross_sum, (size_t)tree_tiles * kCrossMax);
+        GFA2_ALLOC(b.pmass, n <= kSmallTree ? (size_t)n + 1 : (size_t)n / 16 + 1);
         GFA2_ALLOC(b.bmass, tree_tiles);
         GFA2_ALLOC(b.chunk_mass, (tree_tiles + kTileChunk - 1) / kTileChunk);
         GFA2_ALLOC(b.big_rc, kMaxBig);

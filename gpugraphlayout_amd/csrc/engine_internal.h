@@ -13,7 +13,6 @@
 //   rec      float4[V+C] the quadtree in pre-order: {x, y, mass, info}
 //            info == -1: a body; otherwise a cell, (skip << 5) | (level - 1) as unsigned,
 //            skip being the number of records in its subtree (the walk jumps by it)
-//   brec     int[V]      record index of the body at sorted position k
 //   rcount   int[V+C]    body count of each cell record
 // Tree levels: the root is level 0; a key holds 32 levels of 2-bit quadrant digits, so
 // cells exist down to level 32. Bodies that share all 32 digits share one level-32 cell.
@@ -152,9 +151,12 @@ struct Bufs {
     int* S;
     float4* rec;
     int4* kids;             // per cell record: the record indices of its 1-4 children (-1: none)
-    int* kids_part;         // [kids_blocks][8]: per k_kids block, the largest level-4p cell
+    int* kids_part;         // [kids_blocks][8]: per block of k_tile, then of k_cross, the largest level-4p cell
     int kids_blocks = 1;
-    int* brec;
+    int4* cross = nullptr;  // [tree tiles][kCrossMax]: cells that reach past their tile
+    Moment* cross_sum = nullptr;  // their bodies' sums in the tile (as k_tile keeps them)
+    int* ncross = nullptr;  // [tree tiles]
+    signed char* tmin = nullptr;  // [tree tiles, whole groups of 16]: each tile's least lcp
     float4* sbody;          // {x, y, mass, 0} of the body at sorted position k (node k in exact mode)
     float4* pm;             // {x, y, mass, 0} of node v, written with the keys (k_lcp gathers it)
     float* ew_raw = nullptr;    // edge weights per CSR entry (null: unweighted)
@@ -192,7 +194,8 @@ struct Bufs {
     // only heavier cells are summed in quadrant order.
     bool int_mass = false;
     bool no_big = false;              // total mass below 2^24: no cell is summed in quadrant order
-    Moment* pmass = nullptr;          // n + 1
+    Moment* pmass = nullptr;          // the bodies' sums before every 16th sorted position (the small
+                                      // tree: before every one)
     Moment* bmass = nullptr;          // per tree tile
     int* chunk_sum = nullptr;         // per 256 tree tiles (the two-level tile scan)
     Moment* chunk_mass = nullptr;
@@ -220,10 +223,9 @@ constexpr int kSortTile = kSortThreads * kSortItems;
 constexpr int kTreeThreads = 256;
 constexpr int kTreeItems = 2;
 constexpr int kTreeTile = kTreeThreads * kTreeItems;
-// up to this many tiles k_prefix sums the tile totals before it itself (no scan launch)
+// up to this many tiles k_tile sums the tile totals before it itself (no scan launch)
 constexpr int kFuseTiles = 2048;
-// up to this many bodies (all graphs together) k_cells builds the cells and child lists
-constexpr int kCellsNodes = 32768;
+constexpr int kCrossMax = kMaxLevels;  // cells over one position: a level each
 constexpr int kTileChunk = 256;       // tree tiles per block of the two-level tile scan
 
 // Radix sort of (key, value) pairs on 64-bit keys, ascending and stable. Sorts

@@ -227,7 +227,7 @@ __device__ __forceinline__ int xcd_block() {
 //             last body's own d2 below dq rejects. Only the cells left are voted on, body by
 //             body, all lanes at once (lanes = bodies, as in the reference). An accepted record
 //             is appended {x, y, k_r m} to an LDS list; an opened cell pushes all its 1-4
-//             children at once (their record indices, listed per cell by k_kids when the tree is
+//             children at once (their record indices, listed per cell when the tree is
 //             built), so a cell's children are tested in the same round. The children go on
 //             top, so the traversal runs depth-first in blocks of up to 64 records (one record
 //             per round near the stack's capacity, where a depth-first walk adds at most three

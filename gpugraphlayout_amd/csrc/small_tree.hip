@@ -28,71 +28,7 @@ constexpr int kThreads = 1024;
 constexpr int kWaves = kThreads / 64;
 constexpr int kRunCap = 64;          // longest run of tied bodies ordered by counting
 
-// Prefix moments over sorted bodies: q = fixed-point coordinate = 2^31 h + l with 0 <= l < 2^31, so
-// the sums of m h and m l stay within 64 bits for integer masses of under 2^30 together, and
-// 2^31 sum(m h) + sum(m l) is the exact 128-bit moment.
-struct Split {
-    long long xh, xl, yh, yl;
-    unsigned int m;
-};
-
-__device__ __forceinline__ Split split_of(float4 b, float4 c) {
-    const int s = moment_shift(c.z);
-    const long long m = (long long)b.z;
-    const long long qx = fixed_coord(b.x, c.x, s), qy = fixed_coord(b.y, c.y, s);
-    return Split{m * (qx >> 31), m * (qx & 0x7fffffff), m * (qy >> 31), m * (qy & 0x7fffffff), (unsigned int)m};
-}
-
-__device__ __forceinline__ Split operator+(const Split& a, const Split& b) {
-    return Split{a.xh + b.xh, a.xl + b.xl, a.yh + b.yh, a.yl + b.yl, a.m + b.m};
-}
-
-__device__ __forceinline__ Split operator-(const Split& a, const Split& b) {
-    return Split{a.xh - b.xh, a.xl - b.xl, a.yh - b.yh, a.yl - b.yl, a.m - b.m};
-}
-
-// One step of a wave-wide scan by a data-parallel move (no LDS): the value of the lane the control
-// word names, 0 where there is none or the row mask leaves the lane out.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ unsigned int moved(unsigned int v) {
-    return (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, true);
-}
-
-template <int CTRL, int ROWS>
-__device__ __forceinline__ long long moved(long long v) {
-    const unsigned int lo = moved<CTRL, ROWS>((unsigned int)v);
-    const unsigned int hi = moved<CTRL, ROWS>((unsigned int)((unsigned long long)v >> 32));
-    return (long long)(((unsigned long long)hi << 32) | lo);
-}
-
-// Inclusive scan over the wave: within rows of 16 lanes (shifts by 1, 2, 4, 8), then lane 15 of a
-// row into the next, then lane 31 into the upper half.
-template <typename T>
-__device__ __forceinline__ T wave_scan(T v) {
-    v += moved<0x111, 0xf>(v);
-    v += moved<0x112, 0xf>(v);
-    v += moved<0x114, 0xf>(v);
-    v += moved<0x118, 0xf>(v);
-    v += moved<0x142, 0xa>(v);
-    v += moved<0x143, 0xc>(v);
-    return v;
-}
-
-__device__ __forceinline__ Split wave_scan(const Split& v) {
-    return Split{wave_scan(v.xh), wave_scan(v.xl), wave_scan(v.yh), wave_scan(v.yl), wave_scan(v.m)};
-}
-
-// The value of one lane (uniform).
-__device__ __forceinline__ long long from_lane(long long v, int l) {
-    const unsigned int lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, l);
-    const unsigned int hi = (unsigned)__builtin_amdgcn_readlane((int)((unsigned long long)v >> 32), l);
-    return (long long)(((unsigned long long)hi << 32) | lo);
-}
-
-__device__ __forceinline__ Split from_lane(const Split& v, int l) {
-    return Split{from_lane(v.xh, l), from_lane(v.xl, l), from_lane(v.yh, l), from_lane(v.yl, l),
-                 (unsigned)__builtin_amdgcn_readlane((int)v.m, l)};
-}
+using Split = SplitOf<unsigned int>;      // (the launch's rule: under 2^24 in all)
 
 struct SmallArgs {
     const float2* pos;
@@ -438,7 +374,7 @@ __device__ void small_tree(const SmallArgs& A, SmallLds<N>& L) {
         for (int r = 0; r < R; ++r) {
             if (r >= rows) break;                      // uniform
             const int e = base + r * 64 + lane;
-            const Split own = e < n ? split_of(bd[r], root) : Split{0, 0, 0, 0, 0u};
+            const Split own = e < n ? split_of<unsigned int>(bd[r], root) : Split{0, 0, 0, 0, 0u};
             const Split in = wave_scan(own);
             ex[r] = run + (in - own);
             run = run + from_lane(in, 63);
@@ -499,8 +435,7 @@ __device__ void small_tree(const SmallArgs& A, SmallLds<N>& L) {
                 const Split* P = reinterpret_cast<const Split*>(A.pmass);
                 D = P[end] - P[i];
             }
-            const u128 x = ((u128)(__int128)D.xh << 31) + (u128)(__int128)D.xl;
-            const u128 y = ((u128)(__int128)D.yh << 31) + (u128)(__int128)D.yl;
+            const u128 x = moment_x(D), y = moment_y(D);
             const double M = (double)D.m;
             const int e = -moment_shift(root.z);
             A.rec[rc] = make_float4(

@@ -58,4 +58,103 @@ __device__ __forceinline__ double i128_to_double(unsigned long long lo, unsigned
     return neg ? -mag : mag;
 }
 
+// Prefix moments over sorted bodies: q = fixed-point coordinate = 2^31 h + l with 0 <= l < 2^31, so
+// the sums of m h and m l stay within 64 bits for integer masses of under 2^30 together, and
+// 2^31 sum(m h) + sum(m l) is the exact 128-bit moment.
+// (Sums wrap: a difference of two prefix sums is exact if it is within 64 bits itself.)
+template <typename M>
+struct SplitOf {
+    long long xh, xl, yh, yl;
+    M m;
+};
+
+__device__ __forceinline__ long long wrap_add(long long a, long long b) {
+    return (long long)((unsigned long long)a + (unsigned long long)b);
+}
+
+__device__ __forceinline__ long long wrap_sub(long long a, long long b) {
+    return (long long)((unsigned long long)a - (unsigned long long)b);
+}
+
+template <typename M>
+__device__ __forceinline__ SplitOf<M> split_of(float4 b, float4 c) {
+    const int s = moment_shift(c.z);
+    const long long m = (long long)b.z;
+    const long long qx = fixed_coord(b.x, c.x, s), qy = fixed_coord(b.y, c.y, s);
+    return SplitOf<M>{m * (qx >> 31), m * (qx & 0x7fffffff), m * (qy >> 31), m * (qy & 0x7fffffff), (M)m};
+}
+
+template <typename M>
+__device__ __forceinline__ SplitOf<M> operator+(const SplitOf<M>& a, const SplitOf<M>& b) {
+    return SplitOf<M>{wrap_add(a.xh, b.xh), wrap_add(a.xl, b.xl), wrap_add(a.yh, b.yh), wrap_add(a.yl, b.yl), a.m + b.m};
+}
+
+template <typename M>
+__device__ __forceinline__ SplitOf<M> operator-(const SplitOf<M>& a, const SplitOf<M>& b) {
+    return SplitOf<M>{wrap_sub(a.xh, b.xh), wrap_sub(a.xl, b.xl), wrap_sub(a.yh, b.yh), wrap_sub(a.yl, b.yl), a.m - b.m};
+}
+
+// One step of a wave-wide scan by a data-parallel move (no LDS): the value of the lane the control
+// word names, 0 where there is none or the row mask leaves the lane out.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned int moved(unsigned int v) {
+    return (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, true);
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long moved(unsigned long long v) {
+    const unsigned int lo = moved<CTRL, ROWS>((unsigned int)v);
+    const unsigned int hi = moved<CTRL, ROWS>((unsigned int)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+// Inclusive scan over the wave: within rows of 16 lanes (shifts by 1, 2, 4, 8), then lane 15 of a
+// row into the next, then lane 31 into the upper half.
+template <typename T>
+__device__ __forceinline__ T wave_scan(T v) {
+    v += moved<0x111, 0xf>(v);
+    v += moved<0x112, 0xf>(v);
+    v += moved<0x114, 0xf>(v);
+    v += moved<0x118, 0xf>(v);
+    v += moved<0x142, 0xa>(v);
+    v += moved<0x143, 0xc>(v);
+    return v;
+}
+
+template <typename M>
+__device__ __forceinline__ SplitOf<M> wave_scan(const SplitOf<M>& v) {
+    return SplitOf<M>{(long long)wave_scan((unsigned long long)v.xh), (long long)wave_scan((unsigned long long)v.xl),
+                      (long long)wave_scan((unsigned long long)v.yh), (long long)wave_scan((unsigned long long)v.yl),
+                      wave_scan(v.m)};
+}
+
+// The value of one lane (uniform).
+__device__ __forceinline__ unsigned int from_lane(unsigned int v, int l) {
+    return (unsigned)__builtin_amdgcn_readlane((int)v, l);
+}
+
+__device__ __forceinline__ unsigned long long from_lane(unsigned long long v, int l) {
+    const unsigned int lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, l);
+    const unsigned int hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l);
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+template <typename M>
+__device__ __forceinline__ SplitOf<M> from_lane(const SplitOf<M>& v, int l) {
+    return SplitOf<M>{(long long)from_lane((unsigned long long)v.xh, l), (long long)from_lane((unsigned long long)v.xl, l),
+                      (long long)from_lane((unsigned long long)v.yh, l), (long long)from_lane((unsigned long long)v.yl, l),
+                      from_lane(v.m, l)};
+}
+
+// The 128-bit moments.
+template <typename M>
+__device__ __forceinline__ u128 moment_x(const SplitOf<M>& v) {
+    return ((u128)(__int128)v.xh << 31) + (u128)(__int128)v.xl;
+}
+
+template <typename M>
+__device__ __forceinline__ u128 moment_y(const SplitOf<M>& v) {
+    return ((u128)(__int128)v.yh << 31) + (u128)(__int128)v.yl;
+}
+
 }  // namespace gfa2

@@ -1,6 +1,6 @@
-"""Cells and child lists by 16 lanes per cell (graphs and batches of up to 32,768 bodies): cells of
-just under, at and over the 16 bodies one window settles and the 272 the first widening does, the
-size limit and one past it, fractional masses and a batch: the whole tree equal to the oracle's."""
+"""Cells and child lists of graphs past the one-block tree: clumps of just under, at and over 16 and
+272 bodies, 20,000 to 32,769 bodies, fractional masses and a batch: the whole tree equal to the
+oracle's."""
 import numpy as np
 import pytest
 
