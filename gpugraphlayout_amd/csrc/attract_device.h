@@ -164,4 +164,61 @@ __device__ __forceinline__ void attract_medium(int k0, int rows, int lane, const
     }
 }
 
+// Block i of the light and medium ones, which take turns in proportion (256 threads).
+template <bool GEN, int HUB>
+__device__ __forceinline__ void attract_rows(int i, int light_blocks, int medium_blocks, int medium_rows, int tid,
+                                             const AttractArgs& A, const float2* hub) {
+    const unsigned int t = light_blocks + medium_blocks;
+    const int m0 = (int)((unsigned long long)i * medium_blocks / t);          // medium blocks before i
+    const int m1 = (int)((i + 1ull) * medium_blocks / t);
+    if (m1 > m0) attract_medium<GEN, HUB>((m0 * 4 + (tid >> 6)) * medium_rows, medium_rows, tid & 63, A, hub);
+    else attract_light<GEN, HUB>((i - m0) * 256 + tid, A, hub);
+}
+
+// red[0] = the sum over 256 threads. red[0] is written again only by thread 0, and every other
+// entry only after the barriers here, so thread 0 may read it after the call.
+__device__ __forceinline__ void sum_chunk(float2* red, int tid, float ax, float ay) {
+    red[tid] = make_float2(ax, ay);
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (tid < o) {
+            const float2 a = red[tid], b = red[tid + o];
+            red[tid] = make_float2(a.x + b.x, a.y + b.y);
+        }
+        __syncthreads();
+    }
+}
+
+// Chunk c of a heavy row (a block of 256 threads): thread-strided sums, then an LDS tree.
+template <bool GEN, int HUB>
+__device__ __forceinline__ void attract_chunk(int c, const int2* __restrict__ chunks, float2* __restrict__ part, int tid,
+                                              const AttractArgs& A, const float2* hub, float2* red) {
+    const int2 ch = chunks[c];
+    const int v = A.lists[A.nlight + A.nmedium + ch.x];
+    const float2 p = A.pos[v];
+    float ax = 0.0f, ay = 0.0f;
+    const int len = min(kAttrChunk, A.rowptr[v + 1] - ch.y);
+    gather_terms<GEN, 256, HUB>(p, A, hub, Row(A, ch.y, ch.y + len), tid, ax, ay);
+    sum_chunk(red, tid, ax, ay);
+    if (tid == 0) part[c] = red[0];
+}
+
+// What a launch of the attraction covers: chunks, then light and medium blocks (256 threads each).
+struct AttractPlan {
+    int light_blocks, medium_blocks, medium_rows, chunks;
+    int total;
+};
+
+// One of a plan's blocks, without a copy of the hubs.
+template <bool GEN>
+__device__ __forceinline__ void attract_block(int vb, const AttractPlan& w, const int2* __restrict__ chunks,
+                                              float2* __restrict__ part, const AttractArgs& A, float2* red) {
+    if (vb < w.chunks) attract_chunk<GEN, 0>(vb, chunks, part, threadIdx.x, A, nullptr, red);
+    else attract_rows<GEN, 0>(vb - w.chunks, w.light_blocks, w.medium_blocks, w.medium_rows, threadIdx.x, A, nullptr);
+}
+
+AttractPlan attract_plan(const Bufs& b);
+AttractArgs attract_args(const Bufs& b, const Params& p);
+void launch_attract_heavy(const Bufs& b, const Params& p, hipStream_t s);
+
 }  // namespace gfa2

@@ -10,6 +10,7 @@
 // record range. Walk groups, speed state and displacement are per graph, so a graph laid
 // out in a batch follows exactly the trajectory it follows alone.
 #include "engine_internal.h"
+#include "attract_device.h"
 #include "tree_device.h"
 
 #include <algorithm>
@@ -51,21 +52,40 @@ __global__ __launch_bounds__(256) void k_seg_bbox(const float2* __restrict__ pos
     }
 }
 
-__global__ __launch_bounds__(256) void k_seg_keys(const float2* __restrict__ pos, const float* __restrict__ mass, int n,
-                                                  const int* __restrict__ seg_of,
-                                                  const float4* __restrict__ seg_root,
-                                                  unsigned long long* __restrict__ keys,
-                                                  unsigned int* __restrict__ vals,
-                                                  unsigned long long* __restrict__ pkey, float4* __restrict__ pm) {
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        const float4 root = seg_root[seg_of[i]];
-        const float2 p = pos[i];
+struct SegKeysArgs {
+    const float2* pos;
+    const float* mass;
+    int n;
+    const int* seg_of;
+    const float4* seg_root;
+    unsigned long long* keys;
+    unsigned int* vals;
+    unsigned long long* pkey;     // kept for the regather after a global graph sort, or null
+    float4* pm;
+};
+
+__device__ __forceinline__ void seg_keys_block(const SegKeysArgs& K, int block, int blocks) {
+    for (int i = block * 256 + threadIdx.x; i < K.n; i += blocks * 256) {
+        const float4 root = K.seg_root[K.seg_of[i]];
+        const float2 p = K.pos[i];
         const unsigned long long key = path_key(p, root.x, root.y, root.z);
-        keys[i] = key;
-        if (pkey) pkey[i] = key;      // kept for the regather after a global graph sort
-        vals[i] = (unsigned)i;
-        pm[i] = make_float4(p.x, p.y, mass[i], 0.0f);
+        K.keys[i] = key;
+        if (K.pkey) K.pkey[i] = key;
+        K.vals[i] = (unsigned)i;
+        K.pm[i] = make_float4(p.x, p.y, K.mass[i], 0.0f);
     }
+}
+
+__global__ __launch_bounds__(256) void k_seg_keys(const SegKeysArgs K) { seg_keys_block(K, blockIdx.x, gridDim.x); }
+
+// Keys and attraction in one launch (see k_keys_attract).
+template <bool GEN>
+__global__ __launch_bounds__(256) void k_seg_keys_attract(const SegKeysArgs K, int key_blocks, const AttractArgs A,
+                                                          const AttractPlan w, const int2* __restrict__ chunks,
+                                                          float2* __restrict__ part) {
+    __shared__ float2 red[256];
+    if ((int)blockIdx.x < key_blocks) seg_keys_block(K, blockIdx.x, key_blocks);
+    else attract_block<GEN>(blockIdx.x - key_blocks, w, chunks, part, A, red);
 }
 
 // The graph owning node v: the last g with node_off[g] <= v, by binary search over the node
@@ -125,9 +145,25 @@ void launch_seg_bbox(const Bufs& b, hipStream_t s) {
     k_seg_bbox<<<b.nseg, 256, 0, s>>>(b.pos, b.node_off, b.seg_root);
 }
 
+namespace {
+
+SegKeysArgs seg_keys_args(const Bufs& b) {
+    return SegKeysArgs{b.pos, b.mass, b.n, b.seg_of, b.seg_root, b.sort.keys[0], b.sort.vals[0],
+                       b.max_seg <= kSegSortMax ? nullptr : b.pkey, b.pm};
+}
+
+}  // namespace
+
 void launch_seg_keys(const Bufs& b, hipStream_t s) {
-    k_seg_keys<<<grid_for(b.n), 256, 0, s>>>(b.pos, b.mass, b.n, b.seg_of, b.seg_root, b.sort.keys[0], b.sort.vals[0],
-                                             b.max_seg <= kSegSortMax ? nullptr : b.pkey, b.pm);
+    k_seg_keys<<<grid_for(b.n), 256, 0, s>>>(seg_keys_args(b));
+}
+
+void launch_seg_keys_attraction(const Bufs& b, const Params& p, hipStream_t s) {
+    const AttractPlan w = attract_plan(b);
+    const int kb = grid_for(b.n);
+    const auto k = p.linlog || b.ew ? k_seg_keys_attract<true> : k_seg_keys_attract<false>;
+    k<<<kb + w.total, 256, 0, s>>>(seg_keys_args(b), kb, attract_args(b, p), w, b.attr_chunks, b.attr_part);
+    launch_attract_heavy(b, p, s);
 }
 
 void launch_seg_graph_sort(Bufs& b, hipStream_t s) {

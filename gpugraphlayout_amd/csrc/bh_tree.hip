@@ -24,6 +24,7 @@
 //     (src/RPBHKernels.cu:357-506).
 // Nothing waits on another workgroup; every dependency crosses a launch boundary.
 #include "engine_internal.h"
+#include "attract_device.h"
 #include "tree_device.h"
 
 namespace gfa2 {
@@ -143,33 +144,50 @@ __global__ __launch_bounds__(256) void k_new_positions(const float2* __restrict_
 // 16-byte record per sorted body instead of a position and a mass. With dhist (a sort of one
 // launch per pass), also the digit counts of all 8 passes, added to the table the previous
 // iteration's fix-up cleared (the sort's own histogram launches are then skipped).
-__global__ __launch_bounds__(256) void k_keys(const float2* __restrict__ pos, const float* __restrict__ mass, int n,
-                                              const float4* __restrict__ part, DevState* st,
-                                              float4* __restrict__ seg_root,
-                                              unsigned long long* __restrict__ k0, unsigned int* __restrict__ v0,
-                                              unsigned long long* __restrict__ k1, unsigned int* __restrict__ v1,
-                                              float4* __restrict__ pm, int first, unsigned int* __restrict__ dhist,
-                                              const SegState* __restrict__ seg, SegState* __restrict__ seg_cur) {
+struct KeysArgs {
+    const float2* pos;
+    const float* mass;
+    int n;
+    const float4* part;
+    DevState* st;
+    float4* seg_root;
+    unsigned long long *k0, *k1;
+    unsigned int *v0, *v1;
+    float4* pm;
+    int first;
+    unsigned int* dhist;
+    const SegState* seg;
+    SegState* seg_cur;
+};
+
+__device__ __forceinline__ void keys_block(const KeysArgs& K, int block, int blocks) {
+    const float2* __restrict__ pos = K.pos;
+    const float* __restrict__ mass = K.mass;
+    const float4* __restrict__ part = K.part;
+    DevState* st = K.st;
+    float4* __restrict__ pm = K.pm;
+    unsigned int* __restrict__ dhist = K.dhist;
+    const int n = K.n;
     __shared__ float root[3];
     __shared__ unsigned int h[8][256];
     if (dhist)
         for (int p = 0; p < 8; ++p) h[p][threadIdx.x] = 0u;
     // the buffer from which the sort passes that will run (8 less the skipped or unlaunched low
     // ones) end in buffer 0
-    const int low = max(st->sort_skip, first);
+    const int low = max(st->sort_skip, K.first);
     const bool odd = ((8 - low) & 1) != 0;
-    unsigned long long* __restrict__ keys = odd ? k1 : k0;
-    unsigned int* __restrict__ vals = odd ? v1 : v0;
+    unsigned long long* __restrict__ keys = odd ? K.k1 : K.k0;
+    unsigned int* __restrict__ vals = odd ? K.v1 : K.v0;
     reduce_bbox(part, st->nbbox, root);
     const float rootx = root[0], rooty = root[1], radius = root[2];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (block == 0 && threadIdx.x == 0) {
         st->rootx = rootx;
         st->rooty = rooty;
         st->radius = radius;
-        seg_root[0] = make_float4(rootx, rooty, radius, 0.0f);
-        *seg_cur = seg[0];        // for k_advance
+        K.seg_root[0] = make_float4(rootx, rooty, radius, 0.0f);
+        *K.seg_cur = K.seg[0];        // for k_advance
     }
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+    for (int i = block * 256 + threadIdx.x; i < n; i += blocks * 256) {
         const float2 p = pos[i];
         const unsigned long long key = path_key(p, rootx, rooty, radius);
         keys[i] = key;
@@ -187,6 +205,22 @@ __global__ __launch_bounds__(256) void k_keys(const float2* __restrict__ pos, co
             if (c) atomicAdd(&dhist[d * 256 + threadIdx.x], c);
         }
     }
+}
+
+__global__ __launch_bounds__(256) void k_keys(const KeysArgs K) { keys_block(K, blockIdx.x, gridDim.x); }
+
+// The keys and the attraction, which both need the positions only, in one launch: on the first
+// key_blocks blocks the keys, on one block each the attraction's virtual blocks. Up to some ten
+// thousand bodies either is a launch and a few steps in a row, and at any size the one fills the
+// chip while the other ends: 92.0 -> 86.2 us an iteration at 10,000 bodies, 138.8 -> 131.0 at 131,000,
+// 533 -> 523 at 1M.
+template <bool GEN>
+__global__ __launch_bounds__(256) void k_keys_attract(const KeysArgs K, int key_blocks, const AttractArgs A,
+                                                      const AttractPlan w, const int2* __restrict__ chunks,
+                                                      float2* __restrict__ part) {
+    __shared__ float2 red[256];
+    if ((int)blockIdx.x < key_blocks) keys_block(K, blockIdx.x, key_blocks);
+    else attract_block<GEN>(blockIdx.x - key_blocks, w, chunks, part, A, red);
 }
 
 // A graph of a batch starts at sorted position i (always true for i == 0).
@@ -1231,16 +1265,33 @@ void launch_reset(const Bufs& b, float global_speed, float speed_efficiency, flo
     new_positions<true>(b, NewState{global_speed, speed_efficiency, jitter_tolerance, k_s_max, -1}, s);
 }
 
-void launch_keys(const Bufs& b, int first, hipStream_t s) {
-    int blocks = (b.n + 255) / 256;
-    if (blocks > b.grid_cap) blocks = b.grid_cap;
+namespace {
+
+KeysArgs keys_args(const Bufs& b, int first) {
+    return KeysArgs{b.pos, b.mass, b.n, b.bbox_part, b.st, b.seg_root, b.sort.keys[0], b.sort.keys[1], b.sort.vals[0],
+                    b.sort.vals[1], b.pm, first, b.sort.hist_in_keys ? b.sort.digit_hist : nullptr, b.seg_st, b.seg_cur};
+}
+
+int keys_blocks(const Bufs& b) {
+    const int blocks = std::min((b.n + 255) / 256, b.grid_cap);
     // Each block that counts digits adds up to 256 counts per pass to the table: at 131,000 bodies
     // 145.6 us an iteration with 128 blocks, 146.5 with 256, 150.5 with one per 256 bodies; at
     // 262,000 198.2, 196.5, 207.6
-    if (b.sort.hist_in_keys) blocks = std::min(blocks, std::max(128, (b.n + 1023) / 1024));
-    k_keys<<<blocks, 256, 0, s>>>(b.pos, b.mass, b.n, b.bbox_part, b.st, b.seg_root, b.sort.keys[0], b.sort.vals[0],
-                                  b.sort.keys[1], b.sort.vals[1], b.pm, first,
-                                  b.sort.hist_in_keys ? b.sort.digit_hist : nullptr, b.seg_st, b.seg_cur);
+    return b.sort.hist_in_keys ? std::min(blocks, std::max(128, (b.n + 1023) / 1024)) : blocks;
+}
+
+}  // namespace
+
+void launch_keys(const Bufs& b, int first, hipStream_t s) {
+    k_keys<<<keys_blocks(b), 256, 0, s>>>(keys_args(b, first));
+}
+
+void launch_keys_attraction(const Bufs& b, const Params& p, int first, hipStream_t s) {
+    const AttractPlan w = attract_plan(b);
+    const int kb = keys_blocks(b);
+    const auto k = p.linlog || b.ew ? k_keys_attract<true> : k_keys_attract<false>;
+    k<<<kb + w.total, 256, 0, s>>>(keys_args(b, first), kb, attract_args(b, p), w, b.attr_chunks, b.attr_part);
+    launch_attract_heavy(b, p, s);
 }
 
 void launch_tree(Bufs& b, hipStream_t s) {

@@ -192,9 +192,12 @@ void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
         hipEventRecord(h->join, h->side);
     };
     mark(0, s);
+    // one launch with the keys, unless it has a grid or blocks of its own or their times are asked
+    // for one by one
+    const bool keyed = mode == 0 && !h->p.exact && !small && !ev && b.attr_grid == 0 && !attract_wide(b);
     if (mode == 0) {
         mark(1, s);
-        if (!small) launch_attraction(b, h->p, true, s);
+        if (!small && !keyed) launch_attraction(b, h->p, true, s);
         mark(2, s);
     } else if (mode == 2) {
         attraction_on_side();
@@ -203,9 +206,11 @@ void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
     if (!h->p.exact && !small) {
         if (b.nseg > 1) {
             if (!advance_seg(b)) launch_seg_bbox(b, s);
-            launch_seg_keys(b, s);
+            if (keyed) launch_seg_keys_attraction(b, h->p, s);
+            else launch_seg_keys(b, s);
         } else {
-            launch_keys(b, h->sort_first, s);
+            if (keyed) launch_keys_attraction(b, h->p, h->sort_first, s);
+            else launch_keys(b, h->sort_first, s);
         }
     }
     mark(4, s);

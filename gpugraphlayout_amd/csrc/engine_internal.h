@@ -265,6 +265,11 @@ constexpr int kSegSortMax = 32768;
 constexpr int kSegSmall = 2048;
 
 // Launch groups of one iteration, in order.
+// Keys and attraction in one launch (and the heavy rows' sums), for one graph or a batch.
+void launch_keys_attraction(const Bufs& b, const Params& p, int first, hipStream_t s);
+void launch_seg_keys_attraction(const Bufs& b, const Params& p, hipStream_t s);
+// The attraction takes blocks that stay on the chip with the hubs' positions in LDS.
+bool attract_wide(const Bufs& b);
 // alone: no other kernel is to run beside it
 void launch_attraction(const Bufs& b, const Params& p, bool alone, hipStream_t s);
 void launch_col_rank(const Bufs& b, hipStream_t s);

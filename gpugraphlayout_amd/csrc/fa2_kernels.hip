@@ -25,31 +25,6 @@ __global__ __launch_bounds__(256) void k_gather_rank(const int* __restrict__ col
         col_rank[e] = rank[col[e]];
 }
 
-// Block i of the light and medium ones, which take turns in proportion (256 threads).
-template <bool GEN, int HUB>
-__device__ __forceinline__ void attract_rows(int i, int light_blocks, int medium_blocks, int medium_rows, int tid,
-                                             const AttractArgs& A, const float2* hub) {
-    const unsigned int t = light_blocks + medium_blocks;
-    const int m0 = (int)((unsigned long long)i * medium_blocks / t);          // medium blocks before i
-    const int m1 = (int)((i + 1ull) * medium_blocks / t);
-    if (m1 > m0) attract_medium<GEN, HUB>((m0 * 4 + (tid >> 6)) * medium_rows, medium_rows, tid & 63, A, hub);
-    else attract_light<GEN, HUB>((i - m0) * 256 + tid, A, hub);
-}
-
-// red[0] = the sum over 256 threads. red[0] is written again only by thread 0, and every other
-// entry only after the barriers here, so thread 0 may read it after the call.
-__device__ __forceinline__ void sum_chunk(float2* red, int tid, float ax, float ay) {
-    red[tid] = make_float2(ax, ay);
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (tid < o) {
-            const float2 a = red[tid], b = red[tid + o];
-            red[tid] = make_float2(a.x + b.x, a.y + b.y);
-        }
-        __syncthreads();
-    }
-}
-
 // Attraction + gravity, fga[v] = gravity(v) + sum over CSR entries of v (in entry order for the
 // light rows; lane-strided then a shuffle tree for medium rows; see below for heavy rows).
 // Degree classes: light rows (<= 32 entries) one thread each, entries four at a time;
@@ -65,37 +40,23 @@ __device__ __forceinline__ void sum_chunk(float2* red, int tid, float ax, float 
 constexpr int kHubCache = 2048;      // hubs' positions in LDS: 16 KB, so that 8 blocks fit a CU
 
 template <bool GEN, int HUB>
-__global__ __launch_bounds__(256) void k_attract(const float2* __restrict__ pos, const float* __restrict__ mass,
-                                                 int n, const float2* __restrict__ pos_rank,
-                                                 const int* __restrict__ rowptr, const int* __restrict__ col,
-                                                 const int* __restrict__ lists, int nlight, int nmedium,
-                                                 const int2* __restrict__ chunks, int nchunks,
+__global__ __launch_bounds__(256) void k_attract(const AttractArgs A, const int2* __restrict__ chunks, int nchunks,
                                                  int light_blocks, int medium_blocks, int medium_rows,
-                                                 int strong, float k_g, float2* __restrict__ fga,
-                                                 float2* __restrict__ part, int linlog,
-                                                 const float* __restrict__ ew) {
+                                                 float2* __restrict__ part) {
     __shared__ float2 red[256];
     __shared__ float2 hub[HUB > 0 ? HUB : 1];
     const int tid = threadIdx.x;
     if constexpr (HUB > 0) {
-        for (int i = tid; i < HUB && i < n; i += 256) hub[i] = pos_rank[i];
+        for (int i = tid; i < HUB && i < A.n; i += 256) hub[i] = A.pos_rank[i];
         __syncthreads();
     }
-    const AttractArgs A{pos, mass, n, pos_rank, rowptr, col, lists, nlight, nmedium, strong, k_g, fga, linlog, ew};
     const int total = light_blocks + medium_blocks + nchunks;
     for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {   // uniform per block
         if (vb >= nchunks) {
             attract_rows<GEN, HUB>(vb - nchunks, light_blocks, medium_blocks, medium_rows, tid, A, hub);
             continue;
         }
-        const int2 ch = chunks[vb];
-        const int v = lists[nlight + nmedium + ch.x];
-        const float2 p = pos[v];
-        float ax = 0.0f, ay = 0.0f;
-        const int len = min(kAttrChunk, rowptr[v + 1] - ch.y);
-        gather_terms<GEN, 256, HUB>(p, A, hub, Row(A, ch.y, ch.y + len), tid, ax, ay);
-        sum_chunk(red, tid, ax, ay);
-        if (tid == 0) part[vb] = red[0];
+        attract_chunk<GEN, HUB>(vb, chunks, part, tid, A, hub, red);
     }
 }
 
@@ -1079,37 +1040,57 @@ void launch_col_rank(const Bufs& b, hipStream_t s) {
     if (b.nnz > 0) k_gather_rank<<<(int)std::min<long long>((b.nnz + 255) / 256, 16384), 256, 0, s>>>(b.col, b.rank, b.nnz, b.col_rank);
 }
 
-void launch_attraction(const Bufs& b, const Params& p, bool alone, hipStream_t s) {
-    const int lb = (b.nlight + 255) / 256;
+AttractPlan attract_plan(const Bufs& b) {
+    AttractPlan a;
+    a.light_blocks = (b.nlight + 255) / 256;
     // several medium rows to a wave once one each would more than fill the card (8 waves on each
     // of 1,024 SIMDs): with one each, R-MAT 2^18 at 4M entries took 182 us an iteration against 176
-    const int rows = std::max(1, std::min(kMediumBatch, b.nmedium / 8192));
-    const int mb = (b.nmedium + 4 * rows - 1) / (4 * rows);
-    int total = lb + mb + b.nattr_chunks;
+    a.medium_rows = std::max(1, std::min(kMediumBatch, b.nmedium / 8192));
+    a.medium_blocks = (b.nmedium + 4 * a.medium_rows - 1) / (4 * a.medium_rows);
+    a.chunks = b.nattr_chunks;
+    a.total = a.light_blocks + a.medium_blocks + a.chunks;
+    return a;
+}
+
+AttractArgs attract_args(const Bufs& b, const Params& p) {
+    return AttractArgs{b.pos,    b.mass,    b.n,              b.pos_rank, b.rowptr, b.col_rank, b.node_lists,
+                       b.nlight, b.nmedium, p.strong_gravity, p.k_g,      b.fga,    p.linlog,   b.ew};
+}
+
+// The wide blocks stay until all rows are done, which pays where their staging and their uneven
+// ends are small beside the work and hubs hold many entries (R-MAT: 8M entries 252 us an
+// iteration without, 265 with; 20M 402, 397; 64M 1,253, 1,213; BA with 1M bodies, 20M entries,
+// 9% of them of hubs: 667, 753), and nothing is to run beside them.
+bool attract_wide(const Bufs& b) {
+    return b.attr_grid == 0 && b.nnz >= kWideEntries && b.hub_entries >= b.nnz / 4;
+}
+
+void launch_attract_heavy(const Bufs& b, const Params& p, hipStream_t s) {
+    if (b.nheavy > 0)
+        k_attract_heavy<<<(b.nheavy + 255) / 256, 256, 0, s>>>(b.pos, b.mass, b.node_lists + b.nlight + b.nmedium,
+                                                               b.nheavy, b.attr_c0, b.attr_part, p.strong_gravity,
+                                                               p.k_g, b.fga);
+}
+
+void launch_attraction(const Bufs& b, const Params& p, bool alone, hipStream_t s) {
+    const AttractPlan w = attract_plan(b);
+    const AttractArgs A = attract_args(b, p);
     const bool gen = p.linlog || b.ew;
-    // The wide blocks stay until all rows are done, which pays where their staging and their uneven
-    // ends are small beside the work and hubs hold many entries (R-MAT: 8M entries 252 us an
-    // iteration without, 265 with; 20M 402, 397; 64M 1,253, 1,213; BA with 1M bodies, 20M entries,
-    // 9% of them of hubs: 667, 753), and nothing is to run beside them.
-    const bool wide = alone && b.attr_grid == 0 && b.nnz >= kWideEntries && b.hub_entries >= b.nnz / 4;
-    if (wide) {
-        const AttractArgs A{b.pos,    b.mass,    b.n,              b.pos_rank, b.rowptr, b.col_rank, b.node_lists,
-                            b.nlight, b.nmedium, p.strong_gravity, p.k_g,      b.fga,    p.linlog,   b.ew};
-        const int blocks = std::min(2 * b.cus, (total + kWideSubs - 1) / kWideSubs);
-        if (gen) k_attract_wide<true><<<blocks, kWideThreads, 0, s>>>(A, b.attr_chunks, b.nattr_chunks, lb, mb, rows, b.attr_part);
-        else k_attract_wide<false><<<blocks, kWideThreads, 0, s>>>(A, b.attr_chunks, b.nattr_chunks, lb, mb, rows, b.attr_part);
-        total = 0;
-    }
-    if (b.attr_grid > 0 && total > b.attr_grid) total = b.attr_grid;   // the launch grid
-    if (total > 0) {
+    if (alone && attract_wide(b)) {
+        const int blocks = std::min(2 * b.cus, (w.total + kWideSubs - 1) / kWideSubs);
+        if (gen)
+            k_attract_wide<true><<<blocks, kWideThreads, 0, s>>>(A, b.attr_chunks, w.chunks, w.light_blocks,
+                                                                 w.medium_blocks, w.medium_rows, b.attr_part);
+        else
+            k_attract_wide<false><<<blocks, kWideThreads, 0, s>>>(A, b.attr_chunks, w.chunks, w.light_blocks,
+                                                                  w.medium_blocks, w.medium_rows, b.attr_part);
+    } else if (w.total > 0) {
+        const int blocks = b.attr_grid > 0 ? std::min(w.total, b.attr_grid) : w.total;
         // a grid smaller than the work (beside other kernels): every block stages the hubs'
         // positions once and uses them for several virtual blocks
-        const bool hub = b.attr_grid > 0 && lb + mb + b.nattr_chunks > 2 * total;
-#define GFA2_ATTRACT(G, H)                                                                                   \
-    k_attract<G, H><<<total, 256, 0, s>>>(b.pos, b.mass, b.n, b.pos_rank, b.rowptr, b.col_rank, b.node_lists,   \
-                                          b.nlight, b.nmedium, b.attr_chunks, b.nattr_chunks, lb, mb, rows,     \
-                                          p.strong_gravity, p.k_g, b.fga, b.attr_part, G ? p.linlog : 0,      \
-                                          G ? b.ew : nullptr)
+        const bool hub = b.attr_grid > 0 && w.total > 2 * blocks;
+#define GFA2_ATTRACT(G, H) \
+    k_attract<G, H><<<blocks, 256, 0, s>>>(A, b.attr_chunks, w.chunks, w.light_blocks, w.medium_blocks, w.medium_rows, b.attr_part)
         if (gen) {
             if (hub) GFA2_ATTRACT(true, kHubCache);
             else GFA2_ATTRACT(true, 0);
@@ -1119,10 +1100,7 @@ void launch_attraction(const Bufs& b, const Params& p, bool alone, hipStream_t s
         }
 #undef GFA2_ATTRACT
     }
-    if (b.nheavy > 0)
-        k_attract_heavy<<<(b.nheavy + 255) / 256, 256, 0, s>>>(b.pos, b.mass, b.node_lists + b.nlight + b.nmedium,
-                                                               b.nheavy, b.attr_c0, b.attr_part, p.strong_gravity,
-                                                               p.k_g, b.fga);
+    launch_attract_heavy(b, p, s);
 }
 
 void launch_walk(const Bufs& b, const Params& p, bool split, hipStream_t s) {

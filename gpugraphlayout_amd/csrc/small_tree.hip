@@ -543,8 +543,7 @@ void launch_small_tree(const Bufs& b, const Params& p, hipStream_t s) {
     A.pmass = b.pmass;
     A.cap_records = b.cap_records;
     A.int_mass = b.int_mass ? 1 : 0;
-    const AttractArgs at{b.pos,    b.mass,       b.n,   b.pos_rank, b.rowptr, b.col_rank, b.node_lists, b.nlight,
-                         b.nmedium, p.strong_gravity, p.k_g, b.fga,      p.linlog, b.ew};
+    const AttractArgs at = attract_args(b, p);
     const bool apart = b.nheavy > 0;
     const int lb = apart ? 0 : (b.nlight + 255) / 256, vb = apart ? 0 : lb + (b.nmedium + 3) / 4;
     if (apart) launch_attraction(b, p, true, s);
