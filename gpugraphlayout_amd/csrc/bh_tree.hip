@@ -14,13 +14,13 @@
 //  4. with lcp_i the common digits of sorted neighbours i and i+1, the cells are exactly
 //     the prefixes of length <= lcp_i; the cells starting at position i have levels
 //     lcp_{i-1}+1 .. lcp_i. Their pre-order record index follows from an exclusive scan
-//     of those counts, and each cell's extent from a galloping search over the keys;
+//     of those counts, and a cell of level L ends at the first position whose lcp is below L;
 //  5. summaries. Counts are extents. For whole-number masses (the default deg+1) a cell
 //     lighter than 2^24 has the same float mass in every summation order, so its mass and
 //     centroid come from exact integer prefix sums over the sorted bodies (fixed-point
 //     moments, see Moment); heavier cells are summed in quadrant order. Other masses:
-//     bottom-up, one launch per level, children in quadrant order, mass accumulated from
-//     0.0f and centroid (sum m*p)*(1/mass), as the reference's SummarizationKernel
+//     bottom-up, children in quadrant order, mass accumulated from 0.0f
+//     and centroid (sum m*p)*(1/mass), as the reference's SummarizationKernel
 //     (src/RPBHKernels.cu:357-506).
 // Nothing waits on another workgroup; every dependency crosses a launch boundary.
 #include "engine_internal.h"

@@ -578,9 +578,16 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
     GFA2_ALLOC(b.kids, (size_t)cap);
     b.kids_blocks = 2 * tree_tiles;
     GFA2_ALLOC(b.kids_part, (size_t)b.kids_blocks * 8);
-    GFA2_ALLOC(b.cross, (size_t)tree_tiles * kCrossMax);
-    GFA2_ALLOC(b.ncross, tree_tiles);
-    GFA2_ALLOC(b.tmin, (tree_tiles + 15) / 16 * 16);
+    {
+        // the crossing cells' tables, one allocation (each costs a small engine's creation 10-20 us)
+        const size_t slots = ((size_t)tree_tiles * kCrossMax + 1) / 2 * 2, groups = ((size_t)tree_tiles + 15) / 16 * 16;
+        char* tables = nullptr;
+        GFA2_ALLOC(tables, slots * (sizeof(int4) + sizeof(Moment)) + groups * (sizeof(int) + 1));
+        b.cross = reinterpret_cast<int4*>(tables);
+        b.cross_sum = reinterpret_cast<Moment*>(b.cross + slots);
+        b.ncross = reinterpret_cast<int*>(b.cross_sum + slots);
+        b.tmin = reinterpret_cast<signed char*>(b.ncross + groups);
+    }
     GFA2_ALLOC(b.sbody, n);
     GFA2_ALLOC(b.pm, n);
     GFA2_ALLOC(b.rcount, (size_t)cap);
@@ -644,7 +651,6 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
         }
     }
     if (b.int_mass) {
-        GFA2_ALLOC(b.cross_sum, (size_t)tree_tiles * kCrossMax);
         GFA2_ALLOC(b.pmass, n <= kSmallTree ? (size_t)n + 1 : (size_t)n / 16 + 1);
         GFA2_ALLOC(b.bmass, tree_tiles);
         GFA2_ALLOC(b.chunk_mass, (tree_tiles + kTileChunk - 1) / kTileChunk);
