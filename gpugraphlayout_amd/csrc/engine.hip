@@ -194,7 +194,8 @@ void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
     mark(0, s);
     // one launch with the keys, unless it has a grid or blocks of its own or their times are asked
     // for one by one
-    const bool keyed = mode == 0 && !h->p.exact && !small && !ev && b.attr_grid == 0 && !attract_wide(b);
+    const bool apart = ev && h->timing != GFA2_TIMING_WALK;
+    const bool keyed = mode == 0 && !h->p.exact && !small && !apart && b.attr_grid == 0 && !attract_wide(b);
     if (mode == 0) {
         mark(1, s);
         if (!small && !keyed) launch_attraction(b, h->p, true, s);
@@ -579,7 +580,7 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
     b.kids_blocks = 2 * tree_tiles;
     GFA2_ALLOC(b.kids_part, (size_t)b.kids_blocks * 8);
     {
-        // the crossing cells' tables, one allocation (each costs a small engine's creation 10-20 us)
+        // the tables of the crossing cells
         const size_t slots = ((size_t)tree_tiles * kCrossMax + 1) / 2 * 2, groups = ((size_t)tree_tiles + 15) / 16 * 16;
         char* tables = nullptr;
         GFA2_ALLOC(tables, slots * (sizeof(int4) + sizeof(Moment)) + groups * (sizeof(int) + 1));
