@@ -332,15 +332,9 @@ __global__ __launch_bounds__(kTreeThreads) void k_lcp(const unsigned long long* 
                                                       const float4* __restrict__ seg_root,
                                                       Moment* __restrict__ bmass, float4* __restrict__ sbody,
                                                       DevState* __restrict__ st) {
-    if (blockIdx.x == 0) {           // for the launches that follow
-        if (threadIdx.x == 0) {
-            st->max_level = 0;
-            st->nbig = 0;
-        }
-        if (threadIdx.x <= kMaxLevels) {
-            st->level_count[threadIdx.x] = 0;
-            st->level_cursor[threadIdx.x] = 0;
-        }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {       // for the launches that follow
+        st->max_level = 0;
+        st->nbig = 0;
     }
     // the tile's keys (with one on each side), graph ids and body ids, read coalesced into
     // LDS; each thread then takes its kTreeItems consecutive positions from there
@@ -550,8 +544,6 @@ struct TileArgs {
     float4* rec;
     int4* kids;
     int* rcount;
-    int* cell_rec;              // with cell_lvl, for the launches per level: records and levels
-    unsigned char* cell_lvl;
     DevState* st;
     const float4* seg_root;
     TileSplit* pm16;            // the sum over the tile's bodies before every 16th position
@@ -612,7 +604,6 @@ __global__ __launch_bounds__(kTreeTile) void k_tile(const TileArgs A) {
     __shared__ int first[kTreeTile + 1];                       // cells opened before each position
     __shared__ unsigned char level[kTreeTile];                 // the first opened cell's
     __shared__ unsigned short owner[kTileCells];               // a round's cells' positions
-    __shared__ int hist[kMaxLevels + 1];
     __shared__ int rmax[8];
     __shared__ int lmax, lmin, ncross, go;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -633,7 +624,6 @@ __global__ __launch_bounds__(kTreeTile) void k_tile(const TileArgs A) {
     if (A.fused)
         for (int t = tid; t < (int)blockIdx.x; t += kTreeTile) acc += A.blockoff[t];
     else if (tid == 0) acc = A.blockoff[blockIdx.x];
-    if (tid <= kMaxLevels) hist[tid] = 0;
     if (tid < 8) rmax[tid] = 0;
     if (tid == 0) {
         lmax = ncross = 0;
@@ -709,11 +699,6 @@ __global__ __launch_bounds__(kTreeTile) void k_tile(const TileArgs A) {
             const int b = next_bit(rows, L, p);                // the cell's last body
             const int g = A.sg ? A.sg[base + p] : 0;
             if (L == 0) A.rec_begin[g] = rc;
-            if (A.cell_lvl) {
-                A.cell_rec[ord] = rc;
-                A.cell_lvl[ord] = (unsigned char)L;
-                atomicAdd(&hist[L], 1);
-            }
             atomicMax(&lmax, L);
             if (b == kTreeTile) {
                 const int slot = blockIdx.x * kCrossMax + atomicAdd(&ncross, 1);
@@ -746,7 +731,6 @@ __global__ __launch_bounds__(kTreeTile) void k_tile(const TileArgs A) {
         if (any) atomicMin(&lmin, tid - 1);
     }
     __syncthreads();
-    if (A.cell_lvl && tid <= kMaxLevels && hist[tid] != 0) atomicAdd(&A.st->level_count[tid], hist[tid]);
     // every block would hit this one word: only blocks above the value seen so far update it
     // (the maximum only grows, so skipping on a stale value is still correct)
     if (tid == 0 && lmax > 0 && lmax > __hip_atomic_load(&A.st->max_level, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
@@ -922,17 +906,18 @@ __global__ __launch_bounds__(kCrossThreads) void k_cross(const TileArgs A) {
     if (tid < 8) A.kids_part[(gridDim.x + blockIdx.x) * 8 + tid] = rmax[tid];
 }
 
-// Summaries of all cells in two launches, for trees of up to kSumMaxBlocks * kSumBlock records. A
-// block takes kSumBlock records, which lie in preorder, and sums the cells that end inside it in
-// LDS, deepest level first. The few that reach past its end contain its last record, so they are
-// nested and of different levels: each has a slot of its own (block, level), and one block
-// then sums them all, deepest level first, with their other children read beforehand. What bounds
-// both are the levels' dependent steps, which here cost a barrier each and no launch: 20k bodies
-// with fractional masses 31 us, where a launch per level took 82.
-constexpr int kSumBlock = 4096, kSumThreads = 1024, kSumMaxBlocks = 62;
+// Summaries of all cells, bottom-up. A block takes kSumBlock records, which lie in preorder, and sums
+// the cells that end inside it in LDS, deepest level first. The few that reach past its end contain
+// its last record, so they are nested and of different levels: each has a slot of its own (block,
+// level). One block then sums the slots of kSumUnits blocks in the same order, with their other
+// children read beforehand; what reaches past those has a slot among kSumUnits of such groups, and
+// so on to one group. What bounds all are the levels' dependent steps, which here cost a barrier
+// each and no launch: 20k bodies with fractional masses 31 us, where a launch per level took 82;
+// an iteration of 70k bodies 155 us (per level 199), of 1M 497 (583), of 11.5M 5,142 (5,820).
+constexpr int kSumBlock = 4096, kSumThreads = 1024, kSumUnits = 62;
 constexpr int kSumLevels = 33;       // slots per block: the root, then a cell's info level + 1
 constexpr int kSumOwn = kSumBlock / kSumThreads;
-static_assert(kSumMaxBlocks * kSumLevels <= 2 * kSumThreads, "two slots per thread of k_sum_spill");
+static_assert(kSumUnits * kSumLevels <= 2 * kSumThreads, "two slots per thread of k_sum_spill");
 
 constexpr unsigned int kBodyInfo = 0xffffffffu;
 
@@ -1034,12 +1019,22 @@ __global__ __launch_bounds__(kSumThreads) void k_sum_blocks(float4* __restrict__
     }
 }
 
+// Units of span records; a block takes kSumUnits of them, and the cells that reach past its last
+// go to its own slots in up (read by a launch with kSumUnits times the span).
 __global__ __launch_bounds__(kSumThreads) void k_sum_spill(float4* __restrict__ rec, const int* __restrict__ spill,
+                                                           int span, int* __restrict__ up,
                                                            const DevState* __restrict__ st) {
     __shared__ float4 sum[2 * kSumThreads];
+    __shared__ int slot[kSumLevels];
     if (st->err != 0) return;
     const int tid = threadIdx.x, total = st->nrecords;
-    const int slots = (total + kSumBlock - 1) / kSumBlock * kSumLevels;
+    const int unit0 = blockIdx.x * kSumUnits;
+    const int units = min((int)(((long long)total + span - 1) / span) - unit0, kSumUnits);
+    if (units <= 0) return;
+    const int slots = units * kSumLevels;
+    const int stop = (int)min((long long)(unit0 + units) * span, (long long)total);
+    if (tid < kSumLevels) slot[tid] = -1;
+    __syncthreads();
     float4 child[2][4], own[2];
     int ref[2][4];               // a child's slot; -1: it is in child; -2: none
     int cell[2];
@@ -1047,10 +1042,14 @@ __global__ __launch_bounds__(kSumThreads) void k_sum_spill(float4* __restrict__ 
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         const int q = tid + k * kSumThreads;
-        cell[k] = q < slots ? spill[q] : -1;
+        cell[k] = q < slots ? spill[unit0 * kSumLevels + q] : -1;
         if (cell[k] < 0) continue;
         own[k] = rec[cell[k]];
         const int end = min(cell[k] + (int)(__float_as_uint(own[k].w) >> kInfoLevelBits), total);
+        if (end > stop) {
+            slot[q % kSumLevels] = cell[k];
+            continue;
+        }
         int r = cell[k] + 1;
         CellSum s;
 #pragma unroll
@@ -1061,8 +1060,8 @@ __global__ __launch_bounds__(kSumThreads) void k_sum_spill(float4* __restrict__ 
             const unsigned int ci = __float_as_uint(child[k][u].w);
             const int next = r + record_hop(ci);
             ref[k][u] = -1;
-            if (ci != kBodyInfo && r / kSumBlock != (next - 1) / kSumBlock) {
-                ref[k][u] = r / kSumBlock * kSumLevels + info_level(ci) + 1;
+            if (ci != kBodyInfo && r / span != (next - 1) / span) {
+                ref[k][u] = (r / span - unit0) * kSumLevels + info_level(ci) + 1;
                 waits[k] = true;
             }
             s.add(child[k][u]);
@@ -1078,6 +1077,7 @@ __global__ __launch_bounds__(kSumThreads) void k_sum_spill(float4* __restrict__ 
         rec[cell[k]] = sum[q];
     }
     __syncthreads();
+    if (up != nullptr && tid < kSumLevels) up[blockIdx.x * kSumLevels + tid] = slot[tid];
     for (int L = kSumLevels - 1; L >= 0; --L) {
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
@@ -1091,68 +1091,6 @@ __global__ __launch_bounds__(kSumThreads) void k_sum_spill(float4* __restrict__ 
             rec[cell[k]] = sum[q];
         }
         __syncthreads();
-    }
-}
-
-// Larger trees, a launch per level. Bucket cells by level (order inside a level is irrelevant).
-__global__ __launch_bounds__(256) void k_levels(const int* __restrict__ cell_rec,
-                                                const unsigned char* __restrict__ cell_lvl,
-                                                int* __restrict__ level_list, DevState* st) {
-    __shared__ int off[kMaxLevels + 2];
-    __shared__ int hist[kMaxLevels + 1];
-    __shared__ int base[kMaxLevels + 1];
-    const int tid = threadIdx.x;
-    if (tid == 0) {
-        int run = 0;
-        for (int L = 0; L <= kMaxLevels; ++L) {
-            off[L] = run;
-            run += st->level_count[L];
-        }
-        off[kMaxLevels + 1] = run;
-        if (blockIdx.x == 0)
-            for (int L = 0; L <= kMaxLevels + 1; ++L) st->level_offset[L] = off[L];
-    }
-    if (tid <= kMaxLevels) hist[tid] = 0;
-    __syncthreads();
-    const int C = st->err == 0 ? st->ncells : 0;
-    const int t = blockIdx.x * 256 + tid;
-    int L = -1, local = 0, rc = 0;
-    if (t < C) {
-        L = cell_lvl[t];
-        rc = cell_rec[t];
-        local = atomicAdd(&hist[L], 1);
-    }
-    __syncthreads();
-    if (tid <= kMaxLevels && hist[tid] != 0) base[tid] = atomicAdd(&st->level_cursor[tid], hist[tid]);
-    __syncthreads();
-    if (L >= 0) level_list[off[L] + base[L] + local] = rc;
-}
-
-// Summaries of all cells at one level; children are the records between rc+1 and
-// rc+skip, hopped by their own skips, in quadrant order.
-__global__ __launch_bounds__(256) void k_summarize(int L, const int* __restrict__ level_list,
-                                                   float4* __restrict__ rec, const DevState* __restrict__ st) {
-    if (st->err != 0) return;
-    const int beg = st->level_offset[L];
-    const int cnt = st->level_count[L];
-    for (int t = blockIdx.x * 256 + threadIdx.x; t < cnt; t += gridDim.x * 256) {
-        const int rc = level_list[beg + t];
-        const unsigned int info = __float_as_uint(rec[rc].w);
-        const int end = min(rc + (int)(info >> kInfoLevelBits), st->nrecords);
-        float cm = 0.0f, px = 0.0f, py = 0.0f;
-        int r = rc + 1;
-        while (r < end) {
-            const float4 c = rec[r];
-            const unsigned int ci = __float_as_uint(c.w);
-            px = fmaf(c.x, c.z, px);
-            py = fmaf(c.y, c.z, py);
-            cm += c.z;
-            r += ci == 0xffffffffu ? 1 : max((int)(ci >> kInfoLevelBits), 1);
-        }
-        const float inv = 1.0f / cm;
-        rec[rc].x = px * inv;
-        rec[rc].y = py * inv;
-        rec[rc].z = cm;
     }
 }
 
@@ -1312,11 +1250,8 @@ void launch_tree(Bufs& b, hipStream_t s) {
     } else if (!fused) {
         k_scan_blocks<<<1, 1024, 0, s>>>(b.blocksum, tiles, n, b.cap_records, b.rec_begin + b.nseg, b.st, bm);
     }
-    const int max_cells = b.cap_records - n;
-    const int sum_grid = (b.cap_records + kSumBlock - 1) / kSumBlock;
-    const bool by_level = !b.int_mass && sum_grid > kSumMaxBlocks;
     const TileArgs T{b.lcp,       sg,      n,       b.blocksum,  bm,        fused ? 1 : 0, b.S,     b.sbody,
-                     b.rec,       b.kids,         b.rcount, b.cell_rec, by_level ? b.cell_lvl : nullptr, b.st,
+                     b.rec,       b.kids,         b.rcount, b.st,
                      b.seg_root,  reinterpret_cast<TileSplit*>(b.pmass),        b.cap_records, b.rec_begin, b.nseg, b.node_off, b.big_rc, b.big_lvl,
                      b.kids_part, b.cross,        reinterpret_cast<TileSplit*>(b.cross_sum), b.ncross, b.tmin};
     // a wave for each of a tile's cells while the tiles fit the chip once (50,000 bodies: 8.4 us with
@@ -1334,18 +1269,18 @@ void launch_tree(Bufs& b, hipStream_t s) {
         if (!b.no_big) k_big<<<1, 256, 0, s>>>(b.rec, b.big_rc, b.big_lvl, b.st);
         return;
     }
-    // the spilled cells fit one block; larger trees fill the chip with a level each
-    if (!by_level) {
-        k_sum_blocks<<<sum_grid, kSumThreads, 0, s>>>(b.rec, b.level_list, b.st);
-        k_sum_spill<<<1, kSumThreads, 0, s>>>(b.rec, b.level_list, b.st);
-        return;
+    int units = (b.cap_records + kSumBlock - 1) / kSumBlock, span = kSumBlock;
+    int* spill = b.spill;
+    k_sum_blocks<<<units, kSumThreads, 0, s>>>(b.rec, spill, b.st);
+    for (;;) {
+        const int groups = (units + kSumUnits - 1) / kSumUnits;
+        int* up = groups > 1 ? spill + units * kSumLevels : nullptr;
+        k_sum_spill<<<groups, kSumThreads, 0, s>>>(b.rec, spill, span, up, b.st);
+        if (groups == 1) return;
+        spill = up;
+        units = groups;
+        span *= kSumUnits;           // (units of 2^31 records at most: below 62^4 blocks)
     }
-    k_levels<<<(max_cells + 255) / 256, 256, 0, s>>>(b.cell_rec, b.cell_lvl, b.level_list, b.st);
-    int sum_blocks = (max_cells / 4 + 255) / 256;
-    if (sum_blocks < 1) sum_blocks = 1;
-    if (sum_blocks > 1024) sum_blocks = 1024;
-    for (int L = kKeyLevels; L >= 0; --L)
-        k_summarize<<<sum_blocks, 256, 0, s>>>(L, b.level_list, b.rec, b.st);
 }
 
 }  // namespace gfa2

@@ -592,9 +592,8 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
     GFA2_ALLOC(b.sbody, n);
     GFA2_ALLOC(b.pm, n);
     GFA2_ALLOC(b.rcount, (size_t)cap);
-    GFA2_ALLOC(b.cell_rec, maxcells);
     GFA2_ALLOC(b.cell_lvl, maxcells);
-    GFA2_ALLOC(b.level_list, maxcells);
+    GFA2_ALLOC(b.spill, 66 * ((size_t)cap / 4096 + 8));   // (33 slots per block, fewer in all for the groups)
     GFA2_ALLOC(b.bbox_part, kPartBlocks);
     GFA2_ALLOC(b.st, 1);
     // a sort wait that runs out raises the instance's error word, so every later kernel of the

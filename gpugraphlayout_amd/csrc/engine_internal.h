@@ -51,9 +51,6 @@ struct DevState {
     int sort_skip;      // low 8-bit digit passes the next path-key sort skips (0: a full sort)
     int full_sorts;     // iterations after new positions whose next sort is still a full one
     int runmax[8];      // largest body count of a cell at level 4, 8, ..., 32 (the last tree)
-    int level_count[kMaxLevels + 1];
-    int level_offset[kMaxLevels + 2];
-    int level_cursor[kMaxLevels + 1];
 };
 
 // Prefix sums over sorted bodies for the integer-mass summary path: mass, and mass times the
@@ -162,9 +159,8 @@ struct Bufs {
     float* ew_raw = nullptr;    // edge weights per CSR entry (null: unweighted)
     float* ew = nullptr;        // w^delta per CSR entry
     int* rcount;
-    int* cell_rec;
     unsigned char* cell_lvl;
-    int* level_list;
+    int* spill;
     float4* bbox_part;
     WalkPart* walk_part;
     int nwalk_part;

@@ -453,7 +453,7 @@ __device__ void small_tree(const SmallArgs& A, SmallLds<N>& L) {
     if (tid < 8) A.kids_part[tid] = L.rmax[tid];
     if (tid == 0) A.st->max_level = L.lmax;
     if (!A.int_mass) {
-        // bottom-up, children in quadrant order (as k_summarize)
+        // bottom-up, children in quadrant order (as k_sum_blocks)
         for (int lv = L.lmax; lv >= 0; --lv) {
             for (int c = tid; c < cells; c += kThreads) {
                 if (A.cell_lvl[c] != lv) continue;     // this thread's own write
