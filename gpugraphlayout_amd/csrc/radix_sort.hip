@@ -508,9 +508,10 @@ constexpr unsigned int kStatCount = (1u << 27) - 1;
 // threads); of 512 up to 262,144, where fewer tiles have to be read (131,000: 145.6, with 256 threads
 // 151.1). Beyond, three launches per pass are as fast (262,000: 198.5 us an iteration against 196.5;
 // 300,000: 225.7 against 224.8; 2M: 1,118 against 1,159). 1,024 threads were slower
-// throughout, past this line most beside a second stream's kernels, where such large blocks find no
-// room (579,581 bodies, 20M entries: 349 us against 407; alone 404.7 against 400.6). With a look-back from tile to tile the iterations took 104.1 us at 20,000, 121.8 (now
-// 115.0) at 50,000 and 158.2 at 131,000.
+// up to this line. Past it they gain 1% on one stream and lose where a second stream's kernels
+// leave such large blocks no room (579,581 bodies, 20M entries, three launches against one: 404.7
+// and 400.6 us an iteration alone, 349 and 407 beside the attraction). With a look-back from tile to
+// tile the iterations took 104.1 us at 20,000, 121.8 (now 115.0) at 50,000 and 158.2 at 131,000.
 constexpr int kSweepSmall = 32768;
 constexpr int kSweepMost = 262144;
 constexpr int kMaxSpins = 1 << 20;   // per thread and pass: ~1 s at worst, then an error
