@@ -154,9 +154,10 @@ __global__ __launch_bounds__(256) void k_bfs_pairs(const int* __restrict__ tgt, 
                                                    const unsigned long long* __restrict__ next, int level,
                                                    int* __restrict__ dist, const int* __restrict__ changed) {
     if (*changed == 0) return;
-    const int total = nk * T;
-    for (int q = blockIdx.x * 256 + threadIdx.x; q < total; q += gridDim.x * 256) {
-        const int k = q / T;
+    // unsigned: a search's pairs are fewer than 2^31, but a grid stride more may not be
+    const unsigned int total = (unsigned int)nk * T;
+    for (unsigned int q = blockIdx.x * 256u + threadIdx.x; q < total; q += gridDim.x * 256u) {
+        const int k = (int)(q / (unsigned int)T);
         const size_t p = (size_t)k0 * T + q;
         if (dist[p] == 0 && ((next[(size_t)tgt[p] * W + (k >> 6)] >> (k & 63)) & 1ull)) dist[p] = level;
     }
