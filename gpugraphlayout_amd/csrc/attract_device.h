@@ -21,12 +21,15 @@ struct AttractArgs {
     const float* ew;
 };
 
-__device__ __forceinline__ float2 gravity(float2 p, float m, int strong, float k_g) {
+// A node's force from its position, mass and attraction: gravity added. Here and in the other terms
+// every fused multiply-add is written out: left to the compiler, which product of a sum of two is
+// fused differs from kernel to kernel, and with it the last bit.
+__device__ __forceinline__ float2 add_gravity(float2 p, float m, int strong, float k_g, float ax, float ay) {
     float fg;
     if (strong) fg = k_g * m;
-    else if (p.x != 0.0f || p.y != 0.0f) fg = k_g * m * rsqrtf(p.x * p.x + p.y * p.y);
+    else if (p.x != 0.0f || p.y != 0.0f) fg = k_g * m * rsqrtf(fmaf(p.x, p.x, p.y * p.y));
     else fg = 0.0f;
-    return make_float2(-p.x * fg, -p.y * fg);
+    return make_float2(fmaf(-p.x, fg, ax), fmaf(-p.y, fg, ay));
 }
 
 // One edge's attraction term on node p from neighbour q. Linear: q - p. With linlog (the
@@ -44,12 +47,12 @@ __device__ __forceinline__ void attract_term(float2 p, float2 q, int linlog, con
     } else {
         float fa = 1.0f;
         if (linlog) {
-            const float d = sqrtf(dx * dx + dy * dy);
+            const float d = sqrtf(fmaf(dx, dx, dy * dy));
             fa = d == 0.0f ? 0.0f : logf(1.0f + d) / d;
         }
         if (ew) fa *= ew[e];
-        ax += dx * fa;
-        ay += dy * fa;
+        ax = fmaf(dx, fa, ax);
+        ay = fmaf(dy, fa, ay);
     }
 }
 
@@ -113,8 +116,7 @@ __device__ __forceinline__ void attract_light(int k, const AttractArgs& A, const
     const float2 p = A.pos[v];
     float ax = 0.0f, ay = 0.0f;
     gather_terms<GEN, 1, HUB>(p, A, hub, Row(A, A.rowptr[v], A.rowptr[v + 1]), 0, ax, ay);
-    const float2 g = gravity(p, A.mass[v], A.strong, A.k_g);
-    A.fga[v] = make_float2(g.x + ax, g.y + ay);
+    A.fga[v] = add_gravity(p, A.mass[v], A.strong, A.k_g, ax, ay);
 }
 
 // Medium rows k0 to k0 + rows - 1 (one wave, rows <= kMediumBatch): lane-strided sums, then a
@@ -158,10 +160,7 @@ __device__ __forceinline__ void attract_medium(int k0, int rows, int lane, const
         }
         if (lane == r) sum = make_float2(ax, ay);
     }
-    if (lane < nb) {
-        const float2 g = gravity(p, A.mass[v], A.strong, A.k_g);
-        A.fga[v] = make_float2(g.x + sum.x, g.y + sum.y);
-    }
+    if (lane < nb) A.fga[v] = add_gravity(p, A.mass[v], A.strong, A.k_g, sum.x, sum.y);
 }
 
 // Block i of the light and medium ones, which take turns in proportion (256 threads).

@@ -108,8 +108,7 @@ __global__ __launch_bounds__(256) void k_attract_heavy(const float2* __restrict_
         ax += part[c].x;
         ay += part[c].y;
     }
-    const float2 g = gravity(pos[v], mass[v], strong, k_g);
-    fga[v] = make_float2(g.x + ax, g.y + ay);
+    fga[v] = add_gravity(pos[v], mass[v], strong, k_g, ax, ay);
 }
 
 // A body's swing and traction terms (SpeedKernel, src/RPFA2Kernels.cu:111-161) from its total
@@ -688,7 +687,7 @@ __device__ __forceinline__ void mirror_state(DevState* st, const SegState& q, co
 // One node's new position.
 __device__ __forceinline__ float2 displaced(float2 p, float2 F, float2 P, float gs) {
     const float dx = F.x - P.x, dy = F.y - P.y;
-    const float swg = sqrtf(dx * dx + dy * dy);
+    const float swg = sqrtf(fmaf(dx, dx, dy * dy));
     const float factor = (float)((double)gs / (1.0 + (double)sqrtf(gs * swg)));
     p.x = fmaf(F.x, factor, p.x);
     p.y = fmaf(F.y, factor, p.y);
