@@ -147,7 +147,8 @@ struct Bufs {
     int* blocksum;
     int* S;
     float4* rec;
-    int4* kids;             // per cell record: the record indices of its 1-4 children (-1: none)
+    int4* kids;             // per cell record: the record indices of its 1-4 children (-1: none; of a
+                            // level-32 cell's bodies, which follow it in the records, the first four)
     int* kids_part;         // [kids_blocks][8]: per block of k_tile, then of k_cross, the largest level-4p cell
     int kids_blocks = 1;
     int4* cross = nullptr;  // [tree tiles][kCrossMax]: cells that reach past their tile

@@ -188,7 +188,8 @@ __device__ __forceinline__ int xcd_block() {
 //             body, all lanes at once (lanes = bodies, as in the reference). An accepted record
 //             is appended {x, y, k_r m} to an LDS list; an opened cell pushes all its 1-4
 //             children at once (their record indices, listed per cell when the tree is
-//             built), so a cell's children are tested in the same round. The children go on
+//             built), so a cell's children are tested in the same round (a cell of level 32 holds
+//             any number of bodies: those past the fourth go to the list directly). The children go on
 //             top, so the traversal runs depth-first in blocks of up to 64 records (one record
 //             per round near the stack's capacity, where a depth-first walk adds at most three
 //             entries per tree level).
@@ -302,6 +303,24 @@ __global__ __launch_bounds__(BT) void k_walk(const float4* __restrict__ rec, con
     wave_lds_sync();
     float ax = 0.0f, ay = 0.0f;
     const int half = (G == 32) ? (lane >> 5) : 0;
+    auto drain = [&]() {
+        // pad to whole loop trips with massless entries (their terms are exactly 0)
+        const int padded = (nlist + kPad - 1) / kPad * kPad;
+        if (nlist + lane < padded) lst[nlist + lane] = make_float3(0.0f, 0.0f, 0.0f);
+        wave_lds_sync();
+        for (int q0 = 0; q0 < padded; q0 += kPad) {
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                const float3 e = lst[q0 + u * kStride + half];
+                const float dx = px - e.x, dy = py - e.y;
+                const float w = e.z * __builtin_amdgcn_rcpf(fmaf(dx, dx, fmaf(dy, dy, epssq)));
+                ax = fmaf(dx, w, ax);
+                ay = fmaf(dy, w, ay);
+            }
+        }
+        nlist = 0;
+        wave_lds_sync();
+    };
     while (top > 0) {
         // a round takes up to 64 entries; each may push up to 4 children (net +3), so near the
         // capacity the rounds shrink to depth-first steps, whose growth the slack bounds
@@ -369,6 +388,8 @@ __global__ __launch_bounds__(BT) void k_walk(const float4* __restrict__ rec, con
         const unsigned long long m1 = m0 & __builtin_amdgcn_ballot_w64(kd.y >= 0);
         const unsigned long long m2 = m0 & __builtin_amdgcn_ballot_w64(kd.z >= 0);
         const unsigned long long m3 = m0 & __builtin_amdgcn_ballot_w64(kd.w >= 0);
+        // opened cells of level 32 (info level 31): any number of bodies, of which kids lists four
+        unsigned long long mb = m3 & __builtin_amdgcn_ballot_w64((info & 31u) == 31u);
         const bool accept = (okm >> lane) & 1ull;
         const bool open = live && !body && !accept;
         const int p1 = top + __popcll(m0), p2 = p1 + __popcll(m1), p3 = p2 + __popcll(m2);
@@ -394,23 +415,26 @@ __global__ __launch_bounds__(BT) void k_walk(const float4* __restrict__ rec, con
         top = p3 + __popcll(m3);
         nlist += na;
         naccepted += (unsigned int)na;
-        if (nlist > kWalkList - 64 || top == 0) {
-            // pad to whole loop trips with massless entries (their terms are exactly 0)
-            const int padded = (nlist + kPad - 1) / kPad * kPad;
-            if (nlist + lane < padded) lst[nlist + lane] = make_float3(0.0f, 0.0f, 0.0f);
-            wave_lds_sync();
-            for (int q0 = 0; q0 < padded; q0 += kPad) {
-#pragma unroll
-                for (int u = 0; u < kUnroll; ++u) {
-                    const float3 e = lst[q0 + u * kStride + half];
-                    const float dx = px - e.x, dy = py - e.y;
-                    const float w = e.z * __builtin_amdgcn_rcpf(fmaf(dx, dx, fmaf(dy, dy, epssq)));
-                    ax = fmaf(dx, w, ax);
-                    ay = fmaf(dy, w, ay);
+        if (mb != 0ull) {
+            // the bodies of level-32 cells past the fourth follow it in the records
+            do {
+                const int j = __builtin_ctzll(mb);
+                mb &= mb - 1;
+                const int cell = __builtin_amdgcn_readlane(r, j);
+                const int end = cell + (int)((unsigned int)__builtin_amdgcn_readlane((int)info, j) >> kInfoLevelBits);
+                for (int q = cell + 5; q < end; q += 64) {
+                    if (nlist > kWalkList - 64) drain();
+                    const int more = min(end - q, 64);
+                    if (lane < more) {
+                        const float4 b = rec[q + lane];
+                        lst[nlist + lane] = make_float3(b.x, b.y, k_r * b.z);
+                    }
+                    nlist += more;
+                    naccepted += (unsigned int)more;
                 }
-            }
-            nlist = 0;
+            } while (mb != 0ull);
         }
+        if (nlist > kWalkList - 64 || top == 0) drain();
         wave_lds_sync();
     }
     if constexpr (G == 32) {
