@@ -3,6 +3,7 @@
 #include "mpnn_internal.h"
 #include "../../include/gfa2.h"
 
+#include <algorithm>
 #include <cmath>
 #include <new>
 #include <type_traits>
@@ -41,7 +42,12 @@ struct gfa2_mpnn {
 
 namespace {
 
-int st_of(hipError_t e) { return e == hipSuccess ? GFA2_OK : (e == hipErrorOutOfMemory ? GFA2_ERR_OOM : GFA2_ERR_HIP); }
+int st_of(hipError_t e) {
+    if (e == hipSuccess) return GFA2_OK;
+    if (e != hipErrorOutOfMemory) return GFA2_ERR_HIP;
+    (void)hipGetLastError();            // reported here: not again by the next call
+    return GFA2_ERR_OOM;
+}
 
 #define MP_TRY(expr)                           \
     do {                                       \
@@ -75,27 +81,51 @@ void drop_spare(gfa2_mpnn* m) {
     m->spare = GraphBlock{};
 }
 
-// Scratch sized for n nodes (grows, never shrinks).
+void free_scratch(MpnnScratch& s) {
+    for (float** p : {&s.z0, &s.z1, &s.H1, &s.A1, &s.H2, &s.Y, &s.dY, &s.P, &s.Q, &s.dZ1}) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+    }
+    s.cap = 0;
+}
+
+// Scratch for n nodes, before every use of it (it grows and never shrinks, but is gone after a
+// growth that found no memory, so that the next graph finds all of the memory there is).
 int ensure_scratch(gfa2_mpnn* m, int n) {
     MpnnScratch& s = m->s;
     if (n <= s.cap) return GFA2_OK;
     drop_spare(m);
-    for (void* p : {(void*)s.z0, (void*)s.z1, (void*)s.H1, (void*)s.A1, (void*)s.H2, (void*)s.Y, (void*)s.dY,
-                    (void*)s.P, (void*)s.Q, (void*)s.dZ1})
-        if (p) (void)hipFree(p);
-    const size_t nh = (size_t)n * kHid;
-    MP_TRY(hipMalloc(&s.z0, sizeof(float) * (size_t)n * 8));
-    MP_TRY(hipMalloc(&s.z1, sizeof(float) * (size_t)n * 8));
-    MP_TRY(hipMalloc(&s.H1, sizeof(float) * nh));
-    MP_TRY(hipMalloc(&s.A1, sizeof(float) * nh));
-    MP_TRY(hipMalloc(&s.H2, sizeof(float) * nh));
-    MP_TRY(hipMalloc(&s.Y, sizeof(float) * (size_t)n * 2));
-    MP_TRY(hipMalloc(&s.dY, sizeof(float) * (size_t)n * 2));
-    MP_TRY(hipMalloc(&s.P, sizeof(float) * nh));
-    MP_TRY(hipMalloc(&s.Q, sizeof(float) * nh));
-    MP_TRY(hipMalloc(&s.dZ1, sizeof(float) * nh));
-    s.cap = n;
-    return GFA2_OK;
+    free_scratch(s);
+    hipError_t e = hipSuccess;
+    auto take = [&](float*& p, size_t width) {
+        if (e == hipSuccess) e = hipMalloc(&p, sizeof(float) * (size_t)n * width);
+        if (e != hipSuccess) p = nullptr;
+    };
+    take(s.z0, 8);
+    take(s.z1, 8);
+    take(s.H1, kHid);
+    take(s.A1, kHid);
+    take(s.H2, kHid);
+    take(s.Y, 2);
+    take(s.dY, 2);
+    take(s.P, kHid);
+    take(s.Q, kHid);
+    take(s.dZ1, kHid);
+    if (e == hipSuccess) s.cap = n;
+    else free_scratch(s);
+    return st_of(e);
+}
+
+// Room for the training offsets.
+int ensure_offsets(gfa2_mpnn* m, long long count) {
+    if (count <= m->offs_cap) return GFA2_OK;
+    if (m->offs) (void)hipFree(m->offs);
+    m->offs = nullptr;
+    m->offs_cap = 0;
+    const hipError_t e = hipMalloc(&m->offs, sizeof(int) * (size_t)count);
+    if (e == hipSuccess) m->offs_cap = count;
+    else m->offs = nullptr;
+    return st_of(e);
 }
 
 // The block's work is done. The larger of it and the spare one is kept.
@@ -376,11 +406,7 @@ int gfa2_mpnn_loss_grad(gfa2_mpnn_t m, int32_t graph_id, const int32_t* offsets,
     for (int k = 0; k < R; ++k)
         if (offsets[k] < 1 || offsets[k] >= g.n) return GFA2_ERR_INVALID_ARG;
     MP_TRY(hipSetDevice(m->device));
-    if (R > m->offs_cap) {
-        if (m->offs) (void)hipFree(m->offs);
-        MP_TRY(hipMalloc(&m->offs, sizeof(int) * R));
-        m->offs_cap = R;
-    }
+    if ((st = ensure_scratch(m, g.n)) != GFA2_OK || (st = ensure_offsets(m, R)) != GFA2_OK) return st;
     if (R) MP_TRY(hipMemcpyAsync(m->offs, offsets, sizeof(int) * R, hipMemcpyHostToDevice, m->stream));
     mpnn_forward(g, m->w, m->s, true, m->stream);
     if (mpnn_loss_backward(g, m->w, m->s, m->offs, R, loss, m->stream) != 0) return GFA2_ERR_HIP;
@@ -405,11 +431,10 @@ int gfa2_mpnn_train(gfa2_mpnn_t m, int32_t steps, float lr, int32_t R, uint64_t 
         const int n = m->graphs[ids[s % ids.size()]].n;
         for (int k = 0; k < R; ++k) offs[(size_t)s * R + k] = n > 1 ? 1 + (int)(rng.next() % (uint64_t)(n - 1)) : 1;
     }
-    if ((long long)offs.size() > m->offs_cap) {
-        if (m->offs) (void)hipFree(m->offs);
-        MP_TRY(hipMalloc(&m->offs, sizeof(int) * offs.size()));
-        m->offs_cap = (long long)offs.size();
-    }
+    int most = 0;
+    for (int k : ids) most = std::max(most, m->graphs[k].n);
+    int st = ensure_scratch(m, most);
+    if (st != GFA2_OK || (st = ensure_offsets(m, (long long)offs.size())) != GFA2_OK) return st;
     MP_TRY(hipMemcpyAsync(m->offs, offs.data(), sizeof(int) * offs.size(), hipMemcpyHostToDevice, m->stream));
     for (int s = 0; s < steps; ++s) {
         const MpnnGraph& g = m->graphs[ids[s % ids.size()]];
@@ -440,6 +465,7 @@ int gfa2_mpnn_infer(gfa2_mpnn_t m, int32_t graph_id, float scale, float* xy) {
     if (st != GFA2_OK || !xy) return st != GFA2_OK ? st : GFA2_ERR_INVALID_ARG;
     const MpnnGraph& g = m->graphs[graph_id];
     MP_TRY(hipSetDevice(m->device));
+    if ((st = ensure_scratch(m, g.n)) != GFA2_OK) return st;
     mpnn_forward(g, m->w, m->s, false, m->stream);
     mpnn_place(g, m->s, scale, reinterpret_cast<float2*>(m->s.dY), m->stream);
     MP_TRY(hipMemcpyAsync(xy, m->s.dY, sizeof(float) * 2 * g.n, hipMemcpyDeviceToHost, m->stream));
@@ -455,6 +481,7 @@ int gfa2_mpnn_infer_to_engine(gfa2_mpnn_t m, int32_t graph_id, float scale, gfa2
     const MpnnGraph& g = m->graphs[graph_id];
     if (v.n != g.n || v.device != m->device) return GFA2_ERR_INVALID_ARG;
     MP_TRY(hipSetDevice(m->device));
+    if ((st = ensure_scratch(m, g.n)) != GFA2_OK) return st;
     MP_TRY(hipStreamSynchronize(v.stream));
     mpnn_forward(g, m->w, m->s, false, m->stream);
     mpnn_place(g, m->s, scale, v.pos, m->stream);
@@ -471,10 +498,7 @@ int gfa2_mpnn_destroy(gfa2_mpnn_t m) {
         if (b.p) (void)hipFree(b.p);
     drop_spare(m);
     for (void* p : m->allocs) (void)hipFree(p);
-    MpnnScratch& s = m->s;
-    for (void* p : {(void*)s.z0, (void*)s.z1, (void*)s.H1, (void*)s.A1, (void*)s.H2, (void*)s.Y, (void*)s.dY,
-                    (void*)s.P, (void*)s.Q, (void*)s.dZ1})
-        if (p) (void)hipFree(p);
+    free_scratch(m->s);
     if (m->offs) (void)hipFree(m->offs);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
