@@ -112,8 +112,9 @@ namespace {
 
 int hip_status(hipError_t e) {
     if (e == hipSuccess) return GFA2_OK;
-    if (e == hipErrorOutOfMemory) return GFA2_ERR_OOM;
-    return GFA2_ERR_HIP;
+    if (e != hipErrorOutOfMemory) return GFA2_ERR_HIP;
+    (void)hipGetLastError();            // reported here: not again by the next call
+    return GFA2_ERR_OOM;
 }
 
 #define GFA2_TRY(expr)                       \

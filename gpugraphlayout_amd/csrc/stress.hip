@@ -313,7 +313,11 @@ int stress_hop_distances(const Bufs& b, const int* d_src, int K, const int* d_tg
         m.words = nullptr;
     }
     if (e == hipSuccess) e = hipMalloc(&m.flags, sizeof(int) * std::max(kBfsBatch + 1, kCountBlocks));
-    if (e != hipSuccess) return e == hipErrorOutOfMemory ? -2 : -1;
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();               // reported here: not again by the next call
+        return -2;
+    }
+    if (e != hipSuccess) return -1;
     if (hipMemsetAsync(d_dist, 0, sizeof(int) * (size_t)K * T, s) != hipSuccess) return -1;
     int rc = 0;
     switch (W) {
