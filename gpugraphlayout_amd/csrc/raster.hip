@@ -14,9 +14,9 @@
 // there and writes the tile's counts to a copy of the tile of its own (k_raster_tiles), so that
 // no counter is shared; k_shade adds the copies. A tile gets slices in proportion to the samples
 // a part of the lines put there (k_raster_cost, k_raster_plan): in a finished layout one tile of
-// fifty can hold a sixth of them. gfa2_render_noalloc, which has no memory
-// for a list or copies, adds every sample to one counter per pixel with device atomics
-// (k_raster_nodes, k_raster_edges).
+// fifty can hold a sixth of them. Where the tiles' scratch is out of proportion or not to be had, and
+// in gfa2_render_noalloc, which has no memory for a list or copies, every sample is added to one
+// counter per pixel with device atomics (k_raster_nodes, k_raster_edges).
 #include "engine_internal.h"
 #include "../../include/gfa2.h"
 
@@ -147,6 +147,9 @@ constexpr int kTileThreads = 1024;
 constexpr int kTilePixels = kTileW * kTileH;
 constexpr int kQueueGo = 32;                      // a wave walks its tile's lines once it has found this many
 constexpr int kSpareSlices = 1024;                // slices beyond the first of each tile: four per compute unit
+// Scratch up to which tiles are used whatever the picture's shape; beyond, up to four times what
+// the atomics take (a picture of one column has 128 KB of counters for 128 pixels).
+constexpr size_t kTileMemory = 1ull << 30;
 constexpr long long kListEntries = 4ll << 20;     // CSR entries whose lines are listed at a time (64 MB at most)
 constexpr int kLineThreads = 256, kLineItems = 16;
 // Lines with an end this far out (in pixels) are drawn sample by sample (k_raster_lines): below it
@@ -540,6 +543,19 @@ __global__ __launch_bounds__(kTileW) void k_shade_tiles(const unsigned int* __re
     out[p] = brightness(keep_n, nodes, keep_e, edges);
 }
 
+// The picture by a device atomic per sample: cnt holds 2 npix cleared counters, the nodes' first.
+void count_pixels(const Bufs& b, const Frame& f, unsigned int* cnt, unsigned char* img, const gfa2_raster* r,
+                  hipStream_t s) {
+    const long long npix = (long long)f.w * f.h;
+    k_raster_nodes<<<(b.n + 255) / 256, 256, 0, s>>>(b.pos, b.n, f, cnt);
+    long long eb = (b.nnz + 255) / 256;
+    if (eb > 8192) eb = 8192;
+    if (eb > 0) k_raster_edges<<<(int)eb, 256, 0, s>>>(b.pos, b.rowptr, b.col, b.n, b.nnz, f, cnt + npix);
+    long long pb = (npix + 255) / 256;
+    if (pb > 8192) pb = 8192;
+    k_shade<<<(int)pb, 256, 0, s>>>(cnt, cnt + npix, npix, 1.0f - r->node_alpha, 1.0f - r->edge_alpha, img);
+}
+
 }  // namespace
 }  // namespace gfa2
 
@@ -582,9 +598,8 @@ int gfa2_render(gfa2_handle h, const gfa2_raster* r, uint8_t* gray) {
     if (hipSetDevice(device) != hipSuccess) return GFA2_ERR_HIP;
     const long long npix = (long long)r->width * r->height;
     const Frame f{r->x0, r->y0, r->sx, r->sy, r->width, r->height};
-    const int tiles_x = (f.w + kTileW - 1) / kTileW, tiles_y = (f.h + kTileH - 1) / kTileH;
-    const int tiles = tiles_x * tiles_y;
-    const int copies = 2 * tiles + kSpareSlices;
+    const long long across = ((long long)f.w + kTileW - 1) / kTileW, down = ((long long)f.h + kTileH - 1) / kTileH;
+    const long long copies_ll = 2 * across * down + kSpareSlices;
     const long long lists = std::max<long long>(1, (b->nnz + kListEntries - 1) / kListEntries);
     const size_t list = (size_t)std::min<long long>(b->nnz, kListEntries);
     // the scratch: line list, line count, tile costs, far-out lines' counters, plan, copies, picture
@@ -594,42 +609,60 @@ int gfa2_render(gfa2_handle h, const gfa2_raster* r, uint8_t* gray) {
         size += (bytes + 255) & ~(size_t)255;
         return at;
     };
+    const size_t two_tiles = 2 * (size_t)(across * down);
     const size_t at_lines = place(sizeof(float4) * list), at_count = place(sizeof(unsigned int));
-    const size_t at_cost = place(sizeof(unsigned long long) * 2 * (size_t)tiles);
+    const size_t at_cost = place(sizeof(unsigned long long) * two_tiles);
     const size_t at_far = place(sizeof(unsigned int) * (size_t)npix);
-    const size_t at_first = place(sizeof(int) * (2 * (size_t)tiles + 1));
-    const size_t at_copies = place(sizeof(unsigned int) * kTilePixels * (size_t)copies), at_img = place((size_t)npix);
+    const size_t at_first = place(sizeof(int) * (two_tiles + 1));
+    const size_t at_copies = place(sizeof(unsigned int) * kTilePixels * (size_t)copies_ll), at_img = place((size_t)npix);
+    const size_t plain = 9 * (size_t)npix;
     EngineScratch scratch(h);
-    char* mem = static_cast<char*>(scratch.get(size));
-    if (!mem) return GFA2_ERR_OOM;
-    float4* lines = reinterpret_cast<float4*>(mem + at_lines);
-    unsigned int* nlines = reinterpret_cast<unsigned int*>(mem + at_count);
-    unsigned long long* cost = reinterpret_cast<unsigned long long*>(mem + at_cost);
-    unsigned int* far = reinterpret_cast<unsigned int*>(mem + at_far);
-    int* first = reinterpret_cast<int*>(mem + at_first);
-    unsigned int* copy = reinterpret_cast<unsigned int*>(mem + at_copies);
-    unsigned char* img = reinterpret_cast<unsigned char*>(mem + at_img);
-    hipError_t e = hipMemsetAsync(nlines, 0, at_first - at_count, s);      // count, costs and counters
-    for (long long q = 0; q < lists && e == hipSuccess; ++q) {
-        const long long e0 = q * kListEntries, e1 = std::min<long long>(b->nnz, e0 + kListEntries);
-        if (q > 0) e = hipMemsetAsync(nlines, 0, sizeof(unsigned int), s);
-        constexpr long long kPer = kLineThreads * kLineItems;
-        if (e1 > e0)
-            k_raster_lines<<<(int)((e1 - e0 + kPer - 1) / kPer), kLineThreads, 0, s>>>(b->pos, b->rowptr, b->col, b->n, e0,
-                                                                                     e1, f, lines, nlines, far);
-        if (q == 0) {
-            // the plan of the first list serves the others
-            const long long most = std::max<long long>(b->n, (long long)list) / (256 * kCostStride) + 1;
-            k_raster_cost<<<dim3(2 * tiles, (int)std::min<long long>(most, 8)), 256, 0, s>>>(lines, nlines, b->pos, b->n,
-                                                                                           f, tiles, tiles_x, cost);
-            k_raster_plan<<<1, 1024, 0, s>>>(cost, 2 * tiles, kSpareSlices, first);
+    char* mem = nullptr;
+    if (size <= kTileMemory || size / 4 <= plain) mem = static_cast<char*>(scratch.get(size));
+    unsigned char* img = nullptr;
+    hipError_t e = hipSuccess;
+    if (!mem) {
+        mem = static_cast<char*>(scratch.get(plain));
+        if (!mem) return GFA2_ERR_OOM;
+        unsigned int* cnt = reinterpret_cast<unsigned int*>(mem);
+        img = reinterpret_cast<unsigned char*>(cnt + 2 * npix);
+        e = hipMemsetAsync(cnt, 0, sizeof(unsigned int) * 2 * (size_t)npix, s);
+        if (e == hipSuccess) {
+            count_pixels(*b, f, cnt, img, r, s);
+            e = hipGetLastError();
         }
-        k_raster_tiles<<<copies, kTileThreads, 0, s>>>(lines, nlines, b->pos, b->n, f, tiles, tiles_x, first, copy, q > 0);
-    }
-    if (e == hipSuccess) {
-        k_shade_tiles<<<tiles * kTileH, kTileW, 0, s>>>(copy, first, tiles, tiles_x, far, f, 1.0f - r->node_alpha,
-                                                        1.0f - r->edge_alpha, img);
-        e = hipGetLastError();
+    } else {
+        const int tiles_x = (int)across, tiles = (int)(across * down), copies = (int)copies_ll;
+        float4* lines = reinterpret_cast<float4*>(mem + at_lines);
+        unsigned int* nlines = reinterpret_cast<unsigned int*>(mem + at_count);
+        unsigned long long* cost = reinterpret_cast<unsigned long long*>(mem + at_cost);
+        unsigned int* far = reinterpret_cast<unsigned int*>(mem + at_far);
+        int* first = reinterpret_cast<int*>(mem + at_first);
+        unsigned int* copy = reinterpret_cast<unsigned int*>(mem + at_copies);
+        img = reinterpret_cast<unsigned char*>(mem + at_img);
+        e = hipMemsetAsync(nlines, 0, at_first - at_count, s);      // count, costs and counters
+        for (long long q = 0; q < lists && e == hipSuccess; ++q) {
+            const long long e0 = q * kListEntries, e1 = std::min<long long>(b->nnz, e0 + kListEntries);
+            if (q > 0) e = hipMemsetAsync(nlines, 0, sizeof(unsigned int), s);
+            constexpr long long kPer = kLineThreads * kLineItems;
+            if (e1 > e0)
+                k_raster_lines<<<(int)((e1 - e0 + kPer - 1) / kPer), kLineThreads, 0, s>>>(b->pos, b->rowptr, b->col, b->n,
+                                                                                         e0, e1, f, lines, nlines, far);
+            if (q == 0) {
+                // the plan of the first list serves the others
+                const long long most = std::max<long long>(b->n, (long long)list) / (256 * kCostStride) + 1;
+                k_raster_cost<<<dim3(2 * tiles, (int)std::min<long long>(most, 8)), 256, 0, s>>>(
+                    lines, nlines, b->pos, b->n, f, tiles, tiles_x, cost);
+                k_raster_plan<<<1, 1024, 0, s>>>(cost, 2 * tiles, kSpareSlices, first);
+            }
+            k_raster_tiles<<<copies, kTileThreads, 0, s>>>(lines, nlines, b->pos, b->n, f, tiles, tiles_x, first, copy,
+                                                           q > 0);
+        }
+        if (e == hipSuccess) {
+            k_shade_tiles<<<tiles * kTileH, kTileW, 0, s>>>(copy, first, tiles, tiles_x, far, f, 1.0f - r->node_alpha,
+                                                            1.0f - r->edge_alpha, img);
+            e = hipGetLastError();
+        }
     }
     if (e == hipSuccess) e = hipMemcpyAsync(gray, img, (size_t)npix, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -661,13 +694,7 @@ int gfa2_render_noalloc(gfa2_handle h, const gfa2_raster* r, uint8_t* gray) {
     long long zb = (2 * npix + 255) / 256;
     if (zb > 8192) zb = 8192;
     k_fill_zero<<<(int)zb, 256, 0, s>>>(cnt, 2 * npix);
-    k_raster_nodes<<<(b->n + 255) / 256, 256, 0, s>>>(b->pos, b->n, f, cnt);
-    long long eb = (b->nnz + 255) / 256;
-    if (eb > 8192) eb = 8192;
-    if (eb > 0) k_raster_edges<<<(int)eb, 256, 0, s>>>(b->pos, b->rowptr, b->col, b->n, b->nnz, f, cnt + npix);
-    long long pb = (npix + 255) / 256;
-    if (pb > 8192) pb = 8192;
-    k_shade<<<(int)pb, 256, 0, s>>>(cnt, cnt + npix, npix, 1.0f - r->node_alpha, 1.0f - r->edge_alpha, img);
+    count_pixels(*b, f, cnt, img, r, s);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(gray, img, (size_t)npix, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
