@@ -14,9 +14,10 @@
 // there and writes the tile's counts to a copy of the tile of its own (k_raster_tiles), so that
 // no counter is shared; k_shade adds the copies. A tile gets slices in proportion to the samples
 // a part of the lines put there (k_raster_cost, k_raster_plan): in a finished layout one tile of
-// fifty can hold a sixth of them. Where the tiles' scratch is out of proportion or not to be had, and
-// in gfa2_render_noalloc, which has no memory for a list or copies, every sample is added to one
-// counter per pixel with device atomics (k_raster_nodes, k_raster_edges).
+// fifty can hold a sixth of them. Where tiles do not pay (tiles_pay, kFewSamples) or their scratch
+// is out of proportion or not to be had, and in gfa2_render_noalloc, which has no memory for a list
+// or copies, every sample is added to one counter per pixel with device atomics (k_raster_pixels;
+// k_raster_nodes, k_raster_edges).
 #include "engine_internal.h"
 #include "../../include/gfa2.h"
 
@@ -92,16 +93,18 @@ __global__ __launch_bounds__(64) void k_minmax_final(const float4* __restrict__ 
     if (threadIdx.x == 0) *out = m;
 }
 
-// Discs of radius 3 around the rounded node centre.
-__global__ __launch_bounds__(256) void k_raster_nodes(const float2* __restrict__ pos, int n, Frame f,
-                                                      unsigned int* __restrict__ cnt) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float2 p = pos[i];
+// A disc of radius 3 around the rounded node centre.
+__device__ __forceinline__ void node_hits(float2 p, const Frame& f, unsigned int* __restrict__ cnt) {
     const int cx = (int)lroundf(to_px(p.x, f.x0, f.sx)), cy = (int)lroundf(to_px(p.y, f.y0, f.sy));
     for (int dy = -3; dy <= 3; ++dy)
         for (int dx = -3; dx <= 3; ++dx)
             if (dx * dx + dy * dy <= 9) hit(cnt, f, cx + dx, cy + dy);
+}
+
+__global__ __launch_bounds__(256) void k_raster_nodes(const float2* __restrict__ pos, int n, Frame f,
+                                                      unsigned int* __restrict__ cnt) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) node_hits(pos[i], f, cnt);
 }
 
 // One thread per CSR entry (i, j) with i < j: the line from node i to node j, sampled at
@@ -147,6 +150,17 @@ constexpr int kTileThreads = 1024;
 constexpr int kTilePixels = kTileW * kTileH;
 constexpr int kQueueGo = 32;                      // a wave walks its tile's lines once it has found this many
 constexpr int kSpareSlices = 1024;                // slices beyond the first of each tile: four per compute unit
+constexpr int kSliceSamples = 16384;              // least samples for a slice beyond a tile's first: 15 us, as long
+                                                  // as its block takes to clear and write its copy
+// Small pictures of so few lines that they hold no more samples than this are counted by atomics
+// without a list (the tiles' launches take 40 us and more: mesh of 10,000 nodes at 256 x 128 20 us,
+// by tiles 56; 500 nodes and 1,491 random lines 82 and 70).
+constexpr long long kFewSamples = 6ll << 20;
+constexpr int kFewPixels = 256;
+// Least tests of lines and nodes against tiles (0.2 ms) for which the device may choose atomics after
+// all (tiles_pay); below, that form's launch and the totals it needs are left out (40 us of a picture
+// of 71,000 nodes and 1M lines at 1,250 x 1,250; a mesh of 90,000 nodes there takes 120 us for 90).
+constexpr long long kManyTests = 100'000'000;
 // Scratch up to which tiles are used whatever the picture's shape; beyond, up to four times what
 // the atomics take (a picture of one column has 128 KB of counters for 128 pixels).
 constexpr size_t kTileMemory = 1ull << 30;
@@ -197,21 +211,35 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+__device__ __forceinline__ int line_steps(const float4 l) {
+    return (int)ceilf(fmaxf(fabsf(__fsub_rn(l.z, l.x)), fabsf(__fsub_rn(l.w, l.y))));
+}
+
+// What a list holds.
+struct ListTotals {
+    unsigned long long samples;
+    unsigned int lines, longest;       // the longest in samples
+};
+
 // The lines of CSR entries [e0, e1) with i < j, in no order (counts do not depend on it), as
-// {x0, y0, x1, y1} in pixels; the far-out ones are drawn here, into far.
+// {x0, y0, x1, y1} in pixels; the far-out ones are drawn here, into far. totals: the list's samples
+// are wanted too.
 __global__ __launch_bounds__(kLineThreads) void k_raster_lines(const float2* __restrict__ pos,
                                                                const int* __restrict__ rowptr,
                                                                const int* __restrict__ col, int n, long long e0,
                                                                long long e1, Frame f, float4* __restrict__ lines,
-                                                               unsigned int* __restrict__ nlines,
-                                                               unsigned int* __restrict__ far) {
-    __shared__ unsigned int wsum[kLineThreads / 64];
+                                                               ListTotals* __restrict__ list,
+                                                               unsigned int* __restrict__ far, int totals) {
+    __shared__ unsigned int wsum[kLineThreads / 64], wlong[kLineThreads / 64];
+    __shared__ unsigned long long wsamples[kLineThreads / 64];
     __shared__ unsigned int base;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const long long first = e0 + ((long long)blockIdx.x * kLineThreads + tid) * kLineItems;
     const long long last = first + kLineItems < e1 ? first + kLineItems : e1;
     float4 mine[kLineItems];
     unsigned int take = 0u;                         // bit q: mine[q] is a line
+    unsigned long long samples = 0ull;
+    unsigned int longest = 0u;
     if (first < last) {
         int lo = 0, hi = n;                         // row: rowptr[lo] <= first < rowptr[lo + 1]
         while (hi - lo > 1) {
@@ -242,7 +270,14 @@ __global__ __launch_bounds__(kLineThreads) void k_raster_lines(const float2* __r
         const float4 l = mine[q];
         const float out = fmaxf(fmaxf(fabsf(l.x), fabsf(l.y)), fmaxf(fabsf(l.z), fabsf(l.w)));
         const bool nan = l.x != l.x || l.y != l.y || l.z != l.z || l.w != l.w;
-        if (out < kFarOut && !nan) continue;
+        if (out < kFarOut && !nan) {
+            if (totals) {
+                const unsigned int k = (unsigned int)line_steps(l) + 1u;
+                samples += k;
+                longest = max(longest, k);
+            }
+            continue;
+        }
         take &= ~(1u << q);
         const float ddx = __fsub_rn(l.z, l.x), ddy = __fsub_rn(l.w, l.y);
         const float len = fmaxf(fabsf(ddx), fabsf(ddy));
@@ -265,6 +300,17 @@ __global__ __launch_bounds__(kLineThreads) void k_raster_lines(const float2* __r
             hit(far, f, (int)lroundf(sx), (int)lroundf(sy));
         }
     }
+    if (totals) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            samples += __shfl_xor(samples, o, 64);
+            longest = max(longest, (unsigned int)__shfl_xor((int)longest, o, 64));
+        }
+        if (lane == 0) {
+            wsamples[wave] = samples;
+            wlong[wave] = longest;
+        }
+    }
     // the block's lines get one run of the list
     const unsigned int c = (unsigned int)__popc(take);
     unsigned int inc = c;
@@ -281,7 +327,17 @@ __global__ __launch_bounds__(kLineThreads) void k_raster_lines(const float2* __r
         if (w < wave) before += wsum[w];
         total += wsum[w];
     }
-    if (tid == 0) base = total ? atomicAdd(nlines, total) : 0u;
+    if (tid == 0) {
+        base = 0u;
+        if (total) {
+            base = atomicAdd(&list->lines, total);
+            static_assert(kLineThreads / 64 == 4, "four waves");
+            if (totals) {
+                atomicAdd(&list->samples, wsamples[0] + wsamples[1] + wsamples[2] + wsamples[3]);
+                atomicMax(&list->longest, max(max(wlong[0], wlong[1]), max(wlong[2], wlong[3])));
+            }
+        }
+    }
     __syncthreads();
     unsigned int at = base + before + inc - c;
 #pragma unroll
@@ -311,10 +367,6 @@ __device__ __forceinline__ Tile tile_of(int t, int tiles_x, const Frame& f) {
     return a;
 }
 
-__device__ __forceinline__ int line_steps(const float4 l) {
-    return (int)ceilf(fmaxf(fabsf(__fsub_rn(l.z, l.x)), fabsf(__fsub_rn(l.w, l.y))));
-}
-
 __device__ __forceinline__ bool clip_to_tile(const float4 l, const Tile& a, int* k0, int* k1) {
     return clip_line(l, line_steps(l), (float)a.c0, (float)(a.c0 + a.cw), (float)a.ylo, (float)(a.ylo + a.rh), 2.0f, k0,
                      k1);
@@ -326,19 +378,41 @@ __device__ __forceinline__ bool node_in_tile(float2 p, const Frame& f, const Til
     return *cx >= a.c0 - 3 && *cx <= a.c0 + a.cw + 2 && *cy >= a.ylo - 3 && *cy <= a.ylo + a.rh + 2;
 }
 
+// Whether the lines and nodes are counted in tiles or by a device atomic per sample (k_raster_pixels),
+// from the first list's totals: the least times of both forms, in ns, as fitted to pictures of 64 x 64
+// to 8,000 x 8,000. Tiles pay for long lines (100,000 nodes, 1M lines at 1,250 x 1,250: 1.9 ms, 22.4
+// with atomics); every line is tested against every tile, so atomics do for many lines of a few
+// pixels, where their hits spread over the picture (a mesh of 1M nodes and 2M lines: 0.26 and
+// 0.71 ms at 1,250 x 1,250, 0.57 and 3.1 at 4,000 x 4,000, but 0.75 and 0.40 at 500 x 500, 130 hits a
+// pixel). A wave of atomics takes as long as its longest line, hence lines times the longest.
+__device__ __forceinline__ bool tiles_pay(const ListTotals& l, int n, int tiles, const Frame& f) {
+    const float samples = (float)l.samples, lines = (float)l.lines, nodes = (float)n;
+    if (samples + 29.0f * nodes > 32.0f * (float)f.w * (float)f.h) return true;
+    const float plain = 50e3f + 0.04f * lines * (float)l.longest + 0.15f * nodes;
+    const float tiled = 60e3f + 0.002f * (float)tiles * (lines + nodes) + 0.3f * nodes + 0.004f * samples;
+    return tiled < plain;
+}
+
 // Work of tile t (lines, t < tiles; nodes, t - tiles) in samples, from every kCostStride-th line
 // or node: its samples, 8 per line or node that crosses it, and a quarter per one looked at.
 constexpr int kCostStride = 16;
 
 __global__ __launch_bounds__(256) void k_raster_cost(const float4* __restrict__ lines,
-                                                     const unsigned int* __restrict__ nlines,
+                                                     const ListTotals* __restrict__ list,
                                                      const float2* __restrict__ pos, int n, Frame f, int tiles,
-                                                     int tiles_x, unsigned long long* __restrict__ cost) {
+                                                     int tiles_x, unsigned long long* __restrict__ cost,
+                                                     unsigned int* __restrict__ copies, int either) {
     __shared__ unsigned long long wsum[4];
     const int t = blockIdx.x;
+    if (either && !tiles_pay(*list, n, tiles, f)) {
+        // the nodes' counters of k_raster_pixels
+        const long long npix = (long long)f.w * f.h, step = (long long)gridDim.x * gridDim.y * 256;
+        for (long long p = ((long long)blockIdx.y * gridDim.x + t) * 256 + threadIdx.x; p < npix; p += step) copies[p] = 0u;
+        return;
+    }
     const bool nodes = t >= tiles;
     const Tile a = tile_of(nodes ? t - tiles : t, tiles_x, f);
-    const unsigned int total = nodes ? (unsigned int)n : *nlines;
+    const unsigned int total = nodes ? (unsigned int)n : list->lines;
     unsigned long long c = 0ull;
     for (unsigned int i = (blockIdx.y * 256u + threadIdx.x) * kCostStride; i < total; i += gridDim.y * 256u * kCostStride) {
         int k0, k1;
@@ -354,12 +428,17 @@ __global__ __launch_bounds__(256) void k_raster_cost(const float4* __restrict__ 
 }
 
 // first[t]: the first copy of tile t's slices; every tile gets one slice and a share of the spare
-// ones by its cost. One block.
+// ones by its cost; no copies at all where tiles do not pay. One block.
 __global__ __launch_bounds__(1024) void k_raster_plan(const unsigned long long* __restrict__ cost, int count,
-                                                      int spare, int* __restrict__ first) {
+                                                      int spare, const ListTotals* __restrict__ list, int n, Frame f,
+                                                      int* __restrict__ first, int either) {
     __shared__ unsigned long long wcost[16];
     __shared__ int wsum[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (either && !tiles_pay(*list, n, count / 2, f)) {
+        for (int t = tid; t <= count; t += 1024) first[t] = 0;
+        return;
+    }
     unsigned long long c = 0ull;
     for (int t = tid; t < count; t += 1024) c += cost[t];
 #pragma unroll
@@ -368,6 +447,8 @@ __global__ __launch_bounds__(1024) void k_raster_plan(const unsigned long long* 
     __syncthreads();
     unsigned long long total = 1ull;
     for (int w = 0; w < 16; ++w) total += wcost[w];
+    // (costs are quarters of samples, of every kCostStride-th line)
+    spare = (int)min((unsigned long long)spare, total * (kCostStride / 4) / kSliceSamples);
     int carry = 0;
     for (int t0 = 0; t0 < count; t0 += 1024) {
         const int t = t0 + tid;
@@ -400,7 +481,7 @@ __global__ __launch_bounds__(1024) void k_raster_plan(const unsigned long long* 
 // 1250) took 11.9 ms, 23 samples/ns; with equal slices per tile 1.94 ms, with slices by cost and
 // block-wide batches 1.31 ms, as here 1.02 ms, 270 samples/ns.
 __global__ __launch_bounds__(kTileThreads) void k_raster_tiles(const float4* __restrict__ lines,
-                                                               const unsigned int* __restrict__ nlines,
+                                                               const ListTotals* __restrict__ list,
                                                                const float2* __restrict__ pos, int n, Frame f,
                                                                int tiles, int tiles_x, const int* __restrict__ first,
                                                                unsigned int* __restrict__ copies, int more) {
@@ -431,7 +512,7 @@ __global__ __launch_bounds__(kTileThreads) void k_raster_tiles(const float4* __r
         }
     };
     static_assert(kTileW == 256, "a row of the counters is 257 words");
-    const unsigned int total = nodes ? (unsigned int)n : *nlines;
+    const unsigned int total = nodes ? (unsigned int)n : list->lines;
     const unsigned int i0 = (unsigned int)((unsigned long long)total * slice / slices);
     const unsigned int i1 = (unsigned int)((unsigned long long)total * (slice + 1) / slices);
     // nodes: a wave per disc of radius 3 around the rounded centre
@@ -502,6 +583,37 @@ __global__ __launch_bounds__(kTileThreads) void k_raster_tiles(const float4* __r
     }
 }
 
+// The same without tiles: a device atomic per sample, a thread per line and per node (cn: the
+// nodes' counters, far: the lines').
+__global__ __launch_bounds__(256) void k_raster_pixels(const float4* __restrict__ lines,
+                                                       const ListTotals* __restrict__ list,
+                                                       const float2* __restrict__ pos, int n, Frame f, int tiles,
+                                                       const int* __restrict__ first, unsigned int* __restrict__ cn,
+                                                       unsigned int* __restrict__ far, int more) {
+    if (first[2 * tiles] != 0) return;
+    const unsigned int nodes = more ? 0u : (unsigned int)n, total = list->lines + nodes;
+    for (unsigned int q = blockIdx.x * 256u + threadIdx.x; q < total; q += gridDim.x * 256u) {
+        if (q < nodes) {
+            node_hits(pos[q], f, cn);
+            continue;
+        }
+        const float4 l = lines[q - nodes];
+        const int steps = line_steps(l);
+        if (steps == 0) {
+            hit(far, f, round_px(l.x), round_px(l.y));
+            continue;
+        }
+        const double ddx = (double)__fsub_rn(l.z, l.x), ddy = (double)__fsub_rn(l.w, l.y);
+        const double n_steps = (double)steps, y = __ddiv_rn(1.0, n_steps);
+        for (int k = 0; k <= steps; ++k) {
+            const double t = quotient((double)k, n_steps, y);
+            const float sx = (float)__dadd_rn((double)l.x, __dmul_rn(t, ddx));
+            const float sy = (float)__dadd_rn((double)l.y, __dmul_rn(t, ddy));
+            hit(far, f, round_px(sx), round_px(sy));
+        }
+    }
+}
+
 __device__ __forceinline__ float powi(float b, unsigned int k) {
     float r = 1.0f;
     while (k) {
@@ -525,7 +637,8 @@ __global__ __launch_bounds__(256) void k_shade(const unsigned int* __restrict__ 
         out[p] = brightness(keep_n, cn[p], keep_e, ce[p]);
 }
 
-// The same from the tiles' copies and the far-out lines' counters; a block per row of a tile.
+// The same from the tiles' copies and the far-out lines' counters (from k_raster_pixels' counters,
+// the nodes' in place of the copies, if it counted); a block per row of a tile.
 __global__ __launch_bounds__(kTileW) void k_shade_tiles(const unsigned int* __restrict__ copies,
                                                         const int* __restrict__ first, int tiles, int tiles_x,
                                                         const unsigned int* __restrict__ far, Frame f, float keep_n,
@@ -535,7 +648,7 @@ __global__ __launch_bounds__(kTileW) void k_shade_tiles(const unsigned int* __re
     if (row >= a.rh || (int)threadIdx.x >= a.cw) return;
     const size_t p = (size_t)(a.r0 + row) * f.w + a.c0 + threadIdx.x;
     const unsigned int* c = copies + (size_t)row * kTileW + threadIdx.x;
-    unsigned int edges = far[p], nodes = 0u;
+    unsigned int edges = far[p], nodes = first[2 * tiles] == 0 ? copies[p] : 0u;
     const int e1 = first[t + 1], n1 = first[tiles + t + 1];
 #pragma unroll 8
     for (int k = first[t]; k < e1; ++k) edges += c[(size_t)k * kTilePixels];
@@ -599,10 +712,12 @@ int gfa2_render(gfa2_handle h, const gfa2_raster* r, uint8_t* gray) {
     const long long npix = (long long)r->width * r->height;
     const Frame f{r->x0, r->y0, r->sx, r->sy, r->width, r->height};
     const long long across = ((long long)f.w + kTileW - 1) / kTileW, down = ((long long)f.h + kTileH - 1) / kTileH;
-    const long long copies_ll = 2 * across * down + kSpareSlices;
+    const long long most_samples = (b->nnz / 2) * std::max(f.w, f.h);
+    const int spare = (int)std::min<long long>(kSpareSlices, (most_samples + 29ll * b->n) / kSliceSamples);
+    const long long copies_ll = 2 * across * down + spare;
     const long long lists = std::max<long long>(1, (b->nnz + kListEntries - 1) / kListEntries);
-    const size_t list = (size_t)std::min<long long>(b->nnz, kListEntries);
-    // the scratch: line list, line count, tile costs, far-out lines' counters, plan, copies, picture
+    const size_t list_len = (size_t)std::min<long long>(b->nnz, kListEntries);
+    // the scratch: line list, its totals, tile costs, far-out lines' counters, plan, copies, picture
     size_t size = 0;
     auto place = [&](size_t bytes) {
         const size_t at = size;
@@ -610,15 +725,17 @@ int gfa2_render(gfa2_handle h, const gfa2_raster* r, uint8_t* gray) {
         return at;
     };
     const size_t two_tiles = 2 * (size_t)(across * down);
-    const size_t at_lines = place(sizeof(float4) * list), at_count = place(sizeof(unsigned int));
+    const size_t at_lines = place(sizeof(float4) * list_len), at_list = place(sizeof(ListTotals));
     const size_t at_cost = place(sizeof(unsigned long long) * two_tiles);
     const size_t at_far = place(sizeof(unsigned int) * (size_t)npix);
     const size_t at_first = place(sizeof(int) * (two_tiles + 1));
     const size_t at_copies = place(sizeof(unsigned int) * kTilePixels * (size_t)copies_ll), at_img = place((size_t)npix);
-    const size_t plain = 9 * (size_t)npix;
+    const size_t plain = 9 * (size_t)npix + 1024;
+    const bool few = most_samples <= std::min(kFewSamples, 512 * npix) && std::max(f.w, f.h) <= kFewPixels;
+    const bool either = across * down * (b->nnz / 2 + b->n) > kManyTests;
     EngineScratch scratch(h);
     char* mem = nullptr;
-    if (size <= kTileMemory || size / 4 <= plain) mem = static_cast<char*>(scratch.get(size));
+    if (!few && (size <= kTileMemory || size / 4 <= plain)) mem = static_cast<char*>(scratch.get(size));
     unsigned char* img = nullptr;
     hipError_t e = hipSuccess;
     if (!mem) {
@@ -634,29 +751,33 @@ int gfa2_render(gfa2_handle h, const gfa2_raster* r, uint8_t* gray) {
     } else {
         const int tiles_x = (int)across, tiles = (int)(across * down), copies = (int)copies_ll;
         float4* lines = reinterpret_cast<float4*>(mem + at_lines);
-        unsigned int* nlines = reinterpret_cast<unsigned int*>(mem + at_count);
+        ListTotals* list = reinterpret_cast<ListTotals*>(mem + at_list);
         unsigned long long* cost = reinterpret_cast<unsigned long long*>(mem + at_cost);
         unsigned int* far = reinterpret_cast<unsigned int*>(mem + at_far);
         int* first = reinterpret_cast<int*>(mem + at_first);
         unsigned int* copy = reinterpret_cast<unsigned int*>(mem + at_copies);
         img = reinterpret_cast<unsigned char*>(mem + at_img);
-        e = hipMemsetAsync(nlines, 0, at_first - at_count, s);      // count, costs and counters
+        e = hipMemsetAsync(list, 0, at_first - at_list, s);      // totals, costs and counters
         for (long long q = 0; q < lists && e == hipSuccess; ++q) {
             const long long e0 = q * kListEntries, e1 = std::min<long long>(b->nnz, e0 + kListEntries);
-            if (q > 0) e = hipMemsetAsync(nlines, 0, sizeof(unsigned int), s);
+            if (q > 0) e = hipMemsetAsync(list, 0, sizeof(ListTotals), s);
             constexpr long long kPer = kLineThreads * kLineItems;
             if (e1 > e0)
                 k_raster_lines<<<(int)((e1 - e0 + kPer - 1) / kPer), kLineThreads, 0, s>>>(b->pos, b->rowptr, b->col, b->n,
-                                                                                         e0, e1, f, lines, nlines, far);
+                                                                                         e0, e1, f, lines, list, far,
+                                                                                         either && q == 0);
+            const long long most = std::max<long long>(b->n, (long long)list_len);
             if (q == 0) {
                 // the plan of the first list serves the others
-                const long long most = std::max<long long>(b->n, (long long)list) / (256 * kCostStride) + 1;
-                k_raster_cost<<<dim3(2 * tiles, (int)std::min<long long>(most, 8)), 256, 0, s>>>(
-                    lines, nlines, b->pos, b->n, f, tiles, tiles_x, cost);
-                k_raster_plan<<<1, 1024, 0, s>>>(cost, 2 * tiles, kSpareSlices, first);
+                const int per_tile = (int)std::min<long long>(most / (256 * kCostStride) + 1, 8);
+                k_raster_cost<<<dim3(2 * tiles, per_tile), 256, 0, s>>>(lines, list, b->pos, b->n, f, tiles, tiles_x, cost,
+                                                                        copy, either);
+                k_raster_plan<<<1, 1024, 0, s>>>(cost, 2 * tiles, spare, list, b->n, f, first, either);
             }
-            k_raster_tiles<<<copies, kTileThreads, 0, s>>>(lines, nlines, b->pos, b->n, f, tiles, tiles_x, first, copy,
-                                                           q > 0);
+            k_raster_tiles<<<copies, kTileThreads, 0, s>>>(lines, list, b->pos, b->n, f, tiles, tiles_x, first, copy, q > 0);
+            if (either)
+                k_raster_pixels<<<(int)std::min<long long>(most / 256 + 1, 2048), 256, 0, s>>>(lines, list, b->pos, b->n, f,
+                                                                                           tiles, first, copy, far, q > 0);
         }
         if (e == hipSuccess) {
             k_shade_tiles<<<tiles * kTileH, kTileW, 0, s>>>(copy, first, tiles, tiles_x, far, f, 1.0f - r->node_alpha,

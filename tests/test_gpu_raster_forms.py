@@ -1,5 +1,6 @@
-"""gfa2_render's ways of counting: tiles, or atomics where the tiles' scratch would be out of
-proportion or finds no memory. The picture is bytes: equal to the CPU rasteriser's."""
+"""gfa2_render's ways of counting: tiles, atomics from the list (many lines of a few pixels, also of
+more than one list), atomics without a list (small pictures, pictures whose tiles' scratch would be
+out of proportion or finds no memory). The picture is bytes: equal to the CPU rasteriser's."""
 import ctypes
 
 import numpy as np
@@ -27,6 +28,23 @@ def mesh(side):
                               np.concatenate([i[x < side - 1] + 1, i[side:]]))
     at = np.stack([x, i // side], 1) + np.random.default_rng(side).uniform(-0.3, 0.3, (len(i), 2))
     return hg, hg.arrays(), at.astype(np.float32)
+
+
+@pytest.mark.parametrize("side,w,h", [(200, 600, 500), (300, 4000, 3900), (100, 8000, 7900), (1030, 1250, 1250),
+                                      (1000, 600, 500), (100, 200, 256), (12, 256, 1)])
+def test_short_lines(side, w, h):
+    print(f"case raster forms mesh {side} {w}x{h}", flush=True)
+    hg, g, pos = mesh(side)
+    pos[g.n // 2] = pos[g.n // 2 + 1]           # a line of no length
+    eng = Engine(g.n, g.src, g.dst)
+    eng.set_positions(pos)
+    f = png_frame(eng.bbox(), w, h, g.n, g.m)
+    f.node_alpha, f.edge_alpha = 0.02, 0.1
+    got = eng.render(f)
+    np.testing.assert_array_equal(got, render_gray(hg, pos, f))
+    assert got.min() < got.max()
+    np.testing.assert_array_equal(got, eng.render(f))       # from the workspace that is kept
+    eng.close()
 
 
 @pytest.mark.parametrize("w,h", [(1, 1_200_000), (700_000, 2)])
