@@ -168,6 +168,10 @@ struct SplitMix {
 
 constexpr int kStressBlocks = 512;
 
+// Whether the launch shape says where the attraction runs: not where it is part of a small graph's
+// one launch, nor beside all pairs.
+bool attraction_placed(const gfa2_engine* h) { return !h->p.exact && !small_tree(h->b); }
+
 void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
     hipStream_t s = h->stream;
     Bufs& b = h->b;
@@ -183,7 +187,7 @@ void enqueue_iteration(gfa2_engine* h, hipEvent_t* ev) {
     // (mode 2: joined before the walk).
     // A small graph's tree is one launch that carries the attraction along, in every mode.
     const bool small = !h->p.exact && small_tree(b);
-    const int mode = h->p.exact || small ? 0 : h->tune.attraction_stream;
+    const int mode = attraction_placed(h) ? h->tune.attraction_stream : 0;
     auto attraction_on_side = [&]() {
         hipEventRecord(h->fork, s);
         hipStreamWaitEvent(h->side, h->fork, 0);
@@ -1208,9 +1212,10 @@ int gfa2_autotune(gfa2_handle h, int32_t iters, gfa2_launch_config* best) {
             trial(LaunchConfig{shape.walk_bt, bpc, shape.attraction_stream, shape.attraction_bpc});
     const LaunchConfig shape2 = win;
     const int modes[][2] = {{0, 0}, {1, 0}, {2, 0}, {2, 2}, {2, 3}, {2, 4}};
-    for (const auto& m : modes)
-        if (m[0] != shape2.attraction_stream || m[1] != shape2.attraction_bpc)
-            trial(LaunchConfig{shape2.walk_bt, shape2.blocks_per_cu, m[0], m[1]});
+    if (attraction_placed(h))
+        for (const auto& m : modes)
+            if (m[0] != shape2.attraction_stream || m[1] != shape2.attraction_bpc)
+                trial(LaunchConfig{shape2.walk_bt, shape2.blocks_per_cu, m[0], m[1]});
     // Stage 3: the three fastest shapes again, three rounds each over twice the iterations,
     // interleaved so that a drift of the clock or the layout affects them alike.
     std::stable_sort(timed.begin(), timed.end(),
@@ -1243,7 +1248,14 @@ int gfa2_autotune(gfa2_handle h, int32_t iters, gfa2_launch_config* best) {
     if (h->graph) { (void)hipGraphDestroy(h->graph); h->graph = nullptr; }
     {
         std::lock_guard<std::mutex> lock(g_tune_mu);
-        g_tune_table[size_bucket(b.n)] = win;
+        LaunchConfig& entry = g_tune_table[size_bucket(b.n)];
+        LaunchConfig found = win;
+        if (!attraction_placed(h)) {
+            // what others of these nodes measured, or the default
+            found.attraction_stream = entry.attraction_stream;
+            found.attraction_bpc = entry.attraction_bpc;
+        }
+        entry = found;
     }
     if (best) {
         best->walk_block = win.walk_bt;
