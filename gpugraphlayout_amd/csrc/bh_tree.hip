@@ -223,26 +223,6 @@ __global__ __launch_bounds__(256) void k_keys_attract(const KeysArgs K, int key_
     else attract_block<GEN>(blockIdx.x - key_blocks, w, chunks, part, A, red);
 }
 
-// A graph of a batch starts at sorted position i (always true for i == 0).
-__device__ __forceinline__ bool seg_start(const int* __restrict__ sg, int i) {
-    return i == 0 || (sg != nullptr && sg[i - 1] != sg[i]);
-}
-
-// Levels shared by sorted positions i and i+1; -1 at the end of a graph, except for a
-// graph of one body, whose root (level 0) opens at its only position.
-__device__ __forceinline__ int lcp_at(const unsigned long long* __restrict__ keys, const int* __restrict__ sg, int n,
-                                      int i) {
-    if (i < 0) return -1;
-    const bool end = i >= n - 1 || (sg != nullptr && sg[i] != sg[i + 1]);
-    if (end) return seg_start(sg, i) ? 0 : -1;
-    return lcp_levels(keys[i], keys[i + 1]);
-}
-
-// The level below which cells opened at i are shared with position i-1.
-__device__ __forceinline__ int lcp_prev(const signed char* __restrict__ lcp, const int* __restrict__ sg, int i) {
-    return seg_start(sg, i) ? -1 : (int)lcp[i - 1];
-}
-
 // Block-wide exclusive scan of one int per thread (NT threads). Returns the exclusive
 // prefix; *total gets the block sum.
 template <int NT>
@@ -352,8 +332,10 @@ __global__ __launch_bounds__(kTreeThreads) void k_lcp(const unsigned long long* 
         if (t < kTreeTile) sval[t] = base + t < n ? vals[base + t] : 0u;
     }
     __syncthreads();
-    // seg_start and lcp_at over the staged tile (position i at index i - base + 1); the
-    // position before the tile is only asked for its lcp when no graph starts at the tile
+    // over the staged tile (position i at index i - base + 1): whether a graph starts at position i,
+    // and the levels shared by positions i and i + 1 (-1 at the end of a graph, except for a graph of
+    // one body, whose root, level 0, opens at its only position); the position before the tile is
+    // only asked for its lcp when no graph starts at the tile
     auto seg_start_l = [&](int i) { return i == 0 || (sg != nullptr && ssg[i - base] != ssg[i - base + 1]); };
     auto lcp_at_l = [&](int i) -> int {
         if (i < 0) return -1;
@@ -1241,14 +1223,12 @@ void launch_tree(Bufs& b, hipStream_t s) {
                                          b.seg_root, bm, b.sbody, b.st);
     // up to kFuseTiles tiles, k_tile sums the tile totals itself
     const bool fused = tiles <= kFuseTiles;
-    if (tiles > 8 * kTileChunk) {
+    if (!fused) {
         const int chunks = (tiles + kTileChunk - 1) / kTileChunk;
         Moment* cm = b.int_mass ? b.chunk_mass : nullptr;
         k_scan_up<<<chunks, kTileChunk, 0, s>>>(b.blocksum, bm, tiles, b.chunk_sum, cm);
         k_scan_blocks<<<1, 1024, 0, s>>>(b.chunk_sum, chunks, n, b.cap_records, b.rec_begin + b.nseg, b.st, cm);
         k_scan_down<<<chunks, kTileChunk, 0, s>>>(b.blocksum, bm, tiles, b.chunk_sum, cm);
-    } else if (!fused) {
-        k_scan_blocks<<<1, 1024, 0, s>>>(b.blocksum, tiles, n, b.cap_records, b.rec_begin + b.nseg, b.st, bm);
     }
     const TileArgs T{b.lcp,       sg,      n,       b.blocksum,  bm,        fused ? 1 : 0, b.S,     b.sbody,
                      b.rec,       b.kids,         b.rcount, b.st,

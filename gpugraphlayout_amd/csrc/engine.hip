@@ -542,7 +542,6 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
     h->groups_cap = groups_cap;
     const int sort_tiles = (n + kSortTile - 1) / kSortTile;
     const int tree_tiles = (n + kTreeTile - 1) / kTreeTile;
-    const size_t maxcells = (size_t)(cap - n);
     int st = GFA2_OK;
 #define GFA2_ALLOC(ptr, cnt) \
     if ((st = dalloc(h, &(ptr), (cnt))) != GFA2_OK) { free_all(h); return st; }
@@ -576,29 +575,11 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
     // no tile has published counts, ticket 0
     GFA2_TRY(hipMemsetAsync(b.sort.status, 0, sizeof(unsigned int) * 256 * (size_t)sort_tiles, h->stream));
     GFA2_TRY(hipMemsetAsync(b.sort.ticket, 0, sizeof(unsigned long long), h->stream));
-    GFA2_ALLOC(b.lcp, (size_t)tree_tiles * kTreeTile);      // read by whole tiles
-    GFA2_ALLOC(b.blocksum, tree_tiles);
-    GFA2_ALLOC(b.chunk_sum, (tree_tiles + kTileChunk - 1) / kTileChunk);
-    GFA2_ALLOC(b.S, (size_t)n + 1);
     GFA2_ALLOC(b.rec, (size_t)cap);
     GFA2_ALLOC(b.kids, (size_t)cap);
-    b.kids_blocks = 2 * tree_tiles;
-    GFA2_ALLOC(b.kids_part, (size_t)b.kids_blocks * 8);
-    {
-        // the tables of the crossing cells
-        const size_t slots = ((size_t)tree_tiles * kCrossMax + 1) / 2 * 2, groups = ((size_t)tree_tiles + 15) / 16 * 16;
-        char* tables = nullptr;
-        GFA2_ALLOC(tables, slots * (sizeof(int4) + sizeof(Moment)) + groups * (sizeof(int) + 1));
-        b.cross = reinterpret_cast<int4*>(tables);
-        b.cross_sum = reinterpret_cast<Moment*>(b.cross + slots);
-        b.ncross = reinterpret_cast<int*>(b.cross_sum + slots);
-        b.tmin = reinterpret_cast<signed char*>(b.ncross + groups);
-    }
     GFA2_ALLOC(b.sbody, n);
     GFA2_ALLOC(b.pm, n);
     GFA2_ALLOC(b.rcount, (size_t)cap);
-    GFA2_ALLOC(b.cell_lvl, maxcells);
-    GFA2_ALLOC(b.spill, 66 * ((size_t)cap / 4096 + 8));   // (33 slots per block, fewer in all for the groups)
     GFA2_ALLOC(b.bbox_part, kPartBlocks);
     GFA2_ALLOC(b.st, 1);
     // a sort wait that runs out raises the instance's error word, so every later kernel of the
@@ -650,18 +631,40 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
         b.int_mass = whole && total < 16777216.0 * 62.0;
         // no cell (a part of one graph) can reach 2^24
         b.no_big = total < 16777216.0;
-        if (small_tree(b)) {
-            b.kids_blocks = 1;
-            b.sort.hist_in_keys = false;
+    }
+    if (small_tree(b)) {
+        b.kids_blocks = 1;
+        b.sort.hist_in_keys = false;
+        if (b.int_mass) {
+            GFA2_ALLOC(b.pmass, (size_t)n + 1);
+        } else {
+            GFA2_ALLOC(b.cell_lvl, (size_t)(cap - n));
+        }
+    } else {
+        b.kids_blocks = 2 * tree_tiles;
+        GFA2_ALLOC(b.lcp, (size_t)tree_tiles * kTreeTile);      // read by whole tiles
+        GFA2_ALLOC(b.blocksum, tree_tiles);
+        GFA2_ALLOC(b.chunk_sum, (tree_tiles + kTileChunk - 1) / kTileChunk);
+        GFA2_ALLOC(b.S, (size_t)n + 1);
+        // the tables of the crossing cells
+        const size_t slots = ((size_t)tree_tiles * kCrossMax + 1) / 2 * 2, groups = ((size_t)tree_tiles + 15) / 16 * 16;
+        char* tables = nullptr;
+        GFA2_ALLOC(tables, slots * (sizeof(int4) + sizeof(Moment)) + groups * (sizeof(int) + 1));
+        b.cross = reinterpret_cast<int4*>(tables);
+        b.cross_sum = reinterpret_cast<Moment*>(b.cross + slots);
+        b.ncross = reinterpret_cast<int*>(b.cross_sum + slots);
+        b.tmin = reinterpret_cast<signed char*>(b.ncross + groups);
+        if (b.int_mass) {
+            GFA2_ALLOC(b.pmass, (size_t)n / 16 + 1);
+            GFA2_ALLOC(b.bmass, tree_tiles);
+            GFA2_ALLOC(b.chunk_mass, (tree_tiles + kTileChunk - 1) / kTileChunk);
+            GFA2_ALLOC(b.big_rc, kMaxBig);
+            GFA2_ALLOC(b.big_lvl, kMaxBig);
+        } else {
+            GFA2_ALLOC(b.spill, 66 * ((size_t)cap / 4096 + 8));   // (33 slots per block, fewer in all for the groups)
         }
     }
-    if (b.int_mass) {
-        GFA2_ALLOC(b.pmass, n <= kSmallTree ? (size_t)n + 1 : (size_t)n / 16 + 1);
-        GFA2_ALLOC(b.bmass, tree_tiles);
-        GFA2_ALLOC(b.chunk_mass, (tree_tiles + kTileChunk - 1) / kTileChunk);
-        GFA2_ALLOC(b.big_rc, kMaxBig);
-        GFA2_ALLOC(b.big_lvl, kMaxBig);
-    }
+    GFA2_ALLOC(b.kids_part, (size_t)b.kids_blocks * 8);
 #undef GFA2_ALLOC
     b.cus = h->cus;
     b.nlight = nlight;

@@ -163,8 +163,6 @@ struct Bufs {
     unsigned char* cell_lvl;
     int* spill;
     float4* bbox_part;
-    WalkPart* walk_part;
-    int nwalk_part;
     DevState* st;
     // Batched layout of many graphs (nseg > 1). Graph g owns nodes [node_off[g],
     // node_off[g+1]) of the concatenated input and, after the sort, the same range of sorted
