@@ -687,13 +687,12 @@ int set_graph_impl(gfa2_engine* h, int32_t n, const int64_t* rowptr, const int32
         std::vector<int> start((size_t)maxdeg + 2, 0);
         for (int v = 0; v < n; ++v) ++start[(size_t)(maxdeg - (rp32[v + 1] - rp32[v])) + 1];
         for (int d = 0; d <= maxdeg; ++d) start[(size_t)d + 1] += start[(size_t)d];
+        long long hub_entries = 0;
+        for (int d = 0; d <= maxdeg && start[(size_t)d] < kWideHubs; ++d)
+            hub_entries += (long long)(maxdeg - d) * (std::min(start[(size_t)d + 1], kWideHubs) - start[(size_t)d]);
+        b.hub_entries = hub_entries;
         std::vector<int> rank((size_t)n);
-        b.hub_entries = 0;
-        for (int v = 0; v < n; ++v) {
-            const int deg = rp32[v + 1] - rp32[v];
-            rank[v] = start[(size_t)(maxdeg - deg)]++;
-            if (rank[v] < kWideHubs) b.hub_entries += deg;
-        }
+        for (int v = 0; v < n; ++v) rank[v] = start[(size_t)(maxdeg - (rp32[v + 1] - rp32[v]))]++;
         GFA2_TRY(hipMemcpyAsync(b.rank, rank.data(), sizeof(int) * n, hipMemcpyHostToDevice, h->stream));
         launch_col_rank(b, h->stream);
         GFA2_TRY(hipStreamSynchronize(h->stream));   // rank goes out of scope
