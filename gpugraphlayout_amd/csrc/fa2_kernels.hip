@@ -16,7 +16,7 @@ namespace {
 // order and without atomics. Nodes are pre-sorted into degree classes:
 //   light (deg <= 32): one thread per node, sequential sum
 //   medium (deg <= 2048): one wave per node, lane-strided sums + butterfly reduction
-//   heavy: one 256-thread block per node, thread-strided sums + LDS tree reduction
+//   heavy: a 256-thread block per 4,096 entries, thread-strided sums + LDS tree reduction
 // ---------------------------------------------------------------------------------------
 // col_rank[e] = rank[col[e]] (once per graph).
 __global__ __launch_bounds__(256) void k_gather_rank(const int* __restrict__ col, const int* __restrict__ rank,
@@ -664,7 +664,8 @@ __device__ __forceinline__ SegState speed_update(SegState q, const GroupSums& r,
     return q;
 }
 
-// The tree's largest cell at level 4, 8, ..., 32, from the child-list kernel's blocks, into rm
+// The tree's largest cell at level 4, 8, ..., 32, from the blocks of k_tile and k_cross (the small
+// tree: its one block), into rm
 // (8 words of LDS; followed by a barrier).
 template <int NT>
 __device__ __forceinline__ void max_runs(const int* __restrict__ kids_part, int kids_blocks, int* rm) {

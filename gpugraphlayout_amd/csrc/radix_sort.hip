@@ -718,7 +718,7 @@ __device__ void heapsort_pairs(unsigned long long* __restrict__ k, unsigned int*
 // A block takes the runs that start in its kFixTile positions and looks kFixHalo positions past
 // them; each pair's place in its run is the number of the run's pairs before it, counted in LDS.
 // A run past the window (over kFixHalo pairs) is left to the thread at its first position, which
-// sorts it in place (insertion sort up to 32 pairs, heapsort beyond). Where the result replaces
+// heapsorts it in place. Where the result replaces
 // its input, a neighbouring block may read positions while their run's own block reorders them;
 // it uses only their top bits, which all pairs of a run share.
 //

@@ -212,6 +212,8 @@ int gfa2_exact_repulsion(gfa2_handle h, int32_t fp64, double* xy);
  * fills it from gfa2_get_bbox as its CPU writer does. Nodes are discs of radius 3, edges lines
  * from the smaller to the larger node id; a pixel hit by k nodes and l edges gets brightness
  * round(255 (1 - node_alpha)^k (1 - edge_alpha)^l). gray: width*height bytes, top row first.
+ * Device memory of a call: 9 bytes a pixel, or where tiles pay about 13 with up to 200 MB beside
+ * them; up to 256 MB of it stay with the handle until its next graph.
  * Single-graph handles only (GFA2_ERR_UNSUPPORTED for a batch). */
 typedef struct gfa2_raster {
     float x0, y0;
