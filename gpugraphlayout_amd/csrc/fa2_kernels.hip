@@ -284,6 +284,7 @@ __global__ __launch_bounds__(BT) void k_walk(const float4* __restrict__ rec, con
     const int upper4 = (lane >> 5) << 2;    // 4 in the upper half-wave, else 0 (j2 >= j)
     const float two_r = seg_root[g].z * 2;
     const float base = two_r * two_r * itolsq;
+    const bool deep = st->max_level >= kKeyLevels;     // the tree has a level-32 cell
     // the root's children start the walk (a graph of one body has no cell records)
     const int root = rec_begin[g];
     const bool has_root = root + 1 < rec_begin[g + 1];
@@ -388,8 +389,6 @@ __global__ __launch_bounds__(BT) void k_walk(const float4* __restrict__ rec, con
         const unsigned long long m1 = m0 & __builtin_amdgcn_ballot_w64(kd.y >= 0);
         const unsigned long long m2 = m0 & __builtin_amdgcn_ballot_w64(kd.z >= 0);
         const unsigned long long m3 = m0 & __builtin_amdgcn_ballot_w64(kd.w >= 0);
-        // opened cells of level 32 (info level 31): any number of bodies, of which kids lists four
-        unsigned long long mb = m3 & __builtin_amdgcn_ballot_w64((info & 31u) == 31u);
         const bool accept = (okm >> lane) & 1ull;
         const bool open = live && !body && !accept;
         const int p1 = top + __popcll(m0), p2 = p1 + __popcll(m1), p3 = p2 + __popcll(m2);
@@ -415,9 +414,11 @@ __global__ __launch_bounds__(BT) void k_walk(const float4* __restrict__ rec, con
         top = p3 + __popcll(m3);
         nlist += na;
         naccepted += (unsigned int)na;
-        if (mb != 0ull) {
-            // the bodies of level-32 cells past the fourth follow it in the records
-            do {
+        if (deep) {
+            // opened cells of level 32 (info level 31) have any number of bodies: those past the fourth
+            // follow it in the records
+            unsigned long long mb = m3 & __builtin_amdgcn_ballot_w64((info & 31u) == 31u);
+            while (mb != 0ull) {
                 const int j = __builtin_ctzll(mb);
                 mb &= mb - 1;
                 const int cell = __builtin_amdgcn_readlane(r, j);
@@ -432,7 +433,7 @@ __global__ __launch_bounds__(BT) void k_walk(const float4* __restrict__ rec, con
                     nlist += more;
                     naccepted += (unsigned int)more;
                 }
-            } while (mb != 0ull);
+            }
         }
         if (nlist > kWalkList - 64 || top == 0) drain();
         wave_lds_sync();
