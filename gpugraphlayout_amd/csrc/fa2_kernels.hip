@@ -1083,9 +1083,9 @@ AttractArgs attract_args(const Bufs& b, const Params& p) {
 }
 
 // The wide blocks stay until all rows are done, which pays where their staging and their uneven
-// ends are small beside the work and hubs hold many entries (R-MAT: 8M entries 252 us an
-// iteration without, 265 with; 20M 402, 397; 64M 1,253, 1,213; BA with 1M bodies, 20M entries,
-// 9% of them of hubs: 667, 753), and nothing is to run beside them.
+// ends are small beside the work and hubs hold many entries (R-MAT on one stream: 8M entries 252 us
+// an iteration without, 265 with; 17M 292 either way; 20M 398, 400; 64M 1,245, 1,207; BA with 1M
+// bodies, 20M entries, 9% of them of hubs: 667, 753), and nothing is to run beside them.
 bool attract_wide(const Bufs& b) {
     return b.attr_grid == 0 && b.nnz >= kWideEntries && b.hub_entries >= b.nnz / 4;
 }
